@@ -63,8 +63,7 @@ __global__ __launch_bounds__(kThreads) void k_potrf_blk(TS* __restrict__ L, cons
   extern __shared__ __align__(16) unsigned char smem_raw[];
   T* S = reinterpret_cast<T*>(smem_raw);
   T* dinv = S + NP * P;  // 1/L[r][r] for every row
-  T* col = dinv + NP;
-  T* ut = col + 128;  // 32 x 33: the last factored tile's inverse, transposed in full
+  T* ut = dinv + NP;  // 32 x 33: the last factored tile's inverse, transposed in full
   const int tid = threadIdx.x, wave = wave_id(), l = lane_id();
 
   const int nn = n * n;
@@ -199,7 +198,7 @@ __global__ __launch_bounds__(kThreads) void k_potrf_blk(TS* __restrict__ L, cons
     T* D = S + 32 * kb * P + 32 * kb;
     if (wave == 0) {
       if (kb > 0) trail(kb - 1, kb, kb);
-      tile_chol_inv<T>(D, P, dinv + 32 * kb, col, ut);
+      tile_chol_inv<T>(D, P, dinv + 32 * kb, ut);
     } else {
       for (int j = wave - 1; j < NB - 1; j += WS) {
         if (j < kb - 1) inv_finish(kb - 1, j);
@@ -302,7 +301,7 @@ __global__ __launch_bounds__(kThreads) void k_potrf_blk(TS* __restrict__ L, cons
 // its targets are then k_schur_small's, so that a factor_and_solve needs no
 // separate forward-sweep kernels.
 // ---------------------------------------------------------------------------
-constexpr size_t node32_lds(size_t esize) { return esize * (2 * 32 * 33 + 32 + 128); }
+constexpr size_t node32_lds(size_t esize) { return esize * (2 * 32 * 33 + 32); }
 
 // (two wavefronts per SIMD: the register budget is held to 256, which the
 // compiler meets without spills by keeping the MFMA accumulators in VGPRs)
@@ -326,7 +325,6 @@ __global__ __launch_bounds__(64, 2) void k_node32(T* __restrict__ L, T* __restri
   T* S = reinterpret_cast<T*>(smem_raw);  // 32 x 33: the block, then R_i, Lc_i, R_i'
   T* ut = S + 32 * P;                       // 32 x 33: Linv transposed, then Lc_i'
   T* dinv = ut + 32 * P;
-  T* col = dinv + 32;
   const int l = lane_id();
   const int lr = l >> 5, lc = l & 31;  // lane l moves row 2q + lr, column lc of a block
 
@@ -368,7 +366,7 @@ __global__ __launch_bounds__(64, 2) void k_node32(T* __restrict__ L, T* __restri
       }
     }
   };
-  tile_chol_inv<T>(S, P, dinv, col, ut, hook);
+  tile_chol_inv<T>(S, P, dinv, ut, hook);
   // the factor (lower) with the transposed inverse (strict upper)
 #pragma unroll
   for (int q = 0; q < 16; ++q) A[(2 * q + lr) * n + lc] = S[(2 * q + lr) * P + lc];
@@ -1709,7 +1707,7 @@ constexpr size_t apply_fwd_lds(int m) {
 
 template <typename T, int NB>
 constexpr size_t potrf_blk_lds() {
-  return sizeof(T) * ((size_t)(32 * NB) * (32 * NB + 1) + 32 * NB + 128 + 32 * 33);
+  return sizeof(T) * ((size_t)(32 * NB) * (32 * NB + 1) + 32 * NB + 32 * 33);
 }
 template <typename T, int NB>
 constexpr size_t trsm_blk_lds() {

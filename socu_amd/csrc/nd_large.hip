@@ -37,10 +37,6 @@ constexpr int kLP = 33;                       // pitch of an LDS tile
 constexpr int kTileElems = 32 * kLP;
 constexpr int kLargeTiles = kMaxNLarge / 32;  // tiles per block dimension, at most
 
-// LDS operations of one wavefront complete in issue order; this keeps the
-// compiler from moving LDS accesses of the wave across the point.
-__device__ __forceinline__ void wave_lds_order() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
-
 // Tile (r0, c0) of a rows x cols row-major matrix M (leading dimension ld)
 // into the wave's LDS tile Tl: entries outside the matrix read 0, or 1 on
 // the matrix diagonal when pad_diag (identity padding of a diagonal block).
@@ -212,8 +208,8 @@ __device__ __forceinline__ void inverse_bands(T* __restrict__ A, int n, int NB, 
 
 template <typename T>
 constexpr size_t potrf_large_lds() {
-  // diagonal tile, ut, 128 column entries, dinv, two tiles per wavefront
-  return sizeof(T) * (2 * kTileElems + 128 + kMaxNLarge + 8 * kTileElems);
+  // diagonal tile, ut, dinv, two tiles per wavefront
+  return sizeof(T) * (2 * kTileElems + kMaxNLarge + 8 * kTileElems);
 }
 
 // One workgroup of four wavefronts per node of the level (grid (dim, B)).
@@ -228,15 +224,14 @@ __global__ __launch_bounds__(kThreads) void k_potrf_large(T* __restrict__ L, con
   extern __shared__ __align__(16) unsigned char smem_raw[];
   T* D = reinterpret_cast<T*>(smem_raw);
   T* ut = D + kTileElems;
-  T* col = ut + kTileElems;
-  T* dinv = col + 128;
+  T* dinv = ut + kTileElems;
   const int wave = wave_id();
   T* X0 = dinv + kMaxNLarge + 2 * wave * kTileElems;
   T* X1 = X0 + kTileElems;
   for (int kb = 0; kb < NB; ++kb) {
     if (wave == 0) {
       wtile_load(D, A, n, n, n, 32 * kb, 32 * kb, true);
-      tile_chol_inv<T>(D, kLP, dinv + 32 * kb, col, ut);
+      tile_chol_inv<T>(D, kLP, dinv + 32 * kb, ut);
       wave_lds_order();
       wtile_store_diag(D, A, n, 32 * kb);  // L below, Linv^T above the diagonal
     }

@@ -8,12 +8,13 @@
 // * wave_gemm: a 32x32 (2x2 MFMA tiles) accumulation C += A B with A, B
 //   read from LDS through element strides.
 // * tile_chol_inv: Cholesky and inverse of a 32x32 diagonal tile by one
-//   wavefront, row r in lane r's registers, column broadcasts through LDS.
+//   wavefront, as two 16-column panels (nd_panel.h).
 #pragma once
 
 #include <hip/hip_runtime.h>
 
 #include "nd_common.h"
+#include "nd_panel.h"
 
 namespace socu {
 
@@ -49,6 +50,10 @@ __device__ __forceinline__ typename Mfma<T>::acc_t acc_zero() {
   z[0] = z[1] = z[2] = z[3] = T(0);
   return z;
 }
+
+// LDS operations of one wavefront complete in issue order; this keeps the
+// compiler from moving LDS accesses of the wave across the point.
+__device__ __forceinline__ void wave_lds_order() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
 __device__ __forceinline__ int lane_id() { return threadIdx.x & 63; }
 __device__ __forceinline__ int wave_id() { return threadIdx.x >> 6; }
@@ -207,207 +212,95 @@ __device__ __forceinline__ void acc16_foreach(typename Mfma<T>::acc_t& acc, F f)
 // S: tile in LDS, row-major with `pitch`; its lower triangle is the input.
 // On return the lower triangle holds L, the strict upper triangle holds the
 // transposed inverse (S[c][q] = Linv[q][c] for q > c) and dinv[r] = 1/L[r][r].
-// col: 128 entries of wave-private LDS (two buffers of two columns; its
-// first 64 entries are overwritten at the end).
 // ut: a 32 x 33 LDS tile that receives Linv transposed in full (ut[r][c] =
 // Linv[c][r], zeros and diagonal included).
 //
-// Lanes 0-31 keep row r of the tile in u[]; lanes 32-63 keep column r of the
-// inverse (Gauss-Jordan: Linv = L_31^-1 ... L_0^-1).  The pivots are taken two
-// at a time: for the 2x2 pivot block [a b; b c] (from lanes k, k+1 by
-// readlane), 1/sqrt(a) and 1/sqrt(ac - b^2) are computed side by side and
-// 1/sqrt(c - b^2/a) = sqrt(a) / sqrt(ac - b^2) follows with two products, so
-// the serial chain per two columns is one reciprocal square root.  Steps k
-// and k+1 then fuse into one rank-2 update per entry,
-//   u[q] -= (c1 - c2 t) A[q][k] + c2 A[q][k+1],   t = b / a,
-// with each half's coefficients c1 (step k) and c2 (step k+1, from the entry
-// k+1 updated by step k).  Columns k, k+1 come from the LDS buffer (k/2) % 2
-// (LDS operations of one wavefront complete in issue order, so no barrier is
-// needed).  Look-ahead: entries k+2, k+3 are updated first and published as
-// the next pair's columns.  FP32 (EARLY): the next pair's column reads are
-// issued right after (a scheduling barrier keeps them there), so that their
-// LDS latency runs under this pair's remaining updates instead of the next
-// pivot chain; FP64 reads them at the start of the pair step (two sets of FP64
-// columns in registers spill).
-// The coefficients are not masked for row lanes at or above the pair: those
-// lanes only change entries of their strict upper triangle, which nothing
-// reads (not the column buffers, the pivots, nor the store), and their own
-// pivot entries are replaced explicitly.
-// hook(k) runs at the start of pair step k (k even, a compile-time constant
-// after unrolling): a caller can issue loads there, late in the chain, when
-// the column registers of the early steps are free.
+// Two 16-column panels (panel16) with one MFMA update between them.  Payload
+// rows of the first panel: the identity, giving U_11 = L_11^-T, and A_21,
+// giving L_21; of the second: U_12 = -U_11 L_21^T and the identity.  Each DPP
+// row g (16 lanes) loads its payload rows from where it stores them, except
+// that g = 2 repeats the identity rows to store L with U above its diagonal
+// in S, and g = 3 repeats U_12 to store it in ut.
+// hook(k) runs before pivot step k (a compile-time constant after unrolling):
+// a caller can issue loads there.
 struct NoHook {
   __device__ __forceinline__ void operator()(int) const {}
 };
 template <typename T, typename Hook = NoHook>
-__device__ __forceinline__ void tile_chol_inv(T* S, int pitch, T* dinv, T* col, T* ut, Hook hook = Hook()) {
+__device__ __forceinline__ void tile_chol_inv(T* S, int pitch, T* dinv, T* ut, Hook hook = Hook()) {
   const int lane = lane_id();
-  const int r = lane & 31;
-  const bool rowlane = lane < 32;
-  T u[32];
+  const int r = lane & 15, g = lane >> 4;
+  // rows of the diagonal tiles whose L the lane stores beside U (none: -1)
+  const int rl = g == 2 ? r : -1;
+  T u[16], p[1][16];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {  // the identity tiles and the zero tile of ut
+    const T e = (4 * c + g == r) ? T(1) : T(0);
+    ut[(4 * c + g) * 33 + r] = e;
+    ut[(16 + 4 * c + g) * 33 + 16 + r] = e;
+    ut[(16 + 4 * c + g) * 33 + r] = T(0);
+  }
+  typename Mfma<T>::acc_t s22;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) s22[c] = S[(16 + Mfma<T>::row(lane, c)) * pitch + 16 + r];
+  wave_lds_order();
   {
-    // Row lanes take row r as it is, strict upper entries included: those
-    // entries only ever meet the multipliers of their own lane (see below)
-    // and are not stored.  The reads are unconditional (in bounds) and
-    // pinned, so that they are all in flight at once; inverse lanes then
-    // replace theirs by the unit vector e_r.  (Selects on the reads let the
-    // compiler turn every read into a branch with a wait of its own.)
+    const T* urow = S + r * pitch;
+    T* prow = (g & 1) ? S + (16 + r) * pitch : ut + r * 33;
 #pragma unroll
-    for (int c = 0; c < 32; ++c) u[c] = S[r * pitch + c];
+    for (int c = 0; c < 16; ++c) u[c] = urow[c];
 #pragma unroll
-    for (int c = 0; c < 32; ++c) asm volatile("" : "+v"(u[c]));
-    if (!rowlane) {
+    for (int c = 0; c < 16; ++c) p[0][c] = prow[c];
 #pragma unroll
-      for (int c = 0; c < 32; ++c) u[c] = (c == r) ? T(1) : T(0);
+    for (int c = 0; c < 16; ++c) {
+      pin_reg(u[c]);
+      pin_reg(p[0][c]);
     }
+    panel16<T, 1>(u, p, hook);
+    if (g == 2) prow = S + r * pitch;
+#pragma unroll
+    for (int c = 0; c < 16; ++c) prow[c] = (c <= rl) ? u[c] : p[0][c];
   }
-  // one base address in a vector register: every column access below is
-  // that base plus an immediate offset
-  typedef __attribute__((address_space(3))) T lds_t;
-  lds_t* colv = (lds_t*)col;
-  asm volatile("" : "+v"(colv));
-  if (rowlane) {
-    colv[r] = u[0];
-    colv[32 + r] = u[1];
-  }
-  // Publishing a pair's columns: row lanes write buffer p, inverse lanes the
-  // other buffer, whose columns are already in registers (so no branch on
-  // the lane kind): pubv[p] is each lane's target for buffer p.
-  lds_t* pubv0 = colv + (rowlane ? 0 : 64);
-  lds_t* pubv1 = colv + (rowlane ? 64 : 0);
-  asm volatile("" : "+v"(pubv0), "+v"(pubv1));
-  // Row index for the pivot selects below; inverse lanes take one past every
-  // pivot, so that the selects give them the multipliers (no branch).
-  const int rsel = rowlane ? r : 64;
-  constexpr bool EARLY = sizeof(T) == 4;
-  // FP32 column reads are 16-byte vector reads of four entries from an
-  // aligned start (col is 16-byte aligned; entries below the first one
-  // needed are dropped): half the LDS instructions of paired 4-byte reads.
-  typedef T t4 __attribute__((ext_vector_type(4)));
-  typedef __attribute__((address_space(3))) t4 lds_t4;
-  T c0[32], c1[32];
-  if constexpr (EARLY) {
-#pragma unroll
-    for (int q0 = 0; q0 < 32; q0 += 4) {
-      const t4 v0 = *(const lds_t4*)(colv + q0);
-      const t4 v1 = *(const lds_t4*)(colv + 32 + q0);
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (q0 + j >= 2) {
-          c0[q0 + j] = v0[j];
-          c1[q0 + j] = v1[j];
-        }
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < 32; k += 2) {
-    lds_t* nb = colv + 64 * (((k >> 1) + 1) & 1);
-    lds_t* pb = (((k >> 1) + 1) & 1) ? pubv1 : pubv0;
-    if constexpr (!EARLY) {
-      const lds_t* cb = colv + 64 * ((k >> 1) & 1);
-#pragma unroll
-      for (int q = k + 2; q < 32; ++q) {
-        c0[q] = cb[q];
-        c1[q] = cb[32 + q];
-      }
-    }
-    hook(k);
-    const T a = bcast_lane(u[k], k);
-    const T b = bcast_lane(u[k], k + 1);
-    const T c = bcast_lane(u[k + 1], k + 1);
-    const T inv1 = rsqrt_t(a);
-    const T g = rsqrt_t(a * c - b * b);
-    const T inv2 = g * (a * inv1);  // 1 / sqrt(c - b^2 / a)
-    const T t = b * inv1 * inv1;
-    // step k: row lanes l = L[r][k]; inverse lanes z_k
-    const T lk1 = u[k] * inv1;
-    const T cf1 = lk1 * inv1;
-    // step k+1, on entry k+1 as updated by step k (A[k+1][k] = b)
-    const T uk1 = u[k + 1] - cf1 * b;
-    const T lk2 = uk1 * inv2;
-    const T cf2 = lk2 * inv2;
-    const T cf1p = cf1 - cf2 * t;
-    // (explicit fused multiply-adds: two per entry and pair of steps)
-    T ncf1 = -cf1p, ncf2 = -cf2;
-    T n0[32], n1[32];
-    if (k + 2 < 32) {
-      u[k + 2] = fma(ncf2, c1[k + 2], fma(ncf1, c0[k + 2], u[k + 2]));
-      u[k + 3] = fma(ncf2, c1[k + 3], fma(ncf1, c0[k + 3], u[k + 3]));
-      asm volatile("" : "+v"(u[k + 2]), "+v"(u[k + 3]));
-      pb[r] = u[k + 2];
-      pb[32 + r] = u[k + 3];
-      // the remaining updates use the coefficients as pinned here, after the
-      // stores
-      asm volatile("" : "+v"(ncf1), "+v"(ncf2) : : "memory");
-      if constexpr (EARLY) {
-#pragma unroll
-        for (int q0 = (k + 4) & ~3; q0 < 32; q0 += 4) {
-          const t4 v0 = *(const lds_t4*)(nb + q0);
-          const t4 v1 = *(const lds_t4*)(nb + 32 + q0);
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            if (q0 + j >= k + 4) {
-              n0[q0 + j] = v0[j];
-              n1[q0 + j] = v1[j];
-            }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-#pragma unroll
-    for (int q = k + 4; q < 32; ++q) u[q] = fma(ncf2, c1[q], fma(ncf1, c0[q], u[q]));
-    const T pk1 = a * inv1;                // sqrt(a)
-    const T pk2 = (c - b * t) * inv2;      // sqrt(c - b^2 / a)
-    // lane comparisons on a copy of r the compiler cannot see through, so
-    // that they are made here and not hoisted out of the loop (32 hoisted
-    // masks spill to lanes of a vector register)
-    // (rows above k and k+1 take the multipliers too: for them these are
-    // strict-upper entries, which nothing reads)
-    int rk = rsel;
-    asm volatile("" : "+v"(rk));
-    const bool on1 = rk == k, on2 = rk == k + 1;
-    u[k] = on1 ? pk1 : lk1;
-    u[k + 1] = on2 ? pk2 : lk2;
-    // Materialise the registers every step: otherwise the optimiser sinks
-    // the updates to their last use and keeps every broadcast value alive.
-#pragma unroll
-    for (int q = 0; q < 32; ++q) asm volatile("" : "+v"(u[q]));
-    if constexpr (EARLY) {
-#pragma unroll
-      for (int q = k + 4; q < 32; ++q) {
-        c0[q] = n0[q];
-        c1[q] = n1[q];
-      }
-    }
-  }
-  // Lanes r and r + 32 share row r of S: the row lane stores columns c <= r,
-  // the inverse lane columns c > r, i.e. lane stores columns lo .. lo + span
-  // (none for inverse lane 31: lo = 32).  Every lane stores every entry, the
-  // ones outside its range into its own entry of col (free by now; distinct
-  // entries, so no bank conflicts): one compare and one address select per
-  // entry, no branches (the range is hidden from the optimiser, which would
-  // otherwise branch on the lane kind per entry).
+  wave_lds_order();
   {
-    lds_t* srow = (lds_t*)S + r * pitch;
-    lds_t* sink = colv + lane;
-    int lo = rowlane ? 0 : r + 1, span = rowlane ? r : (r < 31 ? 30 - r : 0);
-    asm volatile("" : "+v"(lo), "+v"(span));
+    // A_22 -= L_21 L_21^T and U_12 = -U_11 L_21^T: the B operand of both,
+    // and the A operand of the first, are the same entries of L_21
+    typename Mfma<T>::acc_t u12 = acc_zero<T>();
+    T l21[4], u11[4];
 #pragma unroll
-    for (int c = 0; c < 32; ++c) {
-      lds_t* d = ((unsigned)(c - lo) <= (unsigned)span) ? srow + c : sink;
-      asm volatile("" : "+v"(d));
-      *d = u[c];
+    for (int k = 0; k < 4; ++k) {
+      l21[k] = S[(16 + r) * pitch + 4 * k + g];
+      u11[k] = ut[r * 33 + 4 * k + g];
     }
-  }
-  // ut[r][c] = Linv[c][r] in full (zeros above the diagonal, 1/L[r][r] on
-  // it): the inverse lanes' whole columns, the operand of the panel product
-  if (!rowlane)
 #pragma unroll
-    for (int c = 0; c < 32; ++c) ut[r * 33 + c] = u[c];
-  // dinv from the diagonal of ut (this wavefront's LDS writes above complete
-  // first): tracking 1/L[r][r] through the pair steps by lane selects kept
-  // 32 lane masks alive to the end
-  if (rowlane) dinv[r] = ut[r * 33 + r];
+    for (int k = 0; k < 4; ++k) {
+      s22 = Mfma<T>::mma(-l21[k], l21[k], s22);
+      u12 = Mfma<T>::mma(-u11[k], l21[k], u12);
+    }
+    acc16_foreach<T>(s22, [&](int i, int j, T v) { S[(16 + i) * pitch + 16 + j] = v; });
+    acc16_foreach<T>(u12, [&](int i, int j, T v) { S[i * pitch + 16 + j] = v; });
+  }
+  wave_lds_order();
+  {
+    const T* urow = S + (16 + r) * pitch + 16;
+    T* prow = (g == 1 || g == 2) ? ut + (16 + r) * 33 + 16 : S + r * pitch + 16;
+#pragma unroll
+    for (int c = 0; c < 16; ++c) u[c] = urow[c];
+#pragma unroll
+    for (int c = 0; c < 16; ++c) p[0][c] = prow[c];
+#pragma unroll
+    for (int c = 0; c < 16; ++c) {
+      pin_reg(u[c]);
+      pin_reg(p[0][c]);
+    }
+    panel16<T, 1>(u, p, [&](int k) { hook(16 + k); });
+    if (g == 2) prow = S + (16 + r) * pitch + 16;
+    if (g == 3) prow = ut + r * 33 + 16;
+#pragma unroll
+    for (int c = 0; c < 16; ++c) prow[c] = (c <= rl) ? u[c] : p[0][c];
+  }
+  wave_lds_order();
+  if (lane < 32) dinv[lane] = ut[lane * 33 + lane];
 }
 
 // Inverse of a 32x32 lower-triangular tile (no factorisation), by one
