@@ -148,6 +148,14 @@ int run_op(int op, void* L, void* E, void* x, const uint8_t* mask, int B, int N,
     if (e != hipSuccess) return hip_fail(e, "diagonal-block inverse launch");
     Lt = W;
   }
+  if (n <= socu::kSmallN && (op == SOCU_OP_FACTOR || op == SOCU_OP_FACTOR_AND_SOLVE)) {
+    const bool solve = op == SOCU_OP_FACTOR_AND_SOLVE;
+    const bool with_x = solve && m <= socu::kSmallM;  // (more right-hand sides: the sweeps follow)
+    const hipError_t e = socu::small_factor<T>(Lt, Et, with_x ? xt : nullptr, mask, B, N, n, m, st, Ls, Es);
+    if (e != hipSuccess) return hip_fail(e, "small-block factor launch");
+    if (!solve || (with_x && socu::small_tail_applies(B, n, m))) return SOCU_OK;
+    return run_sweeps<T>(Lt, Et, xt, mask, B, N, n, m, !with_x, true, sw, st);
+  }
   switch (op) {
     case SOCU_OP_FACTOR:
       return run_factor<T>(Lt, Et, mask, B, N, n, st, Ls, Es);
@@ -158,11 +166,6 @@ int run_op(int op, void* L, void* E, void* x, const uint8_t* mask, int B, int N,
     case SOCU_OP_SOLVE:
       return run_sweeps<T>(Lt, Et, xt, mask, B, N, n, m, true, true, sw, st);
     case SOCU_OP_FACTOR_AND_SOLVE:
-      if (socu::fused_forward_applies<T>(n, 0)) {  // forward sweep inside the factor's kernels
-        const hipError_t e = socu::factor_and_forward<T>(Lt, Et, xt, mask, B, N, n, m, 0, st, Ls, Es);
-        if (e != hipSuccess) return hip_fail(e, "factor_and_solve launch");
-        return run_sweeps<T>(Lt, Et, xt, mask, B, N, n, m, false, true, sw, st);
-      }
       if (ov != nullptr) {  // forward sweep alongside the factor, then the backward sweep
         const hipError_t e =
             socu::factor_with_forward<T>(Lt, Et, xt, mask, mask, B, N, n, m, false, *ov, st, nullptr, Ls, Es);
@@ -186,6 +189,7 @@ int ensure_init() {
   if (e == hipSuccess) e = socu::init_batched_kernels();
   if (e == hipSuccess) e = socu::init_sweep_kernels();
   if (e == hipSuccess) e = socu::init_large_kernels();
+  if (e == hipSuccess) e = socu::init_small_kernels();
   if (e != hipSuccess) return hip_fail(e, "kernel set-up (hipFuncSetAttribute)");
   state = 1;
   return SOCU_OK;
@@ -291,7 +295,9 @@ void free_sweep_ws(SweepWs& sw) {
 // includes a substitution with one right-hand side.
 int alloc_sweep_ws(SweepWs& sw, int op, int B, int N, int n, int m, int dtype) {
   const size_t esz = dtype == SOCU_DTYPE_F64 ? sizeof(double) : sizeof(float);
-  if (op == SOCU_OP_FACTOR || m != 1 || B <= 0 || !socu::sweep_persistent_enabled(n, (int)esz)) return SOCU_OK;
+  if (op == SOCU_OP_FACTOR || m != 1 || B <= 0 || !socu::sweep_persistent_enabled(B, n, (int)esz)) return SOCU_OK;
+  // (these sweep inside the factor's kernels)
+  if (op == SOCU_OP_FACTOR_AND_SOLVE && n <= socu::kSmallN && socu::small_tail_applies(B, n, m)) return SOCU_OK;
   hipError_t e = hipMalloc(&sw.ws, sizeof(int) * socu::sweep_ws_ints(B, N));
   if (e == hipSuccess) e = hipMemset(sw.ws, 0, sizeof(int) * socu::sweep_ws_ints(B, N));  // status reads 0 before a run
   if (e == hipSuccess) e = hipMalloc(&sw.slots, esz * socu::sweep_slot_elems(B, N, n));

@@ -17,7 +17,7 @@
 //                :202-228).
 //   k_schur_blk  one workgroup per 64x64 output tile, MFMA, owner computes:
 //                L_j -= R R^T + Lc^T Lc,  F -= R Lc (syrk.py, gemm.py).
-//   k_sweep32, k_sweep_nb, k_apply_fwd  the sweeps, one launch per step and
+//   k_sweep_nb, k_apply_fwd  the sweeps, one launch per step and
 //                direction: the block-times-panel update and the triangular
 //                apply with the stored inverse in one kernel (k_apply_fwd:
 //                the first forward level) (replaces K9-K16,
@@ -275,152 +275,6 @@ __global__ __launch_bounds__(kThreads) void k_potrf_blk(TS* __restrict__ L, cons
       const int r = idx / n, c = idx - r * n;
       A[idx] = (TS)S[r * P + c];
     }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// One whole level-l node step for n == 32, by one wavefront per node:
-//   L_i <- chol(L_i) with the transposed inverse in its strict upper triangle
-//          (as k_potrf_blk),
-//   R_i <- R_i Linv^T,  Lc_i <- Linv Lc_i          (as k_trsm_node),
-//   F   <- -R_i Lc_i    the fill-in block (i+s, i-s) of the next level (the
-//                       fill-in tasks of k_schur_small / k_schur_blk).
-// The reference runs these as separate potrf, trsm and gemm passes over the
-// level (socu/blas/potrf.py:97-119, socu/blas/trsm.py:94-120 and :202-228,
-// block_tridiag_solver.py:797-813).  At n = 32 the pivot chain of the
-// diagonal block is latency-bound and uses little of a compute unit, so the
-// coupling blocks' loads, MFMA products and stores of one node run while the
-// other wavefronts on the same SIMD are in their chains; R_i and Lc_i are
-// read once (the separate kernels read them for the trsm and again for the
-// fill-in) and the factor is not re-read for the trsm.
-// R_i = block (i+s, i) exists when i + s < N, Lc_i = block (i, i-s) when
-// i >= s, F when both do.  Layouts and storage as the separate kernels;
-// Lsrc / Esrc (optional) are the out-of-place sources of L_i, R_i and Lc_i.
-// With x (n x m blocks, optional) the node also takes its forward-sweep step
-// y_i <- Linv y_i (k_apply_fwd); the updates y_j -= ... that level l sends to
-// its targets are then k_schur_small's, so that a factor_and_solve needs no
-// separate forward-sweep kernels.
-// ---------------------------------------------------------------------------
-constexpr size_t node32_lds(size_t esize) { return esize * (2 * 32 * 33 + 32); }
-
-// (two wavefronts per SIMD: the register budget is held to 256, which the
-// compiler meets without spills by keeping the MFMA accumulators in VGPRs)
-template <typename T>
-__global__ __launch_bounds__(64, 2) void k_node32(T* __restrict__ L, T* __restrict__ E, const uint8_t* __restrict__ mask,
-                                              int N, int nE, int s, int off, int next_off,
-                                              const T* __restrict__ Lsrc, const T* __restrict__ Esrc,
-                                              T* __restrict__ x, int m) {
-  constexpr int n = 32, P = 33;
-  constexpr size_t nn = 32 * 32;
-  const int b = blockIdx.y;
-  if (masked_out(mask, b)) return;
-  const int i = s - 1 + 2 * s * blockIdx.x;
-  const bool hasR = i + s < N, hasC = i >= s;
-  T* A = L + ((size_t)b * N + i) * nn;
-  const T* Ain = (Lsrc != nullptr) ? Lsrc + (A - L) : A;
-  T* Eb = E + (size_t)b * nE * nn;
-  T* XR = hasR ? Eb + (size_t)(off + i / s) * nn : nullptr;        // block (i+s, i)
-  T* XC = hasC ? Eb + (size_t)(off + (i - s) / s) * nn : nullptr;  // block (i, i-s)
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  T* S = reinterpret_cast<T*>(smem_raw);  // 32 x 33: the block, then R_i, Lc_i, R_i'
-  T* ut = S + 32 * P;                       // 32 x 33: Linv transposed, then Lc_i'
-  T* dinv = ut + 32 * P;
-  const int l = lane_id();
-  const int lr = l >> 5, lc = l & 31;  // lane l moves row 2q + lr, column lc of a block
-
-  {
-    T v[16];
-#pragma unroll
-    for (int q = 0; q < 16; ++q) v[q] = Ain[(2 * q + lr) * n + lc];
-#pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      const int r = 2 * q + lr;
-      S[r * P + lc] = (lc <= r) ? v[q] : T(0);
-    }
-  }
-  // R_i and Lc_i are loaded late in the pivot chain (pair step 20), when the
-  // chain's column registers of the early steps are free, and land while the
-  // chain finishes (earlier, the kernel needs more than the 256 registers
-  // that let two wavefronts share a SIMD).
-  T rv[16], cv[16];
-  const T* XRin = hasR ? ((Esrc != nullptr) ? Esrc + (XR - E) : XR) : nullptr;
-  const T* XCin = hasC ? ((Esrc != nullptr) ? Esrc + (XC - E) : XC) : nullptr;
-  // y_i (forward sweep): up to 4 columns (128 entries, two per lane) are
-  // loaded with R_i and Lc_i; wider ones at their step
-  T* y = (x != nullptr) ? x + ((size_t)b * N + i) * (size_t)n * m : nullptr;
-  const bool ypre = y != nullptr && m <= 4;
-  T yv0 = T(0), yv1 = T(0);
-  auto hook = [&](int k) {
-    if (k == 20) {
-      if (ypre) {
-        yv0 = y[min(l, 32 * m - 1)];
-        yv1 = y[min(l + 64, 32 * m - 1)];
-      }
-      if (hasR) {
-#pragma unroll
-        for (int q = 0; q < 16; ++q) rv[q] = XRin[(2 * q + lr) * n + lc];
-      }
-      if (hasC) {
-#pragma unroll
-        for (int q = 0; q < 16; ++q) cv[q] = XCin[(2 * q + lr) * n + lc];
-      }
-    }
-  };
-  tile_chol_inv<T>(S, P, dinv, ut, hook);
-  // the factor (lower) with the transposed inverse (strict upper)
-#pragma unroll
-  for (int q = 0; q < 16; ++q) A[(2 * q + lr) * n + lc] = S[(2 * q + lr) * P + lc];
-  if (y != nullptr) {
-    // y_i <- Linv y_i, up to 32 columns at a time staged in S:
-    // out[r][c] = sum_k ut[k][r] y[k][c]; lane l forms row l % 32 of the
-    // columns of its half (l / 32)
-    for (int c0 = 0; c0 < m; c0 += 32) {
-      const int w = min(32, m - c0);
-      if (ypre) {  // entries l and l + 64 of the 32 x m block
-        if (l < 32 * m) S[(l / m) * P + l % m] = yv0;
-        if (l + 64 < 32 * m) S[((l + 64) / m) * P + (l + 64) % m] = yv1;
-      } else {
-        for (int q = l; q < 32 * w; q += 64) {
-          const int k = q / w, c = q - k * w;
-          S[k * P + c] = y[(size_t)k * m + c0 + c];
-        }
-      }
-      for (int c = lr; c < w; c += 2) {
-        T acc = T(0);
-#pragma unroll
-        for (int k = 0; k < 32; ++k) acc = fma(ut[k * P + lc], S[k * P + c], acc);
-        y[(size_t)lc * m + c0 + c] = acc;
-      }
-    }
-  }
-  if (!hasR && !hasC) return;
-
-  // (LDS operations of one wavefront complete in issue order: S and ut are
-  // rewritten below only after the reads of their previous contents.)
-  typename Mfma<T>::acc_t ar[2][2] = {{acc_zero<T>(), acc_zero<T>()}, {acc_zero<T>(), acc_zero<T>()}};
-  typename Mfma<T>::acc_t ac[2][2] = {{acc_zero<T>(), acc_zero<T>()}, {acc_zero<T>(), acc_zero<T>()}};
-  if (hasR) {
-    // R' = R Linv^T: B(k, c) = Linv[c][k] = ut[k][c]
-#pragma unroll
-    for (int q = 0; q < 16; ++q) S[(2 * q + lr) * P + lc] = rv[q];
-    wave_gemm<T>(ar, S, P, 1, ut, P, 1, 32);
-    acc_foreach<T>(ar, [&](int r, int c, T v) { XR[r * n + c] = v; });
-  }
-  if (hasC) {
-    // Lc' = Linv Lc: A(r, k) = Linv[r][k] = ut[k][r]
-#pragma unroll
-    for (int q = 0; q < 16; ++q) S[(2 * q + lr) * P + lc] = cv[q];
-    wave_gemm<T>(ac, ut, 1, P, S, P, 1, 32);
-    acc_foreach<T>(ac, [&](int r, int c, T v) { XC[r * n + c] = v; });
-  }
-  if (hasR && hasC) {
-    // F = -R' Lc' from R' in S and Lc' in ut
-    T* F = Eb + (size_t)(next_off + (i - s) / (2 * s)) * nn;
-    acc_foreach<T>(ar, [&](int r, int c, T v) { S[r * P + c] = v; });
-    acc_foreach<T>(ac, [&](int r, int c, T v) { ut[r * P + c] = v; });
-    typename Mfma<T>::acc_t af[2][2] = {{acc_zero<T>(), acc_zero<T>()}, {acc_zero<T>(), acc_zero<T>()}};
-    wave_gemm<T>(af, S, P, 1, ut, P, 1, 32);
-    acc_foreach<T>(af, [&](int r, int c, T v) { F[r * n + c] = -v; });
   }
 }
 
@@ -1023,11 +877,7 @@ __global__ __launch_bounds__(kThreads) void k_schur_blk(T* __restrict__ L, T* __
 // the MFMA products.  Panels are kept as P[i][k] (pitch NP + 1): row panels
 // are 32 rows of a block, column panels 32 of its columns, transposed.
 // ---------------------------------------------------------------------------
-// four panels of 32 x (NP+1).  (The forward sweep of diagonal tiles stages
-// the two neighbours' right-hand sides, NP x kSmallYc each, and 32 rows of the
-// target's, 32 x kSmallYc, in panel 1, which diagonal tiles do not use.)
-constexpr int kSmallYc = 8;
-static_assert(2 * 32 * kSmallYc + 32 * kSmallYc <= 32 * 33, "right-hand sides fit in one panel");
+// four panels of 32 x (NP+1)
 template <typename T, int NB>
 constexpr size_t schur_small_lds() {
   return sizeof(T) * 4 * 32 * (size_t)(32 * NB + 1);
@@ -1072,18 +922,10 @@ __device__ __forceinline__ void panel_store(T* P, const T* v, bool cols, int i0,
   }
 }
 
-// With x (optional; n x m blocks of right-hand sides) the diagonal-tile
-// tasks of a target j also apply level l's forward-sweep update to rows
-// 32 tr .. of y_j (the forward sweep's update):
-//   y_j -= R_{j-s} y_{j-s} + Lc_{j+s}^T y_{j+s},
-// with the operand panels the Schur product has staged: rows 32 tr.. of R and
-// columns 32 tr.. of Lc.  The nodes' y must have had their level-l step
-// y <- Linv y (k_node32 does it).
 template <typename T, int NB, int NF, bool BF = false>
 __global__ __launch_bounds__(kThreads) void k_schur_small(T* __restrict__ L, T* __restrict__ E,
                                                          const uint8_t* __restrict__ mask, int N, int n_, int nE, int s,
-                                                         int off, int next_off, int nT, const T* __restrict__ Lsrc,
-                                                         T* __restrict__ x, int m) {
+                                                         int off, int next_off, int nT, const T* __restrict__ Lsrc) {
   const int n = NF ? NF : n_;
   constexpr int NP = 32 * NB, PP = NP + 1;
   constexpr int PE = 32 * NP / kThreads;
@@ -1102,7 +944,6 @@ __global__ __launch_bounds__(kThreads) void k_schur_small(T* __restrict__ L, T* 
   T* C;
   int tr, tc;
   bool diag;
-  int jt = -1;  // the target (target tasks only)
   if (task < nT * NTRI) {
     // L_j -= R R^T + Lc^T Lc  (R = block (j, j-s), Lc = block (j+s, j))
     const int u = task / NTRI;
@@ -1111,7 +952,6 @@ __global__ __launch_bounds__(kThreads) void k_schur_small(T* __restrict__ L, T* 
     while (q > tr) { q -= tr + 1; ++tr; }
     tc = q;
     const int j = 2 * s * (u + 1) - 1;
-    jt = j;
     C = L + ((size_t)b * N + j) * nn;
     const T* R = Eb + (size_t)(off + (j - s) / s) * nn;
     const bool hasC = j + s < N;
@@ -1140,36 +980,9 @@ __global__ __launch_bounds__(kThreads) void k_schur_small(T* __restrict__ L, T* 
   }
   const int l = lane_id(), wave = wave_id();
   const int wi = wave >> 1, wj = wave & 1;
-  // forward sweep (diagonal tiles of targets, with x): rows 32 tr .. of y_j
-  // -= R_{j-s} y_{j-s} + Lc_{j+s}^T y_{j+s}, kSmallYc columns at a time
-  const bool ysw = x != nullptr && diag;
-  const size_t nm = (size_t)n * m;
-  const T* ya = nullptr;
-  const T* yc = nullptr;
-  T* yj = nullptr;
-  if (ysw) {
-    T* xb = x + (size_t)b * N * nm;
-    ya = xb + (size_t)(jt - s) * nm;
-    yc = (np == 2) ? xb + (size_t)(jt + s) * nm : ya;
-    yj = xb + (size_t)jt * nm;
-  }
-  constexpr int YA = 32 * NB * kSmallYc / kThreads;  // neighbour entries per thread
-  T yav[YA], ycv[YA], yjv = T(0);
-  // (unconditional loads from clamped addresses; masked when staged)
-  auto yload = [&](int c0, int w) {
-#pragma unroll
-    for (int e = 0; e < YA; ++e) {
-      const int q = threadIdx.x + e * kThreads, k = q / w, c = q - k * w;
-      yav[e] = ya[(size_t)min(k, n - 1) * m + c0 + c];
-      ycv[e] = yc[(size_t)min(k, n - 1) * m + c0 + c];
-    }
-    const int q = threadIdx.x, i = q / w, c = q - i * w;
-    yjv = yj[(size_t)min(32 * tr + i, n - 1) * m + c0 + c];
-  };
-  // every load of the task at once: the first columns of the right-hand
-  // sides, the panels, then this wave's C values.  (Diagonal tiles: panels 1
-  // and 3 equal panels 0 and 2 and are neither loaded nor stored.)
-  if (ysw) yload(0, min(kSmallYc, m));
+  // every load of the task at once: the panels, then this wave's C values.
+  // (Diagonal tiles: panels 1 and 3 equal panels 0 and 2 and are neither
+  // loaded nor stored.)
   T v[4][PE];
 #pragma unroll
   for (int p = 0; p < 4; ++p)
@@ -1195,22 +1008,6 @@ __global__ __launch_bounds__(kThreads) void k_schur_small(T* __restrict__ L, T* 
 #pragma unroll
   for (int p = 0; p < 4; ++p)
     if (p < 2 * np && !(diag && (p & 1))) panel_store<T, NB>(Pn + p * 32 * PP, v[p], cols[p], i0[p], n);
-  const bool hasC = np == 2;
-  T* Ya = Pn + 32 * PP;  // (panel 1) NP x kSmallYc
-  T* Yc = Ya + NP * kSmallYc;
-  T* Yj = Yc + NP * kSmallYc;  // 32 x kSmallYc
-  auto ystage = [&](int w) {
-#pragma unroll
-    for (int e = 0; e < YA; ++e) {
-      const int q = threadIdx.x + e * kThreads, k = q / w, c = q - k * w;
-      if (q < NP * w) {
-        Ya[k * kSmallYc + c] = (k < n) ? yav[e] : T(0);
-        Yc[k * kSmallYc + c] = (hasC && k < n) ? ycv[e] : T(0);
-      }
-    }
-    if ((int)threadIdx.x < 32 * w) Yj[(threadIdx.x / w) * kSmallYc + threadIdx.x % w] = yjv;
-  };
-  if (ysw) ystage(min(kSmallYc, m));  // published by the panels' barrier
   __syncthreads();
   typename Mfma<T>::acc_t acc = acc_zero<T>();
   for (int p = 0; p < np; ++p)
@@ -1221,49 +1018,16 @@ __global__ __launch_bounds__(kThreads) void k_schur_small(T* __restrict__ L, T* 
     const int rr = 32 * tr + 16 * wi + Mfma<T>::row(l, r), cc = 32 * tc + 16 * wj + Mfma<T>::col(l, r);
     if (rr < n && cc < n && (!diag || cc <= rr)) C[rr * n + cc] = cv[r] - acc[r];
   }
-  if (!ysw) return;
-  const T* P0 = Pn;               // P0[i][k] = R[32 tr + i][k]
-  const T* P2 = Pn + 2 * 32 * PP;  // P2[i][k] = Lc[k][32 tr + i]
-  const int tid = threadIdx.x;
-  for (int c0 = 0; c0 < m; c0 += kSmallYc) {
-    const int w = min(kSmallYc, m - c0);
-    if (c0 > 0) {
-      __syncthreads();  // every wave is done with the previous columns
-      yload(c0, w);
-      ystage(w);
-      __syncthreads();
-    }
-    // one output per thread, (i, c) = (tid / w, tid % w): consecutive
-    // threads store consecutive entries of y_j's rows
-    if (tid < 32 * w) {
-      const int i = tid / w, c = tid - i * w;
-      T a0 = T(0), a1 = T(0);
-#pragma unroll 8
-      for (int k = 0; k < NP; k += 2) {
-        a0 = fma(P0[i * PP + k], Ya[k * kSmallYc + c], a0);
-        a1 = fma(P0[i * PP + k + 1], Ya[(k + 1) * kSmallYc + c], a1);
-      }
-      if (hasC) {
-#pragma unroll 8
-        for (int k = 0; k < NP; k += 2) {
-          a0 = fma(P2[i * PP + k], Yc[k * kSmallYc + c], a0);
-          a1 = fma(P2[i * PP + k + 1], Yc[(k + 1) * kSmallYc + c], a1);
-        }
-      }
-      const int r = 32 * tr + i;
-      if (r < n) yj[(size_t)r * m + c0 + c] = Yj[i * kSmallYc + c] - (a0 + a1);
-    }
-  }
 }
 
 // ---------------------------------------------------------------------------
 // solves, with the explicit inverses of the diagonal blocks (see k_potrf_blk)
 //
-// Forward step l (levels ascending), k_sweep32 / k_sweep_nb:
+// Forward step l (levels ascending), k_sweep_nb:
 //   for every receiving block j = 2s(u+1)-1:  y_j -= R_{j-s} y_{j-s} + Lc_{j+s}^T y_{j+s},
 //   then, for the nodes j of level l+1 among them:  y_j <- Linv_j y_j
 //   (k_apply_fwd: the applies of level 0, which no update precedes)
-// Backward level l (levels descending), k_sweep32 / k_sweep_nb:
+// Backward level l (levels descending), k_sweep_nb:
 //   for every node i:  x_i <- Linv_i^T (x_i - R_i^T x_{i+s} - Lc_i x_{i-s})
 // ---------------------------------------------------------------------------
 // Right-hand-side panels in LDS have pitch yp = min(m, kRhsChunk) + 1
@@ -1341,9 +1105,8 @@ __global__ __launch_bounds__(kThreads) void k_apply_fwd(const T* __restrict__ L,
 }
 
 
-// One sweep step for n == 32 in one launch, one workgroup per (block, 16
-// right-hand sides), both products on 16x16 MFMA tiles (waves 0 and 1 take
-// rows 0-15 and 16-31, the right-hand sides are the 16 columns).
+// One sweep step in one launch, one workgroup per (block, 16 right-hand
+// sides).
 // Backward (FWD = false), level l, node i (the reference's backward
 // substitution, block_tridiag_solver.py:581-643; update and apply in one):
 //   t   = x_i - R_i^T x_{i+s} - Lc_i x_{i-s}     (R_i = block (i+s, i) when
@@ -1357,156 +1120,7 @@ __global__ __launch_bounds__(kThreads) void k_apply_fwd(const T* __restrict__ L,
 //   t   = y_j - R_{j-s} y_{j-s} - Lc_{j+s}^T y_{j+s}   (R_{j-s} = block
 //         (j, j-s), Lc_{j+s} = block (j+s, j) when j + s < N),
 //   y_j = t, or Linv_j t = t / L_j[r][r] + U^T t for u even.
-// All three blocks and the three right-hand-side panels are loaded at once
-// and staged in LDS (32 x 33 tiles; panels of pitch rhs_pitch(m)).  Columns
-// at or past w read whatever follows in LDS (a guard keeps those reads in
-// the allocation): they only reach output columns that are not stored.
-template <typename T>
-constexpr size_t sweep32_lds(int m) {
-  return sizeof(T) * (3 * 32 * 33 + 3 * 32 * (size_t)rhs_pitch(m) + 16 + 32);
-}
-
-template <typename T, bool FWD>
-__global__ __launch_bounds__(kThreads) void k_sweep32(const T* __restrict__ L, const T* __restrict__ E,
-                                                     T* __restrict__ x, const uint8_t* __restrict__ mask, int N, int m,
-                                                     int nE, int s, int off, int apply) {
-  constexpr int n = 32, P = 33;
-  constexpr size_t nn = 32 * 32;
-  const int b = blockIdx.z;
-  if (masked_out(mask, b)) return;
-  const int c0 = blockIdx.y * kRhsChunk;
-  const int w = min(kRhsChunk, m - c0);
-  const int yp = rhs_pitch(m);
-  const size_t nm = (size_t)n * m;
-  const T* Eb = E + (size_t)b * nE * nn;
-  T* xb = x + (size_t)b * N * nm;
-  // Blocks used transposed (A(i, k) = M[k][i]) with panel Xp, and as they
-  // stand (A(i, k) = M[i][k]) with panel Xm.
-  int i;
-  bool hasT, hasS, inv;
-  const T* MT;
-  const T* MS;
-  const T* xp;
-  const T* xm;
-  if (!FWD) {
-    i = s - 1 + 2 * s * blockIdx.x;
-    hasT = i + s < N;  // R_i
-    hasS = i >= s;     // Lc_i
-    inv = true;
-  } else {
-    const int u = blockIdx.x;
-    i = 2 * s * (u + 1) - 1;
-    hasT = i + s < N;  // Lc_{j+s}
-    hasS = true;       // R_{j-s}
-    inv = apply != 0 && (u & 1) == 0;
-  }
-  const T* U = L + ((size_t)b * N + i) * nn;
-  T* xi = xb + (size_t)i * nm;
-  if (!FWD) {
-    MT = hasT ? Eb + (size_t)(off + i / s) * nn : U;  // (U: a valid dummy address)
-    MS = hasS ? Eb + (size_t)(off + (i - s) / s) * nn : U;
-  } else {
-    MT = hasT ? Eb + (size_t)(off + i / s) * nn : U;
-    MS = Eb + (size_t)(off + (i - s) / s) * nn;
-  }
-  xp = hasT ? xb + (size_t)(i + s) * nm : xi;
-  xm = hasS ? xb + (size_t)(i - s) * nm : xi;
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  T* Us = reinterpret_cast<T*>(smem_raw);  // 32 x 33 each
-  T* Ts = Us + 32 * P;
-  T* Ss = Ts + 32 * P;
-  T* Xp = Ss + 32 * P;  // 32 x yp each; Xp later holds t
-  T* Xm = Xp + 32 * yp;
-  T* Xi = Xm + 32 * yp;
-  T* dg = Xi + 32 * yp + 16;  // 1 / L[r][r] (after a 16-entry guard)
-  const int tid = threadIdx.x, l = lane_id(), wave = wave_id();
-  // every load at once (unconditional, from valid addresses), then the LDS
-  // stores with the absent operands zeroed
-  constexpr int PT = 32 * 32 / kThreads;
-  T uv[PT], tv[PT], sv[PT];
-#pragma unroll
-  for (int e = 0; e < PT; ++e) {
-    const int idx = tid + e * kThreads;
-    uv[e] = U[idx];
-    tv[e] = MT[idx];
-    sv[e] = MS[idx];
-  }
-  // right-hand-side entries q = tid + kThreads e (row q / w, column q % w)
-  constexpr int PQ = 32 * kRhsChunk / kThreads;
-  T xpv[PQ], xmv[PQ], xiv[PQ];
-#pragma unroll
-  for (int e = 0; e < PQ; ++e) {
-    const int q = tid + e * kThreads, qr = q / w, qc = q - qr * w;
-    const size_t xo = (size_t)min(qr, 31) * m + c0 + qc;
-    xpv[e] = xp[xo];
-    xmv[e] = xm[xo];
-    xiv[e] = xi[xo];
-  }
-#pragma unroll
-  for (int e = 0; e < PT; ++e) {
-    pin_reg(uv[e]);
-    pin_reg(tv[e]);
-    pin_reg(sv[e]);
-  }
-#pragma unroll
-  for (int e = 0; e < PT; ++e) {
-    const int idx = tid + e * kThreads;
-    const int r = idx >> 5, c = idx & 31;
-    Us[r * P + c] = uv[e];
-    Ts[r * P + c] = hasT ? tv[e] : T(0);
-    Ss[r * P + c] = hasS ? sv[e] : T(0);
-    if (r == c) dg[r] = T(1) / uv[e];
-  }
-#pragma unroll
-  for (int e = 0; e < PQ; ++e) {
-    const int q = tid + e * kThreads, qr = q / w, qc = q - qr * w;
-    if (q < 32 * w) {
-      Xp[qr * yp + qc] = hasT ? xpv[e] : T(0);
-      Xm[qr * yp + qc] = hasS ? xmv[e] : T(0);
-      Xi[qr * yp + qc] = xiv[e];
-    }
-  }
-  __syncthreads();
-  // t = x_i - MT^T xp - MS xm: wave rt (0, 1) forms rows 16 rt .. 16 rt + 15
-  const int rt = wave;
-  typename Mfma<T>::acc_t acc = acc_zero<T>();
-  if (rt < 2) {
-    wave_gemm16<T>(acc, Ts + 16 * rt, 1, P, Xp, yp, 1, 32);
-    wave_gemm16<T>(acc, Ss + 16 * rt * P, P, 1, Xm, yp, 1, 32);
-  }
-  if (!inv) {
-    if (rt < 2)
-      acc16_foreach<T>(acc, [&](int r, int c, T v) {
-        if (c < w) xi[(size_t)(16 * rt + r) * m + c0 + c] = Xi[(16 * rt + r) * yp + c] - v;
-      });
-    return;
-  }
-  __syncthreads();  // every read of Xp done
-  if (rt < 2)
-    acc16_foreach<T>(acc, [&](int r, int c, T v) {
-      if (c < w) Xp[(16 * rt + r) * yp + c] = Xi[(16 * rt + r) * yp + c] - v;
-    });
-  __syncthreads();
-  // backward: x_i = A t, A(r, k) = U[r][k] (k > r), 1 / L[r][r] (k = r);
-  // forward: y_j = A t, A(r, k) = U[k][r] (k < r), 1 / L[r][r] (k = r)
-  if (rt < 2) {
-    acc = acc_zero<T>();
-    const int ii = l & 15, kq = l >> 4, row = 16 * rt + ii;
-#pragma unroll
-    for (int k = 0; k < 32; k += 4) {
-      const int kk = k + kq;
-      const T u = FWD ? Us[kk * P + row] : Us[row * P + kk];
-      const T a = (FWD ? kk < row : kk > row) ? u : ((kk == row) ? dg[row] : T(0));
-      acc = Mfma<T>::mma(a, Xp[kk * yp + ii], acc);
-    }
-    acc16_foreach<T>(acc, [&](int r, int c, T v) {
-      if (c < w) xi[(size_t)(16 * rt + r) * m + c0 + c] = v;
-    });
-  }
-}
-
-// The same sweep step for the other block sizes n <= 128 (NB = 1..4; for
-// NB >= 2 three staged blocks would not fit LDS): the block operands are read
+// Three staged blocks would not fit LDS: the block operands are read
 // from global memory
 // in the MFMA operand layout (each element is used once: the right-hand
 // sides are the 16 columns of every product), the three panels and the
@@ -1840,11 +1454,9 @@ static hipError_t set_mixed_attrs() {
 
 hipError_t init_blocked_kernels() {
   hipError_t e;
-  if ((e = set_blk_attrs<float, 1>()) != hipSuccess) return e;
   if ((e = set_blk_attrs<float, 2>()) != hipSuccess) return e;
   if ((e = set_blk_attrs<float, 3>()) != hipSuccess) return e;
   if ((e = set_blk_attrs<float, 4>()) != hipSuccess) return e;
-  if ((e = set_blk_attrs<double, 1>()) != hipSuccess) return e;
   if ((e = set_blk_attrs<double, 2>()) != hipSuccess) return e;
   if ((e = set_blk_attrs<double, 3>()) != hipSuccess) return e;
   if ((e = set_blk_attrs<double, 4>()) != hipSuccess) return e;
@@ -1852,7 +1464,6 @@ hipError_t init_blocked_kernels() {
   if ((e = set_schur_small_attrs<float, 2>()) != hipSuccess) return e;
   if ((e = set_schur_small_attrs<float, 3>()) != hipSuccess) return e;
   if ((e = set_schur_small_attrs<float, 4>()) != hipSuccess) return e;
-  if ((e = set_schur_small_attrs<double, 1>()) != hipSuccess) return e;
   if ((e = set_schur_small_attrs<double, 2>()) != hipSuccess) return e;
   if ((e = set_schur_small_attrs<double, 3>()) != hipSuccess) return e;
   if ((e = set_schur_small_attrs<double, 4>()) != hipSuccess) return e;
@@ -1874,96 +1485,69 @@ hipError_t init_blocked_kernels() {
 template <typename T, int NB, int NF>
 static hipError_t factor_level_nb(T* L, T* E, const uint8_t* mask, int B, int N, int n, int lidx, int prec,
                                   hipStream_t st, hipEvent_t after_potrf, hipEvent_t after_trsm,
-                                  hipEvent_t before_trsm, const T* Lsrc, const T* Esrc, T* x = nullptr,
-                                  int m = 0) {
+                                  hipEvent_t before_trsm, const T* Lsrc, const T* Esrc) {
   const int nE = (int)off_diag_storage_len(N);
   const int Lv = recursive_iterations(N);
   const Level lv = level_info(N, lidx);
   if (lv.dim <= 0 || B <= 0) return hipSuccess;
   const size_t lds_trsm = trsm_blk_lds<T, NB>();
   const bool bf16 = (prec & kPrecBf16Schur) != 0 && sizeof(T) == 4;
-  // n == 32 in the storage precision: one fused node kernel (k_node32) per
-  // level instead of potrf, trsm and the Schur kernel's fill-in tasks (not
-  // when the trsm must wait for other work, nor with FP64 pivots for FP32
-  // blocks or BF16 Schur products, which the separate kernels implement)
-  // With x (fused_forward_applies), the level's forward-sweep steps run in
-  // the same kernels: y_i <- Linv y_i in k_node32, the updates of the targets'
-  // y in k_schur_small.
-  const bool fused = NF == 32 && before_trsm == nullptr && !bf16 &&
-                     !((prec & kPrecF64Pivots) != 0 && sizeof(T) == 4);
-  T* const xf = fused ? x : nullptr;
-  if (fused) {
-    hipEvent_t ea = nullptr, eb = nullptr;
-    if (kt_kernel_events(kKcPotrf, &ea, &eb))
-      hipExtLaunchKernelGGL(k_node32<T>, dim3(lv.dim, B), dim3(64), node32_lds(sizeof(T)), st, ea, eb, 0, L, E, mask, N,
-                            nE, lv.s, lv.off, lv.next_off, Lsrc, Esrc, xf, m);
-    else
-      hipLaunchKernelGGL(k_node32<T>, dim3(lv.dim, B), dim3(64), node32_lds(sizeof(T)), st, L, E, mask, N, nE, lv.s,
-                         lv.off, lv.next_off, Lsrc, Esrc, xf, m);
-    hipError_t e = hipSuccess;
-    if (after_potrf != nullptr) e = hipEventRecord(after_potrf, st);
-    if (e == hipSuccess && after_trsm != nullptr) e = hipEventRecord(after_trsm, st);
+  // under socu_profile_op the launch itself records its start and end
+  // (events of hipExtLaunchKernel: the kernel's own execution interval)
+  auto k = k_potrf_blk<T, NB, NF, T>;
+  size_t lds_potrf = potrf_blk_lds<T, NB>();
+  if ((prec & kPrecF64Pivots) != 0 && sizeof(T) == 4) {
+    k = k_potrf_blk<T, NB, NF, double>;
+    lds_potrf = potrf_blk_lds<double, NB>();
+  }
+  hipEvent_t ea = nullptr, eb = nullptr;
+  if (kt_kernel_events(kKcPotrf, &ea, &eb))
+    hipExtLaunchKernelGGL(k, dim3(lv.dim, B), dim3(potrf_threads(NB)), lds_potrf, st, ea, eb, 0, L, mask, N, n, lv.s,
+                          Lsrc);
+  else
+    hipLaunchKernelGGL(k, dim3(lv.dim, B), dim3(potrf_threads(NB)), lds_potrf, st, L, mask, N, n, lv.s, Lsrc);
+  if (after_potrf != nullptr) {
+    const hipError_t e = hipEventRecord(after_potrf, st);
     if (e != hipSuccess) return e;
-    if (lidx == Lv - 1) return hipGetLastError();
-  } else {
-    // under socu_profile_op the launch itself records its start and end
-    // (events of hipExtLaunchKernel: the kernel's own execution interval)
-    auto k = k_potrf_blk<T, NB, NF, T>;
-    size_t lds_potrf = potrf_blk_lds<T, NB>();
-    if ((prec & kPrecF64Pivots) != 0 && sizeof(T) == 4) {
-      k = k_potrf_blk<T, NB, NF, double>;
-      lds_potrf = potrf_blk_lds<double, NB>();
-    }
-    hipEvent_t ea = nullptr, eb = nullptr;
-    if (kt_kernel_events(kKcPotrf, &ea, &eb))
-      hipExtLaunchKernelGGL(k, dim3(lv.dim, B), dim3(potrf_threads(NB)), lds_potrf, st, ea, eb, 0, L, mask, N, n, lv.s,
-                            Lsrc);
-    else
-      hipLaunchKernelGGL(k, dim3(lv.dim, B), dim3(potrf_threads(NB)), lds_potrf, st, L, mask, N, n, lv.s, Lsrc);
-    if (after_potrf != nullptr) {
-      const hipError_t e = hipEventRecord(after_potrf, st);
-      if (e != hipSuccess) return e;
-    }
-    if (lidx == Lv - 1) return hipGetLastError();
-    if (before_trsm != nullptr) {
-      const hipError_t e = hipStreamWaitEvent(st, before_trsm, 0);
-      if (e != hipSuccess) return e;
-    }
-    kt_begin(kKcTrsm, st);
-    if (B * lv.dim >= trsm_node_min(NB)) {
-      const int cpb = trsm_chunks_per_block();
-      const int groups = (2 * NB + cpb - 1) / cpb;
-      const size_t lds_node = trsm_node_lds<T, NB>();
-      hipLaunchKernelGGL((k_trsm_node<T, NB, NF>), dim3(lv.dim, groups, B), dim3(kTrsmThreads), lds_node, st, L, E,
-                         mask, N, n, nE, lv.s, lv.off, cpb, Esrc);
-    }
-    else
-      hipLaunchKernelGGL((k_trsm_blk<T, NB, NF>), dim3(lv.dim, 2 * NB, B), dim3(trsm_blk_threads(NB)), lds_trsm, st, L,
-                         E, mask, N, n, nE, lv.s, lv.off, Esrc);
-    kt_end(kKcTrsm, st);
-    if (after_trsm != nullptr) {
-      const hipError_t e = hipEventRecord(after_trsm, st);
-      if (e != hipSuccess) return e;
-    }
+  }
+  if (lidx == Lv - 1) return hipGetLastError();
+  if (before_trsm != nullptr) {
+    const hipError_t e = hipStreamWaitEvent(st, before_trsm, 0);
+    if (e != hipSuccess) return e;
+  }
+  kt_begin(kKcTrsm, st);
+  if (B * lv.dim >= trsm_node_min(NB)) {
+    const int cpb = trsm_chunks_per_block();
+    const int groups = (2 * NB + cpb - 1) / cpb;
+    const size_t lds_node = trsm_node_lds<T, NB>();
+    hipLaunchKernelGGL((k_trsm_node<T, NB, NF>), dim3(lv.dim, groups, B), dim3(kTrsmThreads), lds_node, st, L, E,
+                       mask, N, n, nE, lv.s, lv.off, cpb, Esrc);
+  }
+  else
+    hipLaunchKernelGGL((k_trsm_blk<T, NB, NF>), dim3(lv.dim, 2 * NB, B), dim3(trsm_blk_threads(NB)), lds_trsm, st, L,
+                       E, mask, N, n, nE, lv.s, lv.off, Esrc);
+  kt_end(kKcTrsm, st);
+  if (after_trsm != nullptr) {
+    const hipError_t e = hipEventRecord(after_trsm, st);
+    if (e != hipSuccess) return e;
   }
   const int ntile = (n + kSTile - 1) / kSTile;
   const int ntri = ntile * (ntile + 1) / 2;
   const int nT = N / (2 * lv.s);
-  int nF = 0;  // fill-in tasks (k_node32 forms the fill-in blocks itself)
-  if (!fused)
-    for (int t = 1; t < lv.dim; ++t)
-      if (lv.s - 1 + 2 * lv.s * t + lv.s < N) ++nF;
+  int nF = 0;  // fill-in tasks
+  for (int t = 1; t < lv.dim; ++t)
+    if (lv.s - 1 + 2 * lv.s * t + lv.s < N) ++nF;
   const int tasks = nT * ntri + nF * ntile * ntile;
   if (tasks > 0) {
     kt_begin(kKcSchur, st);
-    if (xf != nullptr || use_schur_small(B * (nT + nF), n, (int)sizeof(T))) {
+    if (use_schur_small(B * (nT + nF), n, (int)sizeof(T))) {
       const int nsmall = nT * (NB * (NB + 1) / 2) + nF * NB * NB;
       const size_t lds_small = schur_small_lds<T, NB>();
       auto k = k_schur_small<T, NB, NF, false>;
       if constexpr (sizeof(T) == 4)
         if (bf16) k = k_schur_small<T, NB, NF, true>;
       hipLaunchKernelGGL(k, dim3(nsmall, B), dim3(kThreads), lds_small, st, L, E, mask, N, n, nE, lv.s, lv.off,
-                         lv.next_off, nT, Lsrc, xf, m);
+                         lv.next_off, nT, Lsrc);
     } else {
       auto k = k_schur_blk<T, NF, false>;
       if constexpr (sizeof(T) == 4)
@@ -2021,9 +1605,25 @@ hipError_t factor_level_blocked(T* L, T* E, const uint8_t* mask, int B, int N, i
     return factor_level_large<T>(L, E, mask, B, N, n, lidx, st, after_potrf, after_trsm, before_trsm);
   }
   const int fp = prec;
+  if (n <= kSmallN) {
+    // blocks of n <= 32: FP32 storage with FP64 pivots or BF16 Schur products
+    // takes the separate kernels; else one launch per level (in place; the
+    // level applies the previous level's updates itself)
+    if constexpr (sizeof(T) == 4) {
+      if ((prec & (kPrecF64Pivots | kPrecBf16Schur)) != 0)
+        return n == 32 ? factor_level_nb<T, 1, 32>(L, E, mask, B, N, n, lidx, fp, st, after_potrf, after_trsm,
+                                                   before_trsm, Lsrc, Esrc)
+                       : factor_level_nb<T, 1, 0>(L, E, mask, B, N, n, lidx, fp, st, after_potrf, after_trsm,
+                                                  before_trsm, Lsrc, Esrc);
+    }
+    if (Lsrc != nullptr || Esrc != nullptr) return hipErrorInvalidValue;
+    hipError_t e = before_trsm != nullptr ? hipStreamWaitEvent(st, before_trsm, 0) : hipSuccess;
+    if (e == hipSuccess) e = small_up_level<T>(L, E, nullptr, mask, B, N, n, 0, lidx, st, nullptr, nullptr);
+    if (e == hipSuccess && after_potrf != nullptr) e = hipEventRecord(after_potrf, st);
+    if (e == hipSuccess && after_trsm != nullptr) e = hipEventRecord(after_trsm, st);
+    return e;
+  }
   switch (n) {
-    case 32: return factor_level_nb<T, 1, 32>(L, E, mask, B, N, n, lidx, fp, st, after_potrf, after_trsm, before_trsm, Lsrc,
-                                                   Esrc);
     case 64: return factor_level_nb<T, 2, 64>(L, E, mask, B, N, n, lidx, fp, st, after_potrf, after_trsm, before_trsm, Lsrc,
                                                    Esrc);
     case 96: return factor_level_nb<T, 3, 96>(L, E, mask, B, N, n, lidx, fp, st, after_potrf, after_trsm, before_trsm, Lsrc,
@@ -2033,8 +1633,6 @@ hipError_t factor_level_blocked(T* L, T* E, const uint8_t* mask, int B, int N, i
     default: break;
   }
   switch ((n + 31) / 32) {
-    case 1: return factor_level_nb<T, 1, 0>(L, E, mask, B, N, n, lidx, fp, st, after_potrf, after_trsm, before_trsm, Lsrc,
-                                                   Esrc);
     case 2: return factor_level_nb<T, 2, 0>(L, E, mask, B, N, n, lidx, fp, st, after_potrf, after_trsm, before_trsm, Lsrc,
                                                    Esrc);
     case 3: return factor_level_nb<T, 3, 0>(L, E, mask, B, N, n, lidx, fp, st, after_potrf, after_trsm, before_trsm, Lsrc,
@@ -2086,22 +1684,15 @@ static hipError_t forward_step_nb(const T* L, const T* E, T* x, const uint8_t* m
   const int mch = (m + kRhsChunk - 1) / kRhsChunk;
   if (B <= 0 || mch <= 0) return hipSuccess;
   kt_begin(kKcForward, st);
-  // step l's updates and level l+1's applies in one launch (k_sweep32,
-  // k_sweep_nb)
+  // step l's updates and level l+1's applies in one launch
   if (update && step >= 0) {
     const Level lv = level_info(N, step);
     const int items = N / (2 * lv.s);
     if (items > 0) {
       const int ap = (apply_next && level_info(N, step + 1).dim > 0) ? 1 : 0;
-      if constexpr (NF == 32) {
-        const size_t lds = sweep32_lds<T>(m);
-        hipLaunchKernelGGL((k_sweep32<T, true>), dim3(items, mch, B), dim3(kThreads), lds, st, L, E, x, mask, N, m,
-                           nE, lv.s, lv.off, ap);
-      } else {
-        const size_t lds = sweepnb_lds<T, NB>(m);
-        hipLaunchKernelGGL((k_sweep_nb<T, NB, NF, true>), dim3(items, mch, B), dim3(sweepnb_threads<T, NB, true>()), lds,
-                           st, L, E, x, mask, N, n, m, nE, lv.s, lv.off, ap);
-      }
+      const size_t lds = sweepnb_lds<T, NB>(m);
+      hipLaunchKernelGGL((k_sweep_nb<T, NB, NF, true>), dim3(items, mch, B), dim3(sweepnb_threads<T, NB, true>()), lds,
+                         st, L, E, x, mask, N, n, m, nE, lv.s, lv.off, ap);
     }
     kt_end(kKcForward, st);
     return hipGetLastError();
@@ -2127,15 +1718,14 @@ static hipError_t forward_step_parts(const T* L, const T* E, T* x, const uint8_t
     kt_end(kKcForward, st);
     return e;
   }
+  if (n <= kSmallN) return small_forward_step<T>(L, E, x, mask, B, N, n, m, step, st, u, a);
   switch (n) {
-    case 32: return forward_step_nb<T, 1, 32>(L, E, x, mask, B, N, n, m, step, st, a, u);
     case 64: return forward_step_nb<T, 2, 64>(L, E, x, mask, B, N, n, m, step, st, a, u);
     case 96: return forward_step_nb<T, 3, 96>(L, E, x, mask, B, N, n, m, step, st, a, u);
     case 128: return forward_step_nb<T, 4, 128>(L, E, x, mask, B, N, n, m, step, st, a, u);
     default: break;
   }
   switch ((n + 31) / 32) {
-    case 1: return forward_step_nb<T, 1, 0>(L, E, x, mask, B, N, n, m, step, st, a, u);
     case 2: return forward_step_nb<T, 2, 0>(L, E, x, mask, B, N, n, m, step, st, a, u);
     case 3: return forward_step_nb<T, 3, 0>(L, E, x, mask, B, N, n, m, step, st, a, u);
     case 4: return forward_step_nb<T, 4, 0>(L, E, x, mask, B, N, n, m, step, st, a, u);
@@ -2169,19 +1759,11 @@ static hipError_t backward_level_nb(const T* L, const T* E, T* x, const uint8_t*
   const Level lv = level_info(N, lidx);
   if (lv.dim <= 0 || B <= 0 || mch <= 0) return hipSuccess;
   kt_begin(kKcBackward, st);
-  if constexpr (NF == 32) {  // update and apply in one launch
-    const size_t lds = sweep32_lds<T>(m);
-    hipLaunchKernelGGL((k_sweep32<T, false>), dim3(lv.dim, mch, B), dim3(kThreads), lds, st, L, E, x, mask, N, m, nE,
-                       lv.s, lv.off, 1);
-    kt_end(kKcBackward, st);
-    return hipGetLastError();
-  } else {
-    const size_t lds = sweepnb_lds<T, NB>(m);
-    hipLaunchKernelGGL((k_sweep_nb<T, NB, NF, false>), dim3(lv.dim, mch, B), dim3(sweepnb_threads<T, NB, false>()), lds,
-                       st, L, E, x, mask, N, n, m, nE, lv.s, lv.off, 1);
-    kt_end(kKcBackward, st);
-    return hipGetLastError();
-  }
+  const size_t lds = sweepnb_lds<T, NB>(m);
+  hipLaunchKernelGGL((k_sweep_nb<T, NB, NF, false>), dim3(lv.dim, mch, B), dim3(sweepnb_threads<T, NB, false>()), lds,
+                     st, L, E, x, mask, N, n, m, nE, lv.s, lv.off, 1);
+  kt_end(kKcBackward, st);
+  return hipGetLastError();
 }
 
 template <typename T>
@@ -2196,15 +1778,14 @@ hipError_t backward_level_blocked(const T* L, const T* E, T* x, const uint8_t* m
     kt_end(kKcBackward, st);
     return e;
   }
+  if (n <= kSmallN) return small_backward_level<T>(L, E, x, mask, B, N, n, m, lidx, st);
   switch (n) {
-    case 32: return backward_level_nb<T, 1, 32>(L, E, x, mask, B, N, n, m, lidx, st);
     case 64: return backward_level_nb<T, 2, 64>(L, E, x, mask, B, N, n, m, lidx, st);
     case 96: return backward_level_nb<T, 3, 96>(L, E, x, mask, B, N, n, m, lidx, st);
     case 128: return backward_level_nb<T, 4, 128>(L, E, x, mask, B, N, n, m, lidx, st);
     default: break;
   }
   switch ((n + 31) / 32) {
-    case 1: return backward_level_nb<T, 1, 0>(L, E, x, mask, B, N, n, m, lidx, st);
     case 2: return backward_level_nb<T, 2, 0>(L, E, x, mask, B, N, n, m, lidx, st);
     case 3: return backward_level_nb<T, 3, 0>(L, E, x, mask, B, N, n, m, lidx, st);
     case 4: return backward_level_nb<T, 4, 0>(L, E, x, mask, B, N, n, m, lidx, st);
@@ -2237,23 +1818,6 @@ void overlap_destroy(SweepOverlap& ov) {
   ov = SweepOverlap();
 }
 
-template <typename T>
-bool fused_forward_applies(int n, int prec) {
-  return n == 32 && !(sizeof(T) == 4 && (prec & (kPrecF64Pivots | kPrecBf16Schur)) != 0);
-}
-
-template <typename T>
-hipError_t factor_and_forward(T* L, T* E, T* x, const uint8_t* mask, int B, int N, int n, int m, int prec,
-                              hipStream_t st, const T* Lsrc, const T* Esrc) {
-  if (!fused_forward_applies<T>(n, prec)) return hipErrorInvalidValue;
-  const int Lv = recursive_iterations(N);
-  hipError_t e = hipSuccess;
-  for (int l = 0; l < Lv && e == hipSuccess; ++l)
-    e = factor_level_nb<T, 1, 32>(L, E, mask, B, N, n, l, prec, st, nullptr, nullptr, nullptr, l == 0 ? Lsrc : nullptr,
-                                  l == 0 ? Esrc : nullptr, x, m);
-  return e;
-}
-
 // The reference's fused factor_and_solve likewise interleaves the forward
 // sweep into the factor's levels (block_tridiag_solver.py:926-1233).  Here
 // the sweep runs on a second stream: the inverses of level l follow that
@@ -2265,9 +1829,6 @@ hipError_t factor_with_forward(T* L, T* E, T* x, const uint8_t* factor_mask, con
                                int n, int m, int prec, const SweepOverlap& ov, hipStream_t st,
                                const std::function<hipError_t(hipStream_t)>* side_first, const T* Lsrc,
                                const T* Esrc) {
-  // n == 32: the forward sweep runs inside the factor's own kernels
-  if (side_first == nullptr && factor_mask == sweep_mask && fused_forward_applies<T>(n, prec))
-    return factor_and_forward<T>(L, E, x, factor_mask, B, N, n, m, prec, st, Lsrc, Esrc);
   const int Lv = recursive_iterations(N);
   hipError_t e = hipEventRecord(ov.fork, st);
   if (e == hipSuccess) e = hipStreamWaitEvent(ov.side, ov.fork, 0);
@@ -2288,12 +1849,6 @@ hipError_t factor_with_forward(T* L, T* E, T* x, const uint8_t* factor_mask, con
   return e;
 }
 
-template bool fused_forward_applies<float>(int, int);
-template bool fused_forward_applies<double>(int, int);
-template hipError_t factor_and_forward<float>(float*, float*, float*, const uint8_t*, int, int, int, int, int,
-                                              hipStream_t, const float*, const float*);
-template hipError_t factor_and_forward<double>(double*, double*, double*, const uint8_t*, int, int, int, int, int,
-                                               hipStream_t, const double*, const double*);
 template hipError_t factor_with_forward<float>(float*, float*, float*, const uint8_t*, const uint8_t*, int, int, int,
                                                int, int, const SweepOverlap&, hipStream_t,
                                                const std::function<hipError_t(hipStream_t)>*, const float*,

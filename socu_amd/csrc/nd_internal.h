@@ -135,12 +135,11 @@ hipError_t sweep_persistent(const T* L, const T* E, T* x, const uint8_t* mask, i
 // already satisfied expire at once (for tests of the failure path).
 void set_sweep_spin_limit(int polls);
 int sweep_spin_limit();
-// Whether a plan for block size n and element size dsize uses the persistent
-// sweeps (plans with one right-hand side only): yes, they measured faster than
-// the level kernels for every block size and precision, unless the
-// environment variable SOCU_SWEEP is "level" (never) or "persistent"
-// (always, also the default).
-bool sweep_persistent_enabled(int n, int dsize);
+// Whether a plan for B systems of block size n and element size dsize uses the
+// persistent sweeps (plans with one right-hand side only); the environment
+// variable SOCU_SWEEP = "level" (never) or "persistent" (always) overrides the
+// rule.
+bool sweep_persistent_enabled(int B, int n, int dsize);
 
 // A side stream and per-level events that let the forward sweep of a
 // factor_and_solve run alongside the factor: forward step l waits for level
@@ -164,17 +163,34 @@ hipError_t factor_with_forward(T* L, T* E, T* x, const uint8_t* factor_mask, con
                                const std::function<hipError_t(hipStream_t)>* side_first = nullptr,
                                const T* Lsrc = nullptr, const T* Esrc = nullptr);
 
-// n == 32 (blocks in the storage precision): the factor levels with the
-// forward sweep of x inside the same kernels (k_node32, k_schur_small), one
-// stream, no separate sweep kernels; x then holds y for the backward sweep.
-// fused_forward_applies says whether (n, prec) takes this path;
-// factor_and_forward returns hipErrorInvalidValue otherwise.  Lsrc / Esrc as
-// for factor_level_blocked.
+// Small blocks (nd_small.hip), n <= 32: one launch per level and direction,
+// a level's tasks applying what the level below sends to them (so the levels
+// of a factor or forward sweep are enqueued from 0 up).  small_class: the
+// kernel variant of a system; small_up_tasks: workgroups of a factor level.
+constexpr int kSmallN = 32;
+constexpr int kSmallM = 32;                   // right-hand sides a factor_and_solve takes along
+constexpr int kSmallClasses = kSmallN / 2;  // 2 per multiple of 4
+hipError_t init_small_kernels();
+int small_class(int n, int m);
+int small_up_tasks(int N, int n, int m, int l);
+// Factor level l in the storage precision, with x (m <= kSmallM, or NULL) its
+// forward-sweep step.
 template <typename T>
-bool fused_forward_applies(int n, int prec);
+hipError_t small_up_level(T* L, T* E, T* x, const uint8_t* mask, int B, int N, int n, int m, int l, hipStream_t st,
+                          const T* Lsrc, const T* Esrc);
+// Every factor level, with x the forward sweep and, where small_tail_applies,
+// the backward sweep too.
+bool small_tail_applies(int B, int n, int m);
 template <typename T>
-hipError_t factor_and_forward(T* L, T* E, T* x, const uint8_t* mask, int B, int N, int n, int m, int prec,
-                              hipStream_t st, const T* Lsrc = nullptr, const T* Esrc = nullptr);
+hipError_t small_factor(T* L, T* E, T* x, const uint8_t* mask, int B, int N, int n, int m, hipStream_t st,
+                        const T* Lsrc, const T* Esrc);
+// forward_step_blocked / backward_level_blocked for n <= 32, any m.
+template <typename T>
+hipError_t small_forward_step(const T* L, const T* E, T* x, const uint8_t* mask, int B, int N, int n, int m, int step,
+                              hipStream_t st, bool update, bool apply);
+template <typename T>
+hipError_t small_backward_level(const T* L, const T* E, T* x, const uint8_t* mask, int B, int N, int n, int m,
+                                int lidx, hipStream_t st);
 
 // Mixed-precision factor_and_solve with FP64 refinement (nd_refine.hip).
 struct MixedPlan {

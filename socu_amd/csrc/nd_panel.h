@@ -148,14 +148,19 @@ constexpr PanelPlan panel_plan(int total) {
 // entries c <= lane % 16 hold that row of L (the others are not meaningful;
 // what the tile's strict upper triangle holds on entry is not used either).
 // p[j]: NP payload rows per lane, p[j] <- p[j] L^-T.
+// NC: columns of the panel (a tile whose last 16 - NC rows and columns are
+// identity padding needs no steps for them; entries from NC on are untouched).
 // All 64 lanes must be active.  hook(k) runs before step k.
 //
 // Step k's multiply-adds other than the one that gives the next pivot are
 // spread between the dependent operations of the next pivot's reciprocal
 // square root (left to itself the compiler moves each one down to the first
 // use of its result, and the chain then waits out every latency).
-template <typename T, int NP, typename Hook>
-__device__ __forceinline__ void panel16(T (&u)[16], T (&p)[NP][16], Hook hook) {
+struct NoHook {
+  __device__ __forceinline__ void operator()(int) const {}
+};
+template <typename T, int NP, int NC = 16, typename Hook = NoHook>
+__device__ __forceinline__ void panel16(T (&u)[16], T (&p)[NP][16], Hook hook = Hook()) {
   wait_states<2>();
   T inv = rsqrt_filled(bcast_row<0>(u[0]), [](auto) {});
   T lk = u[0] * inv, pk[NP];
@@ -163,17 +168,17 @@ __device__ __forceinline__ void panel16(T (&u)[16], T (&p)[NP][16], Hook hook) {
   for (int j = 0; j < NP; ++j) pk[j] = p[j][0] * inv;
   __builtin_amdgcn_sched_barrier(0);
   wait_states<2>();
-  static_for<16>([&](auto kc) {
+  static_for<NC>([&](auto kc) {
     constexpr int k = decltype(kc)::value;
     hook(k);
     u[k] = lk;  // row k itself: piv / sqrt(piv)
 #pragma unroll
     for (int j = 0; j < NP; ++j) p[j][k] = pk[j];
-    if constexpr (k + 1 < 16) {
+    if constexpr (k + 1 < NC) {
       fnma_row<k + 1>(u[k + 1], lk, lk);
       // the updates left: payload entry k + 1 of each set (the next step
-      // multiplies it), then u[k+2..15], then the rest of the payload
-      constexpr int nu = 14 - k, total = NP + nu + NP * nu;
+      // multiplies it), then u[k+2..], then the rest of the payload
+      constexpr int nu = NC - 2 - k, total = NP + nu + NP * nu;
       constexpr PanelPlan plan = panel_plan(total);
       auto place = [&](auto pc) {
         constexpr int b = plan.begin[decltype(pc)::value], n = plan.begin[decltype(pc)::value + 1] - b;

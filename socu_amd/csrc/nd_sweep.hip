@@ -566,19 +566,19 @@ hipError_t init_sweep_kernels() {
   return sweep_occupancy<double, 4>(g_sweep_occ[1][3]);
 }
 
-// Measured on MI355X (solve of one right-hand side after the factor, N=512):
-// the persistent upper-level launch beats the level kernels for FP32 blocks
-// with n > 96 (205 vs 208 us per solve, and a converged refinement iteration
-// costs two launches instead of ~40), but loses for smaller blocks and for
-// FP64 (n=64 FP32: 275 vs 133 us; n=128 FP64: 379 vs 339 us): a dependency
-// hop between workgroups costs about as much as a dependent kernel launch.
-bool sweep_persistent_enabled(int n, int dsize) {
+// One launch against one per level and direction: at n > 32 the persistent
+// sweeps are faster for every batch (see sweep_lmin).  At n <= 32 the level
+// kernels are one wavefront per node and their launches 3-4 us: FP64 solves
+// with N=100, persistent / level kernels, n=32: B=1 71.5 / 76.5 us, B=4 81.0 /
+// 87.1, B=16 103.9 / 102.5, B=64 203 / 196; n=20: B=16 86.6 / 80.8; 256 systems
+// of n=20 N=61 (FP32 factor_and_solve) 165 / 157.
+bool sweep_persistent_enabled(int B, int n, int dsize) {
   if (n > kMaxN) return false;  // its node tasks hold whole blocks in LDS
   const char* v = getenv("SOCU_SWEEP");
   if (v != nullptr && strcmp(v, "level") == 0) return false;
   if (v != nullptr && strcmp(v, "persistent") == 0) return true;
   (void)dsize;
-  return true;  // faster than the level kernels for every block size measured (see sweep_lmin)
+  return n > kSmallN || B <= 8;
 }
 
 size_t sweep_ws_ints(int B, int N) { return (size_t)kSweepHeader + 3 * (size_t)B * N; }

@@ -223,9 +223,6 @@ __device__ __forceinline__ void acc16_foreach(typename Mfma<T>::acc_t& acc, F f)
 // in S, and g = 3 repeats U_12 to store it in ut.
 // hook(k) runs before pivot step k (a compile-time constant after unrolling):
 // a caller can issue loads there.
-struct NoHook {
-  __device__ __forceinline__ void operator()(int) const {}
-};
 template <typename T, typename Hook = NoHook>
 __device__ __forceinline__ void tile_chol_inv(T* S, int pitch, T* dinv, T* ut, Hook hook = Hook()) {
   const int lane = lane_id();
