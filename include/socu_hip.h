@@ -241,22 +241,17 @@ int socu_profile_op(int op, void* L, void* E, void* x, const unsigned char* mask
  * entry are ignored, as in socu_cholesky_factor), and x
  * (N,n,m) (ignored for SOCU_OP_FACTOR); `reserved` must be 0.  Needs
  * n <= socu_batched_max_block_size() and m <= 32.  mask is NULL or `count`
- * bytes indexed like `systems`.  One workgroup per system walks all its
- * levels.  Systems fall in size buckets by max(n, m) (<= 8, <= 16, <= 32);
- * each bucket is one launch, with a tile size of at least its bound and
- * workgroups of 1, 2 or 4 wavefronts, the launches on forked streams.  With
- * `tune` the create call times every admissible (tile size, wavefronts) per
- * bucket on a device copy of the batch (the caller's arrays are only read)
- * and keeps the fastest (times within 2% of it are ties, settled for the
- * more wavefronts); results are cached per process and, if the
- * environment variable SOCU_TUNE_CACHE names a file, appended there and
- * reused by later processes.  Without `tune` each bucket uses its own bound
- * and two wavefronts (or the count in the environment variable
- * SOCU_BATCHED_WAVES: 1, 2 or 4), fewer where the LDS does not fit.  create
- * copies the system table to the device and
- * synchronises; execute allocates nothing and synchronises nothing.
- * socu_batched_config returns per bucket the system count, tile size and
- * wavefronts per workgroup. */
+ * bytes indexed like `systems`.  The systems run together, one launch per
+ * dissection level, direction and group of systems with one ceil(n / 4), the
+ * groups on forked streams.  `tune` is accepted and has nothing to choose.
+ * Without `tune`, the environment variable SOCU_BATCHED_WAVES = 1, 2 or 4
+ * runs one workgroup of so many wavefronts per system instead (fewer where
+ * its LDS does not fit), for comparison.  create builds the task lists,
+ * copies them and the system table to the device and synchronises; execute
+ * allocates nothing and synchronises nothing.  socu_batched_config returns
+ * per size bucket (max(n, m) <= 8, <= 16, <= 32) the system count, the tile
+ * size and the wavefronts that work on one node (or, with
+ * SOCU_BATCHED_WAVES, per workgroup). */
 typedef struct socu_batch_system {
   void* L;
   void* E;

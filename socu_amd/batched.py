@@ -74,8 +74,8 @@ class BatchedLaunch:
 
     def config(self) -> dict:
         """Per size bucket (max(n, m) <= 8, 16, 32): the number of systems, the
-        tile size and the wavefronts per workgroup they run with (as chosen
-        by the autotuner when enabled)."""
+        tile size and the wavefronts that work on one node (with
+        SOCU_BATCHED_WAVES: per workgroup)."""
         counts = (ctypes.c_int * 3)()
         tiles = (ctypes.c_int * 3)()
         waves = (ctypes.c_int * 3)()
@@ -103,11 +103,10 @@ def create_batched_cholesky_launch(L: Sequence[torch.Tensor], E: Sequence[torch.
 
     ``mask`` is a bool tensor with one entry per system; a False entry leaves
     that system untouched, as in the reference's mask (README.md:214-235).
-    ``tune`` times every admissible tile size (8, 16, 32, at least the
-    bucket's bound) and workgroup size (1, 2 or 4 wavefronts) for each size
-    bucket on a device copy of the batch when the launch is created and keeps
-    the fastest (cached per process, and in the file named by
-    SOCU_TUNE_CACHE).
+    Every level of all systems with one ceil(n / 4) is one launch.  ``tune`` is
+    accepted and has nothing to choose; with ``tune=False`` the environment
+    variable SOCU_BATCHED_WAVES (1, 2 or 4) runs one workgroup of so many
+    wavefronts per system instead.
     """
     if op not in _OPS:
         raise ValueError(f"unknown op {op!r}; expected one of {sorted(_OPS)}")

@@ -9,7 +9,6 @@
 #include <string.h>
 
 #include <algorithm>
-#include <map>
 #include <mutex>
 #include <stdlib.h>
 #include <string>
@@ -816,43 +815,19 @@ namespace {
 
 constexpr int kClasses = 3;  // tile classes NT = 8, 16, 32
 
-// Process-wide tuning results: key -> chosen (tile class, wavefronts) coded
-// as 8 * waves + class.  Optionally persisted in the file named by
-// SOCU_TUNE_CACHE ("key code" per line).
-std::mutex g_tune_mu;
-std::map<std::string, int> g_tune;
-bool g_tune_loaded = false;
-
-void tune_cache_load() {
-  if (g_tune_loaded) return;
-  g_tune_loaded = true;
-  const char* path = getenv("SOCU_TUNE_CACHE");
-  if (path == nullptr || *path == 0) return;
-  FILE* f = fopen(path, "r");
-  if (f == nullptr) return;
-  char key[256];
-  int c = 0;
-  while (fscanf(f, "%255s %d", key, &c) == 2)
-    if (c >= 0 && (c & 7) < kClasses && ((c >> 3) == 1 || (c >> 3) == 2 || (c >> 3) == 4)) g_tune[key] = c;
-  fclose(f);
-}
-
-void tune_cache_store(const std::string& key, int c) {
-  g_tune[key] = c;
-  const char* path = getenv("SOCU_TUNE_CACHE");
-  if (path == nullptr || *path == 0) return;
-  FILE* f = fopen(path, "a");
-  if (f == nullptr) return;
-  fprintf(f, "%s %d\n", key.c_str(), c);
-  fclose(f);
-}
+// streams a batched plan's launches are spread over (the caller's and side
+// streams; as many as there are hardware queues)
+constexpr int kBatchStreams = 4;
 
 }  // namespace
 
-// Systems are grouped in size buckets b (max(n, m) <= 8, 16, 32); bucket b
-// runs as one launch with tile class tile[b] >= b and workgroups of
-// waves[b] wavefronts.
+// A plan runs level launches over all systems (`levels`).  Untuned plans made
+// with SOCU_BATCHED_WAVES set run one workgroup per system instead: systems
+// are grouped in size buckets b (max(n, m) <= 8, 16, 32), one launch each with
+// tile class tile[b] and workgroups of waves[b] wavefronts.  (With level
+// launches waves[b] is the wavefronts of a node task.)
 struct socu_batched {
+  socu::SmallBatch* levels = nullptr;
   int op = 0, dtype = 0, count = 0;
   const unsigned char* mask = nullptr;
   socu::BatchProblem* dprobs = nullptr;  // device copy of the system table
@@ -862,15 +837,15 @@ struct socu_batched {
   std::vector<long long> cost;           // per system
   std::vector<int> mrhs;                 // per system
   int tile[kClasses] = {0, 1, 2};
-  int waves[kClasses] = {1, 1, 1};
+  int waves[kClasses] = {1, 1, 2};
   int counts[kClasses] = {0, 0, 0};  // per bucket
   int starts[kClasses] = {0, 0, 0};
   int mmax[kClasses] = {1, 1, 1};
   long long bcost[kClasses] = {0, 0, 0};
   int launch_order[kClasses] = {2, 1, 0};  // buckets by decreasing total cost
-  hipStream_t side[kClasses - 1] = {nullptr, nullptr};
+  hipStream_t side[kBatchStreams - 1] = {};
   hipEvent_t fork = nullptr;
-  hipEvent_t join[kClasses - 1] = {nullptr, nullptr};
+  hipEvent_t join[kBatchStreams - 1] = {};
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
 };
@@ -881,11 +856,12 @@ void batched_release(socu_batched* h) {
   if (h == nullptr) return;
   if (h->exec) (void)hipGraphExecDestroy(h->exec);
   if (h->graph) (void)hipGraphDestroy(h->graph);
-  for (int k = 0; k < kClasses - 1; ++k) {
+  for (int k = 0; k < kBatchStreams - 1; ++k) {
     if (h->join[k]) (void)hipEventDestroy(h->join[k]);
     if (h->side[k]) (void)hipStreamDestroy(h->side[k]);
   }
   if (h->fork) (void)hipEventDestroy(h->fork);
+  socu::small_batch_free(h->levels);
   if (h->dprobs) (void)hipFree(h->dprobs);
   if (h->dorder) (void)hipFree(h->dorder);
   delete h;
@@ -917,12 +893,31 @@ int batched_layout(socu_batched* h) {
   return SOCU_OK;
 }
 
-// Launches every non-empty class: the costliest on st, the others on side
-// streams forked from and joined back into st, so their workgroups fill the
-// machine together.
-int batched_enqueue(socu_batched* h, const unsigned char* mask, hipStream_t st,
-                    const socu::BatchProblem* probs = nullptr) {
-  if (probs == nullptr) probs = h->dprobs;
+// The launches of st and of side streams forked from and joined back into it,
+// so that narrow launches of different systems fill the machine together.
+int batched_enqueue_levels(socu_batched* h, const unsigned char* mask, hipStream_t st) {
+  hipError_t e = hipSuccess;
+  bool forked = false;
+  for (int k = 1; k < kBatchStreams && e == hipSuccess; ++k) {
+    if (!socu::small_batch_uses(h->levels, k)) continue;
+    if (!forked) e = hipEventRecord(h->fork, st);
+    forked = true;
+    if (e == hipSuccess) e = hipStreamWaitEvent(h->side[k - 1], h->fork, 0);
+    if (e == hipSuccess)
+      e = socu::small_batch_enqueue(h->levels, h->dprobs, mask, h->op, h->dtype, k, h->side[k - 1]);
+    if (e == hipSuccess) e = hipEventRecord(h->join[k - 1], h->side[k - 1]);
+  }
+  if (e == hipSuccess) e = socu::small_batch_enqueue(h->levels, h->dprobs, mask, h->op, h->dtype, 0, st);
+  for (int k = 1; k < kBatchStreams && e == hipSuccess; ++k)
+    if (socu::small_batch_uses(h->levels, k)) e = hipStreamWaitEvent(st, h->join[k - 1], 0);
+  return e == hipSuccess ? SOCU_OK : hip_fail(e, "batched launch");
+}
+
+// One workgroup per system: launches every non-empty class, the costliest on
+// st, the others on the side streams.
+int batched_enqueue(socu_batched* h, const unsigned char* mask, hipStream_t st) {
+  if (h->levels != nullptr) return batched_enqueue_levels(h, mask, st);
+  const socu::BatchProblem* probs = h->dprobs;
   int first = -1, nside = 0;
   hipError_t e = hipSuccess;
   for (int q = 0; q < kClasses && e == hipSuccess; ++q) {
@@ -946,123 +941,6 @@ int batched_enqueue(socu_batched* h, const unsigned char* mask, hipStream_t st,
   for (int k = 0; k < nside && e == hipSuccess; ++k) e = hipStreamWaitEvent(st, h->join[k], 0);
   if (e != hipSuccess) return hip_fail(e, "batched launch");
   return SOCU_OK;
-}
-
-// For each size bucket, times every admissible (tile class >= the bucket's
-// own, wavefronts 1, 2 or 4) on a device copy of the batch and keeps the
-// fastest, near-ties going to the wider workgroup.  The caller's arrays are
-// only read.  Needs batched_layout first.
-int batched_tune(socu_batched* h, const std::vector<socu::BatchProblem>& probs) {
-  std::lock_guard<std::mutex> lock(g_tune_mu);
-  tune_cache_load();
-  std::string keys[kClasses];
-  bool need = false;
-  for (int b = 0; b < kClasses; ++b) {
-    if (h->counts[b] == 0) continue;
-    char buf[160];
-    snprintf(buf, sizeof buf, "batched4:%s:op%d:bucket%d:count%d:cost%lld", h->dtype == SOCU_DTYPE_F64 ? "f64" : "f32",
-             h->op, b, h->counts[b], h->bcost[b]);
-    keys[b] = buf;
-    auto it = g_tune.find(keys[b]);
-    if (it != g_tune.end() && (it->second & 7) >= b &&
-        socu::batched_fits(it->second & 7, it->second >> 3, h->mmax[b], h->dtype)) {
-      h->tile[b] = it->second & 7;
-      h->waves[b] = it->second >> 3;
-    } else {
-      need = true;
-    }
-  }
-  if (!need) return SOCU_OK;
-  const size_t es = h->dtype == SOCU_DTYPE_F64 ? sizeof(double) : sizeof(float);
-  std::vector<socu::BatchProblem> copy(probs);
-  size_t total = 0;
-  std::vector<size_t> offs(probs.size());
-  for (size_t k = 0; k < probs.size(); ++k) {
-    const auto& P = probs[k];
-    const size_t nn = (size_t)P.n * P.n;
-    offs[k] = total;
-    total += ((size_t)P.N * nn + (size_t)socu::off_diag_storage_len(P.N) * nn + (size_t)P.N * P.n * P.m) * es;
-    total = (total + 255) & ~(size_t)255;
-  }
-  char* arena = nullptr;
-  socu::BatchProblem* dcopy = nullptr;
-  hipStream_t ts = nullptr;
-  hipEvent_t e0 = nullptr, e1 = nullptr;
-  int rc = SOCU_OK;
-  hipError_t e = hipMalloc(&arena, total);
-  if (e == hipSuccess) {
-    for (size_t k = 0; k < probs.size(); ++k) {
-      const auto& P = probs[k];
-      const size_t nn = (size_t)P.n * P.n;
-      char* base = arena + offs[k];
-      copy[k].L = base;
-      copy[k].E = base + (size_t)P.N * nn * es;
-      copy[k].x = (P.x != nullptr) ? base + ((size_t)P.N * nn + (size_t)socu::off_diag_storage_len(P.N) * nn) * es
-                                   : nullptr;
-    }
-    e = hipMalloc(&dcopy, copy.size() * sizeof(socu::BatchProblem));
-  }
-  if (e == hipSuccess) e = hipMemcpy(dcopy, copy.data(), copy.size() * sizeof(socu::BatchProblem), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipStreamCreateWithFlags(&ts, hipStreamNonBlocking);
-  if (e == hipSuccess) e = hipEventCreate(&e0);
-  if (e == hipSuccess) e = hipEventCreate(&e1);
-  for (int b = 0; b < kClasses && e == hipSuccess; ++b) {
-    if (h->counts[b] == 0 ||
-        (g_tune.count(keys[b]) && (g_tune[keys[b]] & 7) >= b &&
-         socu::batched_fits(g_tune[keys[b]] & 7, g_tune[keys[b]] >> 3, h->mmax[b], h->dtype)))
-      continue;
-    struct Cand {
-      int c, w;
-      float ms;
-    };
-    std::vector<Cand> cands;
-    for (int c = b; c < kClasses && e == hipSuccess; ++c) {
-      for (int w : {1, 2, 4}) {
-        if (!socu::batched_fits(c, w, h->mmax[b], h->dtype)) continue;
-        cands.push_back({c, w, 1e30f});
-        for (int rep = 0; rep < 2 && e == hipSuccess; ++rep) {
-          e = socu::batched_copy(h->dprobs, dcopy, h->count, h->op, h->dtype, ts);
-          if (e == hipSuccess) e = hipEventRecord(e0, ts);
-          if (e == hipSuccess)
-            e = socu::batched_launch_class(dcopy, h->dorder + h->starts[b], c, h->counts[b], h->mmax[b], w, nullptr,
-                                           h->op, h->dtype, ts);
-          if (e == hipSuccess) e = hipEventRecord(e1, ts);
-          if (e == hipSuccess) e = hipEventSynchronize(e1);
-          float ms = 0.f;
-          if (e == hipSuccess) e = hipEventElapsedTime(&ms, e0, e1);
-          if (e == hipSuccess && ms < cands.back().ms) cands.back().ms = ms;
-        }
-      }
-    }
-    // Isolated times within kTuneTie of the fastest are ties, settled for
-    // the most wavefronts per system: a wider workgroup runs more of a
-    // system's tasks at once, which shortens the bucket's tail when the
-    // buckets share the GPU in the real launch (measured on the 4096-system
-    // MPC batch: the isolated picks of one and two wavefronts differ by 1-2%,
-    // and two wavefronts for the large buckets make the whole batch 3-5%
-    // faster).
-    if (e == hipSuccess && !cands.empty()) {
-      constexpr float kTuneTie = 0.02f;
-      float tmin = 1e30f;
-      for (const Cand& k : cands) tmin = std::min(tmin, k.ms);
-      const Cand* pick = nullptr;
-      for (const Cand& k : cands)
-        if (k.ms <= tmin * (1.f + kTuneTie) && (pick == nullptr || k.w > pick->w || (k.w == pick->w && k.ms < pick->ms)))
-          pick = &k;
-      h->tile[b] = pick->c;
-      h->waves[b] = pick->w;
-    }
-  }
-  if (e == hipSuccess)
-    for (int b = 0; b < kClasses; ++b)
-      if (h->counts[b] > 0) tune_cache_store(keys[b], 8 * h->waves[b] + h->tile[b]);
-  if (e != hipSuccess) rc = hip_fail(e, "batched autotune");
-  if (e0) (void)hipEventDestroy(e0);
-  if (e1) (void)hipEventDestroy(e1);
-  if (ts) (void)hipStreamDestroy(ts);
-  if (dcopy) (void)hipFree(dcopy);
-  if (arena) (void)hipFree(arena);
-  return rc;
 }
 
 }  // namespace
@@ -1121,7 +999,7 @@ int socu_batched_create(socu_batched** out, int op, const socu_batch_system* sys
   hipError_t e = hipMalloc(&h->dprobs, count * sizeof(socu::BatchProblem));
   if (e == hipSuccess) e = hipMalloc(&h->dorder, count * sizeof(int));
   if (e == hipSuccess) e = hipMemcpy(h->dprobs, probs.data(), count * sizeof(socu::BatchProblem), hipMemcpyHostToDevice);
-  for (int k = 0; k < kClasses - 1 && e == hipSuccess; ++k) {
+  for (int k = 0; k < kBatchStreams - 1 && e == hipSuccess; ++k) {
     e = hipStreamCreateWithFlags(&h->side[k], hipStreamNonBlocking);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&h->join[k], hipEventDisableTiming);
   }
@@ -1131,23 +1009,22 @@ int socu_batched_create(socu_batched** out, int op, const socu_batch_system* sys
     return hip_fail(e, "batched plan set-up");
   }
   rc = batched_layout(h);
-  if (rc == SOCU_OK && !tune) {
-    // SOCU_BATCHED_WAVES=1|2|4 sets the wavefronts per workgroup of an
-    // untuned plan (every variant of the kernels can then be run on purpose),
-    // narrowed where its LDS does not fit the bucket's right-hand sides.
-    // Default 2: two of a system's tasks at a time, the tuner's usual pick
-    // for the 16- and 32-wide buckets (4096-system MPC batch: 10.57 ms
-    // against 10.7-10.8 ms with one wavefront)
-    const char* w = getenv("SOCU_BATCHED_WAVES");
-    const int wv = w ? atoi(w) : 2;
-    if (wv == 1 || wv == 2 || wv == 4)
-      for (int b = 0; b < kClasses; ++b) {
-        int v = wv;
-        while (v > 1 && !socu::batched_fits(h->tile[b], v, h->mmax[b], h->dtype)) v /= 2;
-        h->waves[b] = v;
-      }
+  // Level launches leave nothing to choose by timing: `tune` is accepted and
+  // does not change the plan.  For an untuned plan SOCU_BATCHED_WAVES=1|2|4
+  // asks for one workgroup of so many wavefronts per system, narrowed where
+  // its LDS does not fit the bucket's right-hand sides.
+  const char* w = tune ? nullptr : getenv("SOCU_BATCHED_WAVES");
+  const int wv = w ? atoi(w) : 0;
+  if (rc == SOCU_OK && (wv == 1 || wv == 2 || wv == 4)) {
+    for (int b = 0; b < kClasses; ++b) {
+      int v = wv;
+      while (v > 1 && !socu::batched_fits(h->tile[b], v, h->mmax[b], h->dtype)) v /= 2;
+      h->waves[b] = v;
+    }
+  } else if (rc == SOCU_OK) {
+    e = socu::small_batch_create(&h->levels, probs.data(), count, op, kBatchStreams);
+    if (e != hipSuccess) rc = hip_fail(e, "batched plan set-up (levels)");
   }
-  if (rc == SOCU_OK && tune) rc = batched_tune(h, probs);
   if (rc) {
     batched_release(h);
     return rc;

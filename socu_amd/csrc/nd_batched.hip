@@ -28,7 +28,8 @@
 // runs one or more tasks at once (BShape); block products run on MFMA
 // (16x16 tiles, NT >= 16) or, for NT = 8, as 2x2 register blocks per lane.
 // Small workgroups (W = 1) let several systems share a compute unit, one per
-// SIMD; the tuner picks W per size bucket.
+// SIMD.  Plans run level launches over all systems (nd_small.hip) unless
+// SOCU_BATCHED_WAVES asks for this kernel.
 #include "../../include/socu_hip.h"
 #include "nd_common.h"
 #include "nd_internal.h"
@@ -607,20 +608,6 @@ void launch_nt(const BatchProblem* dprobs, const int* dorder, int count, int mma
   }
 }
 
-// Copies every system's L, E and x from src to dst (same shapes); one
-// workgroup per system.
-template <typename T>
-__global__ __launch_bounds__(256) void k_copy_systems(const BatchProblem* __restrict__ src,
-                                                      const BatchProblem* __restrict__ dst, int op) {
-  const BatchProblem a = src[blockIdx.x], b = dst[blockIdx.x];
-  const size_t nn = (size_t)a.n * a.n;
-  const size_t nL = (size_t)a.N * nn, nE = (size_t)off_diag_storage_len(a.N) * nn;
-  const size_t nx = (op == SOCU_OP_FACTOR) ? 0 : (size_t)a.N * a.n * a.m;
-  for (size_t k = threadIdx.x; k < nL; k += blockDim.x) static_cast<T*>(b.L)[k] = static_cast<const T*>(a.L)[k];
-  for (size_t k = threadIdx.x; k < nE; k += blockDim.x) static_cast<T*>(b.E)[k] = static_cast<const T*>(a.E)[k];
-  for (size_t k = threadIdx.x; k < nx; k += blockDim.x) static_cast<T*>(b.x)[k] = static_cast<const T*>(a.x)[k];
-}
-
 }  // namespace
 
 hipError_t init_batched_kernels() {
@@ -656,16 +643,6 @@ hipError_t batched_launch_class(const BatchProblem* dprobs, const int* dorder, i
     else if (cls == 1) launch_nt<float, 16>(dprobs, dorder, count, mmax, waves, mask, op, st);
     else launch_nt<float, 32>(dprobs, dorder, count, mmax, waves, mask, op, st);
   }
-  return hipGetLastError();
-}
-
-hipError_t batched_copy(const BatchProblem* dsrc, const BatchProblem* ddst, int count, int op, int dtype,
-                        hipStream_t st) {
-  if (count <= 0) return hipSuccess;
-  if (dtype == SOCU_DTYPE_F64)
-    hipLaunchKernelGGL(k_copy_systems<double>, dim3(count), dim3(256), 0, st, dsrc, ddst, op);
-  else
-    hipLaunchKernelGGL(k_copy_systems<float>, dim3(count), dim3(256), 0, st, dsrc, ddst, op);
   return hipGetLastError();
 }
 

@@ -232,6 +232,17 @@ struct BatchProblem {
   void* x;  // (N, n, m), may be NULL for a factor
   int N, n, m, pad;
 };
+// Level launches over uneven systems (nd_small.hip), n, m <= 32: a plan made
+// from the host's table for one operation, its groups of systems spread over
+// `streams` streams; enqueue adds what runs on stream number `stream` of them
+// (small_batch_uses: anything) to st.
+struct SmallBatch;
+hipError_t small_batch_create(SmallBatch** out, const BatchProblem* probs, int count, int op, int streams);
+void small_batch_free(SmallBatch* b);
+bool small_batch_uses(const SmallBatch* b, int stream);
+hipError_t small_batch_enqueue(const SmallBatch* b, const BatchProblem* dprobs, const uint8_t* mask, int op, int dtype,
+                               int stream, hipStream_t st);
+// One workgroup per system (nd_batched.hip).
 hipError_t init_batched_kernels();
 // Tile class of a block size: 0 (tiles of 8), 1 (16), 2 (32).
 int batched_class(int n);
@@ -242,9 +253,6 @@ int batched_class(int n);
 bool batched_fits(int cls, int waves, int mmax, int dtype);
 hipError_t batched_launch_class(const BatchProblem* dprobs, const int* dorder, int cls, int count, int mmax, int waves,
                                 const uint8_t* mask, int op, int dtype, hipStream_t st);
-// Copies L, E (and x unless op is a factor) of count systems src[k] -> dst[k].
-hipError_t batched_copy(const BatchProblem* dsrc, const BatchProblem* ddst, int count, int op, int dtype,
-                        hipStream_t st);
 size_t mixed_residual_lds(int n, int m);
 bool mixed_fits(int n, int m);
 hipError_t mixed_alloc(MixedPlan& p);

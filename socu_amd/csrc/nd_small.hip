@@ -37,6 +37,7 @@
 // 32-bit offsets from a scalar base and no branch per element: with generic
 // pointers and selected loads the n=20 FP32 task took 17 us instead of 6.
 #include <algorithm>
+#include <vector>
 
 #include "../../include/socu_hip.h"
 #include "nd_common.h"
@@ -1030,6 +1031,140 @@ hipError_t small_backward_level(const T* L, const T* E, T* x, const uint8_t* mas
                  lidx, st);
   kt_end(kKcBackward, st);
   return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// Uneven systems: the same kernels, a launch per level and group of systems
+// with one ceil(n / 4), over a list of (system, task) pairs.  (One workgroup
+// per system walking its levels leaves the chip idle behind the long systems
+// and runs the wide levels of each a few tasks at a time.  FP64
+// factor_and_solve of systems of N = 10..200, n = 8..32, the inputs copied in
+// first, one workgroup per system / level launches: 4096 systems 12.8 / 6.0 ms,
+// 32 systems without a graph 1.92 / 0.32 ms; 512 systems in FP32 2.26 / 0.47 ms.)
+// ---------------------------------------------------------------------------
+struct SmallBatch {
+  struct Level {
+    int up = 0, up_count = 0;            // factor: nodes, then targets
+    int fwd = 0, fwd_count = 0, nodes = 0;  // sweeps: nodes, then targets (one per task)
+  };
+  struct Group {
+    int cls = 0, mmax = 0, stream = 0;
+    std::vector<Level> levels;
+  };
+  std::vector<Group> groups;  // by decreasing cost
+  int2* tasks = nullptr;      // device
+};
+
+void small_batch_free(SmallBatch* b) {
+  if (b == nullptr) return;
+  if (b->tasks) (void)hipFree(b->tasks);
+  delete b;
+}
+
+hipError_t small_batch_create(SmallBatch** out, const BatchProblem* probs, int count, int op, int streams) {
+  *out = nullptr;
+  const bool fac = op == SOCU_OP_FACTOR || op == SOCU_OP_FACTOR_AND_SOLVE;
+  const bool solve = op != SOCU_OP_FACTOR;
+  SmallBatch* h = new SmallBatch();
+  std::vector<int> of[kSmallN / 4];
+  double cost[kSmallN / 4] = {};
+  for (int k = 0; k < count; ++k) {
+    const BatchProblem& P = probs[k];
+    const int k4 = small_class(P.n, fac && solve ? P.m : 0) / 2;
+    of[k4].push_back(k);
+    cost[k4] += (double)P.N * P.n * P.n;
+  }
+  std::vector<int> by;
+  for (int k4 = 0; k4 < kSmallN / 4; ++k4)
+    if (!of[k4].empty()) by.push_back(k4);
+  std::stable_sort(by.begin(), by.end(), [&](int x, int y) { return cost[x] > cost[y]; });
+  std::vector<double> load(streams, 0.0);
+  std::vector<int2> tasks;
+  for (int k4 : by) {
+    SmallBatch::Group G;
+    std::vector<int>& sys = of[k4];
+    std::stable_sort(sys.begin(), sys.end(), [&](int x, int y) { return probs[x].N > probs[y].N; });
+    bool exact = true;
+    for (int k : sys) {
+      exact = exact && probs[k].n == 4 * (k4 + 1);
+      if (solve) G.mmax = std::max(G.mmax, probs[k].m);
+    }
+    G.cls = 2 * k4 + (exact ? 1 : 0);
+    G.stream = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+    load[G.stream] += cost[k4];
+    const int per = G.cls < 2 * 4 ? 1 : 2;  // targets per factor task
+    const int Lv = recursive_iterations(probs[sys[0]].N);
+    for (int l = 0; l < Lv; ++l) {
+      SmallBatch::Level V;
+      const int s = 1 << l;
+      V.up = V.fwd = (int)tasks.size();
+      for (int k : sys)
+        for (int t = 0, dim = (probs[k].N + s) / (2 * s); t < dim; ++t) tasks.push_back({k, t});
+      V.nodes = (int)tasks.size() - V.up;
+      auto targets = [&](int each) {
+        if (l > 0)
+          for (int k : sys) {
+            const int dim = (probs[k].N + s) / (2 * s);
+            for (int u = 0; u * each < probs[k].N / (2 * s); ++u) tasks.push_back({k, dim + u});
+          }
+      };
+      if (fac) {
+        targets(per);
+        V.up_count = (int)tasks.size() - V.up;
+      } else {
+        targets(1);
+        V.fwd_count = (int)tasks.size() - V.fwd;
+      }
+      G.levels.push_back(V);
+    }
+    h->groups.push_back(std::move(G));
+  }
+  hipError_t e = hipMalloc(&h->tasks, std::max<size_t>(1, tasks.size()) * sizeof(int2));
+  if (e == hipSuccess) e = hipMemcpy(h->tasks, tasks.data(), tasks.size() * sizeof(int2), hipMemcpyHostToDevice);
+  if (e != hipSuccess) {
+    small_batch_free(h);
+    return e;
+  }
+  *out = h;
+  return hipSuccess;
+}
+
+bool small_batch_uses(const SmallBatch* h, int stream) {
+  for (const auto& G : h->groups)
+    if (G.stream == stream) return true;
+  return false;
+}
+
+template <typename T>
+static hipError_t batch_enqueue(const SmallBatch* h, const BatchProblem* probs, const uint8_t* mask, int op, int stream,
+                                hipStream_t st) {
+  const bool fac = op == SOCU_OP_FACTOR || op == SOCU_OP_FACTOR_AND_SOLVE;
+  for (const auto& G : h->groups) {
+    if (G.stream != stream) continue;
+    SmallArgs<T> A = {};
+    A.probs = probs;
+    A.mask = mask;
+    A.solve = op != SOCU_OP_FACTOR;
+    A.m = G.mmax;
+    for (size_t l = 0; l < G.levels.size(); ++l) {
+      const SmallBatch::Level& V = G.levels[l];
+      A.tasks = h->tasks + V.up;
+      if (fac) launch_up<T>(G.cls, dim3(V.up_count), A, (int)l, st);
+      else if (op != SOCU_OP_BACKWARD) launch_forward<T>(G.cls, dim3(V.fwd_count), A, (int)l, true, true, st);
+    }
+    if (op != SOCU_OP_FACTOR && op != SOCU_OP_FORWARD)
+      for (int l = (int)G.levels.size() - 1; l >= 0; --l) {
+        A.tasks = h->tasks + G.levels[l].up;
+        launch_down<T>(G.cls, dim3(G.levels[l].nodes), A, l, st);
+      }
+  }
+  return hipGetLastError();
+}
+
+hipError_t small_batch_enqueue(const SmallBatch* h, const BatchProblem* dprobs, const uint8_t* mask, int op, int dtype,
+                               int stream, hipStream_t st) {
+  return dtype == SOCU_DTYPE_F64 ? batch_enqueue<double>(h, dprobs, mask, op, stream, st)
+                                 : batch_enqueue<float>(h, dprobs, mask, op, stream, st);
 }
 
 template hipError_t small_up_level<float>(float*, float*, float*, const uint8_t*, int, int, int, int, int, hipStream_t,
