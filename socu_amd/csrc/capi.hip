@@ -147,9 +147,9 @@ int run_op(int op, void* L, void* E, void* x, const uint8_t* mask, int B, int N,
     if (e != hipSuccess) return hip_fail(e, "diagonal-block inverse launch");
     Lt = W;
   }
-  if (n <= socu::kSmallN && (op == SOCU_OP_FACTOR || op == SOCU_OP_FACTOR_AND_SOLVE)) {
+  if (n <= socu::kSmallUpN && (op == SOCU_OP_FACTOR || op == SOCU_OP_FACTOR_AND_SOLVE)) {
     const bool solve = op == SOCU_OP_FACTOR_AND_SOLVE;
-    const bool with_x = solve && m <= socu::kSmallM;  // (more right-hand sides: the sweeps follow)
+    const bool with_x = solve && m <= socu::small_max_rhs(n);  // (more right-hand sides: the sweeps follow)
     const hipError_t e = socu::small_factor<T>(Lt, Et, with_x ? xt : nullptr, mask, B, N, n, m, st, Ls, Es);
     if (e != hipSuccess) return hip_fail(e, "small-block factor launch");
     if (!solve || (with_x && socu::small_tail_applies(B, n, m))) return SOCU_OK;
@@ -189,6 +189,7 @@ int ensure_init() {
   if (e == hipSuccess) e = socu::init_sweep_kernels();
   if (e == hipSuccess) e = socu::init_large_kernels();
   if (e == hipSuccess) e = socu::init_small_kernels();
+  if (e == hipSuccess) e = socu::init_wide_kernels();
   if (e != hipSuccess) return hip_fail(e, "kernel set-up (hipFuncSetAttribute)");
   state = 1;
   return SOCU_OK;

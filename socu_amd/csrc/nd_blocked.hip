@@ -1605,23 +1605,25 @@ hipError_t factor_level_blocked(T* L, T* E, const uint8_t* mask, int B, int N, i
     return factor_level_large<T>(L, E, mask, B, N, n, lidx, st, after_potrf, after_trsm, before_trsm);
   }
   const int fp = prec;
-  if (n <= kSmallN) {
-    // blocks of n <= 32: FP32 storage with FP64 pivots or BF16 Schur products
-    // takes the separate kernels; else one launch per level (in place; the
-    // level applies the previous level's updates itself)
-    if constexpr (sizeof(T) == 4) {
-      if ((prec & (kPrecF64Pivots | kPrecBf16Schur)) != 0)
-        return n == 32 ? factor_level_nb<T, 1, 32>(L, E, mask, B, N, n, lidx, fp, st, after_potrf, after_trsm,
-                                                   before_trsm, Lsrc, Esrc)
-                       : factor_level_nb<T, 1, 0>(L, E, mask, B, N, n, lidx, fp, st, after_potrf, after_trsm,
-                                                  before_trsm, Lsrc, Esrc);
-    }
+  // small blocks in the storage precision (in place): one launch per level,
+  // which applies the previous level's updates itself.  FP32 storage with FP64
+  // pivots or BF16 Schur products takes the separate kernels.
+  const bool separate = sizeof(T) == 4 && (prec & (kPrecF64Pivots | kPrecBf16Schur)) != 0;
+  if (n <= kSmallUpN && !separate) {
     if (Lsrc != nullptr || Esrc != nullptr) return hipErrorInvalidValue;
     hipError_t e = before_trsm != nullptr ? hipStreamWaitEvent(st, before_trsm, 0) : hipSuccess;
     if (e == hipSuccess) e = small_up_level<T>(L, E, nullptr, mask, B, N, n, 0, lidx, st, nullptr, nullptr);
     if (e == hipSuccess && after_potrf != nullptr) e = hipEventRecord(after_potrf, st);
     if (e == hipSuccess && after_trsm != nullptr) e = hipEventRecord(after_trsm, st);
     return e;
+  }
+  if constexpr (sizeof(T) == 4) {
+    if (n == 32)
+      return factor_level_nb<T, 1, 32>(L, E, mask, B, N, n, lidx, fp, st, after_potrf, after_trsm, before_trsm, Lsrc,
+                                       Esrc);
+    if (n < 32)
+      return factor_level_nb<T, 1, 0>(L, E, mask, B, N, n, lidx, fp, st, after_potrf, after_trsm, before_trsm, Lsrc,
+                                      Esrc);
   }
   switch (n) {
     case 64: return factor_level_nb<T, 2, 64>(L, E, mask, B, N, n, lidx, fp, st, after_potrf, after_trsm, before_trsm, Lsrc,

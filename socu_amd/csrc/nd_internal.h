@@ -167,17 +167,25 @@ hipError_t factor_with_forward(T* L, T* E, T* x, const uint8_t* factor_mask, con
 // a level's tasks applying what the level below sends to them (so the levels
 // of a factor or forward sweep are enqueued from 0 up).  small_class: the
 // kernel variant of a system; small_up_tasks: workgroups of a factor level.
+// The factor (with the forward sweep) takes n <= kSmallUpN, above kSmallN by the
+// kernels of nd_wide.hip.
 constexpr int kSmallN = 32;
-constexpr int kSmallM = 32;                   // right-hand sides a factor_and_solve takes along
+constexpr int kSmallUpN = 64;
 constexpr int kSmallClasses = kSmallN / 2;  // 2 per multiple of 4
+// right-hand sides a factor_and_solve takes along
+constexpr int small_max_rhs(int n) { return n <= kSmallN ? 32 : 64; }
 hipError_t init_small_kernels();
+hipError_t init_wide_kernels();
 int small_class(int n, int m);
 int small_up_tasks(int N, int n, int m, int l);
-// Factor level l in the storage precision, with x (m <= kSmallM, or NULL) its
+// Factor level l in the storage precision, with x (m <= small_max_rhs, or NULL) its
 // forward-sweep step.
 template <typename T>
 hipError_t small_up_level(T* L, T* E, T* x, const uint8_t* mask, int B, int N, int n, int m, int l, hipStream_t st,
                           const T* Lsrc, const T* Esrc);
+template <typename T>
+hipError_t wide_up_level(T* L, T* E, T* x, const uint8_t* mask, int B, int N, int n, int m, int l, hipStream_t st,
+                         const T* Lsrc, const T* Esrc);
 // Every factor level, with x the forward sweep and, where small_tail_applies,
 // the backward sweep too.
 bool small_tail_applies(int B, int n, int m);

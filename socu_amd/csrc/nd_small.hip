@@ -42,39 +42,12 @@
 #include "../../include/socu_hip.h"
 #include "nd_common.h"
 #include "nd_internal.h"
+#include "nd_small.h"
 #include "nd_tile.h"
 
 namespace socu {
 
 namespace {
-
-// One system: the arrays of a task, Lin / Ein being where blocks are read
-// that no earlier level has written (the sources of an out-of-place factor).
-template <typename T>
-struct SmallSys {
-  T* L;
-  const T* Lin;
-  T* E;
-  const T* Ein;
-  T* x;
-  int N, n, m;
-};
-
-// What a launch works on: B systems of one shape (probs NULL), or a table of
-// uneven systems with a list of (system, task) pairs, one per workgroup.
-template <typename T>
-struct SmallArgs {
-  T* L;
-  const T* Lsrc;  // NULL: in place
-  T* E;
-  const T* Esrc;
-  T* x;  // NULL: factor only
-  const uint8_t* mask;
-  int N, n, m, nE;
-  const BatchProblem* probs;
-  const int2* tasks;
-  int solve;  // uneven systems: 0 ignores their x
-};
 
 // Kernel variants: K4 = ceil(n / 4).  n <= 16 NB, the last of the NB 16-column
 // panels has NC columns, and products sum over 4 K4 entries.  EX: n == 4 K4
@@ -90,27 +63,6 @@ struct SmallShape {
   static constexpr int kFixed = 3 * kTile + kZ;  // L_k, R_k, Lc_k^T, identity
   static __host__ __device__ constexpr int elems(int m) { return kFixed + m * P; }
 };
-
-// Element `off` of a block with a wave-uniform address (scalar base, 32-bit
-// vector offset).
-template <typename T>
-__device__ __forceinline__ T ldg(const T* base, int off) {
-  typedef const __attribute__((address_space(1))) char* gbytes;
-  typedef const __attribute__((address_space(1))) T* gptr;
-  return *(gptr)((gbytes)base + (unsigned)off * (unsigned)sizeof(T));
-}
-template <typename T>
-__device__ __forceinline__ void stg(T* base, int off, T v) {
-  typedef __attribute__((address_space(1))) char* gbytes;
-  typedef __attribute__((address_space(1))) T* gptr;
-  *(gptr)((gbytes)base + (unsigned)off * (unsigned)sizeof(T)) = v;
-}
-template <typename P>
-__device__ __forceinline__ P* uniform_ptr(P* p) {
-  const unsigned long long v = (unsigned long long)p;
-  const unsigned lo = __builtin_amdgcn_readfirstlane((int)v), hi = __builtin_amdgcn_readfirstlane((int)(v >> 32));
-  return (P*)(((unsigned long long)hi << 32) | lo);
-}
 
 // MFMA operands of an n x n block: [t][b] holds rows 16b + lane % 16 at
 // column 4t + lane / 16 (ROW), or the transpose: columns 16b + lane % 16 at row
@@ -233,8 +185,14 @@ struct Pull {
       typename Mfma<T>::acc_t u[NTRI];
 #pragma unroll
       for (int q = 0; q < NTRI; ++q) u[q] = acc_zero<T>();
-      if (Ra != nullptr) mma_frags<T, K4, EX, true, true, true>(u, fr, fr);
-      if (Lcc != nullptr) mma_frags<T, K4, EX, false, false, true>(u, fc, fc);
+      if (Ra != nullptr) {
+        mma_frags<T, K4, EX, true, true, true>(u, fr, fr);
+        mfma_settle<T>();
+      }
+      if (Lcc != nullptr) {
+        mma_frags<T, K4, EX, false, false, true>(u, fc, fc);
+        mfma_settle<T>();
+      }
 #pragma unroll
       for (int q = 0; q < NTRI; ++q) d[q] -= u[q];
     }
@@ -245,8 +203,14 @@ struct Pull {
     typename Mfma<T>::acc_t u[NB];
 #pragma unroll
     for (int i = 0; i < NB; ++i) u[i] = acc_zero<T>();
-    if (ra) mma_rhs<T, K4, EX, true>(u, fr, va);
-    if (lc) mma_rhs<T, K4, EX, false>(u, fc, vc);
+    if (ra) {
+      mma_rhs<T, K4, EX, true>(u, fr, va);
+      mfma_settle<T>();
+    }
+    if (lc) {
+      mma_rhs<T, K4, EX, false>(u, fc, vc);
+      mfma_settle<T>();
+    }
 #pragma unroll
     for (int i = 0; i < NB; ++i) y[i] -= u[i];
   }
@@ -333,20 +297,6 @@ __device__ __forceinline__ void rhs_to_lds(T* Y, typename Mfma<T>::acc_t (&a)[NB
       for (int r = 0; r < 4; ++r) Y[j * P + 16 * b + Mfma<T>::row(l, r)] = a[b][r];
 }
 
-template <typename T, int NP, int NC>
-__device__ __forceinline__ void run_panel(T (&u)[16], T (&p)[NP][16], const T* urow, const T* prow) {
-#pragma unroll
-  for (int c = 0; c < NC; ++c) u[c] = urow[c];
-#pragma unroll
-  for (int c = 0; c < NC; ++c) p[0][c] = prow[c];
-#pragma unroll
-  for (int c = 0; c < NC; ++c) {
-    pin_reg(u[c]);
-    pin_reg(p[0][c]);
-  }
-  panel16<T, NP, NC>(u, p);
-}
-
 // Second half of 16 rows Q (pitch P) -= X L21^T, X being their first half; b:
 // L21 as the B operand.  rows: how many exist (reads are clamped, writes
 // masked).
@@ -364,13 +314,6 @@ __device__ __forceinline__ void half_update(T* Q, int P, const T (&b)[4], int ro
 #pragma unroll
   for (int r = 0; r < 4; ++r)
     if (Mfma<T>::row(l, r) < rows) Q[Mfma<T>::row(l, r) * P + 16 + (l & 15)] = acc[r];
-}
-
-// Element offset of level l's segment of E, in blocks.
-__device__ __forceinline__ int seg_offset(int N, int l) {
-  int off = 0;
-  for (int q = 0; q < l; ++q) off += (N >> q) - 1;
-  return off;
 }
 
 // One node or target task of level l by the NB wavefronts of a task slot
@@ -653,8 +596,14 @@ __device__ __forceinline__ void forward_task(const SmallSys<T>& Q, int l, int ta
     typename Mfma<T>::acc_t u[NB];
 #pragma unroll
     for (int b = 0; b < NB; ++b) u[b] = acc_zero<T>();
-    if (upd) mma_rhs<T, K4, EX, true>(u, fr, y);
-    if (Lcc != nullptr) mma_rhs<T, K4, EX, false>(u, fc, y2);
+    if (upd) {
+      mma_rhs<T, K4, EX, true>(u, fr, y);
+      mfma_settle<T>();
+    }
+    if (Lcc != nullptr) {
+      mma_rhs<T, K4, EX, false>(u, fc, y2);
+      mfma_settle<T>();
+    }
 #pragma unroll
     for (int b = 0; b < NB; ++b) a[b] -= u[b];
     if (app) {
@@ -664,6 +613,7 @@ __device__ __forceinline__ void forward_task(const SmallSys<T>& Q, int l, int ta
 #pragma unroll
         for (int t = 0; t < min(KU, 4 * b + 4); ++t) u[b] = Mfma<T>::mma(fu[t][b], a[t / 4][t % 4], u[b]);
       }
+      mfma_settle<T>();
 #pragma unroll
       for (int b = 0; b < NB; ++b) a[b] = u[b];
     }
@@ -749,8 +699,14 @@ __device__ __forceinline__ void down_task(const SmallSys<T>& Q, int l, int t0, i
     typename Mfma<T>::acc_t u[NB], o[NB];
 #pragma unroll
     for (int b = 0; b < NB; ++b) u[b] = o[b] = acc_zero<T>();
-    if (hasR) mma_rhs<T, K4, EX, false>(u, fr, y);
-    if (hasC) mma_rhs<T, K4, EX, true>(u, fc, y2);
+    if (hasR) {
+      mma_rhs<T, K4, EX, false>(u, fr, y);
+      mfma_settle<T>();
+    }
+    if (hasC) {
+      mma_rhs<T, K4, EX, true>(u, fc, y2);
+      mfma_settle<T>();
+    }
 #pragma unroll
     for (int b = 0; b < NB; ++b) a[b] -= u[b];
 #pragma unroll
@@ -767,43 +723,6 @@ __device__ __forceinline__ void down_task(const SmallSys<T>& Q, int l, int t0, i
         }
   }
 }
-
-// The system and task of this workgroup; false: nothing to do.
-template <typename T>
-__device__ __forceinline__ bool small_sys(const SmallArgs<T>& A, SmallSys<T>& Q, int& task) {
-  if (A.probs != nullptr) {
-    const int2 st = A.tasks[blockIdx.x];
-    const int p = __builtin_amdgcn_readfirstlane(st.x);
-    if (masked_out(A.mask, p)) return false;
-    const BatchProblem P = A.probs[p];
-    Q.L = uniform_ptr(static_cast<T*>(P.L));
-    Q.E = uniform_ptr(static_cast<T*>(P.E));
-    Q.x = A.solve ? uniform_ptr(static_cast<T*>(P.x)) : nullptr;
-    Q.Lin = Q.L;
-    Q.Ein = Q.E;
-    Q.N = __builtin_amdgcn_readfirstlane(P.N);
-    Q.n = __builtin_amdgcn_readfirstlane(P.n);
-    Q.m = __builtin_amdgcn_readfirstlane(P.m);
-    task = __builtin_amdgcn_readfirstlane(st.y);
-    return true;
-  }
-  const int b = blockIdx.y;
-  if (masked_out(A.mask, b)) return false;
-  const size_t nn = (size_t)A.n * A.n, oL = (size_t)b * A.N * nn, oE = (size_t)b * A.nE * nn;
-  Q.L = A.L + oL;
-  Q.Lin = A.Lsrc != nullptr ? A.Lsrc + oL : Q.L;
-  Q.E = A.E + oE;
-  Q.Ein = A.Esrc != nullptr ? A.Esrc + oE : Q.E;
-  Q.x = A.x != nullptr ? A.x + (size_t)b * A.N * A.n * A.m : nullptr;
-  Q.N = A.N;
-  Q.n = A.n;
-  Q.m = A.m;
-  task = blockIdx.x;
-  return true;
-}
-
-// This wavefront's number, as a scalar.
-__device__ __forceinline__ int wave_uniform() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
 
 template <typename T, int K4, bool EX>
 __global__ __launch_bounds__(64 * ((K4 + 3) / 4)) void k_small_up(SmallArgs<T> A, int l) {
@@ -889,22 +808,6 @@ hipError_t set_small_attrs() {
 }
 
 template <typename T>
-SmallArgs<T> regular_args(T* L, T* E, T* x, const uint8_t* mask, int N, int n, int m, const T* Lsrc, const T* Esrc) {
-  SmallArgs<T> A = {};
-  A.L = L;
-  A.Lsrc = Lsrc;
-  A.E = E;
-  A.Esrc = Esrc;
-  A.x = x;
-  A.mask = mask;
-  A.N = N;
-  A.n = n;
-  A.m = x != nullptr ? m : 0;
-  A.nE = (int)off_diag_storage_len(N);
-  return A;
-}
-
-template <typename T>
 void launch_up(int cls, dim3 grid, const SmallArgs<T>& A, int l, hipStream_t st) {
   with_class(cls, [&](auto k4, auto ex) {
     constexpr int K4 = decltype(k4)::value;
@@ -961,6 +864,7 @@ int small_up_tasks(int N, int n, int m, int l) {
 template <typename T>
 hipError_t small_up_level(T* L, T* E, T* x, const uint8_t* mask, int B, int N, int n, int m, int l, hipStream_t st,
                           const T* Lsrc, const T* Esrc) {
+  if (n > kSmallN) return wide_up_level<T>(L, E, x, mask, B, N, n, m, l, st, Lsrc, Esrc);
   if (B <= 0) return hipSuccess;
   kt_begin(kKcPotrf, st);
   launch_up<T>(small_class(n, x != nullptr ? m : 0), dim3(small_up_tasks(N, n, x != nullptr ? m : 0, l), B),
@@ -977,13 +881,21 @@ hipError_t small_up_level(T* L, T* E, T* x, const uint8_t* mask, int B, int N, i
 // N=40 80.5 / 66.9; 2000 systems of n=4 N=30 117.8 / 154.4.  With two
 // wavefronts per task (n > 16) a compute unit holds too few tasks: n=32 N=100
 // 102 / 117.
-bool small_tail_applies(int B, int n, int m) { return small_class(n, m) < 2 * 4 && B <= kTailMaxSystems; }
+bool small_tail_applies(int B, int n, int m) {
+  return n <= kSmallN && small_class(n, m) < 2 * 4 && B <= kTailMaxSystems;
+}
 
 template <typename T>
 hipError_t small_factor(T* L, T* E, T* x, const uint8_t* mask, int B, int N, int n, int m, hipStream_t st,
                         const T* Lsrc, const T* Esrc) {
   if (B <= 0) return hipSuccess;
   const int Lv = recursive_iterations(N);
+  if (n > kSmallN) {
+    hipError_t e = hipSuccess;
+    for (int l = 0; l < Lv && e == hipSuccess; ++l)
+      e = wide_up_level<T>(L, E, x, mask, B, N, n, m, l, st, Lsrc, Esrc);
+    return e;
+  }
   const int mx = x != nullptr ? m : 0, cls = small_class(n, mx);
   const SmallArgs<T> A = regular_args(L, E, x, mask, N, n, m, Lsrc, Esrc);
   int lo = Lv;

@@ -55,6 +55,18 @@ __device__ __forceinline__ typename Mfma<T>::acc_t acc_zero() {
 // compiler from moving LDS accesses of the wave across the point.
 __device__ __forceinline__ void wave_lds_order() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
+// At the end of a conditional run of MFMAs whose results are read behind it:
+// the wait states such a read needs.  (Along a path that skips a later
+// conditional run the compiler does not always count them, and the hardware
+// does not wait by itself.)
+template <typename T>
+__device__ __forceinline__ void mfma_settle() {
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (sizeof(T) == 8) asm volatile("s_nop 15\n\ts_nop 3" ::: "memory");
+  else asm volatile("s_nop 13" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
 __device__ __forceinline__ int lane_id() { return threadIdx.x & 63; }
 __device__ __forceinline__ int wave_id() { return threadIdx.x >> 6; }
 

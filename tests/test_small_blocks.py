@@ -1,10 +1,10 @@
-"""Small blocks (n <= 32): one launch per level, one or two wavefronts per node.
+"""Small blocks: one launch per level, one, two or four wavefronts per node.
 
-Every kernel variant (one per multiple of four of n, exact and padded, one
-wavefront up to n = 16 and two above), with the narrow levels in one launch
+Every kernel variant (one per multiple of four of n up to 32, of eight up to
+64, exact and padded; one wavefront up to n = 16, two up to 32), with the narrow levels in one launch
 (at most 256 systems of n <= 16) and without, in both precisions, with the
-right-hand sides inside the factor (m <= 32), in one or more column chunks, or
-after it (m > 32), out of place, and the sweeps on their own: against the
+right-hand sides inside the factor (m <= 32, n > 32: 64), in one or more column
+chunks, or after it, out of place, and the sweeps on their own: against the
 oracle.
 """
 import numpy as np
@@ -24,7 +24,8 @@ def _rel(a, b):
 CASES = [(1, 5, 1, 1), (4, 2, 3, 2), (5, 40, 1, 1), (8, 1, 2, 1), (11, 33, 16, 2), (12, 20, 1, 1), (15, 70, 17, 1),
          (16, 64, 16, 1), (16, 3, 33, 2), (17, 20, 1, 1), (20, 61, 4, 3), (23, 7, 32, 1), (24, 100, 1, 1),
          (25, 9, 2, 2), (28, 15, 16, 1), (31, 31, 33, 1), (32, 2, 17, 1), (32, 90, 1, 2), (6, 11, 1, 300),
-         (18, 6, 2, 300)]
+         (18, 6, 2, 300), (33, 20, 1, 1), (36, 7, 17, 2), (40, 33, 3, 1), (41, 12, 64, 1), (48, 25, 16, 2), (49, 9, 1, 1),
+         (56, 16, 65, 1), (60, 40, 4, 1), (64, 31, 16, 1), (64, 2, 33, 2), (57, 1, 2, 1)]
 
 
 @pytest.mark.parametrize("dtype", ["float64", "float32"])
@@ -40,10 +41,10 @@ def test_variants_match_oracle(n, N, m, B, dtype, device):
 
     print(f"small n={n} N={N} m={m} B={B} {dtype}", flush=True)
     tdt = getattr(torch, dtype)
-    # kappa(Psi) <= 1e3 (alpha = 10, n <= 32): 1e3 * N * 2^-53, and 2^-24
+    # kappa(Psi) <= 1e3 (alpha = 10, 16 above n = 32): 1e3 * N * 2^-53, and 2^-24
     tol = 1e-11 if dtype == "float64" else 5e-4
     kinds = min(B, 3)  # distinct systems, repeated over the batch
-    P = [nd.readme_problem(n, N, m, alpha=10.0, seed=17 + k)[:3] for k in range(kinds)]
+    P = [nd.readme_problem(n, N, m, alpha=10.0 if n <= 32 else 16.0, seed=17 + k)[:3] for k in range(kinds)]
     L0, E0, b0 = (np.stack([P[k % kinds][i] for k in range(B)]) for i in range(3))
     L, E, x = (torch.tensor(a, dtype=tdt, device=device) for a in (L0, E0, b0))
     E[:, N - 1:] = 3.0  # the fill-in region's contents on entry are ignored
