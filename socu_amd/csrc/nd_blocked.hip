@@ -17,11 +17,7 @@
 //                :202-228).
 //   k_schur_blk  one workgroup per 64x64 output tile, MFMA, owner computes:
 //                L_j -= R R^T + Lc^T Lc,  F -= R Lc (syrk.py, gemm.py).
-//   k_sweep_nb, k_apply_fwd  the sweeps, one launch per step and
-//                direction: the block-times-panel update and the triangular
-//                apply with the stored inverse in one kernel (k_apply_fwd:
-//                the first forward level) (replaces K9-K16,
-//                block_tridiag_solver.py:425-736).
+// (The sweeps: nd_small.hip, nd_steps.hip, nd_large.hip.)
 #include <stdlib.h>
 
 #include <hip/hip_ext.h>
@@ -1021,304 +1017,8 @@ __global__ __launch_bounds__(kThreads) void k_schur_small(T* __restrict__ L, T* 
 }
 
 // ---------------------------------------------------------------------------
-// solves, with the explicit inverses of the diagonal blocks (see k_potrf_blk)
-//
-// Forward step l (levels ascending), k_sweep_nb:
-//   for every receiving block j = 2s(u+1)-1:  y_j -= R_{j-s} y_{j-s} + Lc_{j+s}^T y_{j+s},
-//   then, for the nodes j of level l+1 among them:  y_j <- Linv_j y_j
-//   (k_apply_fwd: the applies of level 0, which no update precedes)
-// Backward level l (levels descending), k_sweep_nb:
-//   for every node i:  x_i <- Linv_i^T (x_i - R_i^T x_{i+s} - Lc_i x_{i-s})
-// ---------------------------------------------------------------------------
-// Right-hand-side panels in LDS have pitch yp = min(m, kRhsChunk) + 1
-// (dynamic shared memory sized by the launch: few right-hand sides leave room
-// for more workgroups per compute unit).
-__host__ __device__ constexpr int rhs_pitch(int m) { return (m < kRhsChunk ? m : kRhsChunk) + 1; }
-
-
-// y_j <- Linv_j y_j for the nodes j = s-1+2s*t of one level.
-// out[r] = y[r] / L[r][r] + sum_{k<r} U[k][r] y[k]; thread (r, part) reads
-// U[k][r] for its K part (coalesced in r); parts are summed through LDS.
-template <typename T, int NB, int NF>
-__global__ __launch_bounds__(kThreads) void k_apply_fwd(const T* __restrict__ L, T* __restrict__ x,
-                                                       const uint8_t* __restrict__ mask, int N, int n_, int m,
-                                                       int s) {
-  const int n = NF ? NF : n_;
-  constexpr int NP = 32 * NB;
-  constexpr int PARTS = kThreads / NP;
-  constexpr int KP = (NP + PARTS - 1) / PARTS;
-  const int b = blockIdx.z;
-  if (masked_out(mask, b)) return;
-  const int j = s - 1 + 2 * s * blockIdx.x;
-  const int c0 = blockIdx.y * kRhsChunk;
-  const int w = min(kRhsChunk, m - c0);
-  const size_t nn = (size_t)n * n, nm = (size_t)n * m;
-  const T* U = L + ((size_t)b * N + j) * nn;
-  T* y = x + ((size_t)b * N + j) * nm;
-  const int yp = rhs_pitch(m);
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  T* Y = reinterpret_cast<T*>(smem_raw);  // NP x yp
-  T* Pt = Y + NP * yp;                     // PARTS x NP x yp
-  const int tid = threadIdx.x;
-  const int r = tid % NP, part = tid / NP;
-  const bool act = part < PARTS;
-  // All loads are unconditional (clamped addresses) and issued before any is
-  // consumed: pinning them to registers only after the last one is issued
-  // keeps the compiler from turning "cond ? load : 0" into one branch (and
-  // one memory round trip) per load.  Masking follows.
-  T a[KP];
-#pragma unroll
-  for (int e = 0; e < KP; ++e) a[e] = U[(size_t)min(part * KP + e, n - 1) * n + min(r, n - 1)];
-  T dg = U[(size_t)min(r, n - 1) * n + min(r, n - 1)];
-#pragma unroll
-  for (int e = 0; e < KP; ++e) pin_reg(a[e]);
-  pin_reg(dg);
-#pragma unroll
-  for (int e = 0; e < KP; ++e) {
-    const int k = part * KP + e;
-    a[e] = (act && k < r && r < n) ? a[e] : T(0);
-  }
-  for (int q = tid; q < NP * w; q += kThreads) {
-    const int k = q / w, c = q - k * w;
-    Y[k * yp + c] = (k < n) ? y[(size_t)k * m + c0 + c] : T(0);
-  }
-  __syncthreads();
-  if (act) {
-    for (int c = 0; c < w; ++c) {
-      T acc = T(0);
-#pragma unroll
-      for (int e = 0; e < KP; ++e) {
-        const int k = part * KP + e;
-        if (k < NP) acc += a[e] * Y[k * yp + c];
-      }
-      Pt[(part * NP + r) * yp + c] = acc;
-    }
-  }
-  __syncthreads();
-  if (part == 0 && r < n) {
-    for (int c = 0; c < w; ++c) {
-      T acc = Y[r * yp + c] / dg;
-      for (int p = 0; p < PARTS; ++p) acc += Pt[(p * NP + r) * yp + c];
-      y[(size_t)r * m + c0 + c] = acc;
-    }
-  }
-}
-
-
-// One sweep step in one launch, one workgroup per (block, 16 right-hand
-// sides).
-// Backward (FWD = false), level l, node i (the reference's backward
-// substitution, block_tridiag_solver.py:581-643; update and apply in one):
-//   t   = x_i - R_i^T x_{i+s} - Lc_i x_{i-s}     (R_i = block (i+s, i) when
-//         i + s < N, Lc_i = block (i, i-s) when i >= s),
-//   x_i = Linv_i^T t = t / L_i[r][r] + U t       (U: the transposed inverse in
-//         the strict upper triangle of L_i).
-// Forward (FWD = true), step l, target j = 2s(u+1)-1 (the reference's forward
-// substitution, block_tridiag_solver.py:425-485; the update of step l and,
-// for the targets that are level-(l+1) nodes (u even), the apply of level
-// l+1 in one):
-//   t   = y_j - R_{j-s} y_{j-s} - Lc_{j+s}^T y_{j+s}   (R_{j-s} = block
-//         (j, j-s), Lc_{j+s} = block (j+s, j) when j + s < N),
-//   y_j = t, or Linv_j t = t / L_j[r][r] + U^T t for u even.
-// Three staged blocks would not fit LDS: the block operands are read
-// from global memory
-// in the MFMA operand layout (each element is used once: the right-hand
-// sides are the 16 columns of every product), the three panels and the
-// intermediate t are staged in LDS; the triangular apply skips the zero
-// 16-column blocks of Linv.  Four wavefronts take the NP/16 row tiles in turn,
-// except in the FP64 backward sweep (sweepnb_wide): one wavefront per tile,
-// which issues every block load of its tile, the apply's included, before its
-// first MFMA.  Measured against the four-wavefront loop: the FP64 backward
-// sweeps gain (n=64 N=1024 m=16 factor_and_solve 0.612 -> 0.605 ms, n=128
-// N=512 m=8 1.160 -> 1.151 ms); the forward sweep, which runs beside the
-// factor, slowed the factor's kernels more than it gained, and the FP32
-// backward sweeps of the mixed solver's correction solves were slower.
-// Unconditional loads from clamped addresses, masked after.
-template <typename T, bool FWD>
-constexpr bool sweepnb_wide() {
-  return !FWD && sizeof(T) == 8;
-}
-
-template <typename T, int NB, bool FWD>
-constexpr int sweepnb_threads() {
-  return sweepnb_wide<T, FWD>() ? 64 * 2 * NB : kThreads;
-}
-
-template <typename T, int NB>
-constexpr size_t sweepnb_lds(int m) {
-  return sizeof(T) * (4 * (size_t)(32 * NB) * rhs_pitch(m) + 16 + 32 * NB);
-}
-
-template <typename T, int NB, int NF, bool FWD>
-__global__ __launch_bounds__((sweepnb_threads<T, NB, FWD>())) void k_sweep_nb(const T* __restrict__ L,
-                                                                        const T* __restrict__ E, T* __restrict__ x,
-                                                                        const uint8_t* __restrict__ mask, int N,
-                                                                        int n_, int m, int nE, int s, int off,
-                                                                        int apply) {
-  const int n = NF ? NF : n_;
-  constexpr int NP = 32 * NB, RT = NP / 16, KS = NP / 4, kT = sweepnb_threads<T, NB, FWD>();
-  const int b = blockIdx.z;
-  if (masked_out(mask, b)) return;
-  const int c0 = blockIdx.y * kRhsChunk;
-  const int w = min(kRhsChunk, m - c0);
-  const int yp = rhs_pitch(m);
-  const size_t nn = (size_t)n * n, nm = (size_t)n * m;
-  const T* Eb = E + (size_t)b * nE * nn;
-  T* xb = x + (size_t)b * N * nm;
-  int i;
-  bool hasT, hasS, inv;
-  if (!FWD) {
-    i = s - 1 + 2 * s * blockIdx.x;
-    hasT = i + s < N;  // R_i, used transposed
-    hasS = i >= s;     // Lc_i
-    inv = true;
-  } else {
-    const int u = blockIdx.x;
-    i = 2 * s * (u + 1) - 1;
-    hasT = i + s < N;  // Lc_{j+s}, used transposed
-    hasS = true;       // R_{j-s}
-    inv = apply != 0 && (u & 1) == 0;
-  }
-  const T* U = L + ((size_t)b * N + i) * nn;
-  T* xi = xb + (size_t)i * nm;
-  const T* MT = hasT ? Eb + (size_t)(off + i / s) * nn : U;  // (U: a valid dummy address)
-  const T* MS = hasS ? Eb + (size_t)(off + (i - s) / s) * nn : U;
-  const T* xp = hasT ? xb + (size_t)(i + s) * nm : xi;
-  const T* xm = hasS ? xb + (size_t)(i - s) * nm : xi;
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  T* Xp = reinterpret_cast<T*>(smem_raw);  // NP x yp each
-  T* Xm = Xp + NP * yp;
-  T* Xi = Xm + NP * yp;
-  T* Tt = Xi + NP * yp;
-  T* dg = Tt + NP * yp + 16;  // 1 / L[r][r] (after a 16-entry guard)
-  const int tid = threadIdx.x, l = lane_id(), wave = wave_id();
-  const int li = l & 15, kq = l >> 4;
-  auto stage = [&]() {
-    for (int q = tid; q < NP * w; q += kT) {
-      const int k = q / w, c = q - k * w;
-      const size_t xo = (size_t)min(k, n - 1) * m + c0 + c;
-      const T vp = xp[xo], vm = xm[xo], vi = xi[xo];
-      Xp[k * yp + c] = (hasT && k < n) ? vp : T(0);
-      Xm[k * yp + c] = (hasS && k < n) ? vm : T(0);
-      Xi[k * yp + c] = (k < n) ? vi : T(0);
-    }
-    for (int r = tid; r < NP; r += kT) {
-      const T d = U[(size_t)min(r, n - 1) * (n + 1)];
-      dg[r] = (r < n) ? T(1) / d : T(1);
-    }
-  };
-  const int jb = min(li, w - 1);
-  if constexpr (sweepnb_wide<T, FWD>()) {
-    // backward, one wavefront per 16-row tile t (32-bit element offsets from the
-    // wavefront-uniform block addresses)
-    const int t = wave;
-    const int ii = 16 * t + li;
-    const unsigned ic = min(ii, n - 1);
-    T a1[KS], a2[KS], a3[KS];
-#pragma unroll
-    for (int q = 0; q < KS; ++q) {
-      const unsigned kc = min(4 * q + kq, n - 1);
-      a1[q] = MT[kc * (unsigned)n + ic];
-      a2[q] = MS[ic * (unsigned)n + kc];
-    }
-    stage();
-    __syncthreads();
-    // t = x_i - R_i^T x_{i+s} - Lc_i x_{i-s}
-    typename Mfma<T>::acc_t acc = acc_zero<T>();
-#pragma unroll
-    for (int q = 0; q < KS; ++q) {
-      const int kk = 4 * q + kq;
-      pin_reg(a1[q]);
-      pin_reg(a2[q]);
-      const bool ok = kk < n && ii < n;
-      acc = Mfma<T>::mma((hasT && ok) ? a1[q] : T(0), Xp[kk * yp + jb], acc);
-      acc = Mfma<T>::mma((hasS && ok) ? a2[q] : T(0), Xm[kk * yp + jb], acc);
-    }
-    acc16_foreach<T>(acc, [&](int r, int c, T v) {
-      if (c < w) Tt[(16 * t + r) * yp + c] = Xi[(16 * t + r) * yp + c] - v;
-    });
-    // the apply's operands (k >= 16 t), loaded while the other wavefronts
-    // finish t; steps below 4 t load the entries of step 4 t again (the same
-    // addresses: no further traffic) and are not used
-#pragma unroll
-    for (int q = 0; q < KS; ++q) {
-      const unsigned kc = min(4 * max(q, 4 * t) + kq, n - 1);
-      a3[q] = U[ic * (unsigned)n + kc];
-    }
-    __syncthreads();
-    // x_i = A t, A(r, k) = U[r][k] (k > r), 1 / L[r][r] (k = r)
-    acc = acc_zero<T>();
-#pragma unroll
-    for (int q = 0; q < KS; ++q) {
-      if (q >= 4 * t) {  // wavefront-uniform
-        const int kk = 4 * q + kq;
-        pin_reg(a3[q]);
-        const T a = (kk < n && ii < n) ? ((kk > ii) ? a3[q] : ((kk == ii) ? dg[ii] : T(0))) : T(0);
-        acc = Mfma<T>::mma(a, Tt[kk * yp + jb], acc);
-      }
-    }
-    acc16_foreach<T>(acc, [&](int r, int c, T v) {
-      const int row = 16 * t + r;
-      if (row < n && c < w) xi[(size_t)row * m + c0 + c] = v;
-    });
-    return;
-  }
-  stage();
-  __syncthreads();
-  // t = x_i - MT^T xp - MS xm
-  for (int t = wave; t < RT; t += kT / 64) {
-    const int ii = 16 * t + li, ic = min(ii, n - 1);
-    typename Mfma<T>::acc_t acc = acc_zero<T>();
-#pragma unroll 4
-    for (int k = 0; k < NP; k += 4) {
-      const int kk = k + kq, kc = min(kk, n - 1);
-      const T a1 = MT[(size_t)kc * n + ic];
-      const T a2 = MS[(size_t)ic * n + kc];
-      const bool ok = kk < n && ii < n;
-      acc = Mfma<T>::mma((hasT && ok) ? a1 : T(0), Xp[kk * yp + jb], acc);
-      acc = Mfma<T>::mma((hasS && ok) ? a2 : T(0), Xm[kk * yp + jb], acc);
-    }
-    acc16_foreach<T>(acc, [&](int r, int c, T v) {
-      const int row = 16 * t + r;
-      if (c < w) {
-        const T tv = Xi[row * yp + c] - v;
-        if (inv) Tt[row * yp + c] = tv;
-        else if (row < n) xi[(size_t)row * m + c0 + c] = tv;
-      }
-    });
-  }
-  if (!inv) return;
-  __syncthreads();
-  // backward: x_i = A t, A(r, k) = U[r][k] (k > r), 1 / L[r][r] (k = r);
-  // forward: y_j = A t, A(r, k) = U[k][r] (k < r), 1 / L[r][r] (k = r)
-  for (int t = wave; t < RT; t += kT / 64) {
-    const int ii = 16 * t + li, ic = min(ii, n - 1);
-    const int kb = FWD ? 0 : 16 * t, ke = FWD ? 16 * (t + 1) : NP;
-    typename Mfma<T>::acc_t acc = acc_zero<T>();
-#pragma unroll 4
-    for (int k = kb; k < ke; k += 4) {
-      const int kk = k + kq, kc = min(kk, n - 1);
-      const T u = FWD ? U[(size_t)kc * n + ic] : U[(size_t)ic * n + kc];
-      const bool strict = FWD ? kk < ii : kk > ii;
-      const T a = (kk < n && ii < n) ? (strict ? u : ((kk == ii) ? dg[ii] : T(0))) : T(0);
-      acc = Mfma<T>::mma(a, Tt[kk * yp + jb], acc);
-    }
-    acc16_foreach<T>(acc, [&](int r, int c, T v) {
-      const int row = 16 * t + r;
-      if (row < n && c < w) xi[(size_t)row * m + c0 + c] = v;
-    });
-  }
-}
-
-// ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
-// dynamic LDS of the sweep kernels for m right-hand sides
-template <typename T, int NB>
-constexpr size_t apply_fwd_lds(int m) {
-  return sizeof(T) * (1 + kThreads / (32 * NB)) * (size_t)(32 * NB) * rhs_pitch(m);
-}
-
 template <typename T, int NB>
 constexpr size_t potrf_blk_lds() {
   return sizeof(T) * ((size_t)(32 * NB) * (32 * NB + 1) + 32 * NB + 32 * 33);
@@ -1357,17 +1057,6 @@ static hipError_t set_blk_attrs() {
   if (e != hipSuccess) return e;
   e = hipFuncSetAttribute((const void*)k_trsm_node<T, NB, 32 * NB>, hipFuncAttributeMaxDynamicSharedMemorySize,
                           (int)trsm_node_lds<T, NB>());
-  const int lsw = (int)sweepnb_lds<T, NB>(kRhsChunk);  // the widest right-hand-side chunk
-  if (e == hipSuccess)
-    e = hipFuncSetAttribute((const void*)k_sweep_nb<T, NB, 0, true>, hipFuncAttributeMaxDynamicSharedMemorySize, lsw);
-  if (e == hipSuccess)
-    e = hipFuncSetAttribute((const void*)k_sweep_nb<T, NB, 0, false>, hipFuncAttributeMaxDynamicSharedMemorySize, lsw);
-  if (e == hipSuccess)
-    e = hipFuncSetAttribute((const void*)k_sweep_nb<T, NB, 32 * NB, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            lsw);
-  if (e == hipSuccess)
-    e = hipFuncSetAttribute((const void*)k_sweep_nb<T, NB, 32 * NB, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            lsw);
   return e;
 }
 
@@ -1679,36 +1368,6 @@ hipError_t trtri_blocked(const T* L, T* W, const uint8_t* mask, int B, int N, in
   }
 }
 
-template <typename T, int NB, int NF>
-static hipError_t forward_step_nb(const T* L, const T* E, T* x, const uint8_t* mask, int B, int N, int n, int m,
-                                  int step, hipStream_t st, bool apply_next, bool update = true) {
-  const int nE = (int)off_diag_storage_len(N);
-  const int mch = (m + kRhsChunk - 1) / kRhsChunk;
-  if (B <= 0 || mch <= 0) return hipSuccess;
-  kt_begin(kKcForward, st);
-  // step l's updates and level l+1's applies in one launch
-  if (update && step >= 0) {
-    const Level lv = level_info(N, step);
-    const int items = N / (2 * lv.s);
-    if (items > 0) {
-      const int ap = (apply_next && level_info(N, step + 1).dim > 0) ? 1 : 0;
-      const size_t lds = sweepnb_lds<T, NB>(m);
-      hipLaunchKernelGGL((k_sweep_nb<T, NB, NF, true>), dim3(items, mch, B), dim3(sweepnb_threads<T, NB, true>()), lds,
-                         st, L, E, x, mask, N, n, m, nE, lv.s, lv.off, ap);
-    }
-    kt_end(kKcForward, st);
-    return hipGetLastError();
-  }
-  const Level nx = level_info(N, step + 1);
-  if (apply_next && nx.dim > 0) {
-    const size_t lds = apply_fwd_lds<T, NB>(m);
-    hipLaunchKernelGGL((k_apply_fwd<T, NB, NF>), dim3(nx.dim, mch, B), dim3(kThreads), lds, st, L, x, mask, N, n, m,
-                       nx.s);
-  }
-  kt_end(kKcForward, st);
-  return hipGetLastError();
-}
-
 template <typename T>
 static hipError_t forward_step_parts(const T* L, const T* E, T* x, const uint8_t* mask, int B, int N, int n, int m,
                               int step, hipStream_t st, bool a, bool u) {
@@ -1721,18 +1380,7 @@ static hipError_t forward_step_parts(const T* L, const T* E, T* x, const uint8_t
     return e;
   }
   if (n <= kSmallN) return small_forward_step<T>(L, E, x, mask, B, N, n, m, step, st, u, a);
-  switch (n) {
-    case 64: return forward_step_nb<T, 2, 64>(L, E, x, mask, B, N, n, m, step, st, a, u);
-    case 96: return forward_step_nb<T, 3, 96>(L, E, x, mask, B, N, n, m, step, st, a, u);
-    case 128: return forward_step_nb<T, 4, 128>(L, E, x, mask, B, N, n, m, step, st, a, u);
-    default: break;
-  }
-  switch ((n + 31) / 32) {
-    case 2: return forward_step_nb<T, 2, 0>(L, E, x, mask, B, N, n, m, step, st, a, u);
-    case 3: return forward_step_nb<T, 3, 0>(L, E, x, mask, B, N, n, m, step, st, a, u);
-    case 4: return forward_step_nb<T, 4, 0>(L, E, x, mask, B, N, n, m, step, st, a, u);
-    default: return hipErrorInvalidValue;
-  }
+  return wide_forward_step<T>(L, E, x, mask, B, N, n, m, step, st, u, a);
 }
 
 template <typename T>
@@ -1753,21 +1401,6 @@ hipError_t forward_apply_blocked(const T* L, const T* E, T* x, const uint8_t* ma
   return forward_step_parts<T>(L, E, x, mask, B, N, n, m, level - 1, st, true, false);
 }
 
-template <typename T, int NB, int NF>
-static hipError_t backward_level_nb(const T* L, const T* E, T* x, const uint8_t* mask, int B, int N, int n, int m,
-                                    int lidx, hipStream_t st) {
-  const int nE = (int)off_diag_storage_len(N);
-  const int mch = (m + kRhsChunk - 1) / kRhsChunk;
-  const Level lv = level_info(N, lidx);
-  if (lv.dim <= 0 || B <= 0 || mch <= 0) return hipSuccess;
-  kt_begin(kKcBackward, st);
-  const size_t lds = sweepnb_lds<T, NB>(m);
-  hipLaunchKernelGGL((k_sweep_nb<T, NB, NF, false>), dim3(lv.dim, mch, B), dim3(sweepnb_threads<T, NB, false>()), lds,
-                     st, L, E, x, mask, N, n, m, nE, lv.s, lv.off, 1);
-  kt_end(kKcBackward, st);
-  return hipGetLastError();
-}
-
 template <typename T>
 hipError_t backward_level_blocked(const T* L, const T* E, T* x, const uint8_t* mask, int B, int N, int n, int m,
                                   int lidx, hipStream_t st) {
@@ -1781,18 +1414,7 @@ hipError_t backward_level_blocked(const T* L, const T* E, T* x, const uint8_t* m
     return e;
   }
   if (n <= kSmallN) return small_backward_level<T>(L, E, x, mask, B, N, n, m, lidx, st);
-  switch (n) {
-    case 64: return backward_level_nb<T, 2, 64>(L, E, x, mask, B, N, n, m, lidx, st);
-    case 96: return backward_level_nb<T, 3, 96>(L, E, x, mask, B, N, n, m, lidx, st);
-    case 128: return backward_level_nb<T, 4, 128>(L, E, x, mask, B, N, n, m, lidx, st);
-    default: break;
-  }
-  switch ((n + 31) / 32) {
-    case 2: return backward_level_nb<T, 2, 0>(L, E, x, mask, B, N, n, m, lidx, st);
-    case 3: return backward_level_nb<T, 3, 0>(L, E, x, mask, B, N, n, m, lidx, st);
-    case 4: return backward_level_nb<T, 4, 0>(L, E, x, mask, B, N, n, m, lidx, st);
-    default: return hipErrorInvalidValue;
-  }
+  return wide_backward_level<T>(L, E, x, mask, B, N, n, m, lidx, st);
 }
 
 hipError_t overlap_create(SweepOverlap& ov) {

@@ -199,6 +199,13 @@ hipError_t small_forward_step(const T* L, const T* E, T* x, const uint8_t* mask,
 template <typename T>
 hipError_t small_backward_level(const T* L, const T* E, T* x, const uint8_t* mask, int B, int N, int n, int m,
                                 int lidx, hipStream_t st);
+// The same for 32 < n <= 128 (nd_steps.hip).
+template <typename T>
+hipError_t wide_forward_step(const T* L, const T* E, T* x, const uint8_t* mask, int B, int N, int n, int m, int step,
+                             hipStream_t st, bool update, bool apply);
+template <typename T>
+hipError_t wide_backward_level(const T* L, const T* E, T* x, const uint8_t* mask, int B, int N, int n, int m, int lidx,
+                               hipStream_t st);
 
 // Mixed-precision factor_and_solve with FP64 refinement (nd_refine.hip).
 struct MixedPlan {

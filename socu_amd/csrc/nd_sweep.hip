@@ -1,6 +1,6 @@
 // Persistent dataflow solve sweeps for one right-hand side (m = 1), n <= 128.
 //
-// The level-synchronous sweeps (k_sweep32 / k_sweep_nb / k_apply_fwd)
+// The level-synchronous sweeps (nd_small.hip, nd_steps.hip)
 // need a launch per level and direction, each waiting for the slowest
 // workgroup of its level and paying a dispatch gap; at the upper levels, where
 // a level is one or two nodes, those gaps are the whole cost.  Here one launch
