@@ -190,6 +190,7 @@ int ensure_init() {
   if (e == hipSuccess) e = socu::init_large_kernels();
   if (e == hipSuccess) e = socu::init_small_kernels();
   if (e == hipSuccess) e = socu::init_wide_kernels();
+  if (e == hipSuccess) e = socu::init_potrf_kernels();
   if (e != hipSuccess) return hip_fail(e, "kernel set-up (hipFuncSetAttribute)");
   state = 1;
   return SOCU_OK;

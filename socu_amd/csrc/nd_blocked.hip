@@ -3,14 +3,7 @@
 // within the n x n blocks.  One or two kernel launches per phase per level; no
 // atomics, so results are bitwise reproducible.
 //
-//   k_potrf_blk  one workgroup per node:  L_i <- chol(L_i), blocked
-//                right-looking over 32x32 tiles (reference: potrf_blocked,
-//                socu/blas/potrf.py:97-119).  Each diagonal tile is factored
-//                and inverted by one wavefront (tile_chol_inv); panel and
-//                trailing updates run on MFMA.  Then the full inverse Linv_i is
-//                formed (MFMA) and stored transposed in the strict upper
-//                triangle of L_i, which is not part of the factor (the
-//                reference only ever reads tril(L)).
+//   k_potrf_blk  (nd_potrf.hip) L_i and its inverse's transpose.
 //   k_trsm_blk   one workgroup per (node, 32-wide chunk of R rows / Lc cols):
 //                R <- R Linv^T, Lc <- Linv Lc as MFMA products with the stored
 //                inverse (replaces trsm_rltn / trsm_llnn, trsm.py:94-120,
@@ -28,336 +21,9 @@
 
 namespace socu {
 
-// ---------------------------------------------------------------------------
-// potrf
-// ---------------------------------------------------------------------------
 // NF != 0 instantiates the kernels for a fixed block size n == NF (a multiple
 // of 32), so that all index arithmetic is compile-time; NF == 0 is the
 // general (padded) version.
-// TS is the storage type of L; T the compute type (TS = float, T = double
-// factors FP32 blocks with FP64 pivots and updates).
-// One 64-lane wavefront for NB == 1 (the whole factor is wave 0's pivot
-// chain: a workgroup of four would hold registers for three idle waves, and
-// batches of many small blocks are throughput-bound); four otherwise.
-constexpr int potrf_threads(int nb) { return nb == 1 ? 64 : kThreads; }
-
-template <typename TS, int NB, int NF, typename T = TS>
-__global__ __launch_bounds__(kThreads) void k_potrf_blk(TS* __restrict__ L, const uint8_t* __restrict__ mask, int N,
-                                                       int n_, int s, const TS* __restrict__ Lsrc) {
-  const int n = NF ? NF : n_;
-  constexpr int NP = 32 * NB;
-  constexpr int P = NP + 1;
-  constexpr int TH = potrf_threads(NB);
-  constexpr int WS = TH / 64 > 1 ? TH / 64 - 1 : 1;  // stride over waves 1.. (none when TH == 64)
-  const int b = blockIdx.y;
-  if (masked_out(mask, b)) return;
-  const int i = s - 1 + 2 * s * blockIdx.x;
-  TS* A = L + ((size_t)b * N + i) * (size_t)n * n;
-  // out-of-place factor: the block is read from Lsrc (same layout), the
-  // factor written to L
-  const TS* Ain = (Lsrc != nullptr) ? Lsrc + ((size_t)b * N + i) * (size_t)n * n : A;
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  T* S = reinterpret_cast<T*>(smem_raw);
-  T* dinv = S + NP * P;  // 1/L[r][r] for every row
-  T* ut = dinv + NP;  // 32 x 33: the last factored tile's inverse, transposed in full
-  const int tid = threadIdx.x, wave = wave_id(), l = lane_id();
-
-  const int nn = n * n;
-  if constexpr (NF == NP) {
-    // Unpadded block: only the lower tiles are read (every strictly upper
-    // tile is written below before it is read).  Wave 0 reads diagonal tile
-    // (0, 0) alone and starts its pivot chain at once; waves 1..3, idle in
-    // that step, read the other lower tiles meanwhile (the step's barrier
-    // publishes them).  Lane l reads row 2q + l/32, column l%32 of a tile.
-    const int lr = l >> 5, lc = l & 31;
-    if (wave == 0) {
-      TS v[16];
-#pragma unroll
-      for (int q = 0; q < 16; ++q) v[q] = Ain[(2 * q + lr) * NF + lc];
-#pragma unroll
-      for (int q = 0; q < 16; ++q) {
-        const int r = 2 * q + lr;
-        S[r * P + lc] = (lc <= r) ? (T)v[q] : T(0);
-      }
-    } else {
-      constexpr int NT = NB * (NB + 1) / 2 - 1;  // lower tiles other than (0, 0)
-      constexpr int PW = NT > 0 ? (NT + 2) / 3 : 1;
-      TS v[PW][16];
-#pragma unroll
-      for (int k = 0; k < PW; ++k) {
-        int ti = 1, tj = (wave - 1) + 3 * k;
-        while (tj > ti) { tj -= ti + 1; ++ti; }
-        if (ti < NB) {
-#pragma unroll
-          for (int q = 0; q < 16; ++q) v[k][q] = Ain[(32 * ti + 2 * q + lr) * NF + 32 * tj + lc];
-        }
-      }
-#pragma unroll
-      for (int k = 0; k < PW; ++k) {
-        int ti = 1, tj = (wave - 1) + 3 * k;
-        while (tj > ti) { tj -= ti + 1; ++ti; }
-        if (ti < NB) {
-#pragma unroll
-          for (int q = 0; q < 16; ++q) {
-            const int r = 2 * q + lr;
-            S[(32 * ti + r) * P + 32 * tj + lc] = (ti != tj || lc <= r) ? (T)v[k][q] : T(0);
-          }
-        }
-      }
-    }
-  } else {
-    // The block is read as one contiguous n*n run (coalesced, unconditional
-    // loads from clamped addresses) and scattered into the padded LDS square.
-    constexpr int PER = NP * NP / TH;
-    T v[PER];
-#pragma unroll
-    for (int e = 0; e < PER; ++e) {
-      const int idx = tid + e * TH;
-      v[e] = (T)Ain[min(idx, nn - 1)];
-    }
-    for (int idx = tid; idx < NP * NP; idx += TH) {
-      const int r = idx / NP, c = idx - r * NP;
-      S[r * P + c] = (r == c) ? T(1) : T(0);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int e = 0; e < PER; ++e) {
-      const int idx = tid + e * TH;
-      const int r = idx / n, c = idx - r * n;
-      if (idx < nn) S[r * P + c] = (c <= r) ? v[e] : T(0);
-    }
-    __syncthreads();
-  }
-
-  // Off-diagonal tiles of the inverse:
-  //   Linv_ij = -Dinv_i S_ij,  S_ij = sum_{k=j}^{i-1} L_ik Linv_kj  (j < i),
-  //   Linv_jj = Dinv_j.
-  // Linv_ij is kept transposed in the upper tile (j, i):
-  // S[32j+c][32i+r] = Linv_ij[r][c]; S_ij is parked there first and then
-  // overwritten in place.  Column j belongs to wavefront 1 + j, which forms
-  // its blocks while wavefront 0 runs the pivot chain of the next diagonal
-  // tile: in the step of tile kb it finishes Linv_{kb-1,j} and accumulates
-  // S_{kb,j}, whose operands (L_{kb,k} for k < kb, Linv_kj for k < kb) are
-  // final by then.
-  auto inv_partial = [&](int i, int j) {  // S_ij -> upper tile (j, i)
-    typename Mfma<T>::acc_t acc[2][2] = {{acc_zero<T>(), acc_zero<T>()}, {acc_zero<T>(), acc_zero<T>()}};
-    for (int k = j; k < i; ++k) {
-      const T* Lik = S + 32 * i * P + 32 * k;
-      if (k == j) {
-        const T* Dj = S + 32 * j * P + 32 * j;
-        wave_gemm_f<T>(
-            acc, [&](int r, int kk) { return Lik[r * P + kk]; },
-            [&](int kk, int c) { return (kk > c) ? Dj[c * P + kk] : ((kk == c) ? dinv[32 * j + c] : T(0)); }, 32);
-      } else {
-        const T* Ukj = S + 32 * j * P + 32 * k;  // holds Linv_kj transposed
-        wave_gemm<T>(acc, Lik, P, 1, Ukj, 1, P, 32);
-      }
-    }
-    T* Uji = S + 32 * j * P + 32 * i;
-    acc_foreach<T>(acc, [&](int r, int c, T v) { Uji[c * P + r] = v; });
-  };
-  auto inv_finish = [&](int i, int j) {  // Linv_ij = -Dinv_i S_ij, in place
-    T* Uji = S + 32 * j * P + 32 * i;
-    typename Mfma<T>::acc_t inv[2][2] = {{acc_zero<T>(), acc_zero<T>()}, {acc_zero<T>(), acc_zero<T>()}};
-    const T* Di = S + 32 * i * P + 32 * i;
-    wave_gemm_f<T>(
-        inv, [&](int r, int kk) { return (r > kk) ? Di[kk * P + r] : ((r == kk) ? dinv[32 * i + r] : T(0)); },
-        [&](int kk, int c) { return Uji[c * P + kk]; }, 32);
-    acc_foreach<T>(inv, [&](int r, int c, T v) { Uji[c * P + r] = -v; });
-  };
-
-  // 32x32 tile (ti, tj) of S written back to the same tile of A (unpadded
-  // blocks only): lane l stores row 2q + l/32, column l%32.
-  auto store_tile = [&](int ti, int tj) {
-    const int lr = l >> 5, lc = l & 31;
-#pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      const int r = 32 * ti + 2 * q + lr, c = 32 * tj + lc;
-      A[r * n + c] = (TS)S[r * P + c];
-    }
-  };
-
-  // tile (gi, gj) -= L_{gi,kb} L_{gj,kb}^T
-  auto trail = [&](int kb, int gi, int gj) {
-    typename Mfma<T>::acc_t acc[2][2] = {{acc_zero<T>(), acc_zero<T>()}, {acc_zero<T>(), acc_zero<T>()}};
-    wave_gemm<T>(acc, S + 32 * gi * P + 32 * kb, P, 1, S + 32 * gj * P + 32 * kb, 1, P, 32);
-    T* C = S + 32 * gi * P + 32 * gj;
-    acc_foreach<T>(acc, [&](int r, int c, T v) { C[r * P + c] -= v; });
-  };
-
-  // Two phases per diagonal tile kb, with look-ahead: wave 0 applies the
-  // previous step's update to tile (kb, kb) only, then factors it; meanwhile
-  // waves 1..3 apply the rest of that update (tiles (gi, gj), kb <= gj <= gi,
-  // except (kb, kb)) and the inverse-block work.  Then every wave forms the
-  // panel tiles (ti, kb) <- tile (ti, kb) Linv_kb^T.
-  for (int kb = 0; kb < NB; ++kb) {
-    T* D = S + 32 * kb * P + 32 * kb;
-    if (wave == 0) {
-      if (kb > 0) trail(kb - 1, kb, kb);
-      tile_chol_inv<T>(D, P, dinv + 32 * kb, ut);
-    } else {
-      for (int j = wave - 1; j < NB - 1; j += WS) {
-        if (j < kb - 1) inv_finish(kb - 1, j);
-        if (j <= kb - 1) inv_partial(kb, j);
-      }
-      if (kb > 0) {
-        const int m = NB - kb;
-        const int cnt = m * (m + 1) / 2;  // triangle index 0 is (kb, kb)
-        for (int t = wave; t < cnt; t += WS) {
-          int ti = 0, q = t;
-          while (q > ti) { q -= ti + 1; ++ti; }
-          trail(kb - 1, kb + ti, kb + q);
-        }
-      }
-      if constexpr (NF == NP) {
-        // Write-back of the tiles final since the end of step kb - 1 (the
-        // factor's tile column kb - 1 with the inverse of diagonal tile
-        // kb - 1, and the inverse blocks Linv_{kb-2, j}^T), while wave 0 is in
-        // its pivot chain.
-        if (kb > 0) {
-          const int nlow = NB - (kb - 1), nup = kb >= 2 ? kb - 2 : 0;
-          for (int t = wave - 1; t < nlow + nup; t += WS) {
-            if (t < nlow) store_tile(kb - 1 + t, kb - 1);
-            else store_tile(t - nlow, kb - 2);
-          }
-        }
-      }
-    }
-    __syncthreads();
-    // panel: tile (ti, kb) <- tile (ti, kb) Linv^T
-    for (int ti = kb + 1 + wave; ti < NB; ti += TH / 64) {
-      T* X = S + 32 * ti * P + 32 * kb;
-      typename Mfma<T>::acc_t acc[2][2] = {{acc_zero<T>(), acc_zero<T>()}, {acc_zero<T>(), acc_zero<T>()}};
-      const int li = l & 15, kq = l >> 4;
-#pragma unroll
-      for (int k = 0; k < 32; k += 4) {
-        const int kk = k + kq;
-        const T a0 = X[li * P + kk], a1 = X[(li + 16) * P + kk];
-        // B(k, c) = Linv[c][k] = ut[k][c]
-        const int c0 = li, c1 = li + 16;
-        const T b0 = ut[kk * 33 + c0];
-        const T b1 = ut[kk * 33 + c1];
-        acc[0][0] = Mfma<T>::mma(a0, b0, acc[0][0]);
-        acc[0][1] = Mfma<T>::mma(a0, b1, acc[0][1]);
-        acc[1][0] = Mfma<T>::mma(a1, b0, acc[1][0]);
-        acc[1][1] = Mfma<T>::mma(a1, b1, acc[1][1]);
-      }
-      acc_foreach<T>(acc, [&](int r, int c, T v) { X[r * P + c] = v; });
-    }
-    __syncthreads();
-  }
-
-  // The last row of inverse blocks (the others were formed during the
-  // pivot chains above).
-  if (wave > 0)
-    for (int j = wave - 1; j < NB - 1; j += WS) inv_finish(NB - 1, j);
-  __syncthreads();
-
-  // Write-back: tril(L) is the factor; the strict upper triangle, which is
-  // not part of the factor, carries the transposed inverse of the diagonal
-  // block (U[k][r] = Linv[r][k], k < r) for the trsm and solve kernels.
-  if constexpr (NF == NP) {
-    // what the pivot steps have not written yet: diagonal tile NB-1 and the
-    // inverse blocks Linv_{NB-2, j}^T, Linv_{NB-1, j}^T
-    const int n2 = NB >= 2 ? NB - 2 : 0, cnt = 1 + n2 + (NB - 1);
-    for (int t = wave; t < cnt; t += TH / 64) {
-      if (t == 0) store_tile(NB - 1, NB - 1);
-      else if (t - 1 < n2) store_tile(t - 1, NB - 2);
-      else store_tile(t - 1 - n2, NB - 1);
-    }
-  } else {
-    // one contiguous run
-    for (int idx = tid; idx < nn; idx += TH) {
-      const int r = idx / n, c = idx - r * n;
-      A[idx] = (TS)S[r * P + c];
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Inverses of the diagonal factor blocks from tril(L) alone, for solves whose
-// factor may come from anywhere (the reference's sweeps read only tril(L),
-// socu/blas/potrf.py:101-103).  One workgroup of NB wavefronts per block
-// (grid (N, B)): W_i <- tril(L_i) with the transposed inverse in its strict
-// upper triangle, W_i[k][r] = Linv_i[r][k] for k < r -- the layout k_potrf_blk
-// leaves in L_i, which the sweep and apply kernels read.  L is only read.
-//   wave w inverts diagonal tile w (tile_tri_inv);
-//   band d = 1..NB-1: Linv_ij = -Dinv_i sum_{k=j}^{i-1} L_ik Linv_kj, i = j+d,
-//   one wavefront per tile, MFMA.
-// ---------------------------------------------------------------------------
-template <typename T, int NB>
-constexpr size_t trtri_blk_lds() {
-  return sizeof(T) * ((size_t)(32 * NB) * (32 * NB + 1) + 32 * NB);
-}
-
-template <typename T, int NB, int NF>
-__global__ __launch_bounds__(64 * NB) void k_trtri_blk(const T* __restrict__ L, T* __restrict__ W,
-                                                      const uint8_t* __restrict__ mask, int N, int n_) {
-  const int n = NF ? NF : n_;
-  constexpr int NP = 32 * NB;
-  constexpr int P = NP + 1;
-  constexpr int TH = 64 * NB;
-  const int b = blockIdx.y;
-  if (masked_out(mask, b)) return;
-  const int i = blockIdx.x;
-  const size_t nn = (size_t)n * n;
-  const T* A = L + ((size_t)b * N + i) * nn;
-  T* Wb = W + ((size_t)b * N + i) * nn;
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  T* S = reinterpret_cast<T*>(smem_raw);
-  T* dinv = S + NP * P;
-  const int tid = threadIdx.x, wave = wave_id();
-
-  // tril(L_i) into the padded square: zeros above the diagonal and outside
-  // n, ones on the padded part of the diagonal; the block is read as one
-  // contiguous run (upper entries are loaded and dropped).
-  for (int idx = tid; idx < NP * NP; idx += TH) {
-    const int r = idx / NP, c = idx - r * NP;
-    T v = (r == c) ? T(1) : T(0);
-    if (r < n && c < n) v = (c <= r) ? A[r * n + c] : T(0);
-    S[r * P + c] = v;
-  }
-  __syncthreads();
-  tile_tri_inv<T>(S + 32 * wave * P + 32 * wave, P, dinv + 32 * wave);
-  __syncthreads();
-  for (int d = 1; d < NB; ++d) {
-    const int j = wave, ii = wave + d;
-    if (ii < NB) {
-      // S_ij -> upper tile (j, ii), transposed
-      typename Mfma<T>::acc_t acc[2][2] = {{acc_zero<T>(), acc_zero<T>()}, {acc_zero<T>(), acc_zero<T>()}};
-      for (int k = j; k < ii; ++k) {
-        const T* Lik = S + 32 * ii * P + 32 * k;
-        const T* Ukj = S + 32 * j * P + 32 * k;  // Linv_kj transposed (k > j), or tile j's own inverse
-        const T* dj = dinv + 32 * k;
-        wave_gemm_f<T>(
-            acc, [&](int r, int kk) { return Lik[r * P + kk]; },
-            [&](int kk, int c) {
-              if (k != j) return Ukj[c * P + kk];
-              return (kk > c) ? Ukj[c * P + kk] : ((kk == c) ? dj[c] : T(0));
-            },
-            32);
-      }
-      T* Uji = S + 32 * j * P + 32 * ii;
-      acc_foreach<T>(acc, [&](int r, int c, T v) { Uji[c * P + r] = v; });
-      // Linv_ij = -Dinv_i S_ij, in place.  Only this wavefront touches tile
-      // (j, ii), and the LDS operations of one wavefront complete in issue
-      // order, so its stores above precede these reads and these reads the
-      // stores below.
-      const T* Di = S + 32 * ii * P + 32 * ii;
-      const T* di = dinv + 32 * ii;
-      typename Mfma<T>::acc_t inv[2][2] = {{acc_zero<T>(), acc_zero<T>()}, {acc_zero<T>(), acc_zero<T>()}};
-      wave_gemm_f<T>(
-          inv, [&](int r, int kk) { return (r > kk) ? Di[kk * P + r] : ((r == kk) ? di[r] : T(0)); },
-          [&](int kk, int c) { return Uji[c * P + kk]; }, 32);
-      acc_foreach<T>(inv, [&](int r, int c, T v) { Uji[c * P + r] = -v; });
-    }
-    __syncthreads();  // band d is final before band d + 1 reads it
-  }
-  for (int idx = tid; idx < (int)nn; idx += TH) {
-    const int r = idx / n, c = idx - r * n;
-    Wb[idx] = S[r * P + c];
-  }
-}
 
 // ---------------------------------------------------------------------------
 // trsm with the explicit inverse left by k_potrf_blk in the strict upper
@@ -1020,10 +686,6 @@ __global__ __launch_bounds__(kThreads) void k_schur_small(T* __restrict__ L, T* 
 // launchers
 // ---------------------------------------------------------------------------
 template <typename T, int NB>
-constexpr size_t potrf_blk_lds() {
-  return sizeof(T) * ((size_t)(32 * NB) * (32 * NB + 1) + 32 * NB + 32 * 33);
-}
-template <typename T, int NB>
 constexpr size_t trsm_blk_lds() {
   // upper tiles + max(R chunk 32 x (NP+1), Lc chunk NP x 33)
   return sizeof(T) * ((size_t)(NB * (NB + 1) / 2) * 32 * 33 +
@@ -1040,12 +702,6 @@ constexpr size_t trsm_node_lds() {
 template <typename T, int NB>
 static hipError_t set_blk_attrs() {
   hipError_t e;
-  e = hipFuncSetAttribute((const void*)k_potrf_blk<T, NB, 0>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                          (int)potrf_blk_lds<T, NB>());
-  if (e != hipSuccess) return e;
-  e = hipFuncSetAttribute((const void*)k_potrf_blk<T, NB, 32 * NB>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                          (int)potrf_blk_lds<T, NB>());
-  if (e != hipSuccess) return e;
   e = hipFuncSetAttribute((const void*)k_trsm_blk<T, NB, 0>, hipFuncAttributeMaxDynamicSharedMemorySize,
                           (int)trsm_blk_lds<T, NB>());
   if (e != hipSuccess) return e;
@@ -1123,24 +779,6 @@ static bool use_schur_small(int nodes, int n, int esize) {
   return (double)nodes * n * n * esize <= 12.0 * 1024 * 1024;
 }
 
-template <typename T, int NB>
-static hipError_t set_trtri_attrs() {
-  hipError_t e = hipFuncSetAttribute((const void*)k_trtri_blk<T, NB, 0>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     (int)trtri_blk_lds<T, NB>());
-  if (e != hipSuccess) return e;
-  return hipFuncSetAttribute((const void*)k_trtri_blk<T, NB, 32 * NB>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                             (int)trtri_blk_lds<T, NB>());
-}
-
-template <int NB>
-static hipError_t set_mixed_attrs() {
-  hipError_t e = hipFuncSetAttribute((const void*)k_potrf_blk<float, NB, 0, double>,
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)potrf_blk_lds<double, NB>());
-  if (e != hipSuccess) return e;
-  return hipFuncSetAttribute((const void*)k_potrf_blk<float, NB, 32 * NB, double>,
-                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)potrf_blk_lds<double, NB>());
-}
-
 hipError_t init_blocked_kernels() {
   hipError_t e;
   if ((e = set_blk_attrs<float, 2>()) != hipSuccess) return e;
@@ -1156,18 +794,6 @@ hipError_t init_blocked_kernels() {
   if ((e = set_schur_small_attrs<double, 2>()) != hipSuccess) return e;
   if ((e = set_schur_small_attrs<double, 3>()) != hipSuccess) return e;
   if ((e = set_schur_small_attrs<double, 4>()) != hipSuccess) return e;
-  if ((e = set_trtri_attrs<float, 1>()) != hipSuccess) return e;
-  if ((e = set_trtri_attrs<float, 2>()) != hipSuccess) return e;
-  if ((e = set_trtri_attrs<float, 3>()) != hipSuccess) return e;
-  if ((e = set_trtri_attrs<float, 4>()) != hipSuccess) return e;
-  if ((e = set_trtri_attrs<double, 1>()) != hipSuccess) return e;
-  if ((e = set_trtri_attrs<double, 2>()) != hipSuccess) return e;
-  if ((e = set_trtri_attrs<double, 3>()) != hipSuccess) return e;
-  if ((e = set_trtri_attrs<double, 4>()) != hipSuccess) return e;
-  if ((e = set_mixed_attrs<1>()) != hipSuccess) return e;
-  if ((e = set_mixed_attrs<2>()) != hipSuccess) return e;
-  if ((e = set_mixed_attrs<3>()) != hipSuccess) return e;
-  if ((e = set_mixed_attrs<4>()) != hipSuccess) return e;
   return hipSuccess;
 }
 
@@ -1181,20 +807,8 @@ static hipError_t factor_level_nb(T* L, T* E, const uint8_t* mask, int B, int N,
   if (lv.dim <= 0 || B <= 0) return hipSuccess;
   const size_t lds_trsm = trsm_blk_lds<T, NB>();
   const bool bf16 = (prec & kPrecBf16Schur) != 0 && sizeof(T) == 4;
-  // under socu_profile_op the launch itself records its start and end
-  // (events of hipExtLaunchKernel: the kernel's own execution interval)
-  auto k = k_potrf_blk<T, NB, NF, T>;
-  size_t lds_potrf = potrf_blk_lds<T, NB>();
-  if ((prec & kPrecF64Pivots) != 0 && sizeof(T) == 4) {
-    k = k_potrf_blk<T, NB, NF, double>;
-    lds_potrf = potrf_blk_lds<double, NB>();
-  }
-  hipEvent_t ea = nullptr, eb = nullptr;
-  if (kt_kernel_events(kKcPotrf, &ea, &eb))
-    hipExtLaunchKernelGGL(k, dim3(lv.dim, B), dim3(potrf_threads(NB)), lds_potrf, st, ea, eb, 0, L, mask, N, n, lv.s,
-                          Lsrc);
-  else
-    hipLaunchKernelGGL(k, dim3(lv.dim, B), dim3(potrf_threads(NB)), lds_potrf, st, L, mask, N, n, lv.s, Lsrc);
+  hipError_t ep = potrf_level<T>(L, mask, B, N, n, lidx, (prec & kPrecF64Pivots) != 0 && sizeof(T) == 4, Lsrc, 0, n, st);
+  if (ep != hipSuccess) return ep;
   if (after_potrf != nullptr) {
     const hipError_t e = hipEventRecord(after_potrf, st);
     if (e != hipSuccess) return e;
@@ -1334,16 +948,6 @@ hipError_t factor_level_blocked(T* L, T* E, const uint8_t* mask, int B, int N, i
   }
 }
 
-template <typename T, int NB, int NF>
-static hipError_t trtri_nb(const T* L, T* W, const uint8_t* mask, int B, int N, int n, hipStream_t st) {
-  if (B <= 0) return hipSuccess;
-  const size_t lds = trtri_blk_lds<T, NB>();
-  kt_begin(kKcForward, st);
-  hipLaunchKernelGGL((k_trtri_blk<T, NB, NF>), dim3(N, B), dim3(64 * NB), lds, st, L, W, mask, N, n);
-  kt_end(kKcForward, st);
-  return hipGetLastError();
-}
-
 template <typename T>
 hipError_t trtri_blocked(const T* L, T* W, const uint8_t* mask, int B, int N, int n, hipStream_t st) {
   if (n > kMaxN) {
@@ -1352,20 +956,10 @@ hipError_t trtri_blocked(const T* L, T* W, const uint8_t* mask, int B, int N, in
     kt_end(kKcForward, st);
     return e;
   }
-  switch (n) {
-    case 32: return trtri_nb<T, 1, 32>(L, W, mask, B, N, n, st);
-    case 64: return trtri_nb<T, 2, 64>(L, W, mask, B, N, n, st);
-    case 96: return trtri_nb<T, 3, 96>(L, W, mask, B, N, n, st);
-    case 128: return trtri_nb<T, 4, 128>(L, W, mask, B, N, n, st);
-    default: break;
-  }
-  switch ((n + 31) / 32) {
-    case 1: return trtri_nb<T, 1, 0>(L, W, mask, B, N, n, st);
-    case 2: return trtri_nb<T, 2, 0>(L, W, mask, B, N, n, st);
-    case 3: return trtri_nb<T, 3, 0>(L, W, mask, B, N, n, st);
-    case 4: return trtri_nb<T, 4, 0>(L, W, mask, B, N, n, st);
-    default: return hipErrorInvalidValue;
-  }
+  kt_begin(kKcForward, st);
+  const hipError_t e = trtri_blocks<T>(L, W, mask, B, N, n, 0, n, st);
+  kt_end(kKcForward, st);
+  return e;
 }
 
 template <typename T>

@@ -57,6 +57,18 @@ hipError_t factor_level_blocked(T* L, T* E, const uint8_t* mask, int B, int N, i
                                 hipStream_t st, hipEvent_t after_potrf = nullptr, hipEvent_t after_trsm = nullptr,
                                 hipEvent_t before_trsm = nullptr, const T* Lsrc = nullptr, const T* Esrc = nullptr);
 
+hipError_t init_potrf_kernels();
+// Diagonal blocks (nd_potrf.hip): block (r0, r0) of size nb <= kMaxN of each
+// node's block of level lidx <- its Cholesky factor and, in its strict upper
+// triangle, the factor's transposed inverse (f64: FP32 storage computed in FP64;
+// Lsrc: read there instead of in place) ...
+template <typename T>
+hipError_t potrf_level(T* L, const uint8_t* mask, int B, int N, int n, int lidx, bool f64, const T* Lsrc, int r0,
+                       int nb, hipStream_t st);
+// ... and W <- tril(L) with the inverse, for every block.
+template <typename T>
+hipError_t trtri_blocks(const T* L, T* W, const uint8_t* mask, int B, int N, int n, int r0, int nb, hipStream_t st);
+
 // Per-node kernels for kMaxN < n <= kMaxNLarge (nd_large.hip): potrf with the
 // transposed inverse in the strict upper triangle; trsm of level lidx's R and
 // Lc; the forward (U^T x) or backward (U x) apply with U = Linv^T as stored,

@@ -150,7 +150,8 @@ constexpr PanelPlan panel_plan(int total) {
 // p[j]: NP payload rows per lane, p[j] <- p[j] L^-T.
 // NC: columns of the panel (a tile whose last 16 - NC rows and columns are
 // identity padding needs no steps for them; entries from NC on are untouched).
-// All 64 lanes must be active.  hook(k) runs before step k.
+// All 64 lanes must be active.  hook(k) runs before step k (k: an
+// integral_constant).
 //
 // Step k's multiply-adds other than the one that gives the next pivot are
 // spread between the dependent operations of the next pivot's reciprocal
@@ -170,7 +171,7 @@ __device__ __forceinline__ void panel16(T (&u)[16], T (&p)[NP][16], Hook hook = 
   wait_states<2>();
   static_for<NC>([&](auto kc) {
     constexpr int k = decltype(kc)::value;
-    hook(k);
+    hook(kc);
     u[k] = lk;  // row k itself: piv / sqrt(piv)
 #pragma unroll
     for (int j = 0; j < NP; ++j) p[j][k] = pk[j];
