@@ -1053,13 +1053,14 @@ hipError_t factor_with_forward(T* L, T* E, T* x, const uint8_t* factor_mask, con
   if (e == hipSuccess && side_first != nullptr) e = (*side_first)(ov.side);
   if (e == hipSuccess && side_first != nullptr) e = hipEventRecord(ov.ready, ov.side);
   for (int l = 0; l < Lv && e == hipSuccess; ++l) {
+    // one fork per level (each costs the main stream about 4 us in a graph):
+    // behind level l's trsm the side stream applies level l and updates from it
     const bool last = l == Lv - 1;
-    e = factor_level_blocked<T>(L, E, factor_mask, B, N, n, l, prec, st, ov.potrf[l],
+    e = factor_level_blocked<T>(L, E, factor_mask, B, N, n, l, prec, st, last ? ov.potrf[l] : nullptr,
                                 last ? nullptr : ov.trsm[l], (l == 0 && side_first != nullptr) ? ov.ready : nullptr,
                                 l == 0 ? Lsrc : nullptr, l == 0 ? Esrc : nullptr);
-    if (e == hipSuccess) e = hipStreamWaitEvent(ov.side, ov.potrf[l], 0);
+    if (e == hipSuccess) e = hipStreamWaitEvent(ov.side, last ? ov.potrf[l] : ov.trsm[l], 0);
     if (e == hipSuccess) e = forward_apply_blocked<T>(L, E, x, sweep_mask, B, N, n, m, l, ov.side);
-    if (e == hipSuccess && !last) e = hipStreamWaitEvent(ov.side, ov.trsm[l], 0);
     if (e == hipSuccess && !last) e = forward_update_blocked<T>(L, E, x, sweep_mask, B, N, n, m, l, ov.side);
   }
   if (e == hipSuccess) e = hipEventRecord(ov.join, ov.side);
