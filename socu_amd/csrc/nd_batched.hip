@@ -254,8 +254,7 @@ __device__ __forceinline__ void vprod(int n, int m, int kend, FA fa, FX fx, bool
 
 // Cholesky + inverse of every slot's A tile (lower: L, strict upper: L^-T,
 // dinv: 1/L[r][r]); `node` is this thread's task kind (a deferred target task
-// has no factor).  (NT = 32 keeps the 16x16-halves factor: the 32-wide pivot
-// pairs of tile_chol_inv need registers this kernel does not have.)
+// has no factor).
 template <typename T, int NT, int W>
 __device__ __forceinline__ void slots_chol(BSlot<T, NT>* slots, bool node) {
   constexpr int TP = BShape<NT, W>::TP;

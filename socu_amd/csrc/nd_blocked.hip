@@ -863,7 +863,7 @@ static hipError_t factor_level_nb(T* L, T* E, const uint8_t* mask, int B, int N,
   return hipGetLastError();
 }
 
-// One factor level for kMaxN < n <= kMaxNLarge: the tiled potrf and trsm of
+// One factor level for kMaxN < n <= kMaxNLarge: the diagonal blocks, R and Lc by
 // nd_large.hip, then the Schur updates of k_schur_blk (which walks any n).
 template <typename T>
 static hipError_t factor_level_large(T* L, T* E, const uint8_t* mask, int B, int N, int n, int lidx, hipStream_t st,
@@ -872,17 +872,11 @@ static hipError_t factor_level_large(T* L, T* E, const uint8_t* mask, int B, int
   const int Lv = recursive_iterations(N);
   const Level lv = level_info(N, lidx);
   if (lv.dim <= 0 || B <= 0) return hipSuccess;
-  kt_begin(kKcPotrf, st);
-  hipError_t e = potrf_large<T>(L, mask, B, N, n, lidx, st);
-  kt_end(kKcPotrf, st);
+  hipError_t e = before_trsm != nullptr ? hipStreamWaitEvent(st, before_trsm, 0) : hipSuccess;
+  if (e == hipSuccess) e = factor_large<T>(L, E, mask, B, N, n, lidx, st);
   if (e == hipSuccess && after_potrf != nullptr) e = hipEventRecord(after_potrf, st);
-  if (e != hipSuccess || lidx == Lv - 1) return e;
-  if (before_trsm != nullptr && (e = hipStreamWaitEvent(st, before_trsm, 0)) != hipSuccess) return e;
-  kt_begin(kKcTrsm, st);
-  e = trsm_large<T>(L, E, mask, B, N, n, lidx, st);
-  kt_end(kKcTrsm, st);
   if (e == hipSuccess && after_trsm != nullptr) e = hipEventRecord(after_trsm, st);
-  if (e != hipSuccess) return e;
+  if (e != hipSuccess || lidx == Lv - 1) return e;
   const int ntile = (n + kSTile - 1) / kSTile;
   const int ntri = ntile * (ntile + 1) / 2;
   const int nT = N / (2 * lv.s);

@@ -69,16 +69,11 @@ hipError_t potrf_level(T* L, const uint8_t* mask, int B, int N, int n, int lidx,
 template <typename T>
 hipError_t trtri_blocks(const T* L, T* W, const uint8_t* mask, int B, int N, int n, int r0, int nb, hipStream_t st);
 
-// Per-node kernels for kMaxN < n <= kMaxNLarge (nd_large.hip): potrf with the
-// transposed inverse in the strict upper triangle; trsm of level lidx's R and
-// Lc; the forward (U^T x) or backward (U x) apply with U = Linv^T as stored,
-// for level lidx's nodes; the sweep updates of level lidx; the inverse of a
-// factor from tril(L) alone into W.
+// kMaxN < n <= kMaxNLarge (nd_large.hip): a level's diagonal blocks, R and Lc; the
+// sweeps' products with the inverses and with R and Lc; the inverses alone.
 hipError_t init_large_kernels();
 template <typename T>
-hipError_t potrf_large(T* L, const uint8_t* mask, int B, int N, int n, int lidx, hipStream_t st);
-template <typename T>
-hipError_t trsm_large(const T* L, T* E, const uint8_t* mask, int B, int N, int n, int lidx, hipStream_t st);
+hipError_t factor_large(T* L, T* E, const uint8_t* mask, int B, int N, int n, int lidx, hipStream_t st);
 template <typename T>
 hipError_t apply_large(const T* L, T* x, const uint8_t* mask, int B, int N, int n, int m, int lidx, bool bwd,
                        hipStream_t st);

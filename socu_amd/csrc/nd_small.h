@@ -53,6 +53,18 @@ __device__ __forceinline__ void stg(T* base, int off, T v) {
   typedef __attribute__((address_space(1))) T* gptr;
   *(gptr)((gbytes)base + (unsigned)off * (unsigned)sizeof(T)) = v;
 }
+// Elements off, off + 1 of a block (no more than element alignment).
+template <typename T>
+struct Pair {
+  typedef T type __attribute__((ext_vector_type(2)));
+};
+template <typename T>
+__device__ __forceinline__ typename Pair<T>::type ldg2(const T* base, int off) {
+  typedef typename Pair<T>::type v2 __attribute__((aligned(sizeof(T))));
+  typedef const __attribute__((address_space(1))) char* gbytes;
+  typedef const __attribute__((address_space(1))) v2* gptr;
+  return *(gptr)((gbytes)base + (unsigned)off * (unsigned)sizeof(T));
+}
 template <typename P>
 __device__ __forceinline__ P* uniform_ptr(P* p) {
   const unsigned long long v = (unsigned long long)p;

@@ -20,19 +20,6 @@ namespace socu {
 
 namespace {
 
-// Elements off, off + 1 of a block (no more than element alignment).
-template <typename T>
-struct Pair {
-  typedef T type __attribute__((ext_vector_type(2)));
-};
-template <typename T>
-__device__ __forceinline__ typename Pair<T>::type ldg2(const T* base, int off) {
-  typedef typename Pair<T>::type v2 __attribute__((aligned(sizeof(T))));
-  typedef const __attribute__((address_space(1))) char* gbytes;
-  typedef const __attribute__((address_space(1))) v2* gptr;
-  return *(gptr)((gbytes)base + (unsigned)off * (unsigned)sizeof(T));
-}
-
 // What a launch does: a whole step, the updates alone, or the applies of the
 // nodes of level s alone.
 enum StepMode { kStepFull = 0, kStepUpdate = 1, kStepApply = 2 };

@@ -7,8 +7,8 @@
 //                fp64: lane l, reg r holds D[4*r+(l/16)][l%16]
 // * wave_gemm: a 32x32 (2x2 MFMA tiles) accumulation C += A B with A, B
 //   read from LDS through element strides.
-// * tile_chol_inv: Cholesky and inverse of a 32x32 diagonal tile by one
-//   wavefront, as two 16-column panels (nd_panel.h).
+// * tile_chol_inv16, 32b, _grouped: Cholesky and inverse of a diagonal tile by one
+//   wavefront (the strict upper triangle receives the transposed inverse).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -220,140 +220,12 @@ __device__ __forceinline__ void acc16_foreach(typename Mfma<T>::acc_t& acc, F f)
   for (int r = 0; r < 4; ++r) f(Mfma<T>::row(l, r), Mfma<T>::col(l, r), acc[r]);
 }
 
-// Cholesky and inverse of a 32x32 tile, executed by one whole wavefront.
-// S: tile in LDS, row-major with `pitch`; its lower triangle is the input.
-// On return the lower triangle holds L, the strict upper triangle holds the
-// transposed inverse (S[c][q] = Linv[q][c] for q > c) and dinv[r] = 1/L[r][r].
-// ut: a 32 x 33 LDS tile that receives Linv transposed in full (ut[r][c] =
-// Linv[c][r], zeros and diagonal included).
-//
-// Two 16-column panels (panel16) with one MFMA update between them.  Payload
-// rows of the first panel: the identity, giving U_11 = L_11^-T, and A_21,
-// giving L_21; of the second: U_12 = -U_11 L_21^T and the identity.  Each DPP
-// row g (16 lanes) loads its payload rows from where it stores them, except
-// that g = 2 repeats the identity rows to store L with U above its diagonal
-// in S, and g = 3 repeats U_12 to store it in ut.
-// hook(k) runs before pivot step k (a compile-time constant after unrolling):
-// a caller can issue loads there.
-template <typename T, typename Hook = NoHook>
-__device__ __forceinline__ void tile_chol_inv(T* S, int pitch, T* dinv, T* ut, Hook hook = Hook()) {
-  const int lane = lane_id();
-  const int r = lane & 15, g = lane >> 4;
-  // rows of the diagonal tiles whose L the lane stores beside U (none: -1)
-  const int rl = g == 2 ? r : -1;
-  T u[16], p[1][16];
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {  // the identity tiles and the zero tile of ut
-    const T e = (4 * c + g == r) ? T(1) : T(0);
-    ut[(4 * c + g) * 33 + r] = e;
-    ut[(16 + 4 * c + g) * 33 + 16 + r] = e;
-    ut[(16 + 4 * c + g) * 33 + r] = T(0);
-  }
-  typename Mfma<T>::acc_t s22;
-#pragma unroll
-  for (int c = 0; c < 4; ++c) s22[c] = S[(16 + Mfma<T>::row(lane, c)) * pitch + 16 + r];
-  wave_lds_order();
-  {
-    const T* urow = S + r * pitch;
-    T* prow = (g & 1) ? S + (16 + r) * pitch : ut + r * 33;
-#pragma unroll
-    for (int c = 0; c < 16; ++c) u[c] = urow[c];
-#pragma unroll
-    for (int c = 0; c < 16; ++c) p[0][c] = prow[c];
-#pragma unroll
-    for (int c = 0; c < 16; ++c) {
-      pin_reg(u[c]);
-      pin_reg(p[0][c]);
-    }
-    panel16<T, 1>(u, p, hook);
-    if (g == 2) prow = S + r * pitch;
-#pragma unroll
-    for (int c = 0; c < 16; ++c) prow[c] = (c <= rl) ? u[c] : p[0][c];
-  }
-  wave_lds_order();
-  {
-    // A_22 -= L_21 L_21^T and U_12 = -U_11 L_21^T: the B operand of both,
-    // and the A operand of the first, are the same entries of L_21
-    typename Mfma<T>::acc_t u12 = acc_zero<T>();
-    T l21[4], u11[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      l21[k] = S[(16 + r) * pitch + 4 * k + g];
-      u11[k] = ut[r * 33 + 4 * k + g];
-    }
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      s22 = Mfma<T>::mma(-l21[k], l21[k], s22);
-      u12 = Mfma<T>::mma(-u11[k], l21[k], u12);
-    }
-    acc16_foreach<T>(s22, [&](int i, int j, T v) { S[(16 + i) * pitch + 16 + j] = v; });
-    acc16_foreach<T>(u12, [&](int i, int j, T v) { S[i * pitch + 16 + j] = v; });
-  }
-  wave_lds_order();
-  {
-    const T* urow = S + (16 + r) * pitch + 16;
-    T* prow = (g == 1 || g == 2) ? ut + (16 + r) * 33 + 16 : S + r * pitch + 16;
-#pragma unroll
-    for (int c = 0; c < 16; ++c) u[c] = urow[c];
-#pragma unroll
-    for (int c = 0; c < 16; ++c) p[0][c] = prow[c];
-#pragma unroll
-    for (int c = 0; c < 16; ++c) {
-      pin_reg(u[c]);
-      pin_reg(p[0][c]);
-    }
-    panel16<T, 1>(u, p, [&](int k) { hook(16 + k); });
-    if (g == 2) prow = S + (16 + r) * pitch + 16;
-    if (g == 3) prow = ut + r * 33 + 16;
-#pragma unroll
-    for (int c = 0; c < 16; ++c) prow[c] = (c <= rl) ? u[c] : p[0][c];
-  }
-  wave_lds_order();
-  if (lane < 32) dinv[lane] = ut[lane * 33 + lane];
-}
-
-// Inverse of a 32x32 lower-triangular tile (no factorisation), by one
-// wavefront: lane c (of 0-31) forms column c of the inverse by forward
-// substitution, x_r = (delta_rc - sum_{k<r} D[r][k] x_k) / D[r][r], with
-// rows of D read as LDS broadcasts and four partial sums per row; lanes 32-63
-// repeat lanes 0-31 and store nothing.  Output convention of tile_chol_inv:
-// the strict upper triangle receives the transposed inverse
-// (S[c][q] = Dinv[q][c] for q > c), dinv[r] = 1/D[r][r]; the lower triangle
-// (the input) is unchanged.
-template <typename T>
-__device__ __forceinline__ void tile_tri_inv(T* S, int pitch, T* dinv) {
-  const int lane = lane_id();
-  const int c = lane & 31;
-  T x[32];
-#pragma unroll
-  for (int r = 0; r < 32; ++r) {
-    T s0 = T(0), s1 = T(0), s2 = T(0), s3 = T(0);
-#pragma unroll
-    for (int k = 0; k + 3 < r; k += 4) {
-      s0 = fma(S[r * pitch + k], x[k], s0);
-      s1 = fma(S[r * pitch + k + 1], x[k + 1], s1);
-      s2 = fma(S[r * pitch + k + 2], x[k + 2], s2);
-      s3 = fma(S[r * pitch + k + 3], x[k + 3], s3);
-    }
-#pragma unroll
-    for (int k = r & ~3; k < r; ++k) s0 = fma(S[r * pitch + k], x[k], s0);
-    const T dr = T(1) / S[r * pitch + r];
-    x[r] = (((r == c) ? T(1) : T(0)) - ((s0 + s1) + (s2 + s3))) * dr;
-  }
-  if (lane < 32) {
-#pragma unroll
-    for (int q = 0; q < 32; ++q)
-      if (q > c) S[c * pitch + q] = x[q];
-    dinv[c] = x[c];
-  }
-}
-
 // Cholesky and inverse of a 16x16 tile by lanes 0-31 of the wavefront (row
-// lanes 0-15, inverse lanes 16-31; lanes 32-63 must not call it), with the
-// recurrence and in/out convention of tile_chol_inv, one pivot per step.
+// lanes 0-15, inverse lanes 16-31; lanes 32-63 must not call it), one pivot per
+// step.  S's lower triangle is the input; it receives L, the strict upper
+// triangle the transposed inverse, dinv 1 / L[r][r].
 // col: 32 entries of wave-private LDS (the column buffer; all 32 are
-// overwritten at the end).  As in tile_chol_inv, row lanes keep their strict
-// upper entries unmasked (only their own updates touch them and they are not
+// overwritten at the end).  Row lanes keep their strict upper entries unmasked (only their own updates touch them and they are not
 // stored), the lane comparisons are made per step on a copy of the row index
 // the compiler cannot see through, and the loads and stores carry no
 // per-entry branches.
@@ -421,7 +293,7 @@ __device__ __forceinline__ typename Mfma<T>::acc_t mfma16x16x16(FA fa, FB fb) {
 
 // 32x32 Cholesky + inverse by one wavefront through 16x16 halves:
 // A11 = L11 L11^T; L21 = A21 L11^-T; A22 - L21 L21^T = L22 L22^T;
-// Linv21 = -Linv22 L21 Linv11.  Same in/out convention as tile_chol_inv.
+// Linv21 = -Linv22 L21 Linv11.  Same in/out convention.
 template <typename T>
 __device__ __forceinline__ void tile_chol_inv32b(T* S, int pitch, T* dinv, T* col) {
   const int l = lane_id();

@@ -7,7 +7,9 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-EDGES = [1, 7, 16, 17, 31, 32, 33, 48, 49, 64, 65, 79, 80, 81, 96, 97, 101, 112, 113, 127, 128]
+EDGES = [1, 7, 16, 17, 31, 32, 33, 48, 49, 64, 65, 79, 80, 81, 96, 97, 101, 112, 113, 127, 128,
+         # (two halves of 16 ceil(n / 32) rows and the rest)
+         129, 145, 160, 161, 192, 200, 223, 225, 255, 256]
 
 
 def _spd(n, B, seed):
