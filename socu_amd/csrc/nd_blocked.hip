@@ -4,10 +4,8 @@
 // atomics, so results are bitwise reproducible.
 //
 //   k_potrf_blk  (nd_potrf.hip) L_i and its inverse's transpose.
-//   k_trsm_blk   one workgroup per (node, 32-wide chunk of R rows / Lc cols):
-//                R <- R Linv^T, Lc <- Linv Lc as MFMA products with the stored
-//                inverse (replaces trsm_rltn / trsm_llnn, trsm.py:94-120,
-//                :202-228).
+//   k_large_panel (nd_large.hip) R <- R U, Lc <- U^T Lc with the stored inverse
+//                (replaces trsm_rltn / trsm_llnn, trsm.py:94-120, :202-228).
 //   k_schur_blk  one workgroup per 64x64 output tile, MFMA, owner computes:
 //                L_j -= R R^T + Lc^T Lc,  F -= R Lc (syrk.py, gemm.py).
 // (The sweeps: nd_small.hip, nd_steps.hip, nd_large.hip.)
@@ -24,332 +22,6 @@ namespace socu {
 // NF != 0 instantiates the kernels for a fixed block size n == NF (a multiple
 // of 32), so that all index arithmetic is compile-time; NF == 0 is the
 // general (padded) version.
-
-// ---------------------------------------------------------------------------
-// trsm with the explicit inverse left by k_potrf_blk in the strict upper
-// triangle of L_i (U[k][r] = Linv[r][k] for k < r, 1/L[r][r] on the diagonal):
-//   R task  (32 rows of R):   R  <- R Linv^T,   wave q: output columns 32q..
-//   Lc task (32 cols of Lc):  Lc <- Linv Lc,    wave q: output rows 32q..
-// Both are MFMA products with the upper tiles (kb, q), kb <= q, of U; no
-// sequential substitution remains.
-// ---------------------------------------------------------------------------
-// Eight wavefronts: output tile q of the chunk is summed over kb <= q by two
-// of them (kb below and from h(q) = (q + 1) / 2), which meet in LDS, so the
-// longest product chain is half as long as with one wavefront per tile.
-constexpr int kTrsmThreads = 512;
-
-// (output tile q, half) of wavefront w: waves w and w + 4 share a SIMD, and
-// these pairs carry at most three of the ten tile products of NB = 4
-// (q of waves 0..7: 3 3 2 2 0 0 1 1; half: 0 1 1 0 1 0 0 1).
-__device__ __forceinline__ void trsm_wave_task(int w, int& q, int& half) {
-  q = (0x50AF >> (2 * w)) & 3;
-  half = (0x96 >> w) & 1;
-}
-// k_trsm_blk splits only NB = 4 (n > 96); smaller blocks keep one wavefront
-// per output tile (with NB <= 2 most of eight wavefronts would idle, and
-// their workgroups, many per CU in batches, would hold twice the registers).
-constexpr int trsm_blk_threads(int nb) { return nb == 4 ? kTrsmThreads : kThreads; }
-
-template <typename T, int NB, int NF>
-__global__ __launch_bounds__(kTrsmThreads) void k_trsm_blk(const T* __restrict__ L, T* __restrict__ E,
-                                                      const uint8_t* __restrict__ mask, int N, int n_, int nE, int s,
-                                                      int off, const T* __restrict__ Esrc) {
-  const int n = NF ? NF : n_;
-  constexpr int NP = 32 * NB;
-  constexpr int TP = 33;  // tile pitch
-  constexpr int NT = NB * (NB + 1) / 2;
-  const int b = blockIdx.z;
-  if (masked_out(mask, b)) return;
-  const int i = s - 1 + 2 * s * blockIdx.x;
-  const bool isR = (int)blockIdx.y < NB;
-  const int c0 = (isR ? blockIdx.y : blockIdx.y - NB) * 32;
-  if (isR && !(i + s < N)) return;
-  if (!isR && !(i >= s)) return;
-  if (c0 >= n) return;
-  const int w = min(32, n - c0);
-
-  const T* A = L + ((size_t)b * N + i) * (size_t)n * n;
-  T* X = E + ((size_t)b * nE + off + (isR ? i / s : (i - s) / s)) * (size_t)n * n;
-  const T* Xin = (Esrc != nullptr) ? Esrc + (X - E) : X;  // out-of-place: R / Lc read from Esrc
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  T* Ut = reinterpret_cast<T*>(smem_raw);  // NT upper tiles (kb <= q) of U, 32 x TP each
-  T* Xs = Ut + NT * 32 * TP;                // R task: 32 x (NP+1); Lc task: NP x TP
-  constexpr int XP = NP + 1;
-  const int tid = threadIdx.x, wave = wave_id();
-
-  // Issue every load before storing any: upper tiles of U (diagonal entries
-  // turned into reciprocals, lower parts of diagonal tiles zeroed) and the
-  // 32-wide chunk of R or Lc.
-  // (All loads are unconditional from clamped addresses and pinned only
-  // after the last one is issued, so they are in flight together; the
-  // masking and reciprocals follow.)
-  constexpr int TT = trsm_blk_threads(NB);
-  constexpr bool SPLIT = TT == kTrsmThreads;
-  constexpr int PT = 32 * 32 / TT;
-  T uv[NT][PT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    int q = 0, kb = t;
-    while (kb > q) { kb -= q + 1; ++q; }  // t = q(q+1)/2 + kb, kb <= q
-#pragma unroll
-    for (int e = 0; e < PT; ++e) {
-      const int idx = tid + e * TT;
-      const int R = 32 * kb + (idx >> 5), C = 32 * q + (idx & 31);
-      uv[t][e] = A[(size_t)min(R, n - 1) * n + min(C, n - 1)];
-    }
-  }
-  constexpr int PZ = 32 * NP / TT;
-  T zv[PZ];
-#pragma unroll
-  for (int e = 0; e < PZ; ++e) {
-    const int idx = tid + e * TT;
-    const int rr = idx / NP, kr = idx - rr * NP;  // R[c0+rr][kr], row reads
-    const int kc = idx >> 5, cc = idx & 31;       // Lc[kc][c0+cc]
-    const size_t ar = (size_t)(c0 + min(rr, w - 1)) * n + min(kr, n - 1);
-    const size_t ac = (size_t)min(kc, n - 1) * n + c0 + min(cc, w - 1);
-    zv[e] = Xin[isR ? ar : ac];
-  }
-#pragma unroll
-  for (int t = 0; t < NT; ++t)
-#pragma unroll
-    for (int e = 0; e < PT; ++e) pin_reg(uv[t][e]);
-#pragma unroll
-  for (int e = 0; e < PZ; ++e) pin_reg(zv[e]);
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    int q = 0, kb = t;
-    while (kb > q) { kb -= q + 1; ++q; }
-#pragma unroll
-    for (int e = 0; e < PT; ++e) {
-      const int idx = tid + e * TT;
-      const int R = 32 * kb + (idx >> 5), C = 32 * q + (idx & 31);
-      const T g = uv[t][e];
-      uv[t][e] = (R < n && C < n) ? ((R < C) ? g : ((R == C) ? T(1) / g : T(0))) : ((R == C) ? T(1) : T(0));
-    }
-  }
-#pragma unroll
-  for (int e = 0; e < PZ; ++e) {
-    const int idx = tid + e * TT;
-    const int rr = idx / NP, kr = idx - rr * NP;
-    const int kc = idx >> 5, cc = idx & 31;
-    const bool ok = isR ? (rr < w && kr < n) : (cc < w && kc < n);
-    zv[e] = ok ? zv[e] : T(0);
-  }
-#pragma unroll
-  for (int t = 0; t < NT; ++t)
-#pragma unroll
-    for (int e = 0; e < PT; ++e) {
-      const int idx = tid + e * TT;
-      Ut[t * 32 * TP + (idx >> 5) * TP + (idx & 31)] = uv[t][e];
-    }
-#pragma unroll
-  for (int e = 0; e < PZ; ++e) {
-    const int idx = tid + e * TT;
-    if (isR) Xs[(idx / NP) * XP + (idx % NP)] = zv[e];
-    else Xs[(idx >> 5) * TP + (idx & 31)] = zv[e];
-  }
-  __syncthreads();
-
-  int q = wave, half = 0;
-  if constexpr (SPLIT) trsm_wave_task(wave, q, half);
-  const int kb0 = half ? (q + 1) / 2 : 0, kb1 = (half || !SPLIT) ? q + 1 : (q + 1) / 2;
-  typename Mfma<T>::acc_t acc[2][2] = {{acc_zero<T>(), acc_zero<T>()}, {acc_zero<T>(), acc_zero<T>()}};
-  if (q < NB) {
-    for (int kb = kb0; kb < kb1; ++kb) {
-      const T* Utile = Ut + (q * (q + 1) / 2 + kb) * 32 * TP;  // U[32kb.., 32q..]
-      if (isR) {
-        // out[r][c] += sum_k R[r][32kb+k] U[32kb+k][32q+c]
-        wave_gemm<T>(acc, Xs + 32 * kb, XP, 1, Utile, TP, 1, 32);
-      } else {
-        // out[r][c] += sum_k Linv[32q+r][32kb+k] Lc[32kb+k][c],  Linv[32q+r][32kb+k] = U[32kb+k][32q+r]
-        wave_gemm<T>(acc, Utile, 1, TP, Xs + 32 * kb * TP, TP, 1, 32);
-      }
-    }
-  }
-  // the upper half's sums go through the (now free) tiles of U
-  __syncthreads();
-  T* Red = Ut + q * 32 * TP;
-  if (q < NB && half) acc_foreach<T>(acc, [&](int r, int c, T v) { Red[r * TP + c] = v; });
-  __syncthreads();
-  if (q < NB && !half) {
-    if (isR) {
-      acc_foreach<T>(acc, [&](int r, int c, T v) {
-        const int C = 32 * q + c;
-        if (r < w && C < n) X[(size_t)(c0 + r) * n + C] = SPLIT ? v + Red[r * TP + c] : v;
-      });
-    } else {
-      acc_foreach<T>(acc, [&](int r, int c, T v) {
-        const int R = 32 * q + r;
-        if (c < w && R < n) X[(size_t)R * n + c0 + c] = SPLIT ? v + Red[r * TP + c] : v;
-      });
-    }
-  }
-}
-
-// The same products with a few chunks per workgroup, for wide levels:
-// k_trsm_blk reloads the node's upper tiles of U in each of its 2*NB
-// workgroups (8x the block at n=128), which dominates its HBM traffic when
-// every CU has work.  Here a workgroup stages U once and walks `cpb`
-// consecutive chunks of the node's list (its R row chunks, then its Lc column
-// chunks), the next chunk's loads in flight while the current one is
-// multiplied.
-template <typename T, int NB, int NF>
-__global__ __launch_bounds__(kTrsmThreads) void k_trsm_node(const T* __restrict__ L, T* __restrict__ E,
-                                                       const uint8_t* __restrict__ mask, int N, int n_, int nE, int s,
-                                                       int off, int cpb, const T* __restrict__ Esrc) {
-  const int n = NF ? NF : n_;
-  constexpr int NP = 32 * NB;
-  constexpr int TP = 33;
-  constexpr int NT = NB * (NB + 1) / 2;
-  constexpr int XP = NP + 1;
-  constexpr int PT = 32 * 32 / kTrsmThreads;
-  constexpr int PZ = 32 * NP / kTrsmThreads;
-  const int b = blockIdx.z;
-  if (masked_out(mask, b)) return;
-  const int i = s - 1 + 2 * s * blockIdx.x;
-  const bool hasR = i + s < N, hasC = i >= s;
-  const int nbn = (n + 31) / 32;  // chunks per block
-  const int all = (hasR ? nbn : 0) + (hasC ? nbn : 0);
-  // this workgroup's chunks: [q0, q0 + total) of the node's list
-  const int q0 = blockIdx.y * cpb;
-  const int total = min(cpb, all - q0);
-  if (total <= 0) return;
-  const size_t nn = (size_t)n * n;
-  const T* A = L + ((size_t)b * N + i) * nn;
-  T* XR = hasR ? E + ((size_t)b * nE + off + i / s) * nn : nullptr;        // R_i: block (i+s, i)
-  T* XC = hasC ? E + ((size_t)b * nE + off + (i - s) / s) * nn : nullptr;  // Lc_i: block (i, i-s)
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  T* Ut = reinterpret_cast<T*>(smem_raw);
-  T* Xs = Ut + NT * 32 * TP;
-  T* Red = Xs + (32 * XP > NP * TP ? 32 * XP : NP * TP);  // 4 tiles: the upper halves' sums
-  const int tid = threadIdx.x, wave = wave_id();
-  // chunk q: R rows 32c.. for q < nbn (if R exists), then Lc columns 32c..
-  auto chunk = [&](int q, bool& isR, int& c0, int& w, T*& X) {
-    isR = hasR && q < nbn;
-    const int c = isR ? q : q - (hasR ? nbn : 0);
-    c0 = 32 * c;
-    w = min(32, n - c0);
-    X = isR ? XR : XC;
-  };
-  // (out-of-place: R and Lc are read from Esrc, same layout)
-  auto zload = [&](T* zv, bool isR, int c0, int w, const T* Xd) {
-    const T* X = (Esrc != nullptr) ? Esrc + (Xd - E) : Xd;
-#pragma unroll
-    for (int e = 0; e < PZ; ++e) {
-      const int idx = tid + e * kTrsmThreads;
-      const int rr = idx / NP, kr = idx - rr * NP;  // R[c0+rr][kr], row reads
-      const int kc = idx >> 5, cc = idx & 31;       // Lc[kc][c0+cc]
-      const size_t ar = (size_t)(c0 + min(rr, w - 1)) * n + min(kr, n - 1);
-      const size_t ac = (size_t)min(kc, n - 1) * n + c0 + min(cc, w - 1);
-      zv[e] = X[isR ? ar : ac];
-    }
-  };
-  auto zstore = [&](T* zv, bool isR, int w) {
-#pragma unroll
-    for (int e = 0; e < PZ; ++e) {
-      const int idx = tid + e * kTrsmThreads;
-      const int rr = idx / NP, kr = idx - rr * NP;
-      const int kc = idx >> 5, cc = idx & 31;
-      const bool ok = isR ? (rr < w && kr < n) : (cc < w && kc < n);
-      const T v = ok ? zv[e] : T(0);
-      if (isR) Xs[(idx / NP) * XP + (idx % NP)] = v;
-      else Xs[(idx >> 5) * TP + (idx & 31)] = v;
-    }
-  };
-
-  // U tiles and the first chunk: every load issued before any is used
-  T uv[NT][PT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    int q = 0, kb = t;
-    while (kb > q) { kb -= q + 1; ++q; }
-#pragma unroll
-    for (int e = 0; e < PT; ++e) {
-      const int idx = tid + e * kTrsmThreads;
-      const int R = 32 * kb + (idx >> 5), C = 32 * q + (idx & 31);
-      uv[t][e] = A[(size_t)min(R, n - 1) * n + min(C, n - 1)];
-    }
-  }
-  bool isR;
-  int c0, w;
-  T* X;
-  chunk(q0, isR, c0, w, X);
-  T zv[PZ];
-  zload(zv, isR, c0, w, X);
-#pragma unroll
-  for (int t = 0; t < NT; ++t)
-#pragma unroll
-    for (int e = 0; e < PT; ++e) pin_reg(uv[t][e]);
-#pragma unroll
-  for (int e = 0; e < PZ; ++e) pin_reg(zv[e]);
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    int q = 0, kb = t;
-    while (kb > q) { kb -= q + 1; ++q; }
-#pragma unroll
-    for (int e = 0; e < PT; ++e) {
-      const int idx = tid + e * kTrsmThreads;
-      const int R = 32 * kb + (idx >> 5), C = 32 * q + (idx & 31);
-      const T g = uv[t][e];
-      Ut[t * 32 * TP + (idx >> 5) * TP + (idx & 31)] =
-          (R < n && C < n) ? ((R < C) ? g : ((R == C) ? T(1) / g : T(0))) : ((R == C) ? T(1) : T(0));
-    }
-  }
-  zstore(zv, isR, w);
-  __syncthreads();
-
-  for (int q = 0; q < total; ++q) {
-    const bool more = q + 1 < total;
-    bool isRn = false;
-    int c0n = 0, wn = 0;
-    T* Xn = nullptr;
-    if (more) {
-      chunk(q0 + q + 1, isRn, c0n, wn, Xn);
-      zload(zv, isRn, c0n, wn, Xn);  // in flight during the products below
-    }
-    {
-      // output tile qq, summed over kb <= qq by two wavefronts (see
-      // k_trsm_blk); the upper half's sums meet the lower half's in Red
-      int qq, half;
-      trsm_wave_task(wave, qq, half);
-      const int kb0 = half ? (qq + 1) / 2 : 0, kb1 = half ? qq + 1 : (qq + 1) / 2;
-      typename Mfma<T>::acc_t acc[2][2] = {{acc_zero<T>(), acc_zero<T>()}, {acc_zero<T>(), acc_zero<T>()}};
-      if (qq < NB)
-        for (int kb = kb0; kb < kb1; ++kb) {
-          const T* Utile = Ut + (qq * (qq + 1) / 2 + kb) * 32 * TP;  // U[32kb.., 32qq..]
-          if (isR) wave_gemm<T>(acc, Xs + 32 * kb, XP, 1, Utile, TP, 1, 32);
-          else wave_gemm<T>(acc, Utile, 1, TP, Xs + 32 * kb * TP, TP, 1, 32);
-        }
-      T* Rq = Red + qq * 32 * TP;
-      if (qq < NB && half) acc_foreach<T>(acc, [&](int r, int c, T v) { Rq[r * TP + c] = v; });
-      __syncthreads();
-      if (qq < NB && !half) {
-        if (isR) {
-          acc_foreach<T>(acc, [&](int r, int c, T v) {
-            const int C = 32 * qq + c;
-            if (r < w && C < n) X[(size_t)(c0 + r) * n + C] = v + Rq[r * TP + c];
-          });
-        } else {
-          acc_foreach<T>(acc, [&](int r, int c, T v) {
-            const int R = 32 * qq + r;
-            if (c < w && R < n) X[(size_t)R * n + c0 + c] = v + Rq[r * TP + c];
-          });
-        }
-      }
-    }
-    if (more) {
-#pragma unroll
-      for (int e = 0; e < PZ; ++e) pin_reg(zv[e]);
-      __syncthreads();  // every wave is done with the current chunk
-      zstore(zv, isRn, wn);
-      __syncthreads();
-      isR = isRn;
-      c0 = c0n;
-      w = wn;
-      X = Xn;
-    }
-  }
-}
 
 // ---------------------------------------------------------------------------
 // Schur-complement updates, 64x64 output tiles on MFMA
@@ -686,62 +358,6 @@ __global__ __launch_bounds__(kThreads) void k_schur_small(T* __restrict__ L, T* 
 // launchers
 // ---------------------------------------------------------------------------
 template <typename T, int NB>
-constexpr size_t trsm_blk_lds() {
-  // upper tiles + max(R chunk 32 x (NP+1), Lc chunk NP x 33)
-  return sizeof(T) * ((size_t)(NB * (NB + 1) / 2) * 32 * 33 +
-                      ((size_t)32 * (32 * NB + 1) > (size_t)(32 * NB) * 33 ? (size_t)32 * (32 * NB + 1)
-                                                                             : (size_t)(32 * NB) * 33));
-}
-
-// k_trsm_node: k_trsm_blk's LDS and four 32 x 33 tiles for the half sums
-template <typename T, int NB>
-constexpr size_t trsm_node_lds() {
-  return trsm_blk_lds<T, NB>() + sizeof(T) * 4 * 32 * 33;
-}
-
-template <typename T, int NB>
-static hipError_t set_blk_attrs() {
-  hipError_t e;
-  e = hipFuncSetAttribute((const void*)k_trsm_blk<T, NB, 0>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                          (int)trsm_blk_lds<T, NB>());
-  if (e != hipSuccess) return e;
-  e = hipFuncSetAttribute((const void*)k_trsm_blk<T, NB, 32 * NB>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                          (int)trsm_blk_lds<T, NB>());
-  if (e != hipSuccess) return e;
-  e = hipFuncSetAttribute((const void*)k_trsm_node<T, NB, 0>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                          (int)trsm_node_lds<T, NB>());
-  if (e != hipSuccess) return e;
-  e = hipFuncSetAttribute((const void*)k_trsm_node<T, NB, 32 * NB>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                          (int)trsm_node_lds<T, NB>());
-  return e;
-}
-
-// Whether a level's trsm takes k_trsm_node, and with how many chunks per
-// workgroup.  Measured on MI355X (N=512): for n > 96 and levels of at least
-// 64 nodes, two chunks per workgroup cut the n=128 factor by 9 us (FP32) and
-// 35 us (FP64); for n <= 64, or one workgroup per node, it was slower.
-// SOCU_TRSM_NODE=<min nodes> and SOCU_TRSM_CPB=<chunks> override.
-static int trsm_node_min(int nb) {
-  static int v = -2;
-  if (v == -2) {
-    const char* e = getenv("SOCU_TRSM_NODE");
-    v = e ? (atoi(e) < 1 ? 1 : atoi(e)) : -1;
-  }
-  if (v > 0) return v;
-  return nb == 4 ? 64 : (1 << 30);
-}
-
-static int trsm_chunks_per_block() {
-  static int v = -1;
-  if (v < 0) {
-    const char* e = getenv("SOCU_TRSM_CPB");
-    v = e ? atoi(e) : 2;
-    if (v < 1) v = 1;
-  }
-  return v;
-}
-
-template <typename T, int NB>
 static hipError_t set_schur_small_attrs() {
   const int lds = (int)schur_small_lds<T, NB>();
   hipError_t e = hipFuncSetAttribute((const void*)k_schur_small<T, NB, 0>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
@@ -781,12 +397,6 @@ static bool use_schur_small(int nodes, int n, int esize) {
 
 hipError_t init_blocked_kernels() {
   hipError_t e;
-  if ((e = set_blk_attrs<float, 2>()) != hipSuccess) return e;
-  if ((e = set_blk_attrs<float, 3>()) != hipSuccess) return e;
-  if ((e = set_blk_attrs<float, 4>()) != hipSuccess) return e;
-  if ((e = set_blk_attrs<double, 2>()) != hipSuccess) return e;
-  if ((e = set_blk_attrs<double, 3>()) != hipSuccess) return e;
-  if ((e = set_blk_attrs<double, 4>()) != hipSuccess) return e;
   if ((e = set_schur_small_attrs<float, 1>()) != hipSuccess) return e;
   if ((e = set_schur_small_attrs<float, 2>()) != hipSuccess) return e;
   if ((e = set_schur_small_attrs<float, 3>()) != hipSuccess) return e;
@@ -805,7 +415,6 @@ static hipError_t factor_level_nb(T* L, T* E, const uint8_t* mask, int B, int N,
   const int Lv = recursive_iterations(N);
   const Level lv = level_info(N, lidx);
   if (lv.dim <= 0 || B <= 0) return hipSuccess;
-  const size_t lds_trsm = trsm_blk_lds<T, NB>();
   const bool bf16 = (prec & kPrecBf16Schur) != 0 && sizeof(T) == 4;
   hipError_t ep = potrf_level<T>(L, mask, B, N, n, lidx, (prec & kPrecF64Pivots) != 0 && sizeof(T) == 4, Lsrc, 0, n, st);
   if (ep != hipSuccess) return ep;
@@ -818,18 +427,8 @@ static hipError_t factor_level_nb(T* L, T* E, const uint8_t* mask, int B, int N,
     const hipError_t e = hipStreamWaitEvent(st, before_trsm, 0);
     if (e != hipSuccess) return e;
   }
-  kt_begin(kKcTrsm, st);
-  if (B * lv.dim >= trsm_node_min(NB)) {
-    const int cpb = trsm_chunks_per_block();
-    const int groups = (2 * NB + cpb - 1) / cpb;
-    const size_t lds_node = trsm_node_lds<T, NB>();
-    hipLaunchKernelGGL((k_trsm_node<T, NB, NF>), dim3(lv.dim, groups, B), dim3(kTrsmThreads), lds_node, st, L, E,
-                       mask, N, n, nE, lv.s, lv.off, cpb, Esrc);
-  }
-  else
-    hipLaunchKernelGGL((k_trsm_blk<T, NB, NF>), dim3(lv.dim, 2 * NB, B), dim3(trsm_blk_threads(NB)), lds_trsm, st, L,
-                       E, mask, N, n, nE, lv.s, lv.off, Esrc);
-  kt_end(kKcTrsm, st);
+  ep = trsm_level<T>(L, E, Esrc, mask, B, N, n, lidx, st);
+  if (ep != hipSuccess) return ep;
   if (after_trsm != nullptr) {
     const hipError_t e = hipEventRecord(after_trsm, st);
     if (e != hipSuccess) return e;

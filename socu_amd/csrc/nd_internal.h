@@ -74,6 +74,10 @@ hipError_t trtri_blocks(const T* L, T* W, const uint8_t* mask, int B, int N, int
 hipError_t init_large_kernels();
 template <typename T>
 hipError_t factor_large(T* L, T* E, const uint8_t* mask, int B, int N, int n, int lidx, hipStream_t st);
+// n <= kMaxN: R <- R U, Lc <- U^T Lc of a level's nodes (read from Esrc if not NULL).
+template <typename T>
+hipError_t trsm_level(const T* L, T* E, const T* Esrc, const uint8_t* mask, int B, int N, int n, int lidx,
+                      hipStream_t st);
 template <typename T>
 hipError_t apply_large(const T* L, T* x, const uint8_t* mask, int B, int N, int n, int m, int lidx, bool bwd,
                        hipStream_t st);

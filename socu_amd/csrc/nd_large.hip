@@ -18,12 +18,14 @@
 //   kPanelSecond U12 <- U12 U22;  R2 <- R2 U22;  Lc2 <- U22^T Lc2
 //
 // (R1, R2: columns of R; Lc1, Lc2: rows of Lc), then the Schur updates of
-// k_schur_blk, which walks any n.
+// k_schur_blk, which walks any n.  For n <= 128, where the diagonal block is factored
+// whole, kPanelFirst is the level's products with U (R <- R U, Lc <- U^T Lc).
 //
 // Measured (FP64, n = 200, levels of few nodes): one workgroup factoring a whole
 // block, 32x32 tiles through HBM, took 205 us per level and the products with U 34;
 // the five launches take 22 + 7 + 8 + 19 + 7 us.  A sweep's apply took 27 us and its
-// update 36 (32-wide chunks, tiles through LDS one by one): 13 and 9.  What bounds
+// update 36 (32-wide chunks, tiles through LDS one by one): 13 and 9.  For n = 128 the
+// products with U took 12 us (U staged in LDS by each of 8 workgroups per node): 7.  What bounds
 // them now: the halves' pivot chains (see nd_potrf.hip); the products' launches,
 // their loads (one compute unit's misses, 23 bytes/ns).  FP64 factor_and_solve
 // n=200 N=64 m=2: 2468 -> 1062 us.
@@ -37,10 +39,9 @@ namespace socu {
 
 namespace {
 
-constexpr int kPanelThreads = 512;
 constexpr int kPP = 17;  // pitch of a staged chunk: 16 columns
 
-int first_half(int n) { return 16 * ((n + 31) / 32); }
+int first_half(int n) { return n > kMaxN ? 16 * ((n + 31) / 32) : n; }
 
 // The left operand of a product, A(r, k), from a row-major matrix M.
 enum LeftForm {
@@ -134,11 +135,11 @@ __device__ __forceinline__ void stage_chunk(T* X, const Chunk<T>& c, int K) {
 
 // out(r, c) = A X (mode 0), -A X (1) or out - A X (2), row tiles t0 + wavefront, ...
 // of R rows; lower: rows r >= ... of a symmetric result only up to tile tmax.
-template <typename T, int FORM, bool TR>
+template <typename T, int FORM, bool TR, int TH>
 __device__ __forceinline__ void panel_product(const T* M, int ld, int R, int K, const T* X, const Chunk<T>& out,
                                               int mode, int tmax) {
   const int lane = lane_id(), li = lane & 15, w = wave_uniform();
-  for (int t = w; t < tmax; t += kPanelThreads / 64) {
+  for (int t = w; t < tmax; t += TH / 64) {
     typename Mfma<T>::acc_t acc = acc_zero<T>();
     int off[4];
     T c[4];
@@ -168,8 +169,8 @@ enum PanelPhase { kPanelFirst, kPanelUpdate, kPanelSecond, kPanelInverse, kPanel
 // Workgroup (node, chunk of 16 vectors): see above.  kPanelInverse and
 // kPanelInverseSecond: the U12 products alone, for every block (s = 0), L21 being
 // read from Lsrc; kPanelForward / kPanelBackward: x_i <- U^T x_i / U x_i.
-template <typename T>
-__global__ __launch_bounds__(kPanelThreads) void k_large_panel(T* L, const T* Lsrc, T* E, T* x,
+template <typename T, int TH>
+__global__ __launch_bounds__(TH) void k_large_panel(T* L, const T* Lsrc, T* E, const T* Esrc, T* x,
                                                               const uint8_t* __restrict__ mask, int N, int n, int n1,
                                                               int m, int nE, int s, int off, int phase) {
   __shared__ T X[kMaxNLarge * kPP];
@@ -185,10 +186,10 @@ __global__ __launch_bounds__(kPanelThreads) void k_large_panel(T* L, const T* Ls
   if (phase == kPanelForward || phase == kPanelBackward) {
     const int c0 = 16 * y;
     const Chunk<T> v{x + ((size_t)b * N + i) * n * m + c0, m, min(16, m - c0), false};
-    stage_chunk<T, kPanelThreads>(X, v, n);
+    stage_chunk<T, TH>(X, v, n);
     __syncthreads();
-    if (phase == kPanelForward) panel_product<T, kTriCols, false>(A, n, n, n, X, v, 0, cn);
-    else panel_product<T, kTriRows, false>(A, n, n, n, X, v, 0, cn);
+    if (phase == kPanelForward) panel_product<T, kTriCols, false, TH>(A, n, n, n, X, v, 0, cn);
+    else panel_product<T, kTriRows, false, TH>(A, n, n, n, X, v, 0, cn);
     return;
   }
   if (phase == kPanelInverse || phase == kPanelUpdate) {
@@ -196,19 +197,19 @@ __global__ __launch_bounds__(kPanelThreads) void k_large_panel(T* L, const T* Ls
     // (what a chunk reads and writes does not overlap: the cast is for its type)
     if (y < c2) {  // U12 columns 16 y ..
       const Chunk<T> v{const_cast<T*>(L21) + (size_t)16 * y * n, n, min(16, n2 - 16 * y), true};
-      stage_chunk<T, kPanelThreads>(X, v, n1);
+      stage_chunk<T, TH>(X, v, n1);
       __syncthreads();
       const Chunk<T> o{A + n1 + 16 * y, n, v.count, false};
-      panel_product<T, kTriRows, false>(A, n, n1, n1, X, o, 1, c1);
+      panel_product<T, kTriRows, false, TH>(A, n, n1, n1, X, o, 1, c1);
       return;
     }
     y -= c2;
     if (y < c2) {  // A22 rows 16 y .., up to their diagonal tile
       const Chunk<T> v{const_cast<T*>(L21) + (size_t)16 * y * n, n, min(16, n2 - 16 * y), true};
-      stage_chunk<T, kPanelThreads>(X, v, n1);
+      stage_chunk<T, TH>(X, v, n1);
       __syncthreads();
       const Chunk<T> o{A + (size_t)(n1 + 16 * y) * n + n1, n, v.count, true};
-      panel_product<T, kRows, true>(L21, n, n2, n1, X, o, 2, y + 1);
+      panel_product<T, kRows, true, TH>(L21, n, n2, n1, X, o, 2, y + 1);
       return;
     }
     y -= c2;
@@ -216,18 +217,18 @@ __global__ __launch_bounds__(kPanelThreads) void k_large_panel(T* L, const T* Ls
       if (i + s >= N) return;
       T* const R = Eb + (size_t)(off + i / s) * nn + (size_t)16 * y * n;
       const Chunk<T> v{R, n, min(16, n - 16 * y), true}, o{R + n1, n, v.count, true};
-      stage_chunk<T, kPanelThreads>(X, v, n1);
+      stage_chunk<T, TH>(X, v, n1);
       __syncthreads();
-      panel_product<T, kRows, true>(L21, n, n2, n1, X, o, 2, c2);
+      panel_product<T, kRows, true, TH>(L21, n, n2, n1, X, o, 2, c2);
       return;
     }
     y -= cn;
     if (i < s) return;
     T* const C = Eb + (size_t)(off + (i - s) / s) * nn + 16 * y;  // Lc columns
     const Chunk<T> v{C, n, min(16, n - 16 * y), false}, o{C + (size_t)n1 * n, n, v.count, false};
-    stage_chunk<T, kPanelThreads>(X, v, n1);
+    stage_chunk<T, TH>(X, v, n1);
     __syncthreads();
-    panel_product<T, kRows, false>(L21, n, n2, n1, X, o, 2, c2);
+    panel_product<T, kRows, false, TH>(L21, n, n2, n1, X, o, 2, c2);
     return;
   }
   // products with U11 (kPanelFirst) or U22, in place
@@ -246,10 +247,12 @@ __global__ __launch_bounds__(kPanelThreads) void k_large_panel(T* L, const T* Ls
     y -= ct + cn;
     v = Chunk<T>{Eb + (size_t)(off + (i - s) / s) * nn + (size_t)h * n + 16 * y, n, min(16, n - 16 * y), false};
   }
-  stage_chunk<T, kPanelThreads>(X, v, K);
+  Chunk<T> in = v;
+  if (Esrc != nullptr) in.p = const_cast<T*>(Esrc) + (v.p - E);  // (R and Lc alone: n <= kMaxN)
+  stage_chunk<T, TH>(X, in, K);
   __syncthreads();
-  if (v.rows) panel_product<T, kTriCols, true>(U, n, K, K, X, v, 0, (K + 15) / 16);
-  else panel_product<T, kTriCols, false>(U, n, K, K, X, v, 0, (K + 15) / 16);
+  if (v.rows) panel_product<T, kTriCols, true, TH>(U, n, K, K, X, v, 0, (K + 15) / 16);
+  else panel_product<T, kTriCols, false, TH>(U, n, K, K, X, v, 0, (K + 15) / 16);
 }
 
 // Sweep updates, one workgroup per (block, 16-row tile, 16 right-hand sides), grid
@@ -315,11 +318,18 @@ hipError_t set_attrs() {
 }
 
 template <typename T>
-hipError_t launch_panel(T* L, const T* Lsrc, T* E, T* x, const uint8_t* mask, int B, int N, int n, int m, int nodes,
-                        int chunks, int s, int off, int phase, hipStream_t st) {
+hipError_t launch_panel(T* L, const T* Lsrc, T* E, const T* Esrc, T* x, const uint8_t* mask, int B, int N, int n,
+                        int m, int nodes, int chunks, int s, int off, int phase, hipStream_t st) {
   if (nodes <= 0 || chunks <= 0 || B <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_large_panel<T>, dim3(nodes, chunks, B), dim3(kPanelThreads), 0, st, L, Lsrc, E, x, mask, N, n,
-                     first_half(n), m, (int)off_diag_storage_len(N), s, off, phase);
+  auto go = [&](auto th) {
+    constexpr int TH = decltype(th)::value;
+    hipLaunchKernelGGL((k_large_panel<T, TH>), dim3(nodes, chunks, B), dim3(TH), 0, st, L, Lsrc, E, Esrc, x, mask, N, n,
+                       first_half(n), m, (int)off_diag_storage_len(N), s, off, phase);
+  };
+  // (a wavefront per 16-row tile, up to eight)
+  if (n <= 32) go(std::integral_constant<int, 128>{});
+  else if (n <= 64) go(std::integral_constant<int, 256>{});
+  else go(std::integral_constant<int, 512>{});
   return hipGetLastError();
 }
 
@@ -341,14 +351,26 @@ hipError_t factor_large(T* L, T* E, const uint8_t* mask, int B, int N, int n, in
   hipError_t e = potrf_level<T>(L, mask, B, N, n, lidx, false, none, 0, n1, st);
   kt_begin(kKcTrsm, st);
   if (e == hipSuccess)
-    e = launch_panel<T>(L, none, E, none, mask, B, N, n, 1, lv.dim, c2 + ce, lv.s, lv.off, kPanelFirst, st);
+    e = launch_panel<T>(L, none, E, none, none, mask, B, N, n, 1, lv.dim, c2 + ce, lv.s, lv.off, kPanelFirst, st);
   if (e == hipSuccess)
-    e = launch_panel<T>(L, none, E, none, mask, B, N, n, 1, lv.dim, 2 * c2 + ce, lv.s, lv.off, kPanelUpdate, st);
+    e = launch_panel<T>(L, none, E, none, none, mask, B, N, n, 1, lv.dim, 2 * c2 + ce, lv.s, lv.off, kPanelUpdate, st);
   kt_end(kKcTrsm, st);
   if (e == hipSuccess) e = potrf_level<T>(L, mask, B, N, n, lidx, false, none, n1, n2, st);
   kt_begin(kKcTrsm, st);
   if (e == hipSuccess)
-    e = launch_panel<T>(L, none, E, none, mask, B, N, n, 1, lv.dim, c1 + ce, lv.s, lv.off, kPanelSecond, st);
+    e = launch_panel<T>(L, none, E, none, none, mask, B, N, n, 1, lv.dim, c1 + ce, lv.s, lv.off, kPanelSecond, st);
+  kt_end(kKcTrsm, st);
+  return e;
+}
+
+template <typename T>
+hipError_t trsm_level(const T* L, T* E, const T* Esrc, const uint8_t* mask, int B, int N, int n, int lidx,
+                      hipStream_t st) {
+  if (n > kMaxN) return hipErrorInvalidValue;
+  const Level lv = level_info(N, lidx);
+  kt_begin(kKcTrsm, st);
+  const hipError_t e = launch_panel<T>(const_cast<T*>(L), nullptr, E, Esrc, nullptr, mask, B, N, n, 1, lv.dim,
+                                       2 * ((n + 15) / 16), lv.s, lv.off, kPanelFirst, st);
   kt_end(kKcTrsm, st);
   return e;
 }
@@ -358,7 +380,7 @@ hipError_t apply_large(const T* L, T* x, const uint8_t* mask, int B, int N, int 
                        hipStream_t st) {
   const Level lv = level_info(N, lidx);
   // (L is only read in these phases)
-  return launch_panel<T>(const_cast<T*>(L), nullptr, nullptr, x, mask, B, N, n, m, lv.dim, (m + 15) / 16, lv.s, 0,
+  return launch_panel<T>(const_cast<T*>(L), nullptr, nullptr, nullptr, x, mask, B, N, n, m, lv.dim, (m + 15) / 16, lv.s, 0,
                          bwd ? kPanelBackward : kPanelForward, st);
 }
 
@@ -388,14 +410,17 @@ hipError_t trtri_large(const T* L, T* W, const uint8_t* mask, int B, int N, int 
   hipError_t e = trtri_blocks<T>(L, W, mask, B, N, n, 0, n1, st);
   if (e == hipSuccess) e = trtri_blocks<T>(L, W, mask, B, N, n, n1, n2, st);
   if (e == hipSuccess)
-    e = launch_panel<T>(W, L, none, none, mask, B, N, n, 1, N, (n2 + 15) / 16, 0, 0, kPanelInverse, st);
+    e = launch_panel<T>(W, L, none, none, none, mask, B, N, n, 1, N, (n2 + 15) / 16, 0, 0, kPanelInverse, st);
   if (e == hipSuccess)
-    e = launch_panel<T>(W, none, none, none, mask, B, N, n, 1, N, (n1 + 15) / 16, 0, 0, kPanelInverseSecond, st);
+    e = launch_panel<T>(W, none, none, none, none, mask, B, N, n, 1, N, (n1 + 15) / 16, 0, 0, kPanelInverseSecond, st);
   return e;
 }
 
 template hipError_t factor_large<float>(float*, float*, const uint8_t*, int, int, int, int, hipStream_t);
 template hipError_t factor_large<double>(double*, double*, const uint8_t*, int, int, int, int, hipStream_t);
+template hipError_t trsm_level<float>(const float*, float*, const float*, const uint8_t*, int, int, int, int, hipStream_t);
+template hipError_t trsm_level<double>(const double*, double*, const double*, const uint8_t*, int, int, int, int,
+                                       hipStream_t);
 template hipError_t apply_large<float>(const float*, float*, const uint8_t*, int, int, int, int, int, bool,
                                        hipStream_t);
 template hipError_t apply_large<double>(const double*, double*, const uint8_t*, int, int, int, int, int, bool,
