@@ -203,8 +203,7 @@ __global__ __launch_bounds__(kThreads) void k_schur_blk(T* __restrict__ L, T* __
 }
 
 // ---------------------------------------------------------------------------
-// Schur-complement updates for levels with few nodes.  k_schur_blk walks K in
-// chunks, one global round trip per chunk, which at the upper levels (a
+// BF16 Schur products for levels with few nodes.  k_schur_blk walks K in chunks, one global round trip per chunk, which at the upper levels (a
 // handful of tiles) is the whole cost.  Here a task is a 32x32 output tile
 // (4x more tasks) and issues every load it needs at once: the 32-wide panels
 // of its operands (all of K) and its own C values, then one LDS staging and
@@ -357,31 +356,32 @@ __global__ __launch_bounds__(kThreads) void k_schur_small(T* __restrict__ L, T* 
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
-template <typename T, int NB>
+template <int NB>
 static hipError_t set_schur_small_attrs() {
-  const int lds = (int)schur_small_lds<T, NB>();
-  hipError_t e = hipFuncSetAttribute((const void*)k_schur_small<T, NB, 0>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  const int lds = (int)schur_small_lds<float, NB>();
+  hipError_t e = hipFuncSetAttribute((const void*)k_schur_small<float, NB, 0, true>,
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (e == hipSuccess)
-    e = hipFuncSetAttribute((const void*)k_schur_small<T, NB, 32 * NB>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  if constexpr (sizeof(T) == 4) {  // BF16 products (float storage only)
-    if (e == hipSuccess)
-      e = hipFuncSetAttribute((const void*)k_schur_small<T, NB, 0, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              lds);
-    if (e == hipSuccess)
-      e = hipFuncSetAttribute((const void*)k_schur_small<T, NB, 32 * NB, true>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  }
+    e = hipFuncSetAttribute((const void*)k_schur_small<float, NB, 32 * NB, true>,
+                            hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   return e;
 }
 
-// Whether a level's Schur updates (nodes = targets + fill-ins over the batch)
-// take k_schur_small.  Its panel loads repeat each operand per output tile,
-// which only costs where the level streams many blocks; measured on MI355X
-// (N=512, 1024) the small kernel wins up to about 12 MiB of the level's
-// blocks: n=128 FP64 factor 1207 -> 1093 us, FP32 875 -> 767 us, n=32 FP64
-// 265 -> 197 us.  For n <= 32 it is taken at every level: k_schur_blk's
-// 64x64 output tiles leave three of four quarters outside a 32x32 block
-// (B=256 n=32 N=128 m=4 FP64 factor_and_solve: 2.36 -> 1.65 ms).
+// Whether a level's Schur updates (nodes = targets + fill-ins over the batch) take
+// k_schur_blk rather than 16x16 tiles (k_schur_tile, nd_large.hip), which read each
+// operand once per tile: where a level streams many blocks and the 64x64 tiles are
+// all inside the block.  n = 128, FP64, levels of 256, 128, 64 and 32 nodes: 99, 58,
+// 33 us (and 22 in 32x32 tiles with all of K staged in LDS) to 116, 60, 32 and 18;
+// n = 200: 76 us (32 nodes) to 54.
+static bool use_schur_blk(int nodes, int n, int esize) {
+  return (n + 15) / 16 % 4 == 0 && (double)nodes * n * n * esize > 16.0 * 1024 * 1024;
+}
+
+// Whether a level's BF16 Schur products take k_schur_small.  Its panel loads repeat
+// each operand per output tile, which only costs where the level streams many
+// blocks; it wins up to about 12 MiB of the level's blocks (N=512, 1024), and for
+// n <= 32 at every level: k_schur_blk's 64x64 output tiles leave three of four
+// quarters outside a 32x32 block.
 // SOCU_SCHUR_SMALL=<nodes> replaces the rule by a node count (0 disables the
 // small kernel).
 static bool use_schur_small(int nodes, int n, int esize) {
@@ -397,13 +397,10 @@ static bool use_schur_small(int nodes, int n, int esize) {
 
 hipError_t init_blocked_kernels() {
   hipError_t e;
-  if ((e = set_schur_small_attrs<float, 1>()) != hipSuccess) return e;
-  if ((e = set_schur_small_attrs<float, 2>()) != hipSuccess) return e;
-  if ((e = set_schur_small_attrs<float, 3>()) != hipSuccess) return e;
-  if ((e = set_schur_small_attrs<float, 4>()) != hipSuccess) return e;
-  if ((e = set_schur_small_attrs<double, 2>()) != hipSuccess) return e;
-  if ((e = set_schur_small_attrs<double, 3>()) != hipSuccess) return e;
-  if ((e = set_schur_small_attrs<double, 4>()) != hipSuccess) return e;
+  if ((e = set_schur_small_attrs<1>()) != hipSuccess) return e;
+  if ((e = set_schur_small_attrs<2>()) != hipSuccess) return e;
+  if ((e = set_schur_small_attrs<3>()) != hipSuccess) return e;
+  if ((e = set_schur_small_attrs<4>()) != hipSuccess) return e;
   return hipSuccess;
 }
 
@@ -442,20 +439,26 @@ static hipError_t factor_level_nb(T* L, T* E, const uint8_t* mask, int B, int N,
   const int tasks = nT * ntri + nF * ntile * ntile;
   if (tasks > 0) {
     kt_begin(kKcSchur, st);
-    if (use_schur_small(B * (nT + nF), n, (int)sizeof(T))) {
-      const int nsmall = nT * (NB * (NB + 1) / 2) + nF * NB * NB;
-      const size_t lds_small = schur_small_lds<T, NB>();
-      auto k = k_schur_small<T, NB, NF, false>;
-      if constexpr (sizeof(T) == 4)
-        if (bf16) k = k_schur_small<T, NB, NF, true>;
-      hipLaunchKernelGGL(k, dim3(nsmall, B), dim3(kThreads), lds_small, st, L, E, mask, N, n, nE, lv.s, lv.off,
-                         lv.next_off, nT, Lsrc);
-    } else {
-      auto k = k_schur_blk<T, NF, false>;
-      if constexpr (sizeof(T) == 4)
-        if (bf16) k = k_schur_blk<T, NF, true>;
-      hipLaunchKernelGGL(k, dim3(8 * schur_blk_per_xcd(nT, nF, ntile), B), dim3(kThreads), 0, st, L, E, mask, N, n, nE,
-                         lv.s, lv.off, lv.next_off, nT, nF, ntile, Lsrc);
+    const int nodes = B * (nT + nF);
+    const dim3 grid_blk(8 * schur_blk_per_xcd(nT, nF, ntile), B);
+    if (!bf16) {
+      if (!use_schur_blk(nodes, n, (int)sizeof(T))) {
+        ep = schur_tiles<T>(L, Lsrc, E, mask, B, N, n, lidx, nT, nF, st);
+        if (ep != hipSuccess) return ep;
+      } else {
+        hipLaunchKernelGGL((k_schur_blk<T, NF, false>), grid_blk, dim3(kThreads), 0, st, L, E, mask, N, n, nE, lv.s,
+                           lv.off, lv.next_off, nT, nF, ntile, Lsrc);
+      }
+    }
+    if constexpr (sizeof(T) == 4) {
+      if (bf16 && use_schur_small(nodes, n, (int)sizeof(T))) {
+        const int nsmall = nT * (NB * (NB + 1) / 2) + nF * NB * NB;
+        hipLaunchKernelGGL((k_schur_small<T, NB, NF, true>), dim3(nsmall, B), dim3(kThreads),
+                           (schur_small_lds<T, NB>()), st, L, E, mask, N, n, nE, lv.s, lv.off, lv.next_off, nT, Lsrc);
+      } else if (bf16) {
+        hipLaunchKernelGGL((k_schur_blk<T, NF, true>), grid_blk, dim3(kThreads), 0, st, L, E, mask, N, n, nE, lv.s,
+                           lv.off, lv.next_off, nT, nF, ntile, Lsrc);
+      }
     }
     kt_end(kKcSchur, st);
   }
@@ -463,11 +466,10 @@ static hipError_t factor_level_nb(T* L, T* E, const uint8_t* mask, int B, int N,
 }
 
 // One factor level for kMaxN < n <= kMaxNLarge: the diagonal blocks, R and Lc by
-// nd_large.hip, then the Schur updates of k_schur_blk (which walks any n).
+// nd_large.hip, then the Schur updates by 16x16 tiles.
 template <typename T>
 static hipError_t factor_level_large(T* L, T* E, const uint8_t* mask, int B, int N, int n, int lidx, hipStream_t st,
                                      hipEvent_t after_potrf, hipEvent_t after_trsm, hipEvent_t before_trsm) {
-  const int nE = (int)off_diag_storage_len(N);
   const int Lv = recursive_iterations(N);
   const Level lv = level_info(N, lidx);
   if (lv.dim <= 0 || B <= 0) return hipSuccess;
@@ -476,20 +478,14 @@ static hipError_t factor_level_large(T* L, T* E, const uint8_t* mask, int B, int
   if (e == hipSuccess && after_potrf != nullptr) e = hipEventRecord(after_potrf, st);
   if (e == hipSuccess && after_trsm != nullptr) e = hipEventRecord(after_trsm, st);
   if (e != hipSuccess || lidx == Lv - 1) return e;
-  const int ntile = (n + kSTile - 1) / kSTile;
-  const int ntri = ntile * (ntile + 1) / 2;
   const int nT = N / (2 * lv.s);
   int nF = 0;
   for (int t = 1; t < lv.dim; ++t)
     if (lv.s - 1 + 2 * lv.s * t + lv.s < N) ++nF;
-  const int tasks = nT * ntri + nF * ntile * ntile;
-  if (tasks > 0) {
-    kt_begin(kKcSchur, st);
-    hipLaunchKernelGGL((k_schur_blk<T, 0, false>), dim3(8 * schur_blk_per_xcd(nT, nF, ntile), B), dim3(kThreads), 0, st,
-                       L, E, mask, N, n, nE, lv.s, lv.off, lv.next_off, nT, nF, ntile, (const T*)nullptr);
-    kt_end(kKcSchur, st);
-  }
-  return hipGetLastError();
+  kt_begin(kKcSchur, st);
+  e = schur_tiles<T>(L, nullptr, E, mask, B, N, n, lidx, nT, nF, st);
+  kt_end(kKcSchur, st);
+  return e;
 }
 
 template <typename T>

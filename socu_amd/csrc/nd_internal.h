@@ -74,6 +74,10 @@ hipError_t trtri_blocks(const T* L, T* W, const uint8_t* mask, int B, int N, int
 hipError_t init_large_kernels();
 template <typename T>
 hipError_t factor_large(T* L, T* E, const uint8_t* mask, int B, int N, int n, int lidx, hipStream_t st);
+// Any n: a level's Schur updates by 16x16 tiles (targets read from Lsrc if not NULL).
+template <typename T>
+hipError_t schur_tiles(T* L, const T* Lsrc, T* E, const uint8_t* mask, int B, int N, int n, int lidx, int nT, int nF,
+                       hipStream_t st);
 // n <= kMaxN: R <- R U, Lc <- U^T Lc of a level's nodes (read from Esrc if not NULL).
 template <typename T>
 hipError_t trsm_level(const T* L, T* E, const T* Esrc, const uint8_t* mask, int B, int N, int n, int lidx,

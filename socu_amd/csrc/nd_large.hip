@@ -17,18 +17,18 @@
 //   potrf        L22, U22 <- A22
 //   kPanelSecond U12 <- U12 U22;  R2 <- R2 U22;  Lc2 <- U22^T Lc2
 //
-// (R1, R2: columns of R; Lc1, Lc2: rows of Lc), then the Schur updates of
-// k_schur_blk, which walks any n.  For n <= 128, where the diagonal block is factored
-// whole, kPanelFirst is the level's products with U (R <- R U, Lc <- U^T Lc).
+// (R1, R2: columns of R; Lc1, Lc2: rows of Lc), then the Schur updates
+// (k_schur_tile).  For n <= 128, where the diagonal block is factored whole,
+// kPanelFirst is the level's products with U (R <- R U, Lc <- U^T Lc).
 //
 // Measured (FP64, n = 200, levels of few nodes): one workgroup factoring a whole
 // block, 32x32 tiles through HBM, took 205 us per level and the products with U 34;
 // the five launches take 22 + 7 + 8 + 19 + 7 us.  A sweep's apply took 27 us and its
 // update 36 (32-wide chunks, tiles through LDS one by one): 13 and 9.  For n = 128 the
-// products with U took 12 us (U staged in LDS by each of 8 workgroups per node): 7.  What bounds
-// them now: the halves' pivot chains (see nd_potrf.hip); the products' launches,
-// their loads (one compute unit's misses, 23 bytes/ns).  FP64 factor_and_solve
-// n=200 N=64 m=2: 2468 -> 1062 us.
+// products with U took 12 us (U staged in LDS by each of 8 workgroups per node): 7.
+// What bounds them now: the halves' pivot chains (see nd_potrf.hip); the products'
+// launches, their loads (one compute unit's misses, 23 bytes/ns).  FP64 factor_and_solve
+// n=200 N=64 m=2: 2468 -> 1062 us (868 with the Schur tiles).
 #include "../../include/socu_hip.h"
 #include "nd_common.h"
 #include "nd_internal.h"
@@ -303,6 +303,109 @@ __global__ __launch_bounds__(kThreads) void k_update_large(const T* __restrict__
   }
 }
 
+// Schur updates, one workgroup per 16x16 output tile, grid
+// (tasks, B):
+//   targets   j = 2s(u+1)-1, tiles tc <= tr:  L_j -= R R^T + Lc^T Lc
+//   fill-ins  of node i = s-1+2s(f+1):        F = -R Lc
+// (syrk.py, gemm.py).  The wavefronts share the sum: a half of K of one product
+// each, or a quarter of R Lc.  Both operands go from memory to registers in the
+// operand layout.  k_schur_blk's 64x64 tiles walk K with a barrier per 32 columns
+// and leave most of the chip idle on a level of few nodes: n = 200, FP64, levels of
+// 32, 16, 8, 4, 2 nodes 76, 62, 40, 47, 53 -> 54, 29, 17, 10, 7 us (the larger ones
+// at 6.7 ns a tile, 19 TFLOP/s).  FP64 factor_and_solve n=200 N=64 m=2 1059 -> 868 us,
+// n=128 N=512 896 -> 881 us.
+template <typename T, bool COLS>
+__device__ __forceinline__ void pair_load(T (&v)[4][2], const T* M, int n, int rc, int kb, int g) {
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int k = kb + 8 * q + 2 * g;
+    if constexpr (COLS) {
+      v[q][0] = ldg(M, min(k, n - 1) * n + rc);
+      v[q][1] = ldg(M, min(k + 1, n - 1) * n + rc);
+    } else {
+      const int kc = min(k, n - 2);
+      const auto d = ldg2(M, rc * n + kc);
+      v[q][0] = k > kc ? d.y : d.x;
+      v[q][1] = d.y;
+    }
+  }
+}
+
+template <typename T, bool ACOLS, bool BCOLS>
+__device__ __forceinline__ void pair_mma(typename Mfma<T>::acc_t& acc, const T* A, const T* B, int n, int r0, int c0,
+                                         int k0, int k1) {
+  const int lane = lane_id(), g = lane >> 4;
+  const int rc = min(r0 + (lane & 15), n - 1), cc = min(c0 + (lane & 15), n - 1);
+  T a[4][2], b[4][2], na[4][2], nb[4][2];
+  pair_load<T, ACOLS>(a, A, n, rc, k0, g);
+  pair_load<T, BCOLS>(b, B, n, cc, k0, g);
+  for (int kb = k0; kb < k1; kb += 32) {
+    if (kb + 32 < k1) {
+      pair_load<T, ACOLS>(na, A, n, rc, kb + 32, g);
+      pair_load<T, BCOLS>(nb, B, n, cc, kb + 32, g);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const bool in = kb + 8 * q + 2 * g + e < k1;
+        acc = Mfma<T>::mma(in ? a[q][e] : T(0), in ? b[q][e] : T(0), acc);
+        a[q][e] = na[q][e];
+        b[q][e] = nb[q][e];
+      }
+  }
+  mfma_settle<T>();
+}
+
+// (ONE: n = 1, where a row holds no pair; its transpose is read instead)
+template <typename T, bool ONE>
+__global__ __launch_bounds__(kThreads) void k_schur_tile(T* L, const T* Lsrc, T* E,
+                                                        const uint8_t* __restrict__ mask, int N, int n,
+                                                        int nE, int s, int off, int next_off, int nT) {
+  __shared__ T part[4][256];
+  const int b = blockIdx.y;
+  if (masked_out(mask, b)) return;
+  const int nt = (n + 15) / 16, ntri = nt * (nt + 1) / 2;
+  const size_t nn = (size_t)n * n;
+  T* const Eb = E + (size_t)b * nE * nn;
+  const int lane = lane_id(), w = wave_uniform();
+  int task = blockIdx.x, tr, tc;
+  T* C;
+  const bool target = task < nT * ntri;
+  typename Mfma<T>::acc_t acc = acc_zero<T>();
+  if (target) {
+    const int j = 2 * s * (task / ntri + 1) - 1;
+    tc = task % ntri;
+    tr = 0;
+    while (tc > tr) tc -= ++tr;
+    C = L + ((size_t)b * N + j) * nn;
+    const T* const R = Eb + (size_t)(off + (j - s) / s) * nn;
+    const T* const Lc = Eb + (size_t)(off + j / s) * nn;
+    const int half = (n / 2 + 7) & ~7, k0 = (w & 1) ? half : 0, k1 = (w & 1) ? n : min(half, n);
+    if (w < 2) pair_mma<T, ONE, ONE>(acc, R, R, n, 16 * tr, 16 * tc, k0, k1);
+    else if (j + s < N) pair_mma<T, true, true>(acc, Lc, Lc, n, 16 * tr, 16 * tc, k0, k1);
+  } else {
+    task -= nT * ntri;
+    const int i = s - 1 + 2 * s * (task / (nt * nt) + 1);
+    const int q = task % (nt * nt);
+    tr = q / nt;
+    tc = q % nt;
+    C = Eb + (size_t)(next_off + (i - s) / (2 * s)) * nn;
+    const int part4 = (n / 4 + 7) & ~7, k0 = w * part4, k1 = w == 3 ? n : min(k0 + part4, n);
+    pair_mma<T, ONE, true>(acc, Eb + (size_t)(off + i / s) * nn, Eb + (size_t)(off + (i - s) / s) * nn, n, 16 * tr,
+                             16 * tc, k0, k1);
+  }
+  const int row = 16 * tr + Mfma<T>::row(lane, w), col = 16 * tc + (lane & 15);
+  const bool in = row < n && col < n && (!target || col <= row);
+  // (the fill-in block's contents on entry are not read: this is its only update)
+  const T c = target && in ? ldg(Lsrc != nullptr ? Lsrc + (C - L) : C, row * n + col) : T(0);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) part[w][e * 64 + lane] = acc[e];
+  __syncthreads();
+  const int q = w * 64 + lane;
+  if (in) stg(C, row * n + col, c - ((part[0][q] + part[1][q]) + (part[2][q] + part[3][q])));
+}
+
 template <typename T>
 constexpr size_t update_lds(int n) {
   return sizeof(T) * 2 * ((n + 31) & ~31) * kPP;
@@ -364,6 +467,18 @@ hipError_t factor_large(T* L, T* E, const uint8_t* mask, int B, int N, int n, in
 }
 
 template <typename T>
+hipError_t schur_tiles(T* L, const T* Lsrc, T* E, const uint8_t* mask, int B, int N, int n, int lidx, int nT, int nF,
+                       hipStream_t st) {
+  const Level lv = level_info(N, lidx);
+  const int nt = (n + 15) / 16, tasks = nT * (nt * (nt + 1) / 2) + nF * nt * nt;
+  if (tasks <= 0 || B <= 0) return hipSuccess;
+  auto k = n > 1 ? k_schur_tile<T, false> : k_schur_tile<T, true>;
+  hipLaunchKernelGGL(k, dim3(tasks, B), dim3(kThreads), 0, st, L, Lsrc, E, mask, N, n, (int)off_diag_storage_len(N),
+                     lv.s, lv.off, lv.next_off, nT);
+  return hipGetLastError();
+}
+
+template <typename T>
 hipError_t trsm_level(const T* L, T* E, const T* Esrc, const uint8_t* mask, int B, int N, int n, int lidx,
                       hipStream_t st) {
   if (n > kMaxN) return hipErrorInvalidValue;
@@ -418,6 +533,10 @@ hipError_t trtri_large(const T* L, T* W, const uint8_t* mask, int B, int N, int 
 
 template hipError_t factor_large<float>(float*, float*, const uint8_t*, int, int, int, int, hipStream_t);
 template hipError_t factor_large<double>(double*, double*, const uint8_t*, int, int, int, int, hipStream_t);
+template hipError_t schur_tiles<float>(float*, const float*, float*, const uint8_t*, int, int, int, int, int, int,
+                                       hipStream_t);
+template hipError_t schur_tiles<double>(double*, const double*, double*, const uint8_t*, int, int, int, int, int, int,
+                                        hipStream_t);
 template hipError_t trsm_level<float>(const float*, float*, const float*, const uint8_t*, int, int, int, int, hipStream_t);
 template hipError_t trsm_level<double>(const double*, double*, const double*, const uint8_t*, int, int, int, int,
                                        hipStream_t);

@@ -5,6 +5,8 @@ sides of each edge, against numpy; the inverse from a factor made elsewhere
 import numpy as np
 import pytest
 
+from oracle import nd
+
 pytestmark = pytest.mark.gpu
 
 EDGES = [1, 7, 16, 17, 31, 32, 33, 48, 49, 64, 65, 79, 80, 81, 96, 97, 101, 112, 113, 127, 128,
@@ -62,3 +64,31 @@ def test_fp64_pivots(n, device):
     run()
     torch.cuda.synchronize()
     assert problems.rel_residual(L0, E0, x.cpu().numpy(), b0) <= 1e-12
+
+
+# the sum of a Schur tile in halves and quarters of n rounded to 8, the last ones
+# short or empty; FP32 with FP64 pivots takes these tiles for the small n too
+@pytest.mark.parametrize("n", [1, 2, 7, 8, 9, 15, 16, 17, 20, 31, 33, 40, 64, 65, 70, 73, 88, 97, 128, 130, 201, 255])
+def test_schur_tiles(n, device):
+    import torch
+    from socu_amd import _lib
+    from socu_amd.block_tridiag_solver import create_cholesky_factor_launch
+
+    print(f"schur n={n}", flush=True)
+    N = 12
+    L0, E0, _ = nd.readme_problem(n, N, 1, alpha=16.0, seed=n)[:3]
+    Lr, Er = L0.copy(), E0.copy()
+    nd.factor(Lr, Er)
+    if n > 64:
+        L, E = (torch.tensor(a[None], device=device) for a in (L0, E0))
+        create_cholesky_factor_launch(L, E)()
+        for got, want in ((np.tril(L[0].cpu().numpy()), np.tril(Lr)), (E[0].cpu().numpy(), Er)):
+            assert _rel(got, want) < 1e-11
+    if n <= 128:
+        L, E = (torch.tensor(a[None], dtype=torch.float32, device=device) for a in (L0, E0))
+        lib = _lib.load()
+        rc = lib.socu_cholesky_factor_f32(L.data_ptr(), E.data_ptr(), None, 1, N, n, _lib.PREC_FP32, None)
+        torch.cuda.synchronize()
+        assert rc == 0
+        for got, want in ((np.tril(L[0].double().cpu().numpy()), np.tril(Lr)), (E[0].double().cpu().numpy(), Er)):
+            assert _rel(got, want) < 1e-4
