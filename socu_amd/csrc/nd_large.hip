@@ -113,8 +113,9 @@ struct Chunk {
   bool rows;
 };
 
-// X(k, c) <- the chunk, zero to 16 columns and to a multiple of 32 in k.
-template <typename T, int THREADS>
+// X(k, c) <- the chunk, zero to 16 columns and to a multiple of 32 in k.  FAR (here
+// and below): a chunk of right-hand sides of a block row above 4 GiB.
+template <typename T, int THREADS, bool FAR = false>
 __device__ __forceinline__ void stage_chunk(T* X, const Chunk<T>& c, int K) {
   const int kp = (K + 31) & ~31;
 #pragma unroll 4
@@ -128,14 +129,14 @@ __device__ __forceinline__ void stage_chunk(T* X, const Chunk<T>& c, int K) {
       j = idx & 15;
     }
     const int kc = min(k, K - 1), jc = min(j, c.count - 1);
-    const T v = ldg(c.p, c.rows ? jc * c.ld + kc : kc * c.ld + jc);
+    const T v = FAR ? ldx(c.p, kc, c.ld, jc) : ldg(c.p, c.rows ? jc * c.ld + kc : kc * c.ld + jc);
     X[k * kPP + j] = (k < K && j < c.count) ? v : T(0);
   }
 }
 
 // out(r, c) = A X (mode 0), -A X (1) or out - A X (2), row tiles t0 + wavefront, ...
 // of R rows; lower: rows r >= ... of a symmetric result only up to tile tmax.
-template <typename T, int FORM, bool TR, int TH>
+template <typename T, int FORM, bool TR, int TH, bool FAR = false>
 __device__ __forceinline__ void panel_product(const T* M, int ld, int R, int K, const T* X, const Chunk<T>& out,
                                               int mode, int tmax) {
   const int lane = lane_id(), li = lane & 15, w = wave_uniform();
@@ -160,7 +161,10 @@ __device__ __forceinline__ void panel_product(const T* M, int ld, int R, int K, 
     panel_mma<T, FORM, TR>(acc, M, ld, R, K, 16 * t, X, k0, k1);
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-      if (ok[e]) stg(out.p, off[e], mode == 0 ? acc[e] : c[e] - acc[e]);
+      if (ok[e]) {
+        if constexpr (FAR) stx(out.p, 16 * t + Mfma<T>::row(lane, e), out.ld, li, acc[e]);  // (mode 0, not TR)
+        else stg(out.p, off[e], mode == 0 ? acc[e] : c[e] - acc[e]);
+      }
   }
 }
 
@@ -169,7 +173,7 @@ enum PanelPhase { kPanelFirst, kPanelUpdate, kPanelSecond, kPanelInverse, kPanel
 // Workgroup (node, chunk of 16 vectors): see above.  kPanelInverse and
 // kPanelInverseSecond: the U12 products alone, for every block (s = 0), L21 being
 // read from Lsrc; kPanelForward / kPanelBackward: x_i <- U^T x_i / U x_i.
-template <typename T, int TH>
+template <typename T, int TH, bool FAR>
 __global__ __launch_bounds__(TH) void k_large_panel(T* L, const T* Lsrc, T* E, const T* Esrc, T* x,
                                                               const uint8_t* __restrict__ mask, int N, int n, int n1,
                                                               int m, int nE, int s, int off, int phase) {
@@ -186,10 +190,10 @@ __global__ __launch_bounds__(TH) void k_large_panel(T* L, const T* Lsrc, T* E, c
   if (phase == kPanelForward || phase == kPanelBackward) {
     const int c0 = 16 * y;
     const Chunk<T> v{x + ((size_t)b * N + i) * n * m + c0, m, min(16, m - c0), false};
-    stage_chunk<T, TH>(X, v, n);
+    stage_chunk<T, TH, FAR>(X, v, n);
     __syncthreads();
-    if (phase == kPanelForward) panel_product<T, kTriCols, false, TH>(A, n, n, n, X, v, 0, cn);
-    else panel_product<T, kTriRows, false, TH>(A, n, n, n, X, v, 0, cn);
+    if (phase == kPanelForward) panel_product<T, kTriCols, false, TH, FAR>(A, n, n, n, X, v, 0, cn);
+    else panel_product<T, kTriRows, false, TH, FAR>(A, n, n, n, X, v, 0, cn);
     return;
   }
   if (phase == kPanelInverse || phase == kPanelUpdate) {
@@ -261,7 +265,7 @@ __global__ __launch_bounds__(TH) void k_large_panel(T* L, const T* Lsrc, T* E, c
 //   forward (target j = 2s(u+1)-1): y_j -= R_{j-s} y_{j-s} + Lc_{j+s}^T y_{j+s}
 //   backward (node i = s-1+2su):    x_i -= Lc_i x_{i-s} + R_i^T x_{i+s}
 // (gemm_nn / gemm_tn, gemm.py:151-201, :358-408)
-template <typename T, bool BWD>
+template <typename T, bool BWD, bool FAR>
 __global__ __launch_bounds__(kThreads) void k_update_large(const T* __restrict__ E, T* __restrict__ x,
                                                           const uint8_t* __restrict__ mask, int N, int n, int m,
                                                           int nE, int s, int off) {
@@ -281,8 +285,8 @@ __global__ __launch_bounds__(kThreads) void k_update_large(const T* __restrict__
   const int lane = lane_id(), w = wave_uniform(), count = min(16, m - c0);
   const T* const Ma = Eb + (size_t)(off + (j - s) / s) * nn;  // block (j, j-s)
   const T* const Mc = Eb + (size_t)(off + j / s) * nn;        // block (j+s, j)
-  if (below) stage_chunk<T, kThreads>(Xa, Chunk<T>{xb + (j - s) * nm, m, count, false}, n);
-  if (above) stage_chunk<T, kThreads>(Xc, Chunk<T>{xb + (j + s) * nm, m, count, false}, n);
+  if (below) stage_chunk<T, kThreads, FAR>(Xa, Chunk<T>{xb + (j - s) * nm, m, count, false}, n);
+  if (above) stage_chunk<T, kThreads, FAR>(Xc, Chunk<T>{xb + (j + s) * nm, m, count, false}, n);
   __syncthreads();
   const int half = (n / 2 + 31) & ~31, k0 = (w & 1) ? half : 0, k1 = (w & 1) ? n : half;
   typename Mfma<T>::acc_t acc = acc_zero<T>();
@@ -299,7 +303,9 @@ __global__ __launch_bounds__(kThreads) void k_update_large(const T* __restrict__
   const int q = w * 64 + lane;
   if (row < n && col < count) {
     T* const p = xb + j * nm;
-    stg(p, row * m + col, ldg(p, row * m + col) - ((part[0][q] + part[1][q]) + (part[2][q] + part[3][q])));
+    const T sum = (part[0][q] + part[1][q]) + (part[2][q] + part[3][q]);
+    if constexpr (FAR) stx(p, row, m, col, ldx(p, row, m, col) - sum);
+    else stg(p, row * m + col, ldg(p, row * m + col) - sum);
   }
 }
 
@@ -413,11 +419,17 @@ constexpr size_t update_lds(int n) {
 
 template <typename T>
 hipError_t set_attrs() {
-  const int lds = (int)update_lds<T>(kMaxNLarge);
-  hipError_t e = hipFuncSetAttribute((const void*)k_update_large<T, false>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  if (e == hipSuccess)
-    e = hipFuncSetAttribute((const void*)k_update_large<T, true>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  hipError_t e = hipSuccess;
+  for (const void* k : {(const void*)k_update_large<T, false, false>, (const void*)k_update_large<T, false, true>,
+                        (const void*)k_update_large<T, true, false>, (const void*)k_update_large<T, true, true>})
+    if (e == hipSuccess) e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)update_lds<T>(kMaxNLarge));
   return e;
+}
+
+// (64-bit offsets cost 0.4% of a factor_and_solve of n=200 N=64 m=2)
+template <typename T>
+bool far_rhs(int n, int m) {
+  return (size_t)n * m * sizeof(T) > 0xffffffffu;
 }
 
 template <typename T>
@@ -426,8 +438,9 @@ hipError_t launch_panel(T* L, const T* Lsrc, T* E, const T* Esrc, T* x, const ui
   if (nodes <= 0 || chunks <= 0 || B <= 0) return hipSuccess;
   auto go = [&](auto th) {
     constexpr int TH = decltype(th)::value;
-    hipLaunchKernelGGL((k_large_panel<T, TH>), dim3(nodes, chunks, B), dim3(TH), 0, st, L, Lsrc, E, Esrc, x, mask, N, n,
-                       first_half(n), m, (int)off_diag_storage_len(N), s, off, phase);
+    auto k = x != nullptr && far_rhs<T>(n, m) ? k_large_panel<T, TH, true> : k_large_panel<T, TH, false>;
+    hipLaunchKernelGGL(k, dim3(nodes, chunks, B), dim3(TH), 0, st, L, Lsrc, E, Esrc, x, mask, N, n, first_half(n), m,
+                       (int)off_diag_storage_len(N), s, off, phase);
   };
   // (a wavefront per 16-row tile, up to eight)
   if (n <= 32) go(std::integral_constant<int, 128>{});
@@ -507,12 +520,9 @@ hipError_t update_large(const T* E, T* x, const uint8_t* mask, int B, int N, int
   if (items <= 0 || B <= 0) return hipSuccess;
   const dim3 grid(items, ((n + 15) / 16) * ((m + 15) / 16), B);
   const int nE = (int)off_diag_storage_len(N);
-  if (bwd)
-    hipLaunchKernelGGL((k_update_large<T, true>), grid, dim3(kThreads), update_lds<T>(n), st, E, x, mask, N, n, m,
-                       nE, lv.s, lv.off);
-  else
-    hipLaunchKernelGGL((k_update_large<T, false>), grid, dim3(kThreads), update_lds<T>(n), st, E, x, mask, N, n, m,
-                       nE, lv.s, lv.off);
+  auto k = far_rhs<T>(n, m) ? (bwd ? k_update_large<T, true, true> : k_update_large<T, false, true>)
+                            : (bwd ? k_update_large<T, true, false> : k_update_large<T, false, false>);
+  hipLaunchKernelGGL(k, grid, dim3(kThreads), update_lds<T>(n), st, E, x, mask, N, n, m, nE, lv.s, lv.off);
   return hipGetLastError();
 }
 

@@ -65,6 +65,18 @@ __device__ __forceinline__ typename Pair<T>::type ldg2(const T* base, int off) {
   typedef const __attribute__((address_space(1))) v2* gptr;
   return *(gptr)((gbytes)base + (unsigned)off * (unsigned)sizeof(T));
 }
+// Element (row, col) of a block row of right-hand sides, m columns: a 64-bit
+// offset, as the sweeps take any m and n m elements may be more than 4 GiB.
+template <typename T>
+__device__ __forceinline__ T ldx(const T* y, int row, int m, int col) {
+  typedef const __attribute__((address_space(1))) T* gptr;
+  return ((gptr)y)[(unsigned long long)(unsigned)row * (unsigned)m + (unsigned)col];
+}
+template <typename T>
+__device__ __forceinline__ void stx(T* y, int row, int m, int col, T v) {
+  typedef __attribute__((address_space(1))) T* gptr;
+  ((gptr)y)[(unsigned long long)(unsigned)row * (unsigned)m + (unsigned)col] = v;
+}
 template <typename P>
 __device__ __forceinline__ P* uniform_ptr(P* p) {
   const unsigned long long v = (unsigned long long)p;

@@ -108,20 +108,31 @@ struct Frag {
 // Right-hand sides, columns c0 .. c0 + 15: as the MFMA B operand ([t]: row
 // 4t + lane / 16) and in the accumulators' layout.  Entries past n or m repeat
 // others; the first operand is masked in the summed direction and results
-// past n or m are not stored.
-template <typename T, int K4>
+// past n or m are not stored.  FAR: block rows of any size (the factor takes m <= 32).
+template <typename T, int K4, bool FAR = false>
 __device__ __forceinline__ void ld_rhs(T (&f)[K4], const T* y, int n, int m, int c0) {
   const int l = lane_id(), j = min(c0 + (l & 15), m - 1), g = l >> 4;
 #pragma unroll
-  for (int t = 0; t < K4; ++t) f[t] = ldg(y, min(4 * t + g, n - 1) * m + j);
+  for (int t = 0; t < K4; ++t) {
+    const int row = min(4 * t + g, n - 1);
+    f[t] = FAR ? ldx(y, row, m, j) : ldg(y, row * m + j);
+  }
 }
-template <typename T, int NB>
+template <typename T, int NB, bool FAR = false>
 __device__ __forceinline__ void ld_rhs_acc(typename Mfma<T>::acc_t (&a)[NB], const T* y, int n, int m, int c0) {
   const int l = lane_id(), j = min(c0 + (l & 15), m - 1);
 #pragma unroll
   for (int b = 0; b < NB; ++b)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) a[b][r] = ldg(y, min(16 * b + Mfma<T>::row(l, r), n - 1) * m + j);
+    for (int r = 0; r < 4; ++r) {
+      const int row = min(16 * b + Mfma<T>::row(l, r), n - 1);
+      a[b][r] = FAR ? ldx(y, row, m, j) : ldg(y, row * m + j);
+    }
+}
+template <typename T, bool FAR>
+__device__ __forceinline__ void st_rhs(T* y, int row, int m, int col, T v) {
+  if constexpr (FAR) stx(y, row, m, col, v);
+  else stg(y, row * m + col, v);
 }
 
 // acc += A B (tiles i, j of A's and B's rows; LOWER: j <= i only).
@@ -529,13 +540,14 @@ __device__ __forceinline__ void up_task(const SmallSys<T>& Q, int l, int task, b
 // c1 - 1 of the right-hand sides): with upd it receives from level l-1 (nodes
 // of level l, then the other targets of level l-1), with app nodes apply
 // y_k <- L_k^-1 y_k, from the inverse stored above the diagonal.
-template <typename T, int K4, bool EX>
+template <typename T, int K4, bool EX, bool FAR>
 __device__ __forceinline__ void forward_task(const SmallSys<T>& Q, int l, int task, bool upd, bool app, int c0,
                                              int c1) {
   constexpr int NB = (K4 + 3) / 4;
   constexpr int KU = sizeof(T) == 8 ? K4 : 4 * NB;
   const int N = Q.N, n = EX ? 4 * K4 : Q.n, m = Q.m;
-  const int nn = n * n, nm = n * m;
+  const int nn = n * n;
+  const size_t nm = (size_t)n * m;
   const int s = 1 << l, h = s >> 1, dim = (N + s) / (2 * s);
   const bool node = task < dim;
   app = app && node;
@@ -545,7 +557,7 @@ __device__ __forceinline__ void forward_task(const SmallSys<T>& Q, int l, int ta
   const T* Ra = upd ? Q.E + (size_t)(offp + ((k - h) >> (l - 1))) * nn : nullptr;          // (k, k-h)
   const T* Lcc = upd && k + h < N ? Q.E + (size_t)(offp + (k >> (l - 1))) * nn : nullptr;  // (k+h, k)
   const T* Lk = Q.L + (size_t)k * nn;
-  T* yk = Q.x + (size_t)k * nm;
+  T* yk = Q.x + k * nm;
   const int lane = lane_id(), i = lane & 15;
   Frag<T, K4, EX, true> fr;
   Frag<T, K4, EX, false> fc;
@@ -553,13 +565,13 @@ __device__ __forceinline__ void forward_task(const SmallSys<T>& Q, int l, int ta
   typename Mfma<T>::acc_t a[NB];
   if (upd) {
     fr.load(Ra, n);
-    ld_rhs<T, K4>(y, yk - (size_t)h * nm, n, m, c0);
+    ld_rhs<T, K4, FAR>(y, yk - h * nm, n, m, c0);
   }
   if (Lcc != nullptr) {
     fc.load(Lcc, n);
-    ld_rhs<T, K4>(y2, yk + (size_t)h * nm, n, m, c0);
+    ld_rhs<T, K4, FAR>(y2, yk + h * nm, n, m, c0);
   }
-  ld_rhs_acc<T, NB>(a, yk, n, m, c0);
+  ld_rhs_acc<T, NB, FAR>(a, yk, n, m, c0);
   // L_k^-1, rows 16b + i, from the tiles on and above the stored diagonal
   T fu[KU][NB], dg[NB];
   if (app) {
@@ -589,9 +601,9 @@ __device__ __forceinline__ void forward_task(const SmallSys<T>& Q, int l, int ta
   if (Lcc != nullptr) fc.mask_k(n);
   for (const int first = c0; c0 < c1; c0 += 16) {
     if (c0 > first) {
-      if (upd) ld_rhs<T, K4>(y, yk - (size_t)h * nm, n, m, c0);
-      if (Lcc != nullptr) ld_rhs<T, K4>(y2, yk + (size_t)h * nm, n, m, c0);
-      ld_rhs_acc<T, NB>(a, yk, n, m, c0);
+      if (upd) ld_rhs<T, K4, FAR>(y, yk - h * nm, n, m, c0);
+      if (Lcc != nullptr) ld_rhs<T, K4, FAR>(y2, yk + h * nm, n, m, c0);
+      ld_rhs_acc<T, NB, FAR>(a, yk, n, m, c0);
     }
     typename Mfma<T>::acc_t u[NB];
 #pragma unroll
@@ -623,7 +635,7 @@ __device__ __forceinline__ void forward_task(const SmallSys<T>& Q, int l, int ta
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int row = 16 * b + Mfma<T>::row(lane, e);
-          if (row < n) stg(yk, row * m + c0 + i, a[b][e]);
+          if (row < n) st_rhs<T, FAR>(yk, row, m, c0 + i, a[b][e]);
         }
   }
 }
@@ -633,21 +645,22 @@ __device__ __forceinline__ void forward_task(const SmallSys<T>& Q, int l, int ta
 // right-hand sides are the (up to 16) columns of the B operand; the difference
 // goes from the accumulators to the second product's B operand as it is: row
 // kr(t) of lane group g below is the row an accumulator's entry t holds.
-template <typename T, int K4, bool EX>
+template <typename T, int K4, bool EX, bool FAR>
 __device__ __forceinline__ void down_task(const SmallSys<T>& Q, int l, int t0, int c0, int c1) {
   constexpr int NB = (K4 + 3) / 4;
   // steps of the second product (FP32: an accumulator's entry t spans the
   // whole 16-row tile)
   constexpr int KU = sizeof(T) == 8 ? K4 : 4 * NB;
   const int N = Q.N, n = EX ? 4 * K4 : Q.n, m = Q.m;
-  const int nn = n * n, nm = n * m;
+  const int nn = n * n;
+  const size_t nm = (size_t)n * m;
   const int s = 1 << l, k = s - 1 + 2 * s * t0;
   const int off = seg_offset(N, l);
   const bool hasR = k + s < N, hasC = k >= s;
   const T* Rk = Q.E + (size_t)(off + (k >> l)) * nn;
   const T* Lck = Q.E + (size_t)(off + ((k - s) >> l)) * nn;
   const T* Lk = Q.L + (size_t)k * nn;
-  T* xk = Q.x + (size_t)k * nm;
+  T* xk = Q.x + k * nm;
   const int lane = lane_id(), i = lane & 15;
   Frag<T, K4, EX, false> fr;
   Frag<T, K4, EX, true> fc;
@@ -655,13 +668,13 @@ __device__ __forceinline__ void down_task(const SmallSys<T>& Q, int l, int t0, i
   typename Mfma<T>::acc_t a[NB];
   if (hasR) {
     fr.load(Rk, n);
-    ld_rhs<T, K4>(y, xk + (size_t)s * nm, n, m, c0);
+    ld_rhs<T, K4, FAR>(y, xk + s * nm, n, m, c0);
   }
   if (hasC) {
     fc.load(Lck, n);
-    ld_rhs<T, K4>(y2, xk - (size_t)s * nm, n, m, c0);
+    ld_rhs<T, K4, FAR>(y2, xk - s * nm, n, m, c0);
   }
-  ld_rhs_acc<T, NB>(a, xk, n, m, c0);
+  ld_rhs_acc<T, NB, FAR>(a, xk, n, m, c0);
   // U[16b + i][kr]: rows of the stored block above its diagonal (tiles on and
   // above it), and the diagonal
   T fu[KU][NB], dg[NB];
@@ -692,9 +705,9 @@ __device__ __forceinline__ void down_task(const SmallSys<T>& Q, int l, int t0, i
   if (hasC) fc.mask_k(n);
   for (const int first = c0; c0 < c1; c0 += 16) {
     if (c0 > first) {
-      if (hasR) ld_rhs<T, K4>(y, xk + (size_t)s * nm, n, m, c0);
-      if (hasC) ld_rhs<T, K4>(y2, xk - (size_t)s * nm, n, m, c0);
-      ld_rhs_acc<T, NB>(a, xk, n, m, c0);
+      if (hasR) ld_rhs<T, K4, FAR>(y, xk + s * nm, n, m, c0);
+      if (hasC) ld_rhs<T, K4, FAR>(y2, xk - s * nm, n, m, c0);
+      ld_rhs_acc<T, NB, FAR>(a, xk, n, m, c0);
     }
     typename Mfma<T>::acc_t u[NB], o[NB];
 #pragma unroll
@@ -719,7 +732,7 @@ __device__ __forceinline__ void down_task(const SmallSys<T>& Q, int l, int t0, i
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int row = 16 * b + Mfma<T>::row(lane, e);
-          if (row < n) stg(xk, row * m + c0 + i, o[b][e]);
+          if (row < n) st_rhs<T, FAR>(xk, row, m, c0 + i, o[b][e]);
         }
   }
 }
@@ -733,23 +746,23 @@ __global__ __launch_bounds__(64 * ((K4 + 3) / 4)) void k_small_up(SmallArgs<T> A
   up_task<T, K4, EX>(Q, l, task, true, reinterpret_cast<T*>(smem_raw), wave_uniform());
 }
 
-template <typename T, int K4, bool EX>
+template <typename T, int K4, bool EX, bool FAR>
 __global__ __launch_bounds__(64) void k_small_down(SmallArgs<T> A, int l) {
   SmallSys<T> Q;
   int task;
   if (!small_sys(A, Q, task)) return;
   // (grid z: 16 right-hand sides each, or one for all of them)
   const int c0 = 16 * blockIdx.z;
-  down_task<T, K4, EX>(Q, l, task, c0, gridDim.z > 1 ? c0 + 16 : Q.m);
+  down_task<T, K4, EX, FAR>(Q, l, task, c0, gridDim.z > 1 ? c0 + 16 : Q.m);
 }
 
-template <typename T, int K4, bool EX>
+template <typename T, int K4, bool EX, bool FAR>
 __global__ __launch_bounds__(64) void k_small_forward(SmallArgs<T> A, int l, int upd, int app) {
   SmallSys<T> Q;
   int task;
   if (!small_sys(A, Q, task)) return;
   const int c0 = 16 * blockIdx.z;
-  forward_task<T, K4, EX>(Q, l, task, upd != 0, app != 0, c0, gridDim.z > 1 ? c0 + 16 : Q.m);
+  forward_task<T, K4, EX, FAR>(Q, l, task, upd != 0, app != 0, c0, gridDim.z > 1 ? c0 + 16 : Q.m);
 }
 
 // Levels lo .. of one system, up and (with right-hand sides) down again, by
@@ -778,7 +791,7 @@ __global__ __launch_bounds__(64 * kTailWaves) void k_small_tail(SmallArgs<T> A, 
   if (Q.x == nullptr) return;
   for (int l = Lv - 1; l >= lo; --l) {
     const int s = 1 << l, dim = (Q.N + s) / (2 * s);
-    for (int t = wv; t < dim; t += kTailWaves) down_task<T, K4, EX>(Q, l, t, 0, Q.m);
+    for (int t = wv; t < dim; t += kTailWaves) down_task<T, K4, EX, false>(Q, l, t, 0, Q.m);
     __syncthreads();
   }
 }
@@ -817,17 +830,33 @@ void launch_up(int cls, dim3 grid, const SmallArgs<T>& A, int l, hipStream_t st)
     hipLaunchKernelGGL((k_small_up<T, K4, EX>), grid, dim3(64 * Sh::NB), lds, st, A, l);
   });
 }
+// Block rows of right-hand sides of 4 GiB and more take 64-bit offsets, in a variant
+// of their own (every n by its padded form): in the common one they cost 1.5% (256
+// systems of n=20 N=61 m=1, FP32 factor_and_solve, 157.8 / 160.2 us).
+template <typename T>
+bool far_rhs(const SmallArgs<T>& A) {
+  return (size_t)A.n * A.m * sizeof(T) > 0xffffffffu;
+}
 template <typename T>
 void launch_down(int cls, dim3 grid, const SmallArgs<T>& A, int l, hipStream_t st) {
+  if (far_rhs(A))
+    return with_class(cls & ~1, [&](auto k4, auto) {
+      hipLaunchKernelGGL((k_small_down<T, decltype(k4)::value, false, true>), grid, dim3(64), 0, st, A, l);
+    });
   with_class(cls, [&](auto k4, auto ex) {
-    hipLaunchKernelGGL((k_small_down<T, decltype(k4)::value, decltype(ex)::value>), grid, dim3(64), 0, st, A, l);
+    hipLaunchKernelGGL((k_small_down<T, decltype(k4)::value, decltype(ex)::value, false>), grid, dim3(64), 0, st, A, l);
   });
 }
 template <typename T>
 void launch_forward(int cls, dim3 grid, const SmallArgs<T>& A, int l, bool upd, bool app, hipStream_t st) {
+  if (far_rhs(A))
+    return with_class(cls & ~1, [&](auto k4, auto) {
+      hipLaunchKernelGGL((k_small_forward<T, decltype(k4)::value, false, true>), grid, dim3(64), 0, st, A, l, (int)upd,
+                         (int)app);
+    });
   with_class(cls, [&](auto k4, auto ex) {
-    hipLaunchKernelGGL((k_small_forward<T, decltype(k4)::value, decltype(ex)::value>), grid, dim3(64), 0, st, A, l,
-                       (int)upd, (int)app);
+    hipLaunchKernelGGL((k_small_forward<T, decltype(k4)::value, decltype(ex)::value, false>), grid, dim3(64), 0, st, A,
+                       l, (int)upd, (int)app);
   });
 }
 template <typename T>

@@ -74,11 +74,11 @@ __global__ __launch_bounds__(64 * RT) void k_step(const T* __restrict__ L, const
   T sp[4], sm[4], xd[4], a1[Q][2], a2[Q][2], a3[Q][2];
   if (hasT) {
 #pragma unroll
-    for (int p = 0; p < 4; ++p) sp[p] = ldg(xi + s * nm, min(k0 + 4 * RT * p, n - 1) * m + cl);
+    for (int p = 0; p < 4; ++p) sp[p] = ldx(xi + s * nm, min(k0 + 4 * RT * p, n - 1), m, cl);
   }
   if (hasS) {
 #pragma unroll
-    for (int p = 0; p < 4; ++p) sm[p] = ldg(xi - s * nm, min(k0 + 4 * RT * p, n - 1) * m + cl);
+    for (int p = 0; p < 4; ++p) sm[p] = ldx(xi - s * nm, min(k0 + 4 * RT * p, n - 1), m, cl);
   }
   auto rows = [&](T(&v)[2], const T* M, int q) {  // v[e] = M[ii][8 q + 2 g + e]
     const int o = ic * n + 8 * q + 2 * g, oc = q < QT ? o : min(o, nn - 2);
@@ -102,7 +102,7 @@ __global__ __launch_bounds__(64 * RT) void k_step(const T* __restrict__ L, const
     for (int q = 0; q < Q; ++q) rows(a2[q], MS, q);
   }
 #pragma unroll
-  for (int e = 0; e < 4; ++e) xd[e] = ldg(xi, min(16 * t + Mfma<T>::row(lane, e), n - 1) * m + cl);
+  for (int e = 0; e < 4; ++e) xd[e] = ldx(xi, min(16 * t + Mfma<T>::row(lane, e), n - 1), m, cl);
   T diag = T(1);
   if (inv) {
     diag = ldg(U, ic * (n + 1));
@@ -147,7 +147,7 @@ __global__ __launch_bounds__(64 * RT) void k_step(const T* __restrict__ L, const
     const int row = 16 * t + Mfma<T>::row(lane, e);
     const T v = row < n ? xd[e] - (acc[e] + acc2[e]) : T(0);
     if (inv) Tt[row * 16 + li] = v;
-    else if (row < n && li < m - c0) stg(xi, row * m + li, v);
+    else if (row < n && li < m - c0) stx(xi, row, m, li, v);
   }
   if (!inv) return;
   __syncthreads();
@@ -171,7 +171,7 @@ __global__ __launch_bounds__(64 * RT) void k_step(const T* __restrict__ L, const
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const int row = 16 * t + Mfma<T>::row(lane, e);
-    if (row < n && li < m - c0) stg(xi, row * m + li, acc[e]);
+    if (row < n && li < m - c0) stx(xi, row, m, li, acc[e]);
   }
 }
 
