@@ -29,6 +29,10 @@ void kt_end(int cls, hipStream_t st);
 // that records them itself (hipExtLaunchKernel), and true; else false.
 bool kt_kernel_events(int cls, hipEvent_t* start, hipEvent_t* stop);
 
+// Workgroups of one launch along x where a workgroup is one of many tasks: with up
+// to 256 threads each they stay below the 2^32 threads a launch takes.
+constexpr int kMaxGridTasks = 1 << 23;
+
 // One-time per-process kernel set-up (LDS limits above 64 KiB).  Must run
 // before any stream capture.
 hipError_t init_blocked_kernels();

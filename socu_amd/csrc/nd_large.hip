@@ -29,6 +29,8 @@
 // What bounds them now: the halves' pivot chains (see nd_potrf.hip); the products'
 // launches, their loads (one compute unit's misses, 23 bytes/ns).  FP64 factor_and_solve
 // n=200 N=64 m=2: 2468 -> 1062 us (868 with the Schur tiles).
+#include <algorithm>
+
 #include "../../include/socu_hip.h"
 #include "nd_common.h"
 #include "nd_internal.h"
@@ -367,7 +369,7 @@ __device__ __forceinline__ void pair_mma(typename Mfma<T>::acc_t& acc, const T* 
 template <typename T, bool ONE>
 __global__ __launch_bounds__(kThreads) void k_schur_tile(T* L, const T* Lsrc, T* E,
                                                         const uint8_t* __restrict__ mask, int N, int n,
-                                                        int nE, int s, int off, int next_off, int nT) {
+                                                        int nE, int s, int off, int next_off, int nT, int first) {
   __shared__ T part[4][256];
   const int b = blockIdx.y;
   if (masked_out(mask, b)) return;
@@ -375,7 +377,7 @@ __global__ __launch_bounds__(kThreads) void k_schur_tile(T* L, const T* Lsrc, T*
   const size_t nn = (size_t)n * n;
   T* const Eb = E + (size_t)b * nE * nn;
   const int lane = lane_id(), w = wave_uniform();
-  int task = blockIdx.x, tr, tc;
+  int task = first + blockIdx.x, tr, tc;
   T* C;
   const bool target = task < nT * ntri;
   typename Mfma<T>::acc_t acc = acc_zero<T>();
@@ -486,8 +488,11 @@ hipError_t schur_tiles(T* L, const T* Lsrc, T* E, const uint8_t* mask, int B, in
   const int nt = (n + 15) / 16, tasks = nT * (nt * (nt + 1) / 2) + nF * nt * nt;
   if (tasks <= 0 || B <= 0) return hipSuccess;
   auto k = n > 1 ? k_schur_tile<T, false> : k_schur_tile<T, true>;
-  hipLaunchKernelGGL(k, dim3(tasks, B), dim3(kThreads), 0, st, L, Lsrc, E, mask, N, n, (int)off_diag_storage_len(N),
-                     lv.s, lv.off, lv.next_off, nT);
+  // (a launch takes 2^32 threads along x; the 32x32 tiles of long systems of small
+  // blocks are four times as many 16x16 ones)
+  for (int first = 0; first < tasks; first += kMaxGridTasks)
+    hipLaunchKernelGGL(k, dim3(std::min(tasks - first, kMaxGridTasks), B), dim3(kThreads), 0, st, L, Lsrc, E, mask, N, n,
+                       (int)off_diag_storage_len(N), lv.s, lv.off, lv.next_off, nT, first);
   return hipGetLastError();
 }
 
