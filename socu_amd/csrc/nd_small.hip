@@ -37,6 +37,8 @@
 // 32-bit offsets from a scalar base and no branch per element: with generic
 // pointers and selected loads the n=20 FP32 task took 17 us instead of 6.
 #include <algorithm>
+#include <new>
+#include <stdexcept>
 #include <vector>
 
 #include "../../include/socu_hip.h"
@@ -985,8 +987,8 @@ hipError_t small_backward_level(const T* L, const T* E, T* x, const uint8_t* mas
 // ---------------------------------------------------------------------------
 struct SmallBatch {
   struct Level {
-    int up = 0, up_count = 0;            // factor: nodes, then targets
-    int fwd = 0, fwd_count = 0, nodes = 0;  // sweeps: nodes, then targets (one per task)
+    size_t first = 0, count = 0;  // nodes, then targets (factor: several per task)
+    size_t nodes = 0;
   };
   struct Group {
     int cls = 0, mmax = 0, stream = 0;
@@ -1002,11 +1004,9 @@ void small_batch_free(SmallBatch* b) {
   delete b;
 }
 
-hipError_t small_batch_create(SmallBatch** out, const BatchProblem* probs, int count, int op, int streams) {
-  *out = nullptr;
+static hipError_t fill_batch(SmallBatch* h, const BatchProblem* probs, int count, int op, int streams) {
   const bool fac = op == SOCU_OP_FACTOR || op == SOCU_OP_FACTOR_AND_SOLVE;
   const bool solve = op != SOCU_OP_FACTOR;
-  SmallBatch* h = new SmallBatch();
   std::vector<int> of[kSmallN / 4];
   double cost[kSmallN / 4] = {};
   for (int k = 0; k < count; ++k) {
@@ -1033,35 +1033,40 @@ hipError_t small_batch_create(SmallBatch** out, const BatchProblem* probs, int c
     G.cls = 2 * k4 + (exact ? 1 : 0);
     G.stream = (int)(std::min_element(load.begin(), load.end()) - load.begin());
     load[G.stream] += cost[k4];
-    const int per = G.cls < 2 * 4 ? 1 : 2;  // targets per factor task
+    const int per = fac && G.cls >= 2 * 4 ? 2 : 1;  // targets per task
     const int Lv = recursive_iterations(probs[sys[0]].N);
     for (int l = 0; l < Lv; ++l) {
       SmallBatch::Level V;
       const int s = 1 << l;
-      V.up = V.fwd = (int)tasks.size();
+      V.first = tasks.size();
       for (int k : sys)
         for (int t = 0, dim = (probs[k].N + s) / (2 * s); t < dim; ++t) tasks.push_back({k, t});
-      V.nodes = (int)tasks.size() - V.up;
-      auto targets = [&](int each) {
-        if (l > 0)
-          for (int k : sys) {
-            const int dim = (probs[k].N + s) / (2 * s);
-            for (int u = 0; u * each < probs[k].N / (2 * s); ++u) tasks.push_back({k, dim + u});
-          }
-      };
-      if (fac) {
-        targets(per);
-        V.up_count = (int)tasks.size() - V.up;
-      } else {
-        targets(1);
-        V.fwd_count = (int)tasks.size() - V.fwd;
-      }
+      V.nodes = tasks.size() - V.first;
+      if (l > 0)
+        for (int k : sys) {
+          const int dim = (probs[k].N + s) / (2 * s);
+          for (int u = 0; u * per < probs[k].N / (2 * s); ++u) tasks.push_back({k, dim + u});
+        }
+      V.count = tasks.size() - V.first;
       G.levels.push_back(V);
     }
     h->groups.push_back(std::move(G));
   }
   hipError_t e = hipMalloc(&h->tasks, std::max<size_t>(1, tasks.size()) * sizeof(int2));
   if (e == hipSuccess) e = hipMemcpy(h->tasks, tasks.data(), tasks.size() * sizeof(int2), hipMemcpyHostToDevice);
+  return e;
+}
+
+hipError_t small_batch_create(SmallBatch** out, const BatchProblem* probs, int count, int op, int streams) {
+  *out = nullptr;
+  SmallBatch* h = nullptr;
+  hipError_t e = hipErrorOutOfMemory;
+  try {  // (the task list takes host memory of its own: about 12 bytes per block row)
+    h = new SmallBatch();
+    e = fill_batch(h, probs, count, op, streams);
+  } catch (const std::bad_alloc&) {
+  } catch (const std::length_error&) {
+  }
   if (e != hipSuccess) {
     small_batch_free(h);
     return e;
@@ -1087,17 +1092,22 @@ static hipError_t batch_enqueue(const SmallBatch* h, const BatchProblem* probs, 
     A.mask = mask;
     A.solve = op != SOCU_OP_FACTOR;
     A.m = G.mmax;
+    // (several launches for a level of more tasks than one takes)
+    auto pieces = [&](size_t first, size_t count, auto launch) {
+      for (size_t t = 0; t < count; t += kMaxGridTasks) {
+        A.tasks = h->tasks + first + t;
+        launch(dim3((unsigned)std::min<size_t>(count - t, kMaxGridTasks)));
+      }
+    };
     for (size_t l = 0; l < G.levels.size(); ++l) {
       const SmallBatch::Level& V = G.levels[l];
-      A.tasks = h->tasks + V.up;
-      if (fac) launch_up<T>(G.cls, dim3(V.up_count), A, (int)l, st);
-      else if (op != SOCU_OP_BACKWARD) launch_forward<T>(G.cls, dim3(V.fwd_count), A, (int)l, true, true, st);
+      if (fac) pieces(V.first, V.count, [&](dim3 grid) { launch_up<T>(G.cls, grid, A, (int)l, st); });
+      else if (op != SOCU_OP_BACKWARD)
+        pieces(V.first, V.count, [&](dim3 grid) { launch_forward<T>(G.cls, grid, A, (int)l, true, true, st); });
     }
     if (op != SOCU_OP_FACTOR && op != SOCU_OP_FORWARD)
-      for (int l = (int)G.levels.size() - 1; l >= 0; --l) {
-        A.tasks = h->tasks + G.levels[l].up;
-        launch_down<T>(G.cls, dim3(G.levels[l].nodes), A, l, st);
-      }
+      for (int l = (int)G.levels.size() - 1; l >= 0; --l)
+        pieces(G.levels[l].first, G.levels[l].nodes, [&](dim3 grid) { launch_down<T>(G.cls, grid, A, l, st); });
   }
   return hipGetLastError();
 }

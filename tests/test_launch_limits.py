@@ -37,3 +37,29 @@ def test_fp64_pivots_of_a_long_system(device):
         r[:hi - i] += (C[i:hi] * x[i + 1:hi + 1, :, None]).sum(1)
         # kappa <= 3: a few units of 2^-24 of the terms' size
         assert float(r.abs().max()) < 1e-5 * float(b.abs().max()), i
+
+
+def test_batch_of_many_block_rows(device):
+    """69 million block rows in one batch: level 0 has 35 million tasks of two
+    wavefronts (m > 16), 2^32 threads and more.  Equal systems, against the same
+    system in a launch of its own."""
+    import torch
+    from socu_amd.batched import create_batched_cholesky_launch
+    from socu_amd.block_tridiag_solver import calculate_off_diag_storage_len, create_cholesky_factor_and_solve_launch
+
+    N, m, count, dt = 2**21, 17, 33, torch.float32
+    print(f"batch of {count} systems n=1 N={N} m={m}", flush=True)
+    gen = torch.Generator(device=device).manual_seed(2)
+    nE = calculate_off_diag_storage_len(N)
+    L0 = torch.rand(N, 1, 1, generator=gen, device=device) + 3.0
+    E0 = torch.zeros(nE, 1, 1, device=device)
+    E0[: N - 1] = torch.rand(N - 1, 1, 1, generator=gen, device=device)
+    b0 = torch.randn(N, 1, m, generator=gen, device=device)
+    L, E, x = (t.expand(count, *t.shape).contiguous() for t in (L0, E0, b0))
+    create_batched_cholesky_launch(list(L), list(E), list(x), dtype=dt)()
+    create_cholesky_factor_and_solve_launch(L0, E0, b0, dtype=dt)()
+    for k in range(count):
+        for got, want in ((L[k], L0), (E[k], E0), (x[k], b0)):
+            assert float((got - want).abs().max()) <= 1e-5 * float(want.abs().max()), k
+    del L, E, x
+    torch.cuda.empty_cache()
