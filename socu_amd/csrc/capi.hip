@@ -296,7 +296,7 @@ void free_sweep_ws(SweepWs& sw) {
 // includes a substitution with one right-hand side.
 int alloc_sweep_ws(SweepWs& sw, int op, int B, int N, int n, int m, int dtype) {
   const size_t esz = dtype == SOCU_DTYPE_F64 ? sizeof(double) : sizeof(float);
-  if (op == SOCU_OP_FACTOR || m != 1 || B <= 0 || !socu::sweep_persistent_enabled(B, n, (int)esz)) return SOCU_OK;
+  if (op == SOCU_OP_FACTOR || m != 1 || B <= 0 || !socu::sweep_persistent_enabled(B, n, false)) return SOCU_OK;
   // (these sweep inside the factor's kernels)
   if (op == SOCU_OP_FACTOR_AND_SOLVE && n <= socu::kSmallN && socu::small_tail_applies(B, n, m)) return SOCU_OK;
   hipError_t e = hipMalloc(&sw.ws, sizeof(int) * socu::sweep_ws_ints(B, N));

@@ -566,19 +566,21 @@ hipError_t init_sweep_kernels() {
   return sweep_occupancy<double, 4>(g_sweep_occ[1][3]);
 }
 
-// One launch against one per level and direction: at n > 32 the persistent
-// sweeps are faster for every batch (see sweep_lmin).  At n <= 32 the level
-// kernels are one wavefront per node and their launches 3-4 us: FP64 solves
-// with N=100, persistent / level kernels, n=32: B=1 71.5 / 76.5 us, B=4 81.0 /
-// 87.1, B=16 103.9 / 102.5, B=64 203 / 196; n=20: B=16 86.6 / 80.8; 256 systems
-// of n=20 N=61 (FP32 factor_and_solve) 165 / 157.
-bool sweep_persistent_enabled(int B, int n, int dsize) {
+// One launch for the upper levels against one per level and direction.  At n > 32
+// always.  At n <= 32 a level kernel is one wavefront per node and its launch 3-4 us,
+// and the batch decides, by how many levels the one launch takes (sweep_lmin).
+// Level kernels / persistent over 280 plans each (n = 4 .. 32, N = 8 .. 700, in a
+// graph): FP64 solves 1.10 at B=9, 1.05 at 16, 1.00 at 32, 0.97 at 64; FP32 backward
+// sweeps 1.07, 1.04, 1.00, 0.98 (the worst, n=24 N=8 B=9, 61.3 / 51.6 us; at B=32
+// between 0.85 and 1.06).  The mixed solver launches the sweeps of a converged
+// iteration too, where one launch is next to nothing: 1.16 at B=9 (up to 1.57), 1.04
+// at 32, 1.00 at 64, 0.97 at 128.
+bool sweep_persistent_enabled(int B, int n, bool refine) {
   if (n > kMaxN) return false;  // its node tasks hold whole blocks in LDS
   const char* v = getenv("SOCU_SWEEP");
   if (v != nullptr && strcmp(v, "level") == 0) return false;
   if (v != nullptr && strcmp(v, "persistent") == 0) return true;
-  (void)dsize;
-  return n > kSmallN || B <= 8;
+  return n > kSmallN || B <= (refine ? 64 : 32);
 }
 
 size_t sweep_ws_ints(int B, int N) { return (size_t)kSweepHeader + 3 * (size_t)B * N; }
