@@ -150,9 +150,11 @@ int run_op(int op, void* L, void* E, void* x, const uint8_t* mask, int B, int N,
   if (n <= socu::kSmallUpN && (op == SOCU_OP_FACTOR || op == SOCU_OP_FACTOR_AND_SOLVE)) {
     const bool solve = op == SOCU_OP_FACTOR_AND_SOLVE;
     const bool with_x = solve && m <= socu::small_max_rhs(n);  // (more right-hand sides: the sweeps follow)
-    const hipError_t e = socu::small_factor<T>(Lt, Et, with_x ? xt : nullptr, mask, B, N, n, m, st, Ls, Es);
+    // (a plan with a sweep workspace sweeps back by the persistent launch)
+    const bool back = with_x && sw.ws == nullptr && socu::small_tail_applies(B, n, m);
+    const hipError_t e = socu::small_factor<T>(Lt, Et, with_x ? xt : nullptr, mask, B, N, n, m, back, st, Ls, Es);
     if (e != hipSuccess) return hip_fail(e, "small-block factor launch");
-    if (!solve || (with_x && socu::small_tail_applies(B, n, m))) return SOCU_OK;
+    if (!solve || back) return SOCU_OK;
     return run_sweeps<T>(Lt, Et, xt, mask, B, N, n, m, !with_x, true, sw, st);
   }
   switch (op) {
@@ -297,8 +299,10 @@ void free_sweep_ws(SweepWs& sw) {
 int alloc_sweep_ws(SweepWs& sw, int op, int B, int N, int n, int m, int dtype) {
   const size_t esz = dtype == SOCU_DTYPE_F64 ? sizeof(double) : sizeof(float);
   if (op == SOCU_OP_FACTOR || m != 1 || B <= 0 || !socu::sweep_persistent_enabled(B, n, false)) return SOCU_OK;
-  // (these sweep inside the factor's kernels)
-  if (op == SOCU_OP_FACTOR_AND_SOLVE && n <= socu::kSmallN && socu::small_tail_applies(B, n, m)) return SOCU_OK;
+  // (these sweep inside the factor's kernels, unless asked not to)
+  if (op == SOCU_OP_FACTOR_AND_SOLVE && n <= socu::kSmallN && socu::small_tail_applies(B, n, m) &&
+      !socu::sweep_persistent_asked())
+    return SOCU_OK;
   hipError_t e = hipMalloc(&sw.ws, sizeof(int) * socu::sweep_ws_ints(B, N));
   if (e == hipSuccess) e = hipMemset(sw.ws, 0, sizeof(int) * socu::sweep_ws_ints(B, N));  // status reads 0 before a run
   if (e == hipSuccess) e = hipMalloc(&sw.slots, esz * socu::sweep_slot_elems(B, N, n));

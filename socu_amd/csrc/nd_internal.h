@@ -159,6 +159,8 @@ int sweep_spin_limit();
 // variable SOCU_SWEEP = "level" (never) or "persistent" (always) overrides the
 // rule.
 bool sweep_persistent_enabled(int B, int n, bool refine);
+// ... whether the variable asks for them.
+bool sweep_persistent_asked();
 
 // A side stream and per-level events that let the forward sweep of a
 // factor_and_solve run alongside the factor: forward step l waits for level
@@ -205,11 +207,11 @@ hipError_t small_up_level(T* L, T* E, T* x, const uint8_t* mask, int B, int N, i
 template <typename T>
 hipError_t wide_up_level(T* L, T* E, T* x, const uint8_t* mask, int B, int N, int n, int m, int l, hipStream_t st,
                          const T* Lsrc, const T* Esrc);
-// Every factor level, with x the forward sweep and, where small_tail_applies,
-// the backward sweep too.
+// Every factor level, with x the forward sweep and, with `back` where
+// small_tail_applies, the backward sweep too.
 bool small_tail_applies(int B, int n, int m);
 template <typename T>
-hipError_t small_factor(T* L, T* E, T* x, const uint8_t* mask, int B, int N, int n, int m, hipStream_t st,
+hipError_t small_factor(T* L, T* E, T* x, const uint8_t* mask, int B, int N, int n, int m, bool back, hipStream_t st,
                         const T* Lsrc, const T* Esrc);
 // forward_step_blocked / backward_level_blocked for n <= 32, any m.
 template <typename T>

@@ -917,7 +917,7 @@ bool small_tail_applies(int B, int n, int m) {
 }
 
 template <typename T>
-hipError_t small_factor(T* L, T* E, T* x, const uint8_t* mask, int B, int N, int n, int m, hipStream_t st,
+hipError_t small_factor(T* L, T* E, T* x, const uint8_t* mask, int B, int N, int n, int m, bool back, hipStream_t st,
                         const T* Lsrc, const T* Esrc) {
   if (B <= 0) return hipSuccess;
   const int Lv = recursive_iterations(N);
@@ -930,7 +930,7 @@ hipError_t small_factor(T* L, T* E, T* x, const uint8_t* mask, int B, int N, int
   const int mx = x != nullptr ? m : 0, cls = small_class(n, mx);
   const SmallArgs<T> A = regular_args(L, E, x, mask, N, n, m, Lsrc, Esrc);
   int lo = Lv;
-  if (small_tail_applies(B, n, mx)) {
+  if (small_tail_applies(B, n, mx) && (x == nullptr || back)) {
     lo = 0;
     while (lo < Lv && small_up_tasks(N, n, mx, lo) > kTailWaves) ++lo;
   }
@@ -939,7 +939,7 @@ hipError_t small_factor(T* L, T* E, T* x, const uint8_t* mask, int B, int N, int
   if (lo < Lv) launch_tail<T>(cls, dim3(1, B), A, lo, st);
   kt_end(kKcPotrf, st);
   hipError_t e = hipGetLastError();
-  if (x != nullptr && small_tail_applies(B, n, mx))
+  if (x != nullptr && back && small_tail_applies(B, n, mx))
     for (int l = lo - 1; l >= 0 && e == hipSuccess; --l) e = small_backward_level<T>(L, E, x, mask, B, N, n, m, l, st);
   return e;
 }
@@ -1122,14 +1122,14 @@ template hipError_t small_up_level<float>(float*, float*, float*, const uint8_t*
                                           const float*, const float*);
 template hipError_t small_up_level<double>(double*, double*, double*, const uint8_t*, int, int, int, int, int,
                                            hipStream_t, const double*, const double*);
-template hipError_t small_factor<float>(float*, float*, float*, const uint8_t*, int, int, int, int, hipStream_t, const float*,
-                                     const float*);
+template hipError_t small_factor<float>(float*, float*, float*, const uint8_t*, int, int, int, int, bool, hipStream_t,
+                                        const float*, const float*);
 template hipError_t small_forward_step<float>(const float*, const float*, float*, const uint8_t*, int, int, int, int, int,
                                             hipStream_t, bool, bool);
 template hipError_t small_backward_level<float>(const float*, const float*, float*, const uint8_t*, int, int, int, int, int,
                                               hipStream_t);
-template hipError_t small_factor<double>(double*, double*, double*, const uint8_t*, int, int, int, int, hipStream_t, const double*,
-                                     const double*);
+template hipError_t small_factor<double>(double*, double*, double*, const uint8_t*, int, int, int, int, bool, hipStream_t,
+                                         const double*, const double*);
 template hipError_t small_forward_step<double>(const double*, const double*, double*, const uint8_t*, int, int, int, int, int,
                                             hipStream_t, bool, bool);
 template hipError_t small_backward_level<double>(const double*, const double*, double*, const uint8_t*, int, int, int, int, int,

@@ -575,11 +575,15 @@ hipError_t init_sweep_kernels() {
 // between 0.85 and 1.06).  The mixed solver launches the sweeps of a converged
 // iteration too, where one launch is next to nothing: 1.16 at B=9 (up to 1.57), 1.04
 // at 32, 1.00 at 64, 0.97 at 128.
+bool sweep_persistent_asked() {
+  const char* v = getenv("SOCU_SWEEP");
+  return v != nullptr && strcmp(v, "persistent") == 0;
+}
 bool sweep_persistent_enabled(int B, int n, bool refine) {
   if (n > kMaxN) return false;  // its node tasks hold whole blocks in LDS
   const char* v = getenv("SOCU_SWEEP");
   if (v != nullptr && strcmp(v, "level") == 0) return false;
-  if (v != nullptr && strcmp(v, "persistent") == 0) return true;
+  if (sweep_persistent_asked()) return true;
   return n > kSmallN || B <= (refine ? 64 : 32);
 }
 

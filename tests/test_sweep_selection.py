@@ -39,3 +39,32 @@ def test_mixed_solver_by_batch_and_block_size(n, B, want, device, monkeypatch):
     L, E, x = _arrays(n, B, device, torch.float64)
     run = create_cholesky_mixed_factor_and_solve_launch(L, E, x)
     assert run.sweep_status() == (want, False)
+
+
+@pytest.mark.parametrize("graph", [False, True])
+@pytest.mark.parametrize("dtype", ["float64", "float32"])
+@pytest.mark.parametrize("n,N,B", [(1, 1, 1), (4, 20, 1), (12, 20, 2), (16, 70, 3), (16, 2, 1)])
+def test_asked_for_by_small_factor_and_solve(n, N, B, dtype, graph, device, monkeypatch):
+    """factor_and_solve of n <= 16 sweeps back inside the factor's kernels; the
+    variable overrides that too."""
+    import numpy as np
+    import torch
+    from oracle import nd
+    from socu_amd.block_tridiag_solver import create_cholesky_factor_and_solve_launch
+
+    tdt = getattr(torch, dtype)
+    P = [nd.readme_problem(n, N, 1, alpha=10.0, seed=50 + k)[:3] for k in range(B)]
+    for mode, want in (("persistent", True), ("level", False)):
+        monkeypatch.setenv("SOCU_SWEEP", mode)
+        L, E, x = (torch.tensor(np.stack([p[i] for p in P]), dtype=tdt, device=device) for i in range(3))
+        run = create_cholesky_factor_and_solve_launch(L, E, x, dtype=tdt, use_cuda_graph=graph)
+        run()
+        assert run.sweep_status() == (want, False)
+        for k in range(B):
+            Lr, Er, xr = (a.copy() for a in P[k])
+            nd.factor(Lr, Er)
+            nd.solve(Lr, Er, xr)
+            # kappa(Psi) <= 1e3: 1e3 * N * 2^-53, and 2^-24
+            tol = 1e-11 if dtype == "float64" else 5e-4
+            assert np.linalg.norm(x[k].double().cpu().numpy() - xr) < tol * np.linalg.norm(xr)
+            assert np.linalg.norm(np.tril(L[k].double().cpu().numpy()) - np.tril(Lr)) < tol * np.linalg.norm(Lr)
