@@ -827,11 +827,11 @@ constexpr int kBatchStreams = 4;
 
 }  // namespace
 
-// A plan runs level launches over all systems (`levels`).  Untuned plans made
-// with SOCU_BATCHED_WAVES set run one workgroup per system instead: systems
-// are grouped in size buckets b (max(n, m) <= 8, 16, 32), one launch each with
-// tile class tile[b] and workgroups of waves[b] wavefronts.  (With level
-// launches waves[b] is the wavefronts of a node task.)
+// A plan runs level launches over all systems (`levels`) or one workgroup per
+// system (choose_batch): systems are then grouped in size buckets b
+// (max(n, m) <= 8, 16, 32), one launch each with tile class tile[b] and workgroups
+// of waves[b] wavefronts.  (With level launches waves[b] is the wavefronts of a
+// node task.)
 struct socu_batched {
   socu::SmallBatch* levels = nullptr;
   int op = 0, dtype = 0, count = 0;
@@ -897,6 +897,122 @@ int batched_layout(socu_batched* h) {
   const hipError_t e = hipMemcpy(h->dorder, h->order.data(), h->order.size() * sizeof(int), hipMemcpyHostToDevice);
   if (e != hipSuccess) return hip_fail(e, "batched plan set-up (order)");
   return SOCU_OK;
+}
+
+// How a batch runs.
+struct BatchChoice {
+  bool levels = true;
+  int streams = 1;                  // of the level launches
+  int waves[kClasses] = {4, 4, 4};  // per workgroup, without them
+};
+
+// Level launches or one workgroup per system, by an estimate of either's time in
+// microseconds.  One workgroup per system (nd_batched.hip) takes a system's levels
+// in rounds of as many tasks as it has room for (four per wavefront with tiles of 8,
+// else one), so its time goes with the horizon, and a batch of short systems is one
+// launch.  Level launches (nd_small.hip) cost a launch per level, direction and group
+// of systems with one ceil(n / 4), whatever the horizon; on several streams the
+// groups overlap, but forking and joining costs 55 us eager and up to 90 in a graph.
+// Measured over 1316 batches (1 .. 4096 systems, n <= 4 to 32 and mixed, N = 1 .. 200,
+// every operation, eager and graphs).  Where the lines lie: n <= 8 mixed N=15, 12
+// systems, solves, one workgroup each / levels on one stream / on several 28 / 50 /
+// 90 us; n <= 8 N=200 factor_and_solve, 64 systems 193 / 128 / 153; n = 17..32 N=15
+// 256 systems 148 / 209 / 174, N=50 474 / 346 / 219.  The choice is within 10% of the
+// fastest of the three for 1238 of them and within 20% for 1296; level launches on
+// four streams everywhere took up to 4.1 times the faster way's time, one workgroup
+// per system everywhere up to 18 times.
+// (Nothing here depends on the graph: an eager plan and its captured twin give
+// the same bits.)
+BatchChoice choose_batch(const std::vector<socu::BatchProblem>& probs, const std::vector<int>& bucket_of, int op,
+                         int dtype) {
+  const bool fac = op == SOCU_OP_FACTOR || op == SOCU_OP_FACTOR_AND_SOLVE, rhs = op != SOCU_OP_FACTOR;
+  const bool up = op != SOCU_OP_BACKWARD, down = rhs && op != SOCU_OP_FORWARD, f64 = dtype == SOCU_DTYPE_F64;
+  auto nodes = [](int N, int l) { return ((long long)N + (1LL << l)) >> (l + 1); };
+  auto upward = [&](int N, int l) { return nodes(N, l) + (l > 0 ? (long long)N >> (l + 1) : 0); };
+  // horizons and how many systems have them
+  auto lengths = [&](auto in) {
+    std::vector<int> all;
+    for (size_t k = 0; k < probs.size(); ++k)
+      if (in(k)) all.push_back(probs[k].N);
+    std::sort(all.begin(), all.end());
+    std::vector<std::pair<int, int>> h;
+    for (int N : all) {
+      if (h.empty() || h.back().first != N) h.push_back({N, 0});
+      ++h.back().second;
+    }
+    return h;
+  };
+  BatchChoice c;
+
+  // one workgroup per system: a round of node tasks (factor; forward and backward
+  // with one right-hand side, 0.45 times as much for each further one), and how many
+  // workgroups of one wavefront the chip keeps busy
+  static constexpr double kRound[kClasses][3] = {{3.6, 2.3, 2.1}, {4.0, 2.4, 2.3}, {14.5, 5.2, 5.8}};
+  static constexpr double kResident[kClasses][2] = {{1800, 1200}, {1500, 900}, {900, 700}};
+  double longest = 0, work = 0;
+  int buckets = 0;
+  for (int b = 0; b < kClasses; ++b) {
+    const auto h = lengths([&](size_t k) { return bucket_of[k] == b; });
+    if (h.empty()) continue;
+    ++buckets;
+    int m = 1;
+    for (size_t k = 0; k < probs.size(); ++k)
+      if (rhs && bucket_of[k] == b) m = std::max(m, probs[k].m);
+    const double columns = 1 + 0.45 * (m - 1), forward = kRound[b][1] * columns, cd = kRound[b][2] * columns;
+    const double cu = !up ? 0 : (fac ? kRound[b][0] + (rhs ? 0.85 * forward : 0) : forward);
+    double best = -1, best_longest = 0, best_work = 0;
+    for (int w : {4, 2, 1}) {
+      const long long at_once = b == 0 ? 4 * w : w;
+      double t1 = 0, sum = 0;
+      for (const auto& [N, count] : h) {
+        double t = -3;
+        for (int l = 0; N >> l; ++l) {
+          t += cu * (double)((upward(N, l) + at_once - 1) / at_once);
+          if (down) t += cd * (double)((nodes(N, l) + at_once - 1) / at_once);
+        }
+        t = std::max(b == 0 && f64 ? 1.15 * t : t, 5.0);
+        t1 = std::max(t1, t);
+        sum += t * count;
+      }
+      sum *= w / kResident[b][f64 ? 1 : 0];
+      if (best < 0 || std::max(t1, sum) < best) {
+        best = std::max(t1, sum);
+        best_longest = t1;
+        best_work = sum;
+        c.waves[b] = w;
+      }
+    }
+    longest = std::max(longest, best_longest);
+    work += best_work;
+  }
+  const double per_system = 2 + std::max(longest, work) + (buckets > 1 ? 35 : 0);
+
+  // level launches on one stream: a launch and its tasks
+  double levels = 3;
+  int groups = 0;
+  for (int k4 = 1; k4 <= socu::kSmallN / 4; ++k4) {
+    const auto h = lengths([&](size_t k) {
+      return socu::small_class(probs[k].n, fac && rhs ? probs[k].m : 0) / 2 == k4 - 1;
+    });
+    if (h.empty()) continue;
+    ++groups;
+    const double launch_up = fac && k4 > 4 ? 8.0 : (fac && rhs ? (k4 == 1 ? 3.2 : (k4 == 2 ? 3.8 : 4.5)) : (k4 > 4 ? 4.2 : 3.2));
+    const double launch_down = k4 > 4 ? 4.4 : 3.2;
+    const double task = 1e-3 * std::max(0.8, 0.168 * k4 * k4) * (f64 ? 1.0 : 0.6) * (fac && rhs ? 1.0 : 0.6);
+    for (int l = 0; h.back().first >> l; ++l) {
+      double tu = 0, td = 0;
+      for (const auto& [N, count] : h) {
+        tu += (double)count * (double)upward(N, l);
+        td += (double)count * (double)nodes(N, l);
+      }
+      if (up) levels += launch_up + task * tu;
+      if (down) levels += launch_down + 0.4 * task * td;
+    }
+  }
+  const double forked = groups < 2 ? levels : (groups == 2 ? 0.55 * levels + 65 : 0.45 * levels + 72);
+  if (forked < levels) c.streams = std::min(groups, kBatchStreams);
+  c.levels = per_system > 0.95 * std::min(levels, forked);
+  return c;
 }
 
 // The launches of st and of side streams forked from and joined back into it,
@@ -1005,35 +1121,46 @@ int socu_batched_create(socu_batched** out, int op, const socu_batch_system* sys
   hipError_t e = hipMalloc(&h->dprobs, count * sizeof(socu::BatchProblem));
   if (e == hipSuccess) e = hipMalloc(&h->dorder, count * sizeof(int));
   if (e == hipSuccess) e = hipMemcpy(h->dprobs, probs.data(), count * sizeof(socu::BatchProblem), hipMemcpyHostToDevice);
-  for (int k = 0; k < kBatchStreams - 1 && e == hipSuccess; ++k) {
-    e = hipStreamCreateWithFlags(&h->side[k], hipStreamNonBlocking);
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&h->join[k], hipEventDisableTiming);
-  }
-  if (e == hipSuccess) e = hipEventCreateWithFlags(&h->fork, hipEventDisableTiming);
   if (e != hipSuccess) {
     batched_release(h);
     return hip_fail(e, "batched plan set-up");
   }
   rc = batched_layout(h);
-  // Level launches leave nothing to choose by timing: `tune` is accepted and
-  // does not change the plan.  For an untuned plan SOCU_BATCHED_WAVES=1|2|4
-  // asks for one workgroup of so many wavefronts per system, narrowed where
-  // its LDS does not fit the bucket's right-hand sides.
-  const char* w = tune ? nullptr : getenv("SOCU_BATCHED_WAVES");
-  const int wv = w ? atoi(w) : 0;
-  if (rc == SOCU_OK && (wv == 1 || wv == 2 || wv == 4)) {
-    for (int b = 0; b < kClasses; ++b) {
-      int v = wv;
-      while (v > 1 && !socu::batched_fits(h->tile[b], v, h->mmax[b], h->dtype)) v /= 2;
-      h->waves[b] = v;
-    }
-  } else if (rc == SOCU_OK) {
-    e = socu::small_batch_create(&h->levels, probs.data(), count, op, kBatchStreams);
-    if (e != hipSuccess) rc = hip_fail(e, "batched plan set-up (levels)");
-  }
   if (rc) {
     batched_release(h);
     return rc;
+  }
+  // `tune` is accepted and does not change the plan: there is nothing to choose by
+  // timing.  For an untuned plan SOCU_BATCHED_WAVES overrides the choice: 1, 2 or 4
+  // wavefronts per workgroup and system, or 0 for level launches.
+  BatchChoice choice = choose_batch(probs, h->bucket_of, op, dtype);
+  const char* w = tune ? nullptr : getenv("SOCU_BATCHED_WAVES");
+  const int wv = w != nullptr && *w >= '0' && *w <= '9' ? atoi(w) : -1;
+  if (wv == 0) choice.levels = true;
+  if (wv == 1 || wv == 2 || wv == 4) {
+    choice.levels = false;
+    for (int b = 0; b < kClasses; ++b) choice.waves[b] = wv;
+  }
+  int streams = choice.streams;
+  if (choice.levels) {
+    e = socu::small_batch_create(&h->levels, probs.data(), count, op, streams);
+  } else {
+    streams = 0;
+    for (int b = 0; b < kClasses; ++b) {
+      int v = choice.waves[b];  // fewer where the LDS does not fit the right-hand sides
+      while (v > 1 && !socu::batched_fits(h->tile[b], v, h->mmax[b], h->dtype)) v /= 2;
+      h->waves[b] = v;
+      if (h->counts[b] > 0) ++streams;
+    }
+  }
+  for (int k = 0; k + 1 < streams && e == hipSuccess; ++k) {
+    e = hipStreamCreateWithFlags(&h->side[k], hipStreamNonBlocking);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&h->join[k], hipEventDisableTiming);
+  }
+  if (e == hipSuccess && streams > 1) e = hipEventCreateWithFlags(&h->fork, hipEventDisableTiming);
+  if (e != hipSuccess) {
+    batched_release(h);
+    return hip_fail(e, "batched plan set-up (streams, levels)");
   }
   if (use_graph) {
     hipStream_t cs;
