@@ -1,0 +1,84 @@
+"""Schur updates of levels that stream more than 16 MiB: 64x64 tiles, for block sizes
+whose 16-row tiles fill them (n = 49 .. 64 and 113 .. 128, ragged ones among them); and
+the same batch one system short of it, by 16x16 tiles.  In place, out of place and with
+a masked system, against the oracle.
+"""
+import numpy as np
+import pytest
+
+from oracle import nd
+
+pytestmark = pytest.mark.gpu
+
+N = 16  # level 0: 8 targets and 7 fill-ins of each system
+LIMIT = 16 * 2**20
+
+
+def _rel(a, b):
+    return np.linalg.norm((a - b).ravel()) / max(np.linalg.norm(b.ravel()), 1e-300)
+
+
+def _systems(n, size):
+    """Systems from which on level 0 takes the 64x64 tiles."""
+    return LIMIT // (15 * n * n * size) + 1
+
+
+def _problems(n, B):
+    P = [nd.readme_problem(n, N, 1, alpha=16.0, seed=n + k)[:2] for k in range(min(B, 3))]
+    want = []
+    for L0, E0 in P:
+        Lr, Er = L0.copy(), E0.copy()
+        nd.factor(Lr, Er)
+        want.append((np.tril(Lr), Er))
+    return [np.stack([P[k % 3][i] for k in range(B)]) for i in range(2)], want
+
+
+def _check(L, E, want, B, tol, skip=()):
+    L, E = L.double().cpu().numpy(), E.double().cpu().numpy()
+    for b in sorted({0, 1, 2, B // 2, B - 2, B - 1} - set(skip)):
+        assert _rel(np.tril(L[b]), want[b % 3][0]) < tol and _rel(E[b], want[b % 3][1]) < tol, b
+
+
+@pytest.mark.parametrize("n,dtype", [(113, "float64"), (120, "float32"), (127, "float64"), (128, "float64")])
+@pytest.mark.parametrize("short", [0, 1])
+def test_factor(n, dtype, short, device):
+    import torch
+    from socu_amd import _lib
+    from socu_amd.block_tridiag_solver import create_cholesky_factor_launch
+
+    tdt = getattr(torch, dtype)
+    B = _systems(n, 8 if dtype == "float64" else 4) - short
+    print(f"schur n={n} {dtype} B={B}", flush=True)
+    # kappa(Psi) <= 1e3: 1e3 * N * 2^-53, and 2^-24
+    tol = 1e-11 if dtype == "float64" else 5e-4
+    (L0, E0), want = _problems(n, B)
+    Ls, Es = (torch.tensor(a, dtype=tdt, device=device) for a in (L0, E0))
+    mask = torch.ones(B, dtype=torch.bool, device=device)
+    mask[1] = short == 1  # (a masked system counts in the level's size)
+    L, E = Ls.clone(), Es.clone()
+    create_cholesky_factor_launch(L, E, mask=mask, dtype=tdt)()
+    skip = () if short else (1,)
+    _check(L, E, want, B, tol, skip)
+    assert all(torch.equal(L[k], Ls[k]) and torch.equal(E[k], Es[k]) for k in skip)
+    L, E = torch.full_like(Ls, 7.0), torch.full_like(Es, 7.0)
+    code = _lib.DTYPE_F64 if dtype == "float64" else _lib.DTYPE_F32
+    rc = _lib.load().socu_cholesky_factor_from(Ls.data_ptr(), Es.data_ptr(), L.data_ptr(), E.data_ptr(), None, B, N, n,
+                                               code, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    _check(L, E, want, B, tol)
+
+
+@pytest.mark.parametrize("n", [50, 63, 64, 117])
+@pytest.mark.parametrize("short", [0, 1])
+def test_fp64_pivots(n, short, device):
+    import torch
+    from socu_amd import _lib
+
+    B = _systems(n, 4) - short
+    print(f"schur pivots n={n} B={B}", flush=True)
+    (L0, E0), want = _problems(n, B)
+    L, E = (torch.tensor(a, dtype=torch.float32, device=device) for a in (L0, E0))
+    rc = _lib.load().socu_cholesky_factor_f32(L.data_ptr(), E.data_ptr(), None, B, N, n, _lib.PREC_FP32,
+                                              torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    _check(L, E, want, B, 5e-4)
