@@ -589,10 +589,10 @@ int socu_plan_create(socu_plan** out, int op, void* L, void* E, void* x, const u
       rc = hip_fail(e, "hipMalloc (diagonal-block inverse workspace)");
     }
   }
-  // The forward sweep alongside the factor pays inside a graph only: issued
-  // eagerly, its event records and waits cost more host time than the
-  // overlap saves (n=128 N=512 FP64: 1.19 ms without, 1.24 ms with).
-  if (rc == SOCU_OK && op == SOCU_OP_FACTOR_AND_SOLVE && B > 0 && use_graph) {
+  // The forward sweep alongside the factor (n <= 64: inside its kernels) pays inside
+  // a graph only: issued eagerly, its event records and waits cost more host time
+  // than the overlap saves (n=128 N=512 FP64: 1.19 ms without, 1.24 ms with).
+  if (rc == SOCU_OK && op == SOCU_OP_FACTOR_AND_SOLVE && B > 0 && use_graph && n > socu::kSmallUpN) {
     const hipError_t e = socu::overlap_create(p->overlap);
     if (e != hipSuccess) rc = hip_fail(e, "stream / event creation (factor_and_solve)");
     p->has_overlap = e == hipSuccess;

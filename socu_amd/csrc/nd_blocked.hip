@@ -371,8 +371,8 @@ static hipError_t set_schur_small_attrs() {
 // k_schur_blk rather than 16x16 tiles (k_schur_tile, nd_large.hip), which read each
 // operand once per tile: where a level streams many blocks and the 64x64 tiles are
 // all inside the block.  n = 128, FP64, levels of 256, 128, 64 and 32 nodes: 99, 58,
-// 33 us (and 22 in 32x32 tiles with all of K staged in LDS) to 116, 60, 32 and 18;
-// n = 200: 76 us (32 nodes) to 54.
+// 33 us (and 22 in 32x32 tiles with all of K staged in LDS) to 116, 60, 32 and 18.
+// (n > 128 takes 16x16 tiles always, factor_level_large: n = 200, 32 nodes, 76 us to 54.)
 static bool use_schur_blk(int nodes, int n, int esize) {
   return (n + 15) / 16 % 4 == 0 && (double)nodes * n * n * esize > 16.0 * 1024 * 1024;
 }
@@ -442,10 +442,12 @@ static hipError_t factor_level_nb(T* L, T* E, const uint8_t* mask, int B, int N,
     const int nodes = B * (nT + nF);
     const dim3 grid_blk(8 * schur_blk_per_xcd(nT, nF, ntile), B);
     if (!bf16) {
-      if (!use_schur_blk(nodes, n, (int)sizeof(T))) {
+      bool blk = false;
+      if constexpr (NB % 2 == 0) blk = use_schur_blk(nodes, n, (int)sizeof(T));
+      if (!blk) {
         ep = schur_tiles<T>(L, Lsrc, E, mask, B, N, n, lidx, nT, nF, st);
         if (ep != hipSuccess) return ep;
-      } else {
+      } else if constexpr (NB % 2 == 0) {
         hipLaunchKernelGGL((k_schur_blk<T, NF, false>), grid_blk, dim3(kThreads), 0, st, L, E, mask, N, n, nE, lv.s,
                            lv.off, lv.next_off, nT, nF, ntile, Lsrc);
       }
@@ -496,7 +498,6 @@ hipError_t factor_level_blocked(T* L, T* E, const uint8_t* mask, int B, int N, i
     if (Lsrc != nullptr || Esrc != nullptr) return hipErrorInvalidValue;  // in place only
     return factor_level_large<T>(L, E, mask, B, N, n, lidx, st, after_potrf, after_trsm, before_trsm);
   }
-  const int fp = prec;
   // small blocks in the storage precision (in place): one launch per level,
   // which applies the previous level's updates itself.  FP32 storage with FP64
   // pivots or BF16 Schur products takes the separate kernels.
@@ -509,32 +510,22 @@ hipError_t factor_level_blocked(T* L, T* E, const uint8_t* mask, int B, int N, i
     if (e == hipSuccess && after_trsm != nullptr) e = hipEventRecord(after_trsm, st);
     return e;
   }
+  // (FP64 blocks of n <= 64 have returned above)
+  auto level = [&](auto nb, auto nf) {
+    return factor_level_nb<T, decltype(nb)::value, decltype(nf)::value>(L, E, mask, B, N, n, lidx, prec, st, after_potrf,
+                                                                        after_trsm, before_trsm, Lsrc, Esrc);
+  };
+  using std::integral_constant;
   if constexpr (sizeof(T) == 4) {
-    if (n == 32)
-      return factor_level_nb<T, 1, 32>(L, E, mask, B, N, n, lidx, fp, st, after_potrf, after_trsm, before_trsm, Lsrc,
-                                       Esrc);
-    if (n < 32)
-      return factor_level_nb<T, 1, 0>(L, E, mask, B, N, n, lidx, fp, st, after_potrf, after_trsm, before_trsm, Lsrc,
-                                      Esrc);
+    if (n == 32) return level(integral_constant<int, 1>{}, integral_constant<int, 32>{});
+    if (n < 32) return level(integral_constant<int, 1>{}, integral_constant<int, 0>{});
+    if (n == 64) return level(integral_constant<int, 2>{}, integral_constant<int, 64>{});
+    if (n < 64) return level(integral_constant<int, 2>{}, integral_constant<int, 0>{});
   }
-  switch (n) {
-    case 64: return factor_level_nb<T, 2, 64>(L, E, mask, B, N, n, lidx, fp, st, after_potrf, after_trsm, before_trsm, Lsrc,
-                                                   Esrc);
-    case 96: return factor_level_nb<T, 3, 96>(L, E, mask, B, N, n, lidx, fp, st, after_potrf, after_trsm, before_trsm, Lsrc,
-                                                   Esrc);
-    case 128: return factor_level_nb<T, 4, 128>(L, E, mask, B, N, n, lidx, fp, st, after_potrf, after_trsm, before_trsm, Lsrc,
-                                                   Esrc);
-    default: break;
-  }
-  switch ((n + 31) / 32) {
-    case 2: return factor_level_nb<T, 2, 0>(L, E, mask, B, N, n, lidx, fp, st, after_potrf, after_trsm, before_trsm, Lsrc,
-                                                   Esrc);
-    case 3: return factor_level_nb<T, 3, 0>(L, E, mask, B, N, n, lidx, fp, st, after_potrf, after_trsm, before_trsm, Lsrc,
-                                                   Esrc);
-    case 4: return factor_level_nb<T, 4, 0>(L, E, mask, B, N, n, lidx, fp, st, after_potrf, after_trsm, before_trsm, Lsrc,
-                                                   Esrc);
-    default: return hipErrorInvalidValue;
-  }
+  if (n == 96) return level(integral_constant<int, 3>{}, integral_constant<int, 96>{});
+  if (n == 128) return level(integral_constant<int, 4>{}, integral_constant<int, 128>{});
+  if (n < 96) return level(integral_constant<int, 3>{}, integral_constant<int, 0>{});
+  return level(integral_constant<int, 4>{}, integral_constant<int, 0>{});
 }
 
 template <typename T>
@@ -605,19 +596,15 @@ hipError_t overlap_create(SweepOverlap& ov) {
   if (e == hipSuccess) e = hipEventCreateWithFlags(&ov.fork, hipEventDisableTiming);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&ov.join, hipEventDisableTiming);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&ov.ready, hipEventDisableTiming);
-  for (int l = 0; l < kSweepMaxLevels && e == hipSuccess; ++l) {
-    e = hipEventCreateWithFlags(&ov.potrf[l], hipEventDisableTiming);
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&ov.trsm[l], hipEventDisableTiming);
-  }
+  for (int l = 0; l < kSweepMaxLevels && e == hipSuccess; ++l)
+    e = hipEventCreateWithFlags(&ov.level[l], hipEventDisableTiming);
   if (e != hipSuccess) overlap_destroy(ov);
   return e;
 }
 
 void overlap_destroy(SweepOverlap& ov) {
-  for (int l = 0; l < kSweepMaxLevels; ++l) {
-    if (ov.potrf[l]) (void)hipEventDestroy(ov.potrf[l]);
-    if (ov.trsm[l]) (void)hipEventDestroy(ov.trsm[l]);
-  }
+  for (int l = 0; l < kSweepMaxLevels; ++l)
+    if (ov.level[l]) (void)hipEventDestroy(ov.level[l]);
   if (ov.fork) (void)hipEventDestroy(ov.fork);
   if (ov.join) (void)hipEventDestroy(ov.join);
   if (ov.ready) (void)hipEventDestroy(ov.ready);
@@ -645,10 +632,10 @@ hipError_t factor_with_forward(T* L, T* E, T* x, const uint8_t* factor_mask, con
     // one fork per level (each costs the main stream about 4 us in a graph):
     // behind level l's trsm the side stream applies level l and updates from it
     const bool last = l == Lv - 1;
-    e = factor_level_blocked<T>(L, E, factor_mask, B, N, n, l, prec, st, last ? ov.potrf[l] : nullptr,
-                                last ? nullptr : ov.trsm[l], (l == 0 && side_first != nullptr) ? ov.ready : nullptr,
+    e = factor_level_blocked<T>(L, E, factor_mask, B, N, n, l, prec, st, last ? ov.level[l] : nullptr,
+                                last ? nullptr : ov.level[l], (l == 0 && side_first != nullptr) ? ov.ready : nullptr,
                                 l == 0 ? Lsrc : nullptr, l == 0 ? Esrc : nullptr);
-    if (e == hipSuccess) e = hipStreamWaitEvent(ov.side, last ? ov.potrf[l] : ov.trsm[l], 0);
+    if (e == hipSuccess) e = hipStreamWaitEvent(ov.side, ov.level[l], 0);
     if (e == hipSuccess) e = forward_apply_blocked<T>(L, E, x, sweep_mask, B, N, n, m, l, ov.side);
     if (e == hipSuccess && !last) e = forward_update_blocked<T>(L, E, x, sweep_mask, B, N, n, m, l, ov.side);
   }

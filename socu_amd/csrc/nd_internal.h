@@ -163,14 +163,13 @@ bool sweep_persistent_enabled(int B, int n, bool refine);
 bool sweep_persistent_asked();
 
 // A side stream and per-level events that let the forward sweep of a
-// factor_and_solve run alongside the factor: forward step l waits for level
-// l's trsm, the inverses of level l for its potrf (created with a plan,
-// destroyed with it).
+// factor_and_solve run alongside the factor: level l of the sweep waits for
+// level l's trsm, or potrf at the last level (created with a plan for n > kSmallUpN
+// or a mixed handle, destroyed with it).
 struct SweepOverlap {
   hipStream_t side = nullptr;
   hipEvent_t fork = nullptr, join = nullptr, ready = nullptr;
-  hipEvent_t potrf[kSweepMaxLevels] = {};
-  hipEvent_t trsm[kSweepMaxLevels] = {};
+  hipEvent_t level[kSweepMaxLevels] = {};
 };
 hipError_t overlap_create(SweepOverlap& ov);
 void overlap_destroy(SweepOverlap& ov);

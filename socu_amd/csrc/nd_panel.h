@@ -150,18 +150,14 @@ constexpr PanelPlan panel_plan(int total) {
 // p[j]: NP payload rows per lane, p[j] <- p[j] L^-T.
 // NC: columns of the panel (a tile whose last 16 - NC rows and columns are
 // identity padding needs no steps for them; entries from NC on are untouched).
-// All 64 lanes must be active.  hook(k) runs before step k (k: an
-// integral_constant).
+// All 64 lanes must be active.
 //
 // Step k's multiply-adds other than the one that gives the next pivot are
 // spread between the dependent operations of the next pivot's reciprocal
 // square root (left to itself the compiler moves each one down to the first
 // use of its result, and the chain then waits out every latency).
-struct NoHook {
-  __device__ __forceinline__ void operator()(int) const {}
-};
-template <typename T, int NP, int NC = 16, typename Hook = NoHook>
-__device__ __forceinline__ void panel16(T (&u)[16], T (&p)[NP][16], Hook hook = Hook()) {
+template <typename T, int NP, int NC = 16>
+__device__ __forceinline__ void panel16(T (&u)[16], T (&p)[NP][16]) {
   wait_states<2>();
   T inv = rsqrt_filled(bcast_row<0>(u[0]), [](auto) {});
   T lk = u[0] * inv, pk[NP];
@@ -171,7 +167,6 @@ __device__ __forceinline__ void panel16(T (&u)[16], T (&p)[NP][16], Hook hook = 
   wait_states<2>();
   static_for<NC>([&](auto kc) {
     constexpr int k = decltype(kc)::value;
-    hook(kc);
     u[k] = lk;  // row k itself: piv / sqrt(piv)
 #pragma unroll
     for (int j = 0; j < NP; ++j) p[j][k] = pk[j];
