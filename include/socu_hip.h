@@ -172,10 +172,12 @@ int socu_plan_destroy(socu_plan* plan);
  * backward substitution as one persistent launch of node tasks that wait on
  * per-node counters; the wide lower levels keep the level kernels (same
  * arithmetic per block as the reference's sweeps,
- * block_tridiag_solver.py:425-485 and :581-643).  Used by every plan with one
- * right-hand side, in both precisions (it measured faster than the level
- * kernels for every block size); the environment variable SOCU_SWEEP read at
- * creation overrides: "level" (never) or "persistent" (always).  Each wait
+ * block_tridiag_solver.py:425-485 and :581-643).  Used by plans with one
+ * right-hand side, in both precisions, where that measured faster than level
+ * kernels: 32 < n <= 128, or n <= 32 and at most 32 systems (mixed handles: 64),
+ * except by factor_and_solve plans of n <= 16 and at most 256 systems, which sweep
+ * back inside the factor's kernels.  The environment variable SOCU_SWEEP read at
+ * creation overrides: "level" (never) or "persistent" (every n <= 128).  Each wait
  * is bounded; if one expires the launch drains, the tasks that depended on
  * the wait write NaN into their part of x (so the failure shows in the
  * solution), and a host-visible word is raised: the plan's next
@@ -241,17 +243,19 @@ int socu_profile_op(int op, void* L, void* E, void* x, const unsigned char* mask
  * entry are ignored, as in socu_cholesky_factor), and x
  * (N,n,m) (ignored for SOCU_OP_FACTOR); `reserved` must be 0.  Needs
  * n <= socu_batched_max_block_size() and m <= 32.  mask is NULL or `count`
- * bytes indexed like `systems`.  The systems run together, one launch per
- * dissection level, direction and group of systems with one ceil(n / 4), the
- * groups on forked streams.  `tune` is accepted and has nothing to choose.
- * Without `tune`, the environment variable SOCU_BATCHED_WAVES = 1, 2 or 4
- * runs one workgroup of so many wavefronts per system instead (fewer where
- * its LDS does not fit), for comparison.  create builds the task lists,
- * copies them and the system table to the device and synchronises; execute
- * allocates nothing and synchronises nothing.  socu_batched_config returns
- * per size bucket (max(n, m) <= 8, <= 16, <= 32) the system count, the tile
- * size and the wavefronts that work on one node (or, with
- * SOCU_BATCHED_WAVES, per workgroup). */
+ * bytes indexed like `systems`.  Batches of short systems run one workgroup
+ * per system, one launch per size bucket (max(n, m) <= 8, <= 16, <= 32); the
+ * others one launch per dissection level, direction and group of systems with
+ * one ceil(n / 4).  create estimates which is faster from the horizons, the
+ * sizes and the number of systems, and puts buckets or groups on forked
+ * streams where that pays.  `tune` is accepted and changes nothing.  Without
+ * `tune`, the environment variable SOCU_BATCHED_WAVES overrides the choice: 1, 2
+ * or 4 wavefronts per system (fewer where the LDS does not fit), or 0 for level
+ * launches.  create builds the task lists, copies them and the system table to
+ * the device and synchronises; execute allocates nothing and synchronises
+ * nothing.  socu_batched_config returns per size bucket the system count, the
+ * tile size and the wavefronts that work on one node, or of a system's
+ * workgroup. */
 typedef struct socu_batch_system {
   void* L;
   void* E;

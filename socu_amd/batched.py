@@ -74,8 +74,8 @@ class BatchedLaunch:
 
     def config(self) -> dict:
         """Per size bucket (max(n, m) <= 8, 16, 32): the number of systems, the
-        tile size and the wavefronts that work on one node (with
-        SOCU_BATCHED_WAVES: per workgroup)."""
+        tile size and the wavefronts that work on one node (one workgroup per
+        system: the wavefronts of a workgroup)."""
         counts = (ctypes.c_int * 3)()
         tiles = (ctypes.c_int * 3)()
         waves = (ctypes.c_int * 3)()
@@ -103,10 +103,11 @@ def create_batched_cholesky_launch(L: Sequence[torch.Tensor], E: Sequence[torch.
 
     ``mask`` is a bool tensor with one entry per system; a False entry leaves
     that system untouched, as in the reference's mask (README.md:214-235).
-    Every level of all systems with one ceil(n / 4) is one launch.  ``tune`` is
-    accepted and has nothing to choose; with ``tune=False`` the environment
-    variable SOCU_BATCHED_WAVES (1, 2 or 4) runs one workgroup of so many
-    wavefronts per system instead.
+    Batches of short systems run one workgroup per system; otherwise every level of
+    all systems with one ceil(n / 4) is one launch.  The choice goes by the horizons,
+    the sizes and the number of systems.  ``tune`` is accepted and changes nothing;
+    with ``tune=False`` the environment variable SOCU_BATCHED_WAVES overrides the
+    choice (1, 2 or 4 wavefronts per system, or 0 for level launches).
     """
     if op not in _OPS:
         raise ValueError(f"unknown op {op!r}; expected one of {sorted(_OPS)}")

@@ -28,8 +28,8 @@
 // runs one or more tasks at once (BShape); block products run on MFMA
 // (16x16 tiles, NT >= 16) or, for NT = 8, as 2x2 register blocks per lane.
 // Small workgroups (W = 1) let several systems share a compute unit, one per
-// SIMD.  Plans run level launches over all systems (nd_small.hip) unless
-// SOCU_BATCHED_WAVES asks for this kernel.
+// SIMD.  Batches of short systems run by this kernel, the others by level launches
+// over all systems (nd_small.hip): choose_batch in capi.hip.
 #include "../../include/socu_hip.h"
 #include "nd_common.h"
 #include "nd_internal.h"

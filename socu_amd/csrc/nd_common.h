@@ -17,16 +17,16 @@
 
 namespace socu {
 
-// Threads per workgroup for every level kernel: four 64-wide wavefronts.
+// Threads per workgroup where a kernel does not choose its own: four 64-wide
+// wavefronts.
 constexpr int kThreads = 256;
 
-// Largest block size n handled by the LDS-resident kernels (a padded
-// 128x129 fp64 block is 129 KiB of the 160 KiB of LDS per workgroup).
+// Largest block size n whose diagonal block one workgroup factors and inverts
+// (k_potrf_blk: eight 16-row tiles, their columns in registers).
 constexpr int kMaxN = 128;
 
-// Largest block size n of the tiled kernels for larger blocks (the block in
-// HBM, 32 x 32 tiles through LDS; a staged 32-wide chunk of a 256-wide
-// block is 66 KiB of FP64 LDS).
+// Largest block size n: two halves of at most kMaxN (nd_large.hip; a chunk of 16
+// vectors of a 256-wide block is 34 KiB of FP64 LDS).
 constexpr int kMaxNLarge = 256;
 
 // Column chunk of the right-hand sides processed by one workgroup.

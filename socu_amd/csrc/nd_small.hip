@@ -911,7 +911,8 @@ hipError_t small_up_level(T* L, T* E, T* x, const uint8_t* mask, int B, int N, i
 // 35.5 us, n=12 N=100 57.7 / 52.1, n=10 N=1000 87.6 / 82.9, 256 systems of n=12
 // N=40 80.5 / 66.9; 2000 systems of n=4 N=30 117.8 / 154.4.  With two
 // wavefronts per task (n > 16) a compute unit holds too few tasks: n=32 N=100
-// 102 / 117.
+// 102 / 117.  (At n = 13 .. 15 the 1024 threads leave the compiler 9 (FP32) or 12
+// (FP64) registers short, which it spills; these sizes were not timed apart.)
 bool small_tail_applies(int B, int n, int m) {
   return n <= kSmallN && small_class(n, m) < 2 * 4 && B <= kTailMaxSystems;
 }
@@ -982,8 +983,10 @@ hipError_t small_backward_level(const T* L, const T* E, T* x, const uint8_t* mas
 // per system walking its levels leaves the chip idle behind the long systems
 // and runs the wide levels of each a few tasks at a time.  FP64
 // factor_and_solve of systems of N = 10..200, n = 8..32, the inputs copied in
-// first, one workgroup per system / level launches: 4096 systems 12.8 / 6.0 ms,
-// 32 systems without a graph 1.92 / 0.32 ms; 512 systems in FP32 2.26 / 0.47 ms.)
+// first, one workgroup per system / level launches: 4096 systems 11.7 / 6.0 ms,
+// 32 systems without a graph 1.92 / 0.32 ms; 512 systems in FP32 2.26 / 0.47 ms.
+// Where the horizons are short it is the other way round: choose_batch in
+// capi.hip.)
 // ---------------------------------------------------------------------------
 struct SmallBatch {
   struct Level {

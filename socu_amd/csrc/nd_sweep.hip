@@ -567,7 +567,9 @@ hipError_t init_sweep_kernels() {
 }
 
 // One launch for the upper levels against one per level and direction.  At n > 32
-// always.  At n <= 32 a level kernel is one wavefront per node and its launch 3-4 us,
+// always: solves by level kernels took 1.00 to 3.04 times as long over n = 34 .. 128,
+// N = 64 and 512, 1 to 64 systems, both precisions (FP64 N=512: n=34 B=1 129 / 203 us,
+// B=64 1672 / 1684; n=128 B=1 336 / 650, B=8 1809 / 1998).  At n <= 32 a level kernel is one wavefront per node and its launch 3-4 us,
 // and the batch decides, by how many levels the one launch takes (sweep_lmin).
 // Level kernels / persistent over 280 plans each (n = 4 .. 32, N = 8 .. 700, in a
 // graph): FP64 solves 1.10 at B=9, 1.05 at 16, 1.00 at 32, 0.97 at 64; FP32 backward
@@ -596,12 +598,12 @@ size_t sweep_slot_elems(int B, int N, int n) {
 
 // Lowest level swept by the persistent launch: levels pay there while the
 // widest of them has at most W nodes over the batch, with W = 64 for n <= 64,
-// 256 for FP32 and 1024 for FP64 blocks above that.  Measured solve times
-// (N=512, one right-hand side, lmin 0..5 against the level kernels) for
-// B = 1, 4 and n = 32, 64, 96, 128 in both precisions: this choice is the
-// fastest or within 4% of it in each case (FP64 n=128 B=1: 226 us against
-// 341 us with level kernels only, FP32: 127 us against 220 us).  Below lmin
-// the level kernels stream the wide levels.
+// 256 for FP32 and 1024 for FP64 blocks above that.  The lines were drawn between
+// these sweeps and former, slower level kernels (N=512, B = 1 and 4, n = 32, 64, 96,
+// 128: the fastest split or within 4% of it); with today's the sweeps as a whole are
+// still the faster way wherever they are taken (sweep_persistent_enabled), the split
+// itself has not been timed again.  Below lmin the level kernels stream the wide
+// levels.
 int sweep_lmin(int B, int N, int n, int dsize) {
   const int Lv = recursive_iterations(N);
   const long long W = n <= 64 ? 64 : (dsize == 8 ? 1024 : 256);
