@@ -116,7 +116,8 @@ struct Chunk {
 };
 
 // X(k, c) <- the chunk, zero to 16 columns and to a multiple of 32 in k.  FAR (here
-// and below): a chunk of right-hand sides of a block row above 4 GiB.
+// and below): a chunk of right-hand sides of a block row above 4 GiB (64-bit offsets
+// for all cost 0.4% of a factor_and_solve of n=200 N=64 m=2).
 template <typename T, int THREADS, bool FAR = false>
 __device__ __forceinline__ void stage_chunk(T* X, const Chunk<T>& c, int K) {
   const int kp = (K + 31) & ~31;
@@ -131,7 +132,7 @@ __device__ __forceinline__ void stage_chunk(T* X, const Chunk<T>& c, int K) {
       j = idx & 15;
     }
     const int kc = min(k, K - 1), jc = min(j, c.count - 1);
-    const T v = FAR ? ldx(c.p, kc, c.ld, jc) : ldg(c.p, c.rows ? jc * c.ld + kc : kc * c.ld + jc);
+    const T v = FAR ? ld_rhs<true>(c.p, kc, c.ld, jc) : ldg(c.p, c.rows ? jc * c.ld + kc : kc * c.ld + jc);
     X[k * kPP + j] = (k < K && j < c.count) ? v : T(0);
   }
 }
@@ -164,7 +165,7 @@ __device__ __forceinline__ void panel_product(const T* M, int ld, int R, int K, 
 #pragma unroll
     for (int e = 0; e < 4; ++e)
       if (ok[e]) {
-        if constexpr (FAR) stx(out.p, 16 * t + Mfma<T>::row(lane, e), out.ld, li, acc[e]);  // (mode 0, not TR)
+        if constexpr (FAR) st_rhs<true>(out.p, 16 * t + Mfma<T>::row(lane, e), out.ld, li, acc[e]);  // (mode 0, not TR)
         else stg(out.p, off[e], mode == 0 ? acc[e] : c[e] - acc[e]);
       }
   }
@@ -306,8 +307,7 @@ __global__ __launch_bounds__(kThreads) void k_update_large(const T* __restrict__
   if (row < n && col < count) {
     T* const p = xb + j * nm;
     const T sum = (part[0][q] + part[1][q]) + (part[2][q] + part[3][q]);
-    if constexpr (FAR) stx(p, row, m, col, ldx(p, row, m, col) - sum);
-    else stg(p, row * m + col, ldg(p, row * m + col) - sum);
+    st_rhs<FAR>(p, row, m, col, ld_rhs<FAR>(p, row, m, col) - sum);
   }
 }
 
@@ -426,12 +426,6 @@ hipError_t set_attrs() {
                         (const void*)k_update_large<T, true, false>, (const void*)k_update_large<T, true, true>})
     if (e == hipSuccess) e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)update_lds<T>(kMaxNLarge));
   return e;
-}
-
-// (64-bit offsets cost 0.4% of a factor_and_solve of n=200 N=64 m=2)
-template <typename T>
-bool far_rhs(int n, int m) {
-  return (size_t)n * m * sizeof(T) > 0xffffffffu;
 }
 
 template <typename T>

@@ -65,17 +65,24 @@ __device__ __forceinline__ typename Pair<T>::type ldg2(const T* base, int off) {
   typedef const __attribute__((address_space(1))) v2* gptr;
   return *(gptr)((gbytes)base + (unsigned)off * (unsigned)sizeof(T));
 }
-// Element (row, col) of a block row of right-hand sides, m columns: a 64-bit
-// offset, as the sweeps take any m and n m elements may be more than 4 GiB.
-template <typename T>
-__device__ __forceinline__ T ldx(const T* y, int row, int m, int col) {
+// Element (row, col) of a block row of right-hand sides, m columns.  FAR: with a
+// 64-bit offset, for block rows of 4 GiB and more (the sweeps take any m).
+template <bool FAR, typename T>
+__device__ __forceinline__ T ld_rhs(const T* y, int row, int m, int col) {
   typedef const __attribute__((address_space(1))) T* gptr;
-  return ((gptr)y)[(unsigned long long)(unsigned)row * (unsigned)m + (unsigned)col];
+  if constexpr (FAR) return ((gptr)y)[(unsigned long long)(unsigned)row * (unsigned)m + (unsigned)col];
+  else return ldg(y, row * m + col);
 }
-template <typename T>
-__device__ __forceinline__ void stx(T* y, int row, int m, int col, T v) {
+template <bool FAR, typename T>
+__device__ __forceinline__ void st_rhs(T* y, int row, int m, int col, T v) {
   typedef __attribute__((address_space(1))) T* gptr;
-  ((gptr)y)[(unsigned long long)(unsigned)row * (unsigned)m + (unsigned)col] = v;
+  if constexpr (FAR) ((gptr)y)[(unsigned long long)(unsigned)row * (unsigned)m + (unsigned)col] = v;
+  else stg(y, row * m + col, v);
+}
+// Whether a launch needs it.
+template <typename T>
+bool far_rhs(int n, int m) {
+  return (size_t)n * m * sizeof(T) > 0xffffffffu;
 }
 template <typename P>
 __device__ __forceinline__ P* uniform_ptr(P* p) {

@@ -112,13 +112,10 @@ struct Frag {
 // others; the first operand is masked in the summed direction and results
 // past n or m are not stored.  FAR: block rows of any size (the factor takes m <= 32).
 template <typename T, int K4, bool FAR = false>
-__device__ __forceinline__ void ld_rhs(T (&f)[K4], const T* y, int n, int m, int c0) {
+__device__ __forceinline__ void ld_rhs_b(T (&f)[K4], const T* y, int n, int m, int c0) {
   const int l = lane_id(), j = min(c0 + (l & 15), m - 1), g = l >> 4;
 #pragma unroll
-  for (int t = 0; t < K4; ++t) {
-    const int row = min(4 * t + g, n - 1);
-    f[t] = FAR ? ldx(y, row, m, j) : ldg(y, row * m + j);
-  }
+  for (int t = 0; t < K4; ++t) f[t] = ld_rhs<FAR>(y, min(4 * t + g, n - 1), m, j);
 }
 template <typename T, int NB, bool FAR = false>
 __device__ __forceinline__ void ld_rhs_acc(typename Mfma<T>::acc_t (&a)[NB], const T* y, int n, int m, int c0) {
@@ -126,17 +123,8 @@ __device__ __forceinline__ void ld_rhs_acc(typename Mfma<T>::acc_t (&a)[NB], con
 #pragma unroll
   for (int b = 0; b < NB; ++b)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = min(16 * b + Mfma<T>::row(l, r), n - 1);
-      a[b][r] = FAR ? ldx(y, row, m, j) : ldg(y, row * m + j);
-    }
+    for (int r = 0; r < 4; ++r) a[b][r] = ld_rhs<FAR>(y, min(16 * b + Mfma<T>::row(l, r), n - 1), m, j);
 }
-template <typename T, bool FAR>
-__device__ __forceinline__ void st_rhs(T* y, int row, int m, int col, T v) {
-  if constexpr (FAR) stx(y, row, m, col, v);
-  else stg(y, row * m + col, v);
-}
-
 // acc += A B (tiles i, j of A's and B's rows; LOWER: j <= i only).
 template <typename T, int K4, bool EX, bool RA, bool RB, bool LOWER, int NT>
 __device__ __forceinline__ void mma_frags(typename Mfma<T>::acc_t (&acc)[NT], const Frag<T, K4, EX, RA>& A,
@@ -180,8 +168,8 @@ struct Pull {
     if (Lcc != nullptr) fc.load(Lcc, n);
     if (yj != nullptr) {
       ld_rhs_acc<T, NB>(y, yj, n, m, 0);
-      if (Ra != nullptr) ld_rhs<T, K4>(va, ya, n, m, 0);
-      if (Lcc != nullptr) ld_rhs<T, K4>(vc, yc, n, m, 0);
+      if (Ra != nullptr) ld_rhs_b<T, K4>(va, ya, n, m, 0);
+      if (Lcc != nullptr) ld_rhs_b<T, K4>(vc, yc, n, m, 0);
     }
 #pragma unroll
     for (int i = 0; i < NB; ++i)
@@ -232,8 +220,8 @@ struct Pull {
                                            int c0) {
     T va[K4], vc[K4];
     ld_rhs_acc<T, NB>(y, yj, n, m, c0);
-    if (ra) ld_rhs<T, K4>(va, ya, n, m, c0);
-    if (lc) ld_rhs<T, K4>(vc, yc, n, m, c0);
+    if (ra) ld_rhs_b<T, K4>(va, ya, n, m, c0);
+    if (lc) ld_rhs_b<T, K4>(vc, yc, n, m, c0);
     sub_rhs(ra, lc, va, vc);
   }
 };
@@ -549,7 +537,7 @@ __device__ __forceinline__ void forward_task(const SmallSys<T>& Q, int l, int ta
   constexpr int KU = sizeof(T) == 8 ? K4 : 4 * NB;
   const int N = Q.N, n = EX ? 4 * K4 : Q.n, m = Q.m;
   const int nn = n * n;
-  const size_t nm = (size_t)n * m;
+  const std::conditional_t<FAR, size_t, int> nm = (decltype(nm))n * m;
   const int s = 1 << l, h = s >> 1, dim = (N + s) / (2 * s);
   const bool node = task < dim;
   app = app && node;
@@ -559,7 +547,7 @@ __device__ __forceinline__ void forward_task(const SmallSys<T>& Q, int l, int ta
   const T* Ra = upd ? Q.E + (size_t)(offp + ((k - h) >> (l - 1))) * nn : nullptr;          // (k, k-h)
   const T* Lcc = upd && k + h < N ? Q.E + (size_t)(offp + (k >> (l - 1))) * nn : nullptr;  // (k+h, k)
   const T* Lk = Q.L + (size_t)k * nn;
-  T* yk = Q.x + k * nm;
+  T* yk = Q.x + (size_t)k * nm;
   const int lane = lane_id(), i = lane & 15;
   Frag<T, K4, EX, true> fr;
   Frag<T, K4, EX, false> fc;
@@ -567,11 +555,11 @@ __device__ __forceinline__ void forward_task(const SmallSys<T>& Q, int l, int ta
   typename Mfma<T>::acc_t a[NB];
   if (upd) {
     fr.load(Ra, n);
-    ld_rhs<T, K4, FAR>(y, yk - h * nm, n, m, c0);
+    ld_rhs_b<T, K4, FAR>(y, yk - (size_t)h * nm, n, m, c0);
   }
   if (Lcc != nullptr) {
     fc.load(Lcc, n);
-    ld_rhs<T, K4, FAR>(y2, yk + h * nm, n, m, c0);
+    ld_rhs_b<T, K4, FAR>(y2, yk + (size_t)h * nm, n, m, c0);
   }
   ld_rhs_acc<T, NB, FAR>(a, yk, n, m, c0);
   // L_k^-1, rows 16b + i, from the tiles on and above the stored diagonal
@@ -603,8 +591,8 @@ __device__ __forceinline__ void forward_task(const SmallSys<T>& Q, int l, int ta
   if (Lcc != nullptr) fc.mask_k(n);
   for (const int first = c0; c0 < c1; c0 += 16) {
     if (c0 > first) {
-      if (upd) ld_rhs<T, K4, FAR>(y, yk - h * nm, n, m, c0);
-      if (Lcc != nullptr) ld_rhs<T, K4, FAR>(y2, yk + h * nm, n, m, c0);
+      if (upd) ld_rhs_b<T, K4, FAR>(y, yk - (size_t)h * nm, n, m, c0);
+      if (Lcc != nullptr) ld_rhs_b<T, K4, FAR>(y2, yk + (size_t)h * nm, n, m, c0);
       ld_rhs_acc<T, NB, FAR>(a, yk, n, m, c0);
     }
     typename Mfma<T>::acc_t u[NB];
@@ -637,7 +625,7 @@ __device__ __forceinline__ void forward_task(const SmallSys<T>& Q, int l, int ta
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int row = 16 * b + Mfma<T>::row(lane, e);
-          if (row < n) st_rhs<T, FAR>(yk, row, m, c0 + i, a[b][e]);
+          if (row < n) st_rhs<FAR>(yk, row, m, c0 + i, a[b][e]);
         }
   }
 }
@@ -655,14 +643,14 @@ __device__ __forceinline__ void down_task(const SmallSys<T>& Q, int l, int t0, i
   constexpr int KU = sizeof(T) == 8 ? K4 : 4 * NB;
   const int N = Q.N, n = EX ? 4 * K4 : Q.n, m = Q.m;
   const int nn = n * n;
-  const size_t nm = (size_t)n * m;
+  const std::conditional_t<FAR, size_t, int> nm = (decltype(nm))n * m;
   const int s = 1 << l, k = s - 1 + 2 * s * t0;
   const int off = seg_offset(N, l);
   const bool hasR = k + s < N, hasC = k >= s;
   const T* Rk = Q.E + (size_t)(off + (k >> l)) * nn;
   const T* Lck = Q.E + (size_t)(off + ((k - s) >> l)) * nn;
   const T* Lk = Q.L + (size_t)k * nn;
-  T* xk = Q.x + k * nm;
+  T* xk = Q.x + (size_t)k * nm;
   const int lane = lane_id(), i = lane & 15;
   Frag<T, K4, EX, false> fr;
   Frag<T, K4, EX, true> fc;
@@ -670,11 +658,11 @@ __device__ __forceinline__ void down_task(const SmallSys<T>& Q, int l, int t0, i
   typename Mfma<T>::acc_t a[NB];
   if (hasR) {
     fr.load(Rk, n);
-    ld_rhs<T, K4, FAR>(y, xk + s * nm, n, m, c0);
+    ld_rhs_b<T, K4, FAR>(y, xk + (size_t)s * nm, n, m, c0);
   }
   if (hasC) {
     fc.load(Lck, n);
-    ld_rhs<T, K4, FAR>(y2, xk - s * nm, n, m, c0);
+    ld_rhs_b<T, K4, FAR>(y2, xk - (size_t)s * nm, n, m, c0);
   }
   ld_rhs_acc<T, NB, FAR>(a, xk, n, m, c0);
   // U[16b + i][kr]: rows of the stored block above its diagonal (tiles on and
@@ -707,8 +695,8 @@ __device__ __forceinline__ void down_task(const SmallSys<T>& Q, int l, int t0, i
   if (hasC) fc.mask_k(n);
   for (const int first = c0; c0 < c1; c0 += 16) {
     if (c0 > first) {
-      if (hasR) ld_rhs<T, K4, FAR>(y, xk + s * nm, n, m, c0);
-      if (hasC) ld_rhs<T, K4, FAR>(y2, xk - s * nm, n, m, c0);
+      if (hasR) ld_rhs_b<T, K4, FAR>(y, xk + (size_t)s * nm, n, m, c0);
+      if (hasC) ld_rhs_b<T, K4, FAR>(y2, xk - (size_t)s * nm, n, m, c0);
       ld_rhs_acc<T, NB, FAR>(a, xk, n, m, c0);
     }
     typename Mfma<T>::acc_t u[NB], o[NB];
@@ -734,7 +722,7 @@ __device__ __forceinline__ void down_task(const SmallSys<T>& Q, int l, int t0, i
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int row = 16 * b + Mfma<T>::row(lane, e);
-          if (row < n) st_rhs<T, FAR>(xk, row, m, c0 + i, o[b][e]);
+          if (row < n) st_rhs<FAR>(xk, row, m, c0 + i, o[b][e]);
         }
   }
 }
@@ -836,12 +824,8 @@ void launch_up(int cls, dim3 grid, const SmallArgs<T>& A, int l, hipStream_t st)
 // of their own (every n by its padded form): in the common one they cost 1.5% (256
 // systems of n=20 N=61 m=1, FP32 factor_and_solve, 157.8 / 160.2 us).
 template <typename T>
-bool far_rhs(const SmallArgs<T>& A) {
-  return (size_t)A.n * A.m * sizeof(T) > 0xffffffffu;
-}
-template <typename T>
 void launch_down(int cls, dim3 grid, const SmallArgs<T>& A, int l, hipStream_t st) {
-  if (far_rhs(A))
+  if (far_rhs<T>(A.n, A.m))
     return with_class(cls & ~1, [&](auto k4, auto) {
       hipLaunchKernelGGL((k_small_down<T, decltype(k4)::value, false, true>), grid, dim3(64), 0, st, A, l);
     });
@@ -851,7 +835,7 @@ void launch_down(int cls, dim3 grid, const SmallArgs<T>& A, int l, hipStream_t s
 }
 template <typename T>
 void launch_forward(int cls, dim3 grid, const SmallArgs<T>& A, int l, bool upd, bool app, hipStream_t st) {
-  if (far_rhs(A))
+  if (far_rhs<T>(A.n, A.m))
     return with_class(cls & ~1, [&](auto k4, auto) {
       hipLaunchKernelGGL((k_small_forward<T, decltype(k4)::value, false, true>), grid, dim3(64), 0, st, A, l, (int)upd,
                          (int)app);

@@ -40,7 +40,9 @@ enum StepMode { kStepFull = 0, kStepUpdate = 1, kStepApply = 2 };
 // forward step and 20 us a backward level there.  FP64 solve n=100 N=200 m=8
 // 518 -> 232 us, factor_and_solve n=64 N=1024 m=16 472 -> 442 us, n=128 N=512
 // 975 -> 959 us, FP32 n=36 N=100 B=8 197 -> 171 us.
-template <typename T, int RT, bool FWD>
+// FAR: 64-bit offsets, for block rows of right-hand sides above 4 GiB (0.3% of a
+// factor_and_solve of n=64 N=1024 m=16).
+template <typename T, int RT, bool FWD, bool FAR>
 __global__ __launch_bounds__(64 * RT) void k_step(const T* __restrict__ L, const T* __restrict__ E,
                                                   T* __restrict__ x, const uint8_t* __restrict__ mask, int N, int n,
                                                   int m, int nE, int s, int off, int mode) {
@@ -74,11 +76,11 @@ __global__ __launch_bounds__(64 * RT) void k_step(const T* __restrict__ L, const
   T sp[4], sm[4], xd[4], a1[Q][2], a2[Q][2], a3[Q][2];
   if (hasT) {
 #pragma unroll
-    for (int p = 0; p < 4; ++p) sp[p] = ldx(xi + s * nm, min(k0 + 4 * RT * p, n - 1), m, cl);
+    for (int p = 0; p < 4; ++p) sp[p] = ld_rhs<FAR>(xi + s * nm, min(k0 + 4 * RT * p, n - 1), m, cl);
   }
   if (hasS) {
 #pragma unroll
-    for (int p = 0; p < 4; ++p) sm[p] = ldx(xi - s * nm, min(k0 + 4 * RT * p, n - 1), m, cl);
+    for (int p = 0; p < 4; ++p) sm[p] = ld_rhs<FAR>(xi - s * nm, min(k0 + 4 * RT * p, n - 1), m, cl);
   }
   auto rows = [&](T(&v)[2], const T* M, int q) {  // v[e] = M[ii][8 q + 2 g + e]
     const int o = ic * n + 8 * q + 2 * g, oc = q < QT ? o : min(o, nn - 2);
@@ -102,7 +104,7 @@ __global__ __launch_bounds__(64 * RT) void k_step(const T* __restrict__ L, const
     for (int q = 0; q < Q; ++q) rows(a2[q], MS, q);
   }
 #pragma unroll
-  for (int e = 0; e < 4; ++e) xd[e] = ldx(xi, min(16 * t + Mfma<T>::row(lane, e), n - 1), m, cl);
+  for (int e = 0; e < 4; ++e) xd[e] = ld_rhs<FAR>(xi, min(16 * t + Mfma<T>::row(lane, e), n - 1), m, cl);
   T diag = T(1);
   if (inv) {
     diag = ldg(U, ic * (n + 1));
@@ -147,7 +149,7 @@ __global__ __launch_bounds__(64 * RT) void k_step(const T* __restrict__ L, const
     const int row = 16 * t + Mfma<T>::row(lane, e);
     const T v = row < n ? xd[e] - (acc[e] + acc2[e]) : T(0);
     if (inv) Tt[row * 16 + li] = v;
-    else if (row < n && li < m - c0) stx(xi, row, m, li, v);
+    else if (row < n && li < m - c0) st_rhs<FAR>(xi, row, m, li, v);
   }
   if (!inv) return;
   __syncthreads();
@@ -171,7 +173,7 @@ __global__ __launch_bounds__(64 * RT) void k_step(const T* __restrict__ L, const
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const int row = 16 * t + Mfma<T>::row(lane, e);
-    if (row < n && li < m - c0) stx(xi, row, m, li, acc[e]);
+    if (row < n && li < m - c0) st_rhs<FAR>(xi, row, m, li, acc[e]);
   }
 }
 
@@ -184,8 +186,8 @@ hipError_t launch_step(const T* L, const T* E, T* x, const uint8_t* mask, int B,
   const int nE = (int)off_diag_storage_len(N);
   auto go = [&](auto rt) {
     constexpr int RT = decltype(rt)::value;
-    hipLaunchKernelGGL((k_step<T, RT, FWD>), dim3(blocks, mch, B), dim3(64 * RT), 0, st, L, E, x, mask, N, n, m, nE,
-                       s, off, mode);
+    auto k = far_rhs<T>(n, m) ? k_step<T, RT, FWD, true> : k_step<T, RT, FWD, false>;
+    hipLaunchKernelGGL(k, dim3(blocks, mch, B), dim3(64 * RT), 0, st, L, E, x, mask, N, n, m, nE, s, off, mode);
   };
   switch ((n + 15) / 16) {
     case 3: go(std::integral_constant<int, 3>{}); break;
