@@ -874,8 +874,8 @@ void batched_release(socu_batched* h) {
 }
 
 // Groups the systems by bucket (each by decreasing cost: long systems start
-// first) and uploads the order.
-int batched_layout(socu_batched* h) {
+// first).
+void batched_layout(socu_batched* h) {
   h->order.clear();
   for (int b = kClasses - 1; b >= 0; --b) {
     std::vector<int> o;
@@ -894,9 +894,6 @@ int batched_layout(socu_batched* h) {
   }
   for (int b = 0; b < kClasses; ++b) h->launch_order[b] = b;
   std::sort(h->launch_order, h->launch_order + kClasses, [&](int x, int y) { return h->bcost[x] > h->bcost[y]; });
-  const hipError_t e = hipMemcpy(h->dorder, h->order.data(), h->order.size() * sizeof(int), hipMemcpyHostToDevice);
-  if (e != hipSuccess) return hip_fail(e, "batched plan set-up (order)");
-  return SOCU_OK;
 }
 
 // How a batch runs.
@@ -1119,17 +1116,12 @@ int socu_batched_create(socu_batched** out, int op, const socu_batch_system* sys
     return rc;
   }
   hipError_t e = hipMalloc(&h->dprobs, count * sizeof(socu::BatchProblem));
-  if (e == hipSuccess) e = hipMalloc(&h->dorder, count * sizeof(int));
   if (e == hipSuccess) e = hipMemcpy(h->dprobs, probs.data(), count * sizeof(socu::BatchProblem), hipMemcpyHostToDevice);
   if (e != hipSuccess) {
     batched_release(h);
     return hip_fail(e, "batched plan set-up");
   }
-  rc = batched_layout(h);
-  if (rc) {
-    batched_release(h);
-    return rc;
-  }
+  batched_layout(h);
   // `tune` is accepted and does not change the plan: there is nothing to choose by
   // timing.  For an untuned plan SOCU_BATCHED_WAVES overrides the choice: 1, 2 or 4
   // wavefronts per workgroup and system, or 0 for level launches.
@@ -1145,6 +1137,8 @@ int socu_batched_create(socu_batched** out, int op, const socu_batch_system* sys
   if (choice.levels) {
     e = socu::small_batch_create(&h->levels, probs.data(), count, op, streams);
   } else {
+    e = hipMalloc(&h->dorder, count * sizeof(int));
+    if (e == hipSuccess) e = hipMemcpy(h->dorder, h->order.data(), count * sizeof(int), hipMemcpyHostToDevice);
     streams = 0;
     for (int b = 0; b < kClasses; ++b) {
       int v = choice.waves[b];  // fewer where the LDS does not fit the right-hand sides
