@@ -59,7 +59,9 @@ def build_library(verbose: bool = False, jobs: int = 0) -> str:
         for f in [ex.submit(_run, c, w) for c, w in cmds]:
             f.result()
     tmp = OUT + ".tmp"
-    link = [hipcc(), "--offload-arch=gfx950", "-fPIC", "-shared", "-o", tmp, *objs]
+    # -Bsymbolic: the package opens the library with global scope, and a second build
+    # of it in one process must call its own functions, not those of the first.
+    link = [hipcc(), "--offload-arch=gfx950", "-fPIC", "-shared", "-Wl,-Bsymbolic", "-o", tmp, *objs]
     if verbose:
         print(" ".join(link), flush=True)
     _run(link, f"linking {OUT}")
