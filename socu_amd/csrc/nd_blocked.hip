@@ -11,6 +11,9 @@
 // (The sweeps: nd_small.hip, nd_steps.hip, nd_large.hip.)
 #include <stdlib.h>
 
+#include <algorithm>
+#include <type_traits>
+
 #include <hip/hip_ext.h>
 
 #include "nd_common.h"
@@ -203,9 +206,10 @@ __global__ __launch_bounds__(kThreads) void k_schur_blk(T* __restrict__ L, T* __
 }
 
 // ---------------------------------------------------------------------------
-// BF16 Schur products for levels with few nodes.  k_schur_blk walks K in chunks, one global round trip per chunk, which at the upper levels (a
-// handful of tiles) is the whole cost.  Here a task is a 32x32 output tile
-// (4x more tasks) and issues every load it needs at once: the 32-wide panels
+// BF16 Schur products for levels with few nodes, and those of FP32 blocks of
+// 16 < n <= 32.  k_schur_blk walks K in chunks, one global round trip per chunk,
+// which at the upper levels (a handful of tiles) is the whole cost.  Here a task is
+// a 32x32 output tile (4x more tasks) and issues every load it needs at once: the 32-wide panels
 // of its operands (all of K) and its own C values, then one LDS staging and
 // the MFMA products.  Panels are kept as P[i][k] (pitch NP + 1): row panels
 // are 32 rows of a block, column panels 32 of its columns, transposed.
@@ -258,7 +262,8 @@ __device__ __forceinline__ void panel_store(T* P, const T* v, bool cols, int i0,
 template <typename T, int NB, int NF, bool BF = false>
 __global__ __launch_bounds__(kThreads) void k_schur_small(T* __restrict__ L, T* __restrict__ E,
                                                          const uint8_t* __restrict__ mask, int N, int n_, int nE, int s,
-                                                         int off, int next_off, int nT, const T* __restrict__ Lsrc) {
+                                                         int off, int next_off, int nT, int first,
+                                                         const T* __restrict__ Lsrc) {
   const int n = NF ? NF : n_;
   constexpr int NP = 32 * NB, PP = NP + 1;
   constexpr int PE = 32 * NP / kThreads;
@@ -269,7 +274,7 @@ __global__ __launch_bounds__(kThreads) void k_schur_small(T* __restrict__ L, T* 
   T* Pn = reinterpret_cast<T*>(smem_raw);  // four panels of 32 x PP
   const size_t nn = (size_t)n * n;
   T* Eb = E + (size_t)b * nE * nn;
-  int task = blockIdx.x;
+  int task = first + blockIdx.x;
   const T* M[4];
   bool cols[4];
   int i0[4];
@@ -277,7 +282,8 @@ __global__ __launch_bounds__(kThreads) void k_schur_small(T* __restrict__ L, T* 
   T* C;
   int tr, tc;
   bool diag;
-  if (task < nT * NTRI) {
+  const bool target = task < nT * NTRI;
+  if (target) {
     // L_j -= R R^T + Lc^T Lc  (R = block (j, j-s), Lc = block (j+s, j))
     const int u = task / NTRI;
     int q = task - u * NTRI;
@@ -323,7 +329,7 @@ __global__ __launch_bounds__(kThreads) void k_schur_small(T* __restrict__ L, T* 
   // C values: the target's (the fill-in block receives its only update here,
   // F = -R Lc, so its entry contents are not read)
   T cv[4] = {T(0), T(0), T(0), T(0)};
-  if (blockIdx.x < nT * NTRI) {
+  if (target) {
     // (out-of-place: the target is read from Lsrc, same layout)
     const T* Cin = (Lsrc != nullptr) ? Lsrc + (C - L) : C;
 #pragma unroll
@@ -377,22 +383,28 @@ static bool use_schur_blk(int nodes, int n, int esize) {
   return (n + 15) / 16 % 4 == 0 && (double)nodes * n * n * esize > 16.0 * 1024 * 1024;
 }
 
-// Whether a level's BF16 Schur products take k_schur_small.  Its panel loads repeat
-// each operand per output tile, which only costs where the level streams many
-// blocks; it wins up to about 12 MiB of the level's blocks (N=512, 1024), and for
-// n <= 32 at every level: k_schur_blk's 64x64 output tiles leave three of four
-// quarters outside a 32x32 block.
-// SOCU_SCHUR_SMALL=<nodes> replaces the rule by a node count (0 disables the
-// small kernel).
-static bool use_schur_small(int nodes, int n, int esize) {
+// Whether a level's FP32 or BF16 Schur products take k_schur_small.
+// FP32: blocks of one 32x32 tile that are not one 16x16 tile.  k_schur_tile reads
+// each operand twice per output row of tiles and a wavefront has a quarter or a half
+// of a short sum.  FP32 factor with FP64 pivots, n = 32, 8, 100, 16 x 64, 256 x 61 and
+// 1024 x 64 blocks: 46, 81, 106, 430, 1610 us to 44, 78, 92, 287, 972; n = 17: 45, 80, 95,
+// 356, 1279 to 45, 80, 88, 266, 868; n = 16, where three of four quarters of the tile are
+// padding, 37, 64, 68, 154, 459 to 38, 65, 70, 164, 495.
+// BF16: its panel loads repeat each operand per output tile, which only costs where
+// the level streams many blocks; it wins up to about 12 MiB of the level's blocks
+// (N=512, 1024), and for n <= 32 at every level: k_schur_blk's 64x64 output tiles
+// leave three of four quarters outside a 32x32 block.  SOCU_SCHUR_SMALL=<nodes>
+// replaces this rule by a node count (0 disables the small kernel).
+static bool use_schur_small(int nodes, int n, bool bf16) {
   static int env = -2;
   if (env == -2) {
     const char* e = getenv("SOCU_SCHUR_SMALL");
     env = e ? (atoi(e) < 0 ? 0 : atoi(e)) : -1;
   }
+  if (!bf16) return n > 16 && n <= 32;
   if (env >= 0) return nodes <= env;
   if (n <= 32) return true;
-  return (double)nodes * n * n * esize <= 12.0 * 1024 * 1024;
+  return (double)nodes * n * n * sizeof(float) <= 12.0 * 1024 * 1024;
 }
 
 hipError_t init_blocked_kernels() {
@@ -441,7 +453,23 @@ static hipError_t factor_level_nb(T* L, T* E, const uint8_t* mask, int B, int N,
     kt_begin(kKcSchur, st);
     const int nodes = B * (nT + nF);
     const dim3 grid_blk(8 * schur_blk_per_xcd(nT, nF, ntile), B);
-    if (!bf16) {
+    // (pieces: as in schur_tiles)
+    auto small = [&](auto bf) {
+      const int count = nT * (NB * (NB + 1) / 2) + nF * NB * NB;
+      for (int first = 0; first < count; first += kMaxGridTasks)
+        hipLaunchKernelGGL((k_schur_small<T, NB, NF, decltype(bf)::value>), dim3(std::min(count - first, kMaxGridTasks), B),
+                           dim3(kThreads), (schur_small_lds<T, NB>()), st, L, E, mask, N, n, nE, lv.s, lv.off, lv.next_off,
+                           nT, first, Lsrc);
+    };
+    bool done = false;
+    if constexpr (sizeof(T) == 4) {
+      if (use_schur_small(nodes, n, bf16)) {
+        if (bf16) small(std::true_type{});
+        else if constexpr (NB == 1) small(std::false_type{});
+        done = true;
+      }
+    }
+    if (!bf16 && !done) {
       bool blk = false;
       if constexpr (NB % 2 == 0) blk = use_schur_blk(nodes, n, (int)sizeof(T));
       if (!blk) {
@@ -453,14 +481,9 @@ static hipError_t factor_level_nb(T* L, T* E, const uint8_t* mask, int B, int N,
       }
     }
     if constexpr (sizeof(T) == 4) {
-      if (bf16 && use_schur_small(nodes, n, (int)sizeof(T))) {
-        const int nsmall = nT * (NB * (NB + 1) / 2) + nF * NB * NB;
-        hipLaunchKernelGGL((k_schur_small<T, NB, NF, true>), dim3(nsmall, B), dim3(kThreads),
-                           (schur_small_lds<T, NB>()), st, L, E, mask, N, n, nE, lv.s, lv.off, lv.next_off, nT, Lsrc);
-      } else if (bf16) {
+      if (bf16 && !done)
         hipLaunchKernelGGL((k_schur_blk<T, NF, true>), grid_blk, dim3(kThreads), 0, st, L, E, mask, N, n, nE, lv.s,
                            lv.off, lv.next_off, nT, nF, ntile, Lsrc);
-      }
     }
     kt_end(kKcSchur, st);
   }

@@ -4,13 +4,14 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-def test_fp64_pivots_of_a_long_system(device):
-    """n = 17 with 4.9 million blocks: level 0 has 17 million 16x16 Schur tiles,
-    2^32 threads and more.  Checked by the residual of a solve."""
+@pytest.mark.parametrize("n,N", [(17, 4_900_000), (8, 17_000_000)])
+def test_fp64_pivots_of_a_long_system(n, N, device):
+    """n = 17 with 4.9 million blocks: 17 million 16x16 tiles of a level's Schur updates
+    would be 2^32 threads and more (it takes 32x32 ones); n = 8 with 17 million blocks:
+    so many 16x16 tiles.  Checked by the residual of a solve."""
     import torch
     from socu_amd import _lib
 
-    n, N = 17, 4_900_000
     print(f"long system n={n} N={N}", flush=True)
     gen = torch.Generator(device=device).manual_seed(1)
     # diagonally dominant: couplings of norm <= 2, diagonal blocks 8 I + (norm <= 1)
@@ -37,6 +38,33 @@ def test_fp64_pivots_of_a_long_system(device):
         r[:hi - i] += (C[i:hi] * x[i + 1:hi + 1, :, None]).sum(1)
         # kappa <= 3: a few units of 2^-24 of the terms' size
         assert float(r.abs().max()) < 1e-5 * float(b.abs().max()), i
+
+
+def test_bf16_schur_of_a_long_system(device):
+    """n = 1 with 2^24 blocks and more: as many tasks of 256 threads.  Checked by the
+    residual of a solve."""
+    import torch
+    from socu_amd import _lib
+
+    N = 2**24 + 5
+    print(f"long system bf16 n=1 N={N}", flush=True)
+    gen = torch.Generator(device=device).manual_seed(3)
+    D = 8 + torch.rand(N, generator=gen, device=device)
+    C = 2 * torch.rand(N - 1, generator=gen, device=device) - 1
+    b = torch.randn(N, generator=gen, device=device)
+    nE = sum((N >> l) - 1 for l in range(N.bit_length()))
+    L, E, x = D.clone(), torch.empty(nE, device=device), b.clone()
+    E[: N - 1] = C
+    lib, st = _lib.load(), torch.cuda.current_stream().cuda_stream
+    assert lib.socu_cholesky_factor_f32(L.data_ptr(), E.data_ptr(), None, 1, N, 1, _lib.PREC_BF16, st) == 0
+    assert lib.socu_cholesky_solve_with_inverses(L.data_ptr(), E.data_ptr(), x.data_ptr(), None, 1, N, 1, 1,
+                                                 _lib.DTYPE_F32, st) == 0
+    r = D * x - b
+    r[1:] += C * x[:-1]
+    r[:-1] += C * x[1:]
+    # products of two numbers rounded to 2^-9: of |C|^2 / D <= 1/6, two into a diagonal
+    # block and one into a fill-in, 2e-3 and 7e-4 over the levels; |x| <= max |b| / 6
+    assert float(r.abs().max()) < 1e-3 * float(b.abs().max())
 
 
 def test_batch_of_many_block_rows(device):

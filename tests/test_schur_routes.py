@@ -1,7 +1,7 @@
 """Schur updates of levels that stream more than 16 MiB: 64x64 tiles, for block sizes
 whose 16-row tiles fill them (n = 49 .. 64 and 113 .. 128, ragged ones among them); and
-the same batch one system short of it, by 16x16 tiles.  In place, out of place and with
-a masked system, against the oracle.
+the same batch one system short of it, by 16x16 tiles.  FP32 blocks about 16 < n <= 32
+take 32x32 tiles.  In place, out of place and with a masked system, against the oracle.
 """
 import numpy as np
 import pytest
@@ -82,3 +82,25 @@ def test_fp64_pivots(n, short, device):
                                               torch.cuda.current_stream().cuda_stream)
     assert rc == 0
     _check(L, E, want, B, 5e-4)
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 24, 31, 32, 33])
+@pytest.mark.parametrize("N", [2, 3, 13])
+def test_fp64_pivots_small_blocks(n, N, device):
+    import torch
+    from socu_amd import _lib
+
+    print(f"schur pivots n={n} N={N}", flush=True)
+    P = [nd.readme_problem(n, N, 1, alpha=16.0, seed=n + k)[:2] for k in range(3)]
+    Ls, Es = (torch.tensor(np.stack([p[i] for p in P]), dtype=torch.float32, device=device) for i in range(2))
+    L, E = Ls.clone(), Es.clone()
+    mask = torch.tensor([True, False, True], device=device)
+    rc = _lib.load().socu_cholesky_factor_f32(L.data_ptr(), E.data_ptr(), mask.data_ptr(), 3, N, n, _lib.PREC_FP32,
+                                              torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    assert torch.equal(L[1], Ls[1]) and torch.equal(E[1], Es[1])
+    for b in (0, 2):
+        Lr, Er = P[b][0].copy(), P[b][1].copy()
+        nd.factor(Lr, Er)
+        assert _rel(np.tril(L[b].double().cpu().numpy()), np.tril(Lr)) < 5e-4, b
+        assert _rel(E[b].double().cpu().numpy(), Er) < 5e-4, b
