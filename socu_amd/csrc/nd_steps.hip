@@ -40,8 +40,11 @@ enum StepMode { kStepFull = 0, kStepUpdate = 1, kStepApply = 2 };
 // forward step and 20 us a backward level there.  FP64 solve n=100 N=200 m=8
 // 518 -> 232 us, factor_and_solve n=64 N=1024 m=16 472 -> 442 us, n=128 N=512
 // 975 -> 959 us, FP32 n=36 N=100 B=8 197 -> 171 us.
-// FAR: 64-bit offsets, for block rows of right-hand sides above 4 GiB (0.3% of a
-// factor_and_solve of n=64 N=1024 m=16).
+// FAR: 64-bit offsets, for block rows of right-hand sides above 4 GiB.  A variant of
+// its own, so that the common one has no instruction for it; that they would cost
+// time there was not shown (factor_and_solve n=64 N=1024 m=16: without FAR 441.8 us,
+// 64-bit offsets for all 443.2, this variant, whose instructions are those of the
+// first, 443.3).
 template <typename T, int RT, bool FWD, bool FAR>
 __global__ __launch_bounds__(64 * RT) void k_step(const T* __restrict__ L, const T* __restrict__ E,
                                                   T* __restrict__ x, const uint8_t* __restrict__ mask, int N, int n,
