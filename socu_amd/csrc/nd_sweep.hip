@@ -596,17 +596,18 @@ size_t sweep_slot_elems(int B, int N, int n) {
   return (size_t)B * (size_t)(k > 0 ? k : 1) * n;
 }
 
-// Lowest level swept by the persistent launch: levels pay there while the
-// widest of them has at most W nodes over the batch, with W = 64 for n <= 64,
-// 256 for FP32 and 1024 for FP64 blocks above that.  The lines were drawn between
-// these sweeps and former, slower level kernels (N=512, B = 1 and 4, n = 32, 64, 96,
-// 128: the fastest split or within 4% of it); with today's the sweeps as a whole are
-// still the faster way wherever they are taken (sweep_persistent_enabled), the split
-// itself has not been timed again.  Below lmin the level kernels stream the wide
-// levels.
+// Lowest level swept by the persistent launch: levels pay there while the widest of
+// them has at most W nodes over the batch; the level kernels stream the wider ones
+// below.  Every split timed (solves in a graph, n = 34, 64, 100, 128, N = 64 .. 2000,
+// 1 to 64 systems, both precisions): W = 64 for n <= 64 is within 4% of the best one,
+// 320 for larger blocks within 5%.  FP64 blocks of 64 < n <= 96 do better with 1024:
+// n=80, 700 and 800 nodes at level 0, 234 and 189 us, with 320 256 and 217.  For n > 96
+// 1024 took longer, a compute unit holding one FP64 task: n=100 N=512 B=4 655 us, with
+// 320 589; n=128 N=2000 B=1 798 / 731; and for FP32 256 was too few: n=100 N=200 B=3
+// 154 / 149, the mixed solver there 807 / 754.
 int sweep_lmin(int B, int N, int n, int dsize) {
   const int Lv = recursive_iterations(N);
-  const long long W = n <= 64 ? 64 : (dsize == 8 ? 1024 : 256);
+  const long long W = n <= 64 ? 64 : (dsize == 8 && n <= 96 ? 1024 : 320);
   int lmin = 0;
   while (lmin < Lv - 1 && (long long)B * ((N + (1 << lmin)) >> (lmin + 1)) > W) ++lmin;
   return lmin;

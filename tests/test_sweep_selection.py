@@ -68,3 +68,34 @@ def test_asked_for_by_small_factor_and_solve(n, N, B, dtype, graph, device, monk
             tol = 1e-11 if dtype == "float64" else 5e-4
             assert np.linalg.norm(x[k].double().cpu().numpy() - xr) < tol * np.linalg.norm(xr)
             assert np.linalg.norm(np.tril(L[k].double().cpu().numpy()) - np.tril(Lr)) < tol * np.linalg.norm(Lr)
+
+
+@pytest.mark.parametrize("n,dtype,W", [(65, "float64", 1024), (96, "float64", 1024), (97, "float64", 320),
+                                       (128, "float64", 320), (65, "float32", 320), (128, "float32", 320),
+                                       (33, "float64", 64), (64, "float32", 64)])
+@pytest.mark.parametrize("over", [0, 1])
+def test_solve_on_both_sides_of_the_split(n, dtype, W, over, device, monkeypatch):
+    """W nodes at level 0 sweep persistently, W + 1 by the level kernels and the upper
+    level persistently: against the oracle (three systems, repeated over the batch)."""
+    import numpy as np
+    import torch
+    from oracle import nd
+    from socu_amd.block_tridiag_solver import create_cholesky_factor_launch, create_cholesky_solve_launch
+
+    monkeypatch.delenv("SOCU_SWEEP", raising=False)
+    tdt, B = getattr(torch, dtype), W + over  # N = 2: one node a system at level 0
+    P = [nd.readme_problem(n, 2, 1, alpha=16.0, seed=60 + k)[:3] for k in range(3)]
+    pick = torch.arange(B) % 3
+    L, E, x = (torch.tensor(np.stack([p[i] for p in P]), dtype=tdt)[pick].to(device) for i in range(3))
+    create_cholesky_factor_launch(L, E, dtype=tdt)()
+    run = create_cholesky_solve_launch(L, E, x, dtype=tdt)
+    run()
+    assert run.sweep_status() == (True, False)
+    # kappa(Psi) <= 1e3: 1e3 * N * 2^-53, and 2^-24
+    tol = 1e-11 if dtype == "float64" else 5e-4
+    for k in range(3):
+        Lr, Er, xr = (a.copy() for a in P[k])
+        nd.factor(Lr, Er)
+        nd.solve(Lr, Er, xr)
+        got = x[pick == k].double().cpu().numpy()
+        assert np.abs(got - xr).max() <= tol * np.abs(xr).max()
