@@ -174,9 +174,10 @@ int socu_plan_destroy(socu_plan* plan);
  * arithmetic per block as the reference's sweeps,
  * block_tridiag_solver.py:425-485 and :581-643).  Used by plans with one
  * right-hand side, in both precisions, where that measured faster than level
- * kernels: 32 < n <= 128, or n <= 32 and at most 32 systems (mixed handles: 64),
- * except by factor_and_solve plans of n <= 16 and at most 256 systems, which sweep
- * back inside the factor's kernels.  The environment variable SOCU_SWEEP read at
+ * kernels: 32 < n <= 128; n <= 32 and at most 32 systems without a graph; FP64,
+ * 24 < n <= 32 and at most 6 systems with one; mixed handles of n <= 32 and at most
+ * 64 systems; except by factor_and_solve plans of n <= 16 and at most 256 systems,
+ * which sweep back inside the factor's kernels.  (The two ways round differently.)  The environment variable SOCU_SWEEP read at
  * creation overrides: "level" (never) or "persistent" (every n <= 128).  Each wait
  * is bounded; if one expires the launch drains, the tasks that depended on
  * the wait write NaN into their part of x (so the failure shows in the

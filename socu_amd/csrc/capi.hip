@@ -296,9 +296,9 @@ void free_sweep_ws(SweepWs& sw) {
 
 // Allocates the persistent-sweep workspace of a plan whose operation
 // includes a substitution with one right-hand side.
-int alloc_sweep_ws(SweepWs& sw, int op, int B, int N, int n, int m, int dtype) {
+int alloc_sweep_ws(SweepWs& sw, int op, int B, int N, int n, int m, int dtype, bool graph) {
   const size_t esz = dtype == SOCU_DTYPE_F64 ? sizeof(double) : sizeof(float);
-  if (op == SOCU_OP_FACTOR || m != 1 || B <= 0 || !socu::sweep_persistent_enabled(B, n, false)) return SOCU_OK;
+  if (op == SOCU_OP_FACTOR || m != 1 || B <= 0 || !socu::sweep_persistent_enabled(B, n, (int)esz, graph)) return SOCU_OK;
   // (these sweep inside the factor's kernels, unless asked not to)
   if (op == SOCU_OP_FACTOR_AND_SOLVE && n <= socu::kSmallN && socu::small_tail_applies(B, n, m) &&
       !socu::sweep_persistent_asked())
@@ -581,7 +581,7 @@ int socu_plan_create(socu_plan** out, int op, void* L, void* E, void* x, const u
   }
   socu_plan* p = new socu_plan{op, L, E, x, mask, B, N, n, need_x ? m : 1, dtype, nullptr, nullptr, SweepWs(),
                                socu::SweepOverlap(), false, nullptr};
-  rc = alloc_sweep_ws(p->sweep, op, B, N, n, p->m, dtype);
+  rc = alloc_sweep_ws(p->sweep, op, B, N, n, p->m, dtype, use_graph != 0);
   if (rc == SOCU_OK && op_needs_inverse(op) && B > 0) {
     const hipError_t e = hipMalloc(&p->inv, inverse_ws_bytes(B, N, n, dtype));
     if (e != hipSuccess) {

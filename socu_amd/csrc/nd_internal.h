@@ -154,11 +154,13 @@ hipError_t sweep_persistent(const T* L, const T* E, T* x, const uint8_t* mask, i
 // already satisfied expire at once (for tests of the failure path).
 void set_sweep_spin_limit(int polls);
 int sweep_spin_limit();
-// Whether a plan for B systems of block size n (refine: the mixed solver's) uses the
+// Whether a plan for B systems of block size n, run eagerly or as a graph, uses the
 // persistent sweeps (plans with one right-hand side only); the environment
 // variable SOCU_SWEEP = "level" (never) or "persistent" (always) overrides the
 // rule.
-bool sweep_persistent_enabled(int B, int n, bool refine);
+bool sweep_persistent_enabled(int B, int n, int dsize, bool graph);
+// The same for the mixed solver.
+bool sweep_persistent_refine(int B, int n);
 // ... whether the variable asks for them.
 bool sweep_persistent_asked();
 

@@ -544,7 +544,7 @@ hipError_t mixed_alloc(MixedPlan& p) {
     if ((e = hipMalloc(&p.res_c, sizeof(double) * rows * residual_slices(p.n))) != hipSuccess) return e;
     if ((e = hipMalloc(&p.res_ticket, sizeof(int) * p.B)) != hipSuccess) return e;
   }
-  if (p.m == 1 && sweep_persistent_enabled(p.B, p.n, true)) {
+  if (p.m == 1 && sweep_persistent_refine(p.B, p.n)) {
     if ((e = hipMalloc(&p.sweep_ws, sizeof(int) * sweep_ws_ints(p.B, p.N))) != hipSuccess) return e;
     if ((e = hipMemset(p.sweep_ws, 0, sizeof(int) * sweep_ws_ints(p.B, p.N))) != hipSuccess) return e;
     if ((e = hipMalloc(&p.sweep_slots, sizeof(float) * sweep_slot_elems(p.B, p.N, p.n))) != hipSuccess) return e;

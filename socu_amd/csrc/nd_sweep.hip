@@ -566,27 +566,40 @@ hipError_t init_sweep_kernels() {
   return sweep_occupancy<double, 4>(g_sweep_occ[1][3]);
 }
 
-// One launch for the upper levels against one per level and direction.  At n > 32
-// always: solves by level kernels took 1.00 to 3.04 times as long over n = 34 .. 128,
-// N = 64 and 512, 1 to 64 systems, both precisions (FP64 N=512: n=34 B=1 129 / 203 us,
-// B=64 1672 / 1684; n=128 B=1 336 / 650, B=8 1809 / 1998).  At n <= 32 a level kernel is one wavefront per node and its launch 3-4 us,
-// and the batch decides, by how many levels the one launch takes (sweep_lmin).
-// Level kernels / persistent over 280 plans each (n = 4 .. 32, N = 8 .. 700, in a
-// graph): FP64 solves 1.10 at B=9, 1.05 at 16, 1.00 at 32, 0.97 at 64; FP32 backward
-// sweeps 1.07, 1.04, 1.00, 0.98 (the worst, n=24 N=8 B=9, 61.3 / 51.6 us; at B=32
-// between 0.85 and 1.06).  The mixed solver launches the sweeps of a converged
-// iteration too, where one launch is next to nothing: 1.16 at B=9 (up to 1.57), 1.04
-// at 32, 1.00 at 64, 0.97 at 128.
 bool sweep_persistent_asked() {
   const char* v = getenv("SOCU_SWEEP");
   return v != nullptr && strcmp(v, "persistent") == 0;
 }
-bool sweep_persistent_enabled(int B, int n, bool refine) {
-  if (n > kMaxN) return false;  // its node tasks hold whole blocks in LDS
+static int persistent_by_variable(int n) {  // 0 or 1; -1: not set
+  if (n > kMaxN) return 0;  // its node tasks hold whole blocks in LDS
   const char* v = getenv("SOCU_SWEEP");
-  if (v != nullptr && strcmp(v, "level") == 0) return false;
-  if (sweep_persistent_asked()) return true;
-  return n > kSmallN || B <= (refine ? 64 : 32);
+  if (v != nullptr && strcmp(v, "level") == 0) return 0;
+  return sweep_persistent_asked() ? 1 : -1;
+}
+// One launch for the upper levels against one per level and direction.  At n > 32
+// always: solves by level kernels took 1.00 to 3.04 times as long over n = 34 .. 128,
+// N = 64 and 512, 1 to 64 systems, both precisions (FP64 N=512: n=34 B=1 129 / 203 us,
+// B=64 1672 / 1684; n=128 B=1 336 / 650, B=8 1809 / 1998).  At n <= 32 a level kernel is
+// one wavefront per node and 3-4 us, and it is the launches that decide.
+// Eager, one call at a time, the host issues 3 us a launch: solves by level kernels
+// 1.26 times the persistent sweeps' time at B=1, 1.12 at 9, 1.03 at 32 (means over
+// n = 4 .. 32, N = 8 .. 700; n=24 N=8 B=9 61.3 / 46.5 us), 0.97 at 64.
+// In a graph level kernels win: n=12 N=20 B=1 45 / 55 us, means over N and B 0.8 at
+// n <= 16, 0.9 .. 0.97 at n = 24 and FP32 n = 32.  But for FP64 blocks above 24 (level
+// kernels 1.02 .. 1.09 at n=25 .. 32 B=1, n=32: B=2 1.07, 4 1.04, 6 1.01, 8 1.00, 12 0.97).
+bool sweep_persistent_enabled(int B, int n, int dsize, bool graph) {
+  const int asked = persistent_by_variable(n);
+  if (asked >= 0) return asked != 0;
+  if (n > kSmallN) return true;
+  return graph ? dsize == 8 && n > 24 && B <= 6 : B <= 32;
+}
+// The mixed solver launches the sweeps of a converged iteration too, where one launch
+// is next to nothing, in a graph as well: with up to 10 iterations level kernels took
+// 1.84 times as long at B=1, 1.40 at 9, 1.13 at 32, 1.04 at 64 (n = 4 .. 32, N = 8 .. 700;
+// with up to 3 1.14, 1.04, 0.99, 0.96).
+bool sweep_persistent_refine(int B, int n) {
+  const int asked = persistent_by_variable(n);
+  return asked >= 0 ? asked != 0 : n > kSmallN || B <= 64;
 }
 
 size_t sweep_ws_ints(int B, int N) { return (size_t)kSweepHeader + 3 * (size_t)B * N; }

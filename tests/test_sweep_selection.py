@@ -30,6 +30,38 @@ def test_solves_by_batch_and_block_size(n, B, want, dtype, device, monkeypatch):
         assert create(L, E, x, dtype=tdt).sweep_status() == (want, False)
 
 
+@pytest.mark.parametrize("n,B,dtype,want", [(1, 1, "float64", False), (24, 1, "float64", False),
+                                            (25, 6, "float64", True), (32, 6, "float64", True),
+                                            (32, 7, "float64", False), (25, 1, "float32", False),
+                                            (32, 1, "float32", False), (33, 65, "float32", True),
+                                            (128, 9, "float64", True), (129, 1, "float64", False)])
+def test_captured_solves_by_batch_and_block_size(n, B, dtype, want, device, monkeypatch):
+    import numpy as np
+    import torch
+    from oracle import nd
+    from socu_amd.block_tridiag_solver import create_cholesky_factor_launch, create_cholesky_solve_launch
+
+    monkeypatch.delenv("SOCU_SWEEP", raising=False)
+    tdt = getattr(torch, dtype)
+    P = [nd.readme_problem(n, 5, 1, alpha=16.0, seed=70 + k)[:3] for k in range(2)]
+    pick = torch.arange(B) % 2
+    L, E, b = (torch.tensor(np.stack([p[i] for p in P]), dtype=tdt)[pick].to(device) for i in range(3))
+    create_cholesky_factor_launch(L, E, dtype=tdt)()
+    x = b.clone()
+    run = create_cholesky_solve_launch(L, E, x, dtype=tdt, use_cuda_graph=True)
+    # kappa(Psi) <= 1e3: 1e3 * N * 2^-53, and 2^-24
+    tol = 1e-11 if dtype == "float64" else 5e-4
+    for _ in range(2):
+        x.copy_(b)
+        run()
+        assert run.sweep_status() == (want, False)
+        for k in range(min(B, 2)):
+            Lr, Er, xr = (a.copy() for a in P[k])
+            nd.factor(Lr, Er)
+            nd.solve(Lr, Er, xr)
+            assert np.abs(x[pick == k].double().cpu().numpy() - xr).max() <= tol * np.abs(xr).max()
+
+
 @pytest.mark.parametrize("n,B,want", [(4, 9, True), (16, 64, True), (16, 65, False), (32, 64, True), (33, 65, True)])
 def test_mixed_solver_by_batch_and_block_size(n, B, want, device, monkeypatch):
     import torch
