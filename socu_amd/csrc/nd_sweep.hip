@@ -579,8 +579,11 @@ static int persistent_by_variable(int n) {  // 0 or 1; -1: not set
 // One launch for the upper levels against one per level and direction.  At n > 32
 // always: solves by level kernels took 1.00 to 3.04 times as long over n = 34 .. 128,
 // N = 64 and 512, 1 to 64 systems, both precisions (FP64 N=512: n=34 B=1 129 / 203 us,
-// B=64 1672 / 1684; n=128 B=1 336 / 650, B=8 1809 / 1998).  At n <= 32 a level kernel is
-// one wavefront per node and 3-4 us, and it is the launches that decide.
+// B=64 1672 / 1684; n=128 B=1 336 / 650, B=8 1809 / 1998).  (Not over all sizes: captured
+// solves of many systems are up to 1.18 times slower for it where the horizons are
+// short, n=33 N=8 B=64 FP32 66 / 57 us, 1.05 times faster in the mean over n = 33 .. 128,
+// N = 8 .. 512, 1 to 300 systems.)  At n <= 32 a level kernel is one wavefront per node and
+// 3-4 us, and it is the launches that decide.
 // Eager, one call at a time, the host issues 3 us a launch: solves by level kernels
 // 1.26 times the persistent sweeps' time at B=1, 1.12 at 9, 1.03 at 32 (means over
 // n = 4 .. 32, N = 8 .. 700; n=24 N=8 B=9 61.3 / 46.5 us), 0.97 at 64.
